@@ -152,6 +152,22 @@ int tmx_small_linear(void* stream, const void* x, const void* norm_w, float eps,
                      const void* residual, void* y, int M, int K, int N, int G, int r, int r_pad,
                      float lora_scale, int swiglu);
 
+/* LoRA weight sync (tunix/generate/sampler.py:361-392): writes n adapter tensors, row-major on the device, into the
+ * operands the projections read, rounded to bf16 (nearest even); 64 tensors per launch.  `descs_host` is a HOST array,
+ * read during the call only.
+ *   is_a != 0: src [rows = K, cols = r] -> columns col0 .. col0 + r - 1 of lora_a_t (K % 64 == 0, ld = r_pad)
+ *   is_a == 0: src [rows = r, cols = n] -> columns col0 .. col0 + n - 1 of lora_b [r, ld]
+ * rows * cols < 2^30. */
+#define TMX_DTYPE_F32 0
+#define TMX_DTYPE_BF16 1
+#define TMX_DTYPE_F16 2
+typedef struct {
+  const void* src;
+  void* dst;
+  int rows, cols, col0, ld, is_a, dtype;
+} tmx_lora_pack_desc;
+int tmx_lora_pack(void* stream, const tmx_lora_pack_desc* descs_host, int n);
+
 /* ---- row-wise kernels between the matrix products ------------------------- */
 
 /* y[M, D] = RMSNorm(x) * w.  TMX_FAMILY_LLAMA3: bf16(bf16(w * x) / rms)

@@ -996,3 +996,35 @@ def test_small_linear_rejects_what_it_cannot_take():
   assert lib.tmx_small_linear(S(), p, p, 1e-5, 0, p, p, None, None, None, p, 4, 8192, 64, 64, 0, 0, 0.0, 0) == -2  # M K too large for the norm
   assert lib.tmx_small_linear(S(), p, None, 1e-5, 0, p, p, None, None, None, p, 1, 256, 64, 64, 0, 0, 0.0, 1) == -4  # SwiGLU needs the norm prologue
   assert lib.tmx_small_linear(S(), None, None, 1e-5, 0, p, p, None, None, None, p, 1, 256, 64, 64, 0, 0, 0.0, 0) == -1
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('K,r,widths', [(64, 1, (32,)), (192, 5, (40, 24)), (256, 16, (64, 32, 32)), (2048, 32, (64,)),
+                                        (128, 11, (33, 31))])
+def test_adapter_sync_writes_both_operands(K, r, widths, dtype):
+  """tmx_lora_pack against the host packing: every segment of a fused projection, odd ranks and widths (the
+  element-wise store), more tensors than one launch takes, and the padding columns of A untouched."""
+  from tunix_amd import quant
+  g = torch.Generator(device=G.DEV).manual_seed(K + r)
+  n = sum(widths)
+  a = [torch.randn(K, r, generator=g, device=G.DEV).to(dtype) for _ in widths]
+  b = [torch.randn(r, w, generator=g, device=G.DEV).to(dtype) for w in widths]
+  want_a = quant.pack_lora_a([x.to(torch.bfloat16) for x in a], K)
+  want_b = torch.cat([x.to(torch.bfloat16) for x in b], dim=1)
+  code = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dtype]
+  from tunix_amd.model import _LORA_PACK_DESC
+  copies = 30
+  got_a = [torch.zeros_like(want_a) for _ in range(copies)]
+  got_b = [torch.full_like(want_b, 7.0) for _ in range(copies)]
+  rows = []
+  for ga, gb in zip(got_a, got_b):
+    col = 0
+    for j, w in enumerate(widths):
+      rows.append((a[j].data_ptr(), ga.data_ptr(), K, r, j * r, want_a.shape[1] * 32, 1, code))
+      rows.append((b[j].data_ptr(), gb.data_ptr(), r, w, col, n, 0, code))
+      col += w
+  descs = np.array(rows, dtype=_LORA_PACK_DESC)
+  G.call('tmx_lora_pack', S(), descs.ctypes.data, len(rows))
+  G.sync()
+  for ga, gb in zip(got_a, got_b):
+    assert torch.equal(ga, want_a) and torch.equal(gb, want_b)

@@ -24,6 +24,7 @@ SIGNATURES = {
     'tmx_qlora_linear_num_splits': [ci, ci, ci],
     'tmx_qlora_linear_num_lora_splits': [ci, ci],
     'tmx_qlora_linear_planes': [vp, vp, vp, vp, vp, vp, vp, ci, ci, ci, ci, ci, ci],
+    'tmx_lora_pack': [vp, vp, ci],
     'tmx_rmsnorm': [vp, vp, vp, vp, ci, ci, cf, ci],
     'tmx_lora_residual_rmsnorm': [vp, vp, vp, ci, vp, ci, ci, vp, ci, cf, vp, vp, vp, vp, ci, ci, cf, ci],
     'tmx_rope_kv_write': [vp, vp, vp, ci, vp, ci, ci, vp, ci, cf, vp, vp, vp, vp, ci, vp, vp, vp, ci, ci,

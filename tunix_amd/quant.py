@@ -119,11 +119,12 @@ class PackedLinear:
     return cls(k, n, group, pack_q4t(q), pack_scales(s.to(torch.bfloat16)), [x.shape[1] for x in qs],
                rank, a_t, b, lora_scale)
 
-  def set_lora(self, loras):
-    """Replaces A/B in place (the LoRA-only weight sync of Sampler.update_params)."""
-    a_t = pack_lora_a([l[0].to(self.lora_a_t.device) for l in loras], self.k)
-    b = torch.cat([l[1].to(self.lora_b.device).to(torch.bfloat16) for l in loras], dim=1)
-    if a_t.shape != self.lora_a_t.shape or b.shape != self.lora_b.shape:
-      raise ValueError('New state must have the same shape, dtype and sharding as the old state.')
-    self.lora_a_t.copy_(a_t)
-    self.lora_b.copy_(b)
+  def set_adapter(self, is_a, col0, value):
+    """Replaces one adapter in place by torch operations (weights that are not on a GPU)."""
+    if is_a:
+      a = self.lora_a_dense().clone()
+      a[:, col0:col0 + self.rank] = value.reshape(self.k, self.rank)
+      self.lora_a_t.copy_(pack_lora_a([a], self.k))
+    else:
+      b = value.reshape(self.rank, -1)
+      self.lora_b[:, col0:col0 + b.shape[1]] = b

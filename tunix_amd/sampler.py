@@ -154,6 +154,10 @@ class Sampler:
     reference's "same structure" / "same shape" errors."""
     del filter_types
     flat = utils.flatten_state(updated_weights)
+    if hasattr(self._transformer, 'merge_lora'):
+      self._transformer.merge_lora(flat)
+      return
+    # a transformer that only has the reference's surface: the whole state, merged
     merged = dict(self._transformer.lora_state())
     unknown = set(flat) - set(merged)
     if unknown:

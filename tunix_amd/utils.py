@@ -179,26 +179,39 @@ def flatten_state(tree):
   hands over: nested mappings or state objects (anything with .items()), mappings keyed by
   path tuples, lists / tuples (index as path part), leaves that are arrays or variable-like
   objects with the array in `.value`.  Integer path parts (layer indices) print as digits."""
+  import torch
   out = {}
 
   def is_node(x):
     return hasattr(x, 'items') and callable(x.items) and not hasattr(x, 'shape')
 
-  def walk(prefix, node):
-    if is_node(node):
+  def put(name, leaf):
+    if name.endswith('.value'):  # pure-dict dumps of variable objects
+      name = name[:-len('.value')]
+    if name in out:
+      raise ValueError(f'duplicate parameter path {name!r}')
+    out[name] = leaf
+
+  def walk(prefix, node):  # prefix: the dotted path so far with its closing dot
+    if isinstance(node, torch.Tensor):
+      put(prefix[:-1], node)
+    elif is_node(node):
       for k, v in node.items():
-        parts = tuple(k) if isinstance(k, tuple) else (k,)
-        walk(prefix + tuple(str(getattr(p, 'key', p)) for p in parts), v)
+        if isinstance(k, str):
+          name = prefix + k
+        elif isinstance(k, tuple):
+          name = prefix + '.'.join([str(getattr(p, 'key', p)) for p in k])
+        else:
+          name = prefix + str(getattr(k, 'key', k))
+        if isinstance(v, torch.Tensor):  # most leaves of a weight sync
+          put(name, v)
+        else:
+          walk(name + '.', v)
     elif isinstance(node, (list, tuple)) and not (node and isinstance(node[0], (int, float, np.number))):
       for i, v in enumerate(node):
-        walk(prefix + (str(i),), v)
+        walk(prefix + str(i) + '.', v)
     else:
-      name = '.'.join(prefix)
-      if name.endswith('.value'):  # pure-dict dumps of variable objects
-        name = name[:-len('.value')]
-      if name in out:
-        raise ValueError(f'duplicate parameter path {name!r}')
-      out[name] = _leaf_array(node)
+      put(prefix[:-1], _leaf_array(node))
 
-  walk((), tree)
+  walk('', tree)
   return out
