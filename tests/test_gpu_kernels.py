@@ -1028,3 +1028,28 @@ def test_adapter_sync_writes_both_operands(K, r, widths, dtype):
   G.sync()
   for ga, gb in zip(got_a, got_b):
     assert torch.equal(ga, want_a) and torch.equal(gb, want_b)
+
+
+# row tiles x column tiles of the many-rows kernel that these shapes take on 256 compute units (wide_plan), ragged in
+# rows and columns; the reference is the f32 product of the dequantised matrix
+@pytest.mark.parametrize('M,K,N', [
+    (129, 256, 96), (257, 384, 4128),                      # 2 x 4
+    (190, 512, 28704), (250, 1024, 32768), (150, 256, 28672), (224, 256, 28672),  # 6 x 4, 8 x 4, 5 x 4, 7 x 4
+    (777, 512, 16416), (384, 512, 56000),                  # 4 x 4, 3 x 4
+    (129, 256, 32800), (383, 1024, 57344), (223, 1024, 57344), (1793, 384, 4128), (1000, 1024, 16384),  # 5, 6, 7, 4, 8 x 8
+    (300, 2048, 1024), (140, 8192, 256)])                  # K-slices
+def test_many_rows_projection_tiles(M, K, N):
+  from tunix_amd import quant
+  lib = _lib.lib()
+  g = torch.Generator(device=G.DEV).manual_seed(M + N)
+  w = (torch.randn(K, N, generator=g, device=G.DEV) * 0.02).to(torch.bfloat16)
+  x = torch.randn(M, K, generator=g, device=G.DEV).to(torch.bfloat16)
+  pl = quant.PackedLinear.from_dense([w], 64, G.DEV)
+  dense = torch.empty(K, N, dtype=torch.bfloat16, device=G.DEV)
+  G.call('tmx_int4_dequant', S(), G.p(pl.qweight), G.p(pl.scales), G.p(dense), K, N, 64)
+  ns = lib.tmx_qlora_linear_num_splits(M, K, N)
+  y = torch.full((ns, M, N), float('nan'), device=G.DEV)
+  G.call('tmx_qlora_linear_planes', S(), G.p(x), G.p(pl.qweight), G.p(pl.scales), None, G.p(y), None, M, K, N, 64, 0, ns)
+  got = y.sum(0)
+  want = x.float() @ dense.float()
+  assert (got - want).norm() <= 1e-5 * want.norm() and (got - want).abs().max() <= 1e-4 * want.abs().max()

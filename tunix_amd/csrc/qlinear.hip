@@ -1532,274 +1532,12 @@ static int launch_qlinear_dma(hipStream_t st, QLinearArgs a) {
   return check_launch();
 }
 
-// ---------------------------------------------------------------------------
-// Many rows (cache fill over whole prompts: more than 128 rows per pass).  At this size the
-// bound is what a CU can pull through its vector memory path (about 30 GB/s per CU, L2 hits
-// included), so the block is as large as the registers allow: 256 rows x 256 columns, 0.31 bytes
-// loaded per kFLOP.  Wave ct owns column tile ct and multiplies both k-tiles of every 2-tile step
-// against all 8 row tiles (128 accumulator registers), so a dequantised weight fragment feeds 8
-// MFMAs.  Same buffer loads and direct-to-LDS slab as the k-way block above, with 256-byte slab
-// rows (four rows per 1 KiB transfer), chunks XOR-swizzled by row % 16.  Two waves per SIMD: one
-// dequantises while the other multiplies.  Row blocks are blockIdx.z, K-slices blockIdx.y.
-struct KW {
-  static constexpr int MT = 8, ROWS = 256, COLS = 256, TS = 2, XS = 128;
-  static constexpr size_t LDS = (size_t)2 * ROWS * XS * 2;  // 128 KiB
-};
-
-template <bool LORA>
-__device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* smem, int bx, int by, int bz) {
-  constexpr int MT = KW::MT, TS = KW::TS, XS = KW::XS, ROWS = KW::ROWS;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int ct = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int h = lane >> 5, nl = lane & 31;
-  const int KT = a.K >> 6;
-  const int slice = LORA ? (bx - a.n_main_blocks) + a.lora_blocks_per_split * by : by;
-  const int per = LORA ? a.kt_per_lora_split : a.kt_per_split;
-  const int kb0 = slice * per;
-  const int kb1 = (kb0 + per < KT) ? kb0 + per : KT;
-  const int nsteps = (kb1 - kb0) / TS, last_step = nsteps - 1;  // host: whole steps
-  if (nsteps <= 0) return;
-  const int row0 = bz * ROWS;
-  const int rows = a.M - row0 < ROWS ? a.M - row0 : ROWS;  // host: >= 1
-  const int gs = __builtin_ctz(a.G >> 6), KG = a.K / a.G;
-  const int NT = LORA ? (a.Rpad >> 5) : (a.N >> 5);
-  const int nb = LORA ? ct : bx * 8 + ct;
-  const bool tile_ok = nb < NT;  // waves past the last tile only help with the slab
-
-  const __amdgpu_buffer_rsrc_t rw =
-      LORA ? make_rsrc(a.a_t, (uint32_t)KT * NT * 4096u) : make_rsrc(a.qw, (uint32_t)NT * KT * 1024u);
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.scales, LORA ? 0u : (uint32_t)NT * KG * 64u);
-  const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x + (size_t)row0 * a.ldx, (uint32_t)rows * a.ldx * 2u);
-  const int wv = LORA ? nb * 4096 + lane * 16 : (nb * KT * 64 + lane) * 16;
-  const int wstep = LORA ? NT * 4096 : 1024;  // bytes between consecutive k-tiles
-  const int sv = (nb * KG * 32 + nl) * 2;
-  // slab transfer: 8 loads per wave and step; load i moves rows 4 wave + 32 i .. + 3 (16 lanes
-  // each), lane l delivering chunk (l % 16) ^ (row % 16) of the step to slot l % 16
-  constexpr int XR = ROWS / 32;
-  int xoff[XR];  // per-lane byte offset in the row block (rows past the end repeat the last)
-#pragma unroll
-  for (int i = 0; i < XR; ++i) {
-    const int row_l = 4 * ct + 32 * i + (lane >> 4);
-    xoff[i] = (row_l < rows ? row_l : rows - 1) * a.ldx * 2 + (((lane & 15) ^ (row_l & 15)) * 16) + kb0 * 128;
-  }
-
-  f32x16_t acc[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
-  constexpr int WPT = LORA ? 4 : 1;  // 16-byte words per lane and tile
-  u32x4_t wring[TS][WPT];
-  uint16_t sring[TS];
-
-  auto load_w_tile = [&](int step, auto jc) __attribute__((always_inline)) {
-    constexpr int j = decltype(jc)::value;
-    step = step < last_step ? step : last_step;
-    const int kt = kb0 + step * TS + j;
-#pragma unroll
-    for (int t = 0; t < WPT; ++t) wring[j][t] = __builtin_amdgcn_raw_buffer_load_b128(rw, wv + t * 1024, kt * wstep, 0);
-    if (!LORA) sring[j] = __builtin_amdgcn_raw_buffer_load_b16(rs, sv, (kt >> gs) * 64, 0);
-  };
-  auto dma_x = [&](int step, int buf) __attribute__((always_inline)) {
-    step = step < last_step ? step : last_step;
-    uint16_t* base = smem + (size_t)buf * ROWS * XS + ct * 4 * XS;
-#pragma unroll
-    for (int i = 0; i < XR; ++i) load_row_to_lds(rx, base + i * 32 * XS, xoff[i], step * (TS * 128));
-  };
-  // One step: 8 fragment groups g = 4 j + t (k-tile j, 16-wide k-block t) of 8 MFMAs, one per row
-  // tile.  Between the MFMAs of group g the wave reads the x fragments of group g + 1 (one LDS
-  // read per MFMA; chunk 2 g + h of a row sits at slot (2 g + h) ^ (row % 16)) and dequantises its
-  // weight fragment a quarter at a time, so the matrix pipe waits neither for LDS nor for the
-  // VALU, also when both waves of a SIMD run in phase after a barrier.  The order is pinned.
-  auto step_math = [&](int step, int buf) __attribute__((always_inline)) {
-    u32x4_t wc[TS][WPT];
-    float s_c[TS], m8s[TS];
-    static_for<TS>([&](auto jc) __attribute__((always_inline)) {
-      constexpr int j = decltype(jc)::value;
-#pragma unroll
-      for (int t = 0; t < WPT; ++t) wc[j][t] = wring[j][t];
-      s_c[j] = LORA ? 0.f : bf2f(sring[j]);
-      m8s[j] = -8.f * s_c[j];
-      load_w_tile(step + 1, jc);  // registers consumed: refill them one step ahead
-    });
-    const uint16_t* xb = smem + (size_t)buf * ROWS * XS + nl * XS;
-    auto word_of = [&](auto gc) __attribute__((always_inline)) {
-      constexpr int g = decltype(gc)::value, j = g / 4, t = g % 4;
-      return t == 0 ? wc[j][0].x : (t == 1 ? wc[j][0].y : (t == 2 ? wc[j][0].z : wc[j][0].w));
-    };
-    bf16x8_t xq[2][MT];
-    u32x4_t bq[2];
-    {
-      const int slot = (h ^ (nl & 15)) * 8;
-#pragma unroll
-      for (int m = 0; m < MT; ++m) xq[0][m] = *reinterpret_cast<const bf16x8_t*>(xb + m * 32 * XS + slot);
-      if (LORA) bq[0] = wc[0][0];
-      else bq[0] = __builtin_bit_cast(u32x4_t, dequant_word(word_of(IC<0>{}), s_c[0], m8s[0]));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    static_for<4 * TS>([&](auto gc) __attribute__((always_inline)) {
-      constexpr int g = decltype(gc)::value, cur = g & 1, nxt = cur ^ 1;
-      constexpr bool more = g + 1 < 4 * TS;
-      constexpr int jn = (g + 1) / 4 % TS, tn = (g + 1) % 4;
-      const int slot = ((2 * (g + 1) + h) ^ (nl & 15)) * 8;
-      uint32_t lo = 0, hi = 0;
-      static_for<MT>([&](auto mc) __attribute__((always_inline)) {
-        constexpr int m = decltype(mc)::value;
-        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xq[cur][m], __builtin_bit_cast(bf16x8_t, bq[cur]), acc[m],
-                                                         0, 0, 0);
-        if constexpr (more) {
-          xq[nxt][m] = *reinterpret_cast<const bf16x8_t*>(xb + m * 32 * XS + slot);
-          if (LORA) {
-            if (m == 0) bq[nxt] = wc[jn][tn % WPT];
-          } else {
-            if (m == 0) dequant_masks(word_of(IC<g + 1>{}), lo, hi);
-            if (m == 1) bq[nxt].x = dequant_part<0>(lo, hi, s_c[jn], m8s[jn]);
-            if (m == 2) bq[nxt].y = dequant_part<1>(lo, hi, s_c[jn], m8s[jn]);
-            if (m == 3) bq[nxt].z = dequant_part<2>(lo, hi, s_c[jn], m8s[jn]);
-            if (m == 4) bq[nxt].w = dequant_part<3>(lo, hi, s_c[jn], m8s[jn]);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      });
-    });
-  };
-  // loads of a step younger than its slab transfer (in-order counter)
-  constexpr int kYounger = TS * (LORA ? 4 : 2);
-  auto wait_slab = [&]() __attribute__((always_inline)) {
-    __builtin_amdgcn_sched_barrier(0);
-    if (tile_ok) __builtin_amdgcn_s_waitcnt(0x0F70 | (kYounger & 15) | ((kYounger >> 4) << 14));
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-  };
-
-  dma_x(0, 0);
-  if (tile_ok) static_for<TS>([&](auto jc) __attribute__((always_inline)) { load_w_tile(0, jc); });
-  wait_slab();
-  for (int step = 0; step < nsteps; ++step) {
-    const int buf = step & 1;
-    dma_x(step + 1, buf ^ 1);
-    __builtin_amdgcn_sched_barrier(0);
-    if (tile_ok) step_math(step, buf);
-    wait_slab();
-  }
-  if (!tile_ok) return;
-  const int col = nb * 32 + nl;
-  if (!LORA && a.t16) {
-    // LoRA in the epilogue: delta tile [32 rows, 32 columns] = t16 rows . B columns, 16 ranks per
-    // MFMA (t rows are the A operand, so the delta lands in the accumulator layout of acc[m]);
-    // y = bf16(bf16(base) + bf16(bf16(delta) ls))
-    const int seg = nb * 32 >= a.seg_end[0] ? (nb * 32 >= a.seg_end[1] ? 2 : 1) : 0;
-    const int tc0 = seg * a.lora_r;
-    const int nkb = (a.lora_r + 15) >> 4;  // host: <= 4
-    u32x4_t bfr[4];
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      uint32_t w[4] = {0, 0, 0, 0};
-      if (kb < nkb) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int rr = kb * 16 + 8 * h + j;
-          const uint32_t e = rr < a.lora_r ? a.lora_b[(size_t)rr * a.N + col] : 0u;
-          w[j >> 1] |= e << (16 * (j & 1));
-        }
-      }
-      bfr[kb] = u32x4_t{w[0], w[1], w[2], w[3]};
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const int trow = row0 + m * 32 + nl;
-      const uint16_t* tp = a.t16 + (size_t)(trow < a.M ? trow : a.M - 1) * a.ldt16 + tc0 + 8 * h;
-      f32x16_t d;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) d[r] = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-        if (kb < nkb) {
-          const bf16x8_t tf = *reinterpret_cast<const bf16x8_t*>(tp + kb * 16);
-          d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tf, __builtin_bit_cast(bf16x8_t, bfr[kb]), d, 0, 0, 0);
-        }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = row0 + m * 32 + acc_row(r, lane);
-        if (row >= a.M) continue;
-        a.y_bf16[(size_t)row * a.ldy + col] = f2bf(rbf(acc[m][r]) + rbf(rbf(d[r]) * a.lora_ls));
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = row0 + m * 32 + acc_row(r, lane);
-      if (row >= a.M) continue;
-      const float v = acc[m][r];
-      if (LORA) a.t_part[((size_t)slice * a.M + row) * a.ldt + col] = v;
-      else if (a.y_bf16) a.y_bf16[(size_t)row * a.ldy + col] = f2bf(v);
-      else a.y_part[((size_t)slice * a.M + row) * a.N + col] = v;
-    }
-}
-
-// Workgroups are dispatched round-robin over the 8 XCDs (linear id % 8), each with its own L2.
-// The launch is one-dimensional and maps ids so that the workgroups of an XCD share row blocks:
-// with S = gcd(row blocks, 8), XCD x works on row blocks x % S, x % S + S, ... in turn, all column
-// blocks and K-slices of one before the next, so the activation slab of a step is fetched into
-// that L2 once and the other workgroups of the XCD hit it.  Ids past the end do nothing.
-__global__ __launch_bounds__(512, 1) void qlinear_mfma_wide_kernel(QLinearArgs a, int blocks, int row_blocks, int S) {
-  extern __shared__ __align__(16) uint16_t smem[];
-  const int id = (int)blockIdx.x, xcd = id & 7, idx = id >> 3;
-  const int per_rb = blocks * a.nsplit;
-  const int p = xcd / S + (8 / S) * idx;
-  // an XCD with an even number of row blocks takes them two at a time, the same column block on both in
-  // consecutive workgroups, so that a weight tile fetched for one is an L2 hit for the other
-  const int R = (row_blocks + S - 1) / S, Gr = (R & 1) ? 1 : 2;
-  const int blk = p / (per_rb * Gr), within = p % (per_rb * Gr);
-  const int bz = xcd % S + S * (blk * Gr + within % Gr);
-  if (bz >= row_blocks) return;
-  const int cb = within / Gr, bx = cb % blocks, by = cb / blocks;
-  if (bx >= a.n_main_blocks) gemm_block_wide<true>(a, smem, bx, by, bz);
-  else gemm_block_wide<false>(a, smem, bx, by, bz);
-}
-
-// t16[m][c] = bf16(sum of the planes' values) for c < cols, 0 up to the row stride ldt
-__global__ __launch_bounds__(256) void lora_t_reduce_kernel(const float* t_part, int nsplit, int M, int ldt,
-                                                            uint16_t* t16, int cols) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= M * ldt) return;
-  const int m = i / ldt, c = i - m * ldt;
-  float t = 0.f;
-  if (c < cols)
-    for (int sp = 0; sp < nsplit; ++sp) t += t_part[((size_t)sp * M + m) * ldt + c];
-  t16[(size_t)m * ldt + c] = f2bf(t);
-}
-
-// part: 0 = main blocks and LoRA blocks in one launch, 1 = LoRA blocks only, 2 = main blocks only
-static int launch_qlinear_wide(hipStream_t st, QLinearArgs a, int part = 0) {
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&qlinear_mfma_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-      (int)KW::LDS);
-  if (attr != hipSuccess) return TMX_ERR_LAUNCH;
-  a.n_main_blocks = part == 1 ? 0 : (a.N + KW::COLS - 1) / KW::COLS;
-  const int blocks = a.n_main_blocks + ((a.a_t && part != 2) ? a.lora_blocks_per_split : 0);
-  const int row_blocks = (a.M + KW::ROWS - 1) / KW::ROWS;
-  int S = 8;
-  while (row_blocks % S) S >>= 1;  // gcd(row_blocks, 8)
-  // ids cover 8 / S XCDs x (row_blocks / S) row blocks x blocks x nsplit per residue, rounded up to 8
-  const long total = (long)blocks * a.nsplit * row_blocks;
-  const int ids = (int)((total + 7) / 8 * 8);
-  hipLaunchKernelGGL(qlinear_mfma_wide_kernel, dim3(ids), dim3(512), KW::LDS, st, a, blocks, row_blocks, S);
-  return check_launch();
-}
-
 // Which kernel serves a projection: narrow ones (fewer than 16 column blocks) with K % 256 == 0
 // below 8192 run the 4-wave kernel; everything else a k-way kernel: the direct-to-LDS one when
 // K % 256 == 0 (measured faster than the 4-wave kernel on the o, q|k|v, down and unsplit gate|up
 // shapes of the 8B and 30B-A3B models at 1, 32, 64 and 128 rows), the plain one otherwise.
 static bool four_wave_shape(int K) { return K % 256 == 0 && K < 8192; }
 static bool four_wave(int K, int N) { return four_wave_shape(K) && (N + 127) / 128 < 16; }
-
-static int slice_len(int KT, int s) { return ((KT + s - 1) / s + 3) / 4 * 4; }
-static bool slices_ok(int KT, int s) { return (KT + slice_len(KT, s) - 1) / slice_len(KT, s) == s; }
 
 // Number of K-slices for a projection: the count that minimises (rounds of workgroups over the
 // device's CUs: 256 on the MI355X, also assumed when no device is present) x (steps per slice + fixed
@@ -1824,13 +1562,7 @@ static int num_splits4(int K, int N) {
 
 int qlinear_num_lora_splits(int K, int N);
 int qlinear_num_splits(int K, int N, int M) {
-  if (M > 128) {
-    // 256-row blocks: K-slices only while the launch has fewer workgroups than CUs
-    const int wgs = (N + 255) / 256 * ((M + 255) / 256);
-    int s = 1;
-    while (wgs * s < device_cus() * 3 / 4 && s * 2 <= TMX_MAX_SPLITS && slices_ok(K / 64, s * 2) && slice_len(K / 64, s * 2) >= 8) s *= 2;
-    return s;
-  }
+  if (M > 128) return wide_plan(M, N, K, 0).nsplit;
   if (four_wave(K, N)) return num_splits4(K, N);
   const int nblocks = (N + 127) / 128;
   const int KT = K / 64;
@@ -2025,7 +1757,7 @@ int qlinear_base(hipStream_t st, const void* x, int ldx, const void* qw, const v
     if (K % 128 || a.kt_per_split % 2 || (a_t && a.kt_per_lora_split % 2) || (size_t)256 * ldx * 2 >= (1u << 31) ||
         (size_t)K * N / 2 >= (1u << 31) || (size_t)K * Rpad * 2 >= (1u << 31))
       return TMX_ERR_SHAPE;
-    return launch_qlinear_wide(st, a);
+    return qwide_launch(st, a, 0);
   }
   if (four_wave(K, N)) {
     if (M <= 32) return launch_qlinear4<1>(st, a);
@@ -2071,11 +1803,9 @@ int qlinear_wide_lora(hipStream_t st, const void* x, int ldx, const void* qw, co
   a.kt_per_lora_split = lora_slice_len(K, N);
   if (a_t) {
     if (a.kt_per_lora_split % 2) return TMX_ERR_UNSUPPORTED;
-    int rc = launch_qlinear_wide(st, a, 1);
+    int rc = qwide_launch(st, a, 1);
     if (rc != TMX_OK) return rc;
-    hipLaunchKernelGGL(lora_t_reduce_kernel, dim3((M * TMX_MAX_RPAD + 255) / 256), dim3(256), 0, st, t_part, nls, M,
-                       TMX_MAX_RPAD, t16, Rpad);
-    if ((rc = check_launch()) != TMX_OK) return rc;
+    if ((rc = lora_t_reduce(st, t_part, nls, M, t16, Rpad)) != TMX_OK) return rc;
     a.t16 = t16;
     a.ldt16 = TMX_MAX_RPAD;
     a.lora_b = (const uint16_t*)lora_b;
@@ -2083,7 +1813,7 @@ int qlinear_wide_lora(hipStream_t st, const void* x, int ldx, const void* qw, co
     a.lora_ls = ls;
     for (int i = 0; i < 3; ++i) a.seg_end[i] = seg_end ? seg_end[i] : N;
   }
-  return launch_qlinear_wide(st, a, 2);
+  return qwide_launch(st, a, 2);
 }
 
 // ---------------------------------------------------------------------------

@@ -309,6 +309,14 @@ int zero_words(hipStream_t st, uint32_t* p, int n);  // p[0 .. n) = 0 by a small
 int device_cus();  // compute units of the current device (256 when none answers)
 // 0 when the fused gate | up launch cannot hand its LoRA projection over for this shape on this device
 size_t qlinear_gate_up_handover_bytes(int M, int K, int F, int r);
+// K-slices are whole groups of 4 k-tiles; slices_ok: s slices and none of them empty
+inline int slice_len(int KT, int s) { return ((KT + s - 1) / s + 3) / 4 * 4; }
+inline bool slices_ok(int KT, int s) { return (KT + slice_len(KT, s) - 1) / slice_len(KT, s) == s; }
+// Projections of more than 128 rows (qwide.hip): mt row tiles x ct column tiles per workgroup, K in nsplit slices
+struct WidePlan { int mt, ct, nsplit; };
+WidePlan wide_plan(int M, int N, int K, int nsplit);  // nsplit 0: its choice
+int qwide_launch(hipStream_t st, const QLinearArgs& a, int part);
+int lora_t_reduce(hipStream_t st, const float* t_part, int nsplit, int M, uint16_t* t16, int cols);
 // Many rows (M > 128), unsplit: y_bf16 = bf16(bf16(x . W) + bf16(bf16(t . B) ls)) in one pass, t = bf16(x . A)
 // computed by a LoRA-only launch of the same kernel and a small reduction (t_part: f32 planes, t16: bf16
 // [M][TMX_MAX_RPAD] scratch).  seg_end: column ends of the fused matrices (q | k | v, gate | up), unused
