@@ -1053,3 +1053,33 @@ def test_many_rows_projection_tiles(M, K, N):
   got = y.sum(0)
   want = x.float() @ dense.float()
   assert (got - want).norm() <= 1e-5 * want.norm() and (got - want).abs().max() <= 1e-4 * want.abs().max()
+
+
+# one and several K-slices of x . A, one to four column tiles of A, a ragged last row tile
+@pytest.mark.parametrize('M,K,N,r', [(129, 256, 96, 8), (300, 4096, 12288, 16), (161, 5120, 28672, 32), (416, 2048, 16384, 64),
+                                     (1000, 4224, 4096, 24)])
+def test_many_rows_projection_with_adapter(M, K, N, r):
+  from tunix_amd import quant
+  lib = _lib.lib()
+  assert lib.tmx_qlora_linear_num_splits(M, K, N) == 1  # LoRA in the epilogue of the launch
+  g = torch.Generator(device=G.DEV).manual_seed(M + r)
+  rnd = lambda *s: torch.randn(*s, generator=g, device=G.DEV)
+  w, a, b = (rnd(K, N) * 0.02).to(torch.bfloat16), (rnd(K, r) * 0.02).to(torch.bfloat16), (rnd(r, N) * 0.1).to(torch.bfloat16)
+  x = rnd(M, K).to(torch.bfloat16)
+  pl = quant.PackedLinear.from_dense([w], 64, G.DEV, [(a, b)], 2.0)
+  dense = torch.empty(K, N, dtype=torch.bfloat16, device=G.DEV)
+  G.call('tmx_int4_dequant', S(), G.p(pl.qweight), G.p(pl.scales), G.p(dense), K, N, 64)
+  ws = torch.empty(lib.tmx_qlora_linear_workspace_bytes(M, K, N), dtype=torch.uint8, device=G.DEV)
+  y = torch.empty(M, N, dtype=torch.bfloat16, device=G.DEV)
+  rb = lambda t: t.to(torch.bfloat16).float()
+  base, t = rb(x.float() @ dense.float()), rb(x.float() @ a.float())
+  delta = rb(rb(t @ b.float()) * 2.0)
+  want = rb(base + delta)
+  for _ in range(2):  # the second call finds the hand-over words as the first left them
+    G.call('tmx_qlora_linear', S(), G.p(x), G.p(pl.qweight), G.p(pl.scales), G.p(pl.lora_a_t), G.p(pl.lora_b), None, G.p(y),
+           G.p(ws), M, K, N, 64, r, pl.r_pad, 2.0)
+    G.sync()
+    # values of t, of the base and of the delta that round the other way each move the result by a bf16 step of a term
+    err = (y.float() - want).abs()
+    assert (err > 2.0 ** -6 * (base.abs() + delta.abs() + 1.0)).sum() == 0
+    assert (y.float() - want).norm() <= 2e-3 * want.norm()

@@ -22,7 +22,9 @@ struct Workspace {
   uint32_t* status;  // first 256 bytes, the same place for every batch size: word 0 is set when a bounded wait inside a kernel runs out
   uint16_t *x, *xn, *q, *attn, *act, *y16;
   float *y_part, *t_part, *rope_tab;
-  uint16_t* t16;  // bf16 LoRA projection of a many-rows pass
+  uint16_t* t16;  // many-rows pass: LoRA projection in bf16, the same in f32, two hand-over areas that take turns
+  float* t_fin;
+  uint32_t* wide_sync;
   void* gu_sync;  // hand-over area of the fused gate | up launch (LoRA projection computed once per launch)
   float* sb_tparts;        // small-batch step: parts of the down projection's t left by gate | up
   float* sb_attn_partial;  // small-batch step: split results of the attention kernel
@@ -105,6 +107,8 @@ static Workspace carve(const tmx_model_desc* m, int B, int C, char* base) {
   w.y_part = (float*)take((size_t)B * ypart * 4);
   w.t_part = (float*)take((size_t)TMX_MAX_LORA_SPLITS * B * TMX_MAX_RPAD * 4);
   w.t16 = (uint16_t*)take(B > 128 ? (size_t)B * TMX_MAX_RPAD * 2 : 0);
+  w.t_fin = (float*)take(B > 128 ? (size_t)B * TMX_MAX_RPAD * 4 : 0);
+  w.wide_sync = (uint32_t*)take(B > 128 ? 2 * wide_sync_words() * 4 : 0);
   {
     w.delta = (uint16_t*)take(B <= 128 ? (size_t)B * D * 2 : 0);
     w.dsync = take(B <= 128 ? qlinear_delta_sync_bytes(B, TMX_MAX_RPAD) : 0);
@@ -216,9 +220,9 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
   auto lora_of = [&](const tmx_qlinear_desc& l, int) {
     LoraIn li = {};
     if (l.lora_a_t) {
-      li.t_part = w.t_part;
+      li.t_part = B > 128 ? w.t_fin : w.t_part;
       li.ldt = TMX_MAX_RPAD;
-      li.nsplit = qlinear_num_lora_splits(l.K, l.N);
+      li.nsplit = B > 128 ? 1 : qlinear_num_lora_splits(l.K, l.N);
       li.b = (const uint16_t*)l.lora_b;
       li.r = l.rank;
       li.ls = l.lora_scale;
@@ -242,13 +246,19 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
     rc = zero_words(st, (uint32_t*)w.dsync, 64);
     if (rc != TMX_OK) return rc;
   }
-  // Many rows (B > 128): projection + LoRA in one pass into w.y16 where the shape allows it (unsplit,
-  // rank % 8 == 0); returns TMX_ERR_UNSUPPORTED (nothing launched) when the caller must take the planes path.
-  auto wide_linear = [&](const void* x, int ldx, const tmx_qlinear_desc& l, int e0, int e1) {
-    if (B <= 128) return (int)TMX_ERR_UNSUPPORTED;
+  // Many rows (B > 128): the projection and its LoRA half in one launch; `fused`: LoRA applied, bf16 in w.y16
+  int wide_turn = 0;  // which hand-over area the next launch uses
+  auto wide_linear = [&](const void* x, int ldx, const tmx_qlinear_desc& l, int e0, int e1, int nsplit, bool* fused) {
     const int seg_end[3] = {e0, e1, l.N};
-    return qlinear_wide_lora(st, x, ldx, l.qweight, l.scales, l.lora_a_t, l.lora_b, l.rank, l.lora_scale, seg_end,
-                             w.y16, w.t_part, w.t16, B, l.K, l.N, l.G, l.r_pad);
+    WideLora wl = {};
+    if (l.lora_a_t) {
+      wl.t_part = w.t_part; wl.t16 = w.t16; wl.t_fin = w.t_fin; wl.status = w.status;
+      wl.sync = w.wide_sync + wide_turn * wide_sync_words();
+      wide_turn ^= 1;
+      wl.sync_clear = w.wide_sync + wide_turn * wide_sync_words();
+    }
+    return qlinear_wide(st, x, ldx, l.qweight, l.scales, l.lora_a_t, l.lora_b, l.rank, l.lora_scale, seg_end, w.y16,
+                        w.y_part, wl, B, l.K, l.N, l.G, l.r_pad, nsplit, fused);
   };
   // the hand-over words of the fused gate | up launch start at zero (the kernel leaves them so)
   if (!moe && B <= kFusedGateUpMaxRows && w.gu_sync && n_steps > 0) {
@@ -258,6 +268,11 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
   // samples of one prompt in consecutive rows: decode attention reads the prompt slots once per group
   const bool share_walk = T == 1 && !small && w.attn_partial && attn_share_ok(B, N, Kh, H, C, s->share_group, s->share_len);
   for (int it = 0; it < n_steps; ++it) {
+    if (w.wide_sync) {  // both areas start a step at zero, whichever the last launch of the step before used
+      rc = zero_words(st, w.wide_sync, 2 * (int)wide_sync_words());
+      if (rc != TMX_OK) return rc;
+      wide_turn = 0;
+    }
     {  // embedding gather + first input norm + this step's RoPE table
       RowNormArgs a = {};
       a.embed = (const uint16_t*)m->embed;
@@ -353,14 +368,17 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
                             (!l.gate_up.lora_a_t || (2 * l.gate_up.rank <= 32 && l.gate_up.r_pad == 32));
       uint16_t* kc = (uint16_t*)s->kv_cache + (size_t)(2 * i) * kv_elems;
       uint16_t* vc = kc + kv_elems;
-      bool fused;  // this projection ran with LoRA in its epilogue: the consumer reads bf16, no LoRA left
+      bool fused;  // this projection ran with LoRA in its epilogue: no LoRA left for the consumer
+      // the projection wrote bf16 to w.y16 instead of f32 planes (many rows, one K-slice)
+      auto whole = [&](int nsplit) { return B > 128 && nsplit == 1; };
       LoraDelta ld;
       bool with_delta = false;  // the projection's LoRA blocks made the delta: the consumer adds it
       {
         if (prof) prof->before(TMX_K_QKV, st);
-        rc = wide_linear(w.xn, D, l.qkv, NH, NH + Kh * H);
-        fused = rc != TMX_ERR_UNSUPPORTED;
-        if (!fused)
+        fused = false;
+        if (B > 128)
+          rc = wide_linear(w.xn, D, l.qkv, NH, NH + Kh * H, sp.qkv, &fused);
+        else
           rc = qlinear_base(st, w.xn, D, l.qkv.qweight, l.qkv.scales, l.qkv.lora_a_t, nullptr, w.y_part, w.t_part,
                             TMX_MAX_RPAD, B, D, QKV, l.qkv.G, l.qkv.r_pad, sp.qkv);
         if (prof) prof->after(TMX_K_QKV, st);
@@ -368,13 +386,13 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       }
       {
         RopeArgs a = {};
-        if (fused) {
+        if (whole(sp.qkv)) {
           a.qkv_bf16 = w.y16;
         } else {
           a.qkv_part = w.y_part;
           a.nsplit = sp.qkv;
-          a.lora = lora_of(l.qkv, sp.qkv);
         }
+        if (!fused) a.lora = lora_of(l.qkv, sp.qkv);
         a.q_norm_w = (const uint16_t*)l.q_norm_w;
         a.k_norm_w = (const uint16_t*)l.k_norm_w;
         a.positions = s->positions; a.step = s->step; a.buf_len = L; a.tpp = T;
@@ -396,9 +414,10 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       }
       {
         if (prof) prof->before(TMX_K_O, st);
-        rc = wide_linear(w.attn, NH, l.o, D, D);
-        fused = rc != TMX_ERR_UNSUPPORTED;
-        if (!fused) {
+        fused = false;
+        if (B > 128) {
+          rc = wide_linear(w.attn, NH, l.o, D, D, sp.o, &fused);
+        } else {
           with_delta = delta_of(l.o, sp.o, D, D, ld);
           rc = qlinear_base(st, w.attn, NH, l.o.qweight, l.o.scales, l.o.lora_a_t, nullptr, w.y_part, w.t_part,
                             TMX_MAX_RPAD, B, NH, D, l.o.G, l.o.r_pad, sp.o, with_delta ? &ld : nullptr);
@@ -408,14 +427,14 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       }
       {
         RowNormArgs a = {};
-        if (fused) {
+        if (whole(sp.o)) {
           a.y_bf16 = w.y16;
         } else {
           a.y_part = w.y_part;
           a.nsplit = sp.o;
-          if (with_delta) a.delta = w.delta;
-          else a.lora = lora_of(l.o, sp.o);
         }
+        if (with_delta) a.delta = w.delta;
+        else if (!fused) a.lora = lora_of(l.o, sp.o);
         a.residual = w.x; a.x_out = w.x;
         a.norm_w = (const uint16_t*)l.norm2_w; a.xn_out = w.xn;
         a.D = D; a.eps = m->norm_eps; a.family = m->family;
@@ -460,9 +479,10 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
         const bool gu16 = sp.gate_up == 1;
         {
           if (prof) prof->before(TMX_K_GATE_UP, st);
-          rc = wide_linear(w.xn, D, l.gate_up, F, 2 * F);
-          fused = rc != TMX_ERR_UNSUPPORTED;
-          if (!fused)
+          fused = false;
+          if (B > 128)
+            rc = wide_linear(w.xn, D, l.gate_up, F, 2 * F, sp.gate_up, &fused);
+          else
             rc = qlinear_base(st, w.xn, D, l.gate_up.qweight, l.gate_up.scales, l.gate_up.lora_a_t,
                               gu16 ? w.y16 : nullptr, w.y_part, w.t_part, TMX_MAX_RPAD, B, D, 2 * F, l.gate_up.G,
                               l.gate_up.r_pad, sp.gate_up);
@@ -471,7 +491,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
         }
         {
           SwigluArgs a = {};
-          a.gu_bf16 = (gu16 || fused) ? w.y16 : nullptr;
+          a.gu_bf16 = gu16 ? w.y16 : nullptr;
           a.gu_part = w.y_part;
           a.nsplit = sp.gate_up;
           if (!fused) a.lora = lora_of(l.gate_up, sp.gate_up);
@@ -481,9 +501,10 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
         }
         {
           if (prof) prof->before(TMX_K_DOWN, st);
-          rc = wide_linear(w.act, F, l.down, D, D);
-          fused = rc != TMX_ERR_UNSUPPORTED;
-          if (!fused) {
+          fused = false;
+          if (B > 128) {
+            rc = wide_linear(w.act, F, l.down, D, D, sp.down, &fused);
+          } else {
             with_delta = delta_of(l.down, sp.down, D, D, ld);
             rc = qlinear_base(st, w.act, F, l.down.qweight, l.down.scales, l.down.lora_a_t, nullptr, w.y_part,
                               w.t_part, TMX_MAX_RPAD, B, F, D, l.down.G, l.down.r_pad, sp.down, with_delta ? &ld : nullptr);
@@ -493,14 +514,14 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
         }
         {
           RowNormArgs a = {};
-          if (fused) {
+          if (whole(sp.down)) {
             a.y_bf16 = w.y16;
           } else {
             a.y_part = w.y_part;
             a.nsplit = sp.down;
-            if (with_delta) a.delta = w.delta;
-            else a.lora = lora_of(l.down, sp.down);
           }
+          if (with_delta) a.delta = w.delta;
+          else if (!fused) a.lora = lora_of(l.down, sp.down);
           a.residual = w.x; a.x_out = w.x;
           a.norm_w = (const uint16_t*)(i + 1 < m->num_layers ? m->layers[i + 1].norm1_w : m->final_norm_w);
           a.xn_out = w.xn;

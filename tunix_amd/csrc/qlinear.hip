@@ -1754,10 +1754,11 @@ int qlinear_base(hipStream_t st, const void* x, int ldx, const void* qw, const v
   }
   if (M > 128) {
     // more than 128 rows: the 256-row block (whole 2-tile steps, 32-bit byte offsets per row block)
-    if (K % 128 || a.kt_per_split % 2 || (a_t && a.kt_per_lora_split % 2) || (size_t)256 * ldx * 2 >= (1u << 31) ||
+    if (K % 128 || a.kt_per_split % 2 || (size_t)256 * ldx * 2 >= (1u << 31) ||
         (size_t)K * N / 2 >= (1u << 31) || (size_t)K * Rpad * 2 >= (1u << 31))
       return TMX_ERR_SHAPE;
-    return qwide_launch(st, a, 0);
+    a.n_lora_slices = nls;  // planes only: the caller adds them
+    return qwide_launch(st, a);
   }
   if (four_wave(K, N)) {
     if (M <= 32) return launch_qlinear4<1>(st, a);
@@ -1773,17 +1774,19 @@ int qlinear_base(hipStream_t st, const void* x, int ldx, const void* qw, const v
   return launch_qlinear<4, 2>(st, a);
 }
 
-int qlinear_wide_lora(hipStream_t st, const void* x, int ldx, const void* qw, const void* scales, const void* a_t,
-                      const void* lora_b, int r, float ls, const int* seg_end, void* y_bf16, float* t_part,
-                      uint16_t* t16, int M, int K, int N, int G, int Rpad) {
-  if (!x || !qw || !scales || !y_bf16) return TMX_ERR_ARG;
-  if (a_t && (!lora_b || !t_part || !t16 || r <= 0)) return TMX_ERR_ARG;
+int qlinear_wide(hipStream_t st, const void* x, int ldx, const void* qw, const void* scales, const void* a_t,
+                 const void* lora_b, int r, float ls, const int* seg_end, void* y_bf16, float* y_part, const WideLora& w,
+                 int M, int K, int N, int G, int Rpad, int nsplit, bool* fused) {
+  if (!x || !qw || !scales || (nsplit == 1 ? !y_bf16 : !y_part)) return TMX_ERR_ARG;
+  *fused = nsplit == 1 && (!a_t || r % 8 == 0);
+  if (a_t && (!lora_b || !w.t_part || !(*fused ? (void*)w.t16 : (void*)w.t_fin) || !w.sync || !w.sync_clear || r <= 0))
+    return TMX_ERR_ARG;
   if (M <= 128 || K % 128 || N % 32 || G % 64 || (G & (G - 1)) || K % G || ldx % 8) return TMX_ERR_SHAPE;
-  if (a_t && (r % 8 || r > 64 || Rpad <= 0 || Rpad % 32 || Rpad > TMX_MAX_RPAD)) return TMX_ERR_UNSUPPORTED;
-  if (qlinear_num_splits(K, N, M) != 1) return TMX_ERR_UNSUPPORTED;
+  if (a_t && (r > 64 || Rpad <= 0 || Rpad % 32 || Rpad > TMX_MAX_RPAD)) return TMX_ERR_SHAPE;
+  const int KT = K / 64;
+  if (nsplit < 1 || nsplit > TMX_MAX_SPLITS || !slices_ok(KT, nsplit)) return TMX_ERR_SHAPE;
   if ((size_t)256 * ldx * 2 >= (1u << 31) || (size_t)K * N / 2 >= (1u << 31) || (size_t)K * Rpad * 2 >= (1u << 31))
     return TMX_ERR_SHAPE;
-  const int KT = K / 64;
   QLinearArgs a = {};
   a.fixed_slice = -1;
   a.ldy = N;
@@ -1791,29 +1794,34 @@ int qlinear_wide_lora(hipStream_t st, const void* x, int ldx, const void* qw, co
   a.ldx = ldx;
   a.qw = (const uint4*)qw;
   a.scales = (const uint16_t*)scales;
-  a.a_t = (const uint16_t*)a_t;
-  a.y_bf16 = (uint16_t*)y_bf16;
-  a.t_part = t_part;
-  a.ldt = TMX_MAX_RPAD;
+  a.y_bf16 = nsplit == 1 ? (uint16_t*)y_bf16 : nullptr;
+  a.y_part = y_part;
   a.M = M; a.K = K; a.N = N; a.G = G; a.Rpad = Rpad;
-  a.nsplit = 1;
-  a.kt_per_split = slice_len(KT, 1);
-  const int nls = qlinear_num_lora_splits(K, N);
-  a.lora_blocks_per_split = nls;
-  a.kt_per_lora_split = lora_slice_len(K, N);
+  a.nsplit = nsplit;
+  a.kt_per_split = slice_len(KT, nsplit);
   if (a_t) {
-    if (a.kt_per_lora_split % 2) return TMX_ERR_UNSUPPORTED;
-    int rc = qwide_launch(st, a, 1);
-    if (rc != TMX_OK) return rc;
-    if ((rc = lora_t_reduce(st, t_part, nls, M, t16, Rpad)) != TMX_OK) return rc;
-    a.t16 = t16;
-    a.ldt16 = TMX_MAX_RPAD;
-    a.lora_b = (const uint16_t*)lora_b;
-    a.lora_r = r;
-    a.lora_ls = ls;
-    for (int i = 0; i < 3; ++i) a.seg_end[i] = seg_end ? seg_end[i] : N;
+    a.a_t = (const uint16_t*)a_t;
+    a.t_part = w.t_part;
+    a.ldt = TMX_MAX_RPAD;
+    // K-slices of 32 k-tiles: 2 for 4096 rows of W, 7 for 14336; a wave then has 4 to 16 k-tiles
+    const int n = KT / 32 < 1 ? 1 : (KT / 32 > 8 ? 8 : KT / 32);
+    a.kt_per_lora_split = (KT + n - 1) / n;
+    a.n_lora_slices = (KT + a.kt_per_lora_split - 1) / a.kt_per_lora_split;
+    a.sync = w.sync;
+    a.sync_clear = w.sync_clear;
+    a.sync_status = w.status;
+    if (*fused) {
+      a.t16 = w.t16;
+      a.ldt16 = TMX_MAX_RPAD;
+      a.lora_b = (const uint16_t*)lora_b;
+      a.lora_r = r;
+      a.lora_ls = ls;
+      for (int i = 0; i < 3; ++i) a.seg_end[i] = seg_end ? seg_end[i] : N;
+    } else {
+      a.t_fin = w.t_fin;
+    }
   }
-  return qwide_launch(st, a, 2);
+  return qwide_launch(st, a);
 }
 
 // ---------------------------------------------------------------------------
@@ -1886,9 +1894,9 @@ extern "C" int tmx_int4_dequant(void* stream, const void* qweight, const void* s
 
 extern "C" size_t tmx_qlora_linear_workspace_bytes(int M, int K, int N) {
   const size_t s = qlinear_num_splits(K, N, M);
-  // f32 K-slice planes, f32 LoRA planes, bf16 LoRA projection (many rows)
+  // f32 K-slice planes, f32 LoRA planes; many rows: bf16 LoRA projection and its hand-over areas
   return (s * (size_t)M * N + (size_t)TMX_MAX_LORA_SPLITS * M * TMX_MAX_RPAD) * sizeof(float) +
-         (size_t)M * TMX_MAX_RPAD * 2;
+         (M > 128 ? (size_t)M * TMX_MAX_RPAD * 2 + 2 * wide_sync_words() * 4 : 0);
 }
 
 extern "C" int tmx_qlora_linear_num_splits(int M, int K, int N) { return qlinear_num_splits(K, N, M); }
@@ -1952,13 +1960,21 @@ extern "C" int tmx_qlora_linear(void* stream, const void* x, const void* qweight
   const int ns = qlinear_num_splits(K, N, M);
   float* y_part = (float*)workspace;
   float* t_part = y_part + (size_t)ns * M * N;
-  if (M > 128 && !residual && ns == 1) {
+  if (M > 128 && M <= TMX_MAX_FILL_ROWS && !residual && ns == 1 && (!lora || (r % 8 == 0 && r <= 64))) {
     // many rows, unsplit: LoRA in the projection's epilogue
-    uint16_t* t16 = (uint16_t*)(t_part + (size_t)TMX_MAX_LORA_SPLITS * M * TMX_MAX_RPAD);
+    WideLora w = {};
+    w.t_part = t_part;
+    w.t16 = (uint16_t*)(t_part + (size_t)TMX_MAX_LORA_SPLITS * M * TMX_MAX_RPAD);
+    if (lora) {
+      w.sync = (uint32_t*)(w.t16 + (size_t)M * TMX_MAX_RPAD);
+      w.sync_clear = w.sync + wide_sync_words();
+      const int zrc = zero_words(st, w.sync, (int)wide_sync_words());
+      if (zrc != TMX_OK) return zrc;
+    }
     const int seg_end[3] = {N, N, N};
-    const int rc = qlinear_wide_lora(st, x, K, qweight, scales, lora ? lora_a_t : nullptr, lora_b, r, lora_scale,
-                                     seg_end, y, t_part, t16, M, K, N, G, r_pad);
-    if (rc != TMX_ERR_UNSUPPORTED) return rc;
+    bool fused = false;
+    return qlinear_wide(st, x, K, qweight, scales, lora ? lora_a_t : nullptr, lora_b, r, lora_scale, seg_end, y, nullptr,
+                        w, M, K, N, G, r_pad, 1, &fused);
   }
   int rc = qlinear_base(st, x, K, qweight, scales, lora ? lora_a_t : nullptr, nullptr, y_part, t_part,
                         TMX_MAX_RPAD, M, K, N, G, r_pad, ns);

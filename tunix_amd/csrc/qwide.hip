@@ -11,20 +11,21 @@ namespace tmx {
 // two buffers: slab rows are 256 bytes (four per 1 KiB transfer), their 16-byte chunks XOR-swizzled by row % 16.  With
 // KW = 2 a wave takes one k-tile of every step, and the two halves of a column tile meet through LDS at the end.
 constexpr int kWideTS = 2, kWideXS = 128;
+constexpr int kWideTiles32 = TMX_MAX_FILL_ROWS / 32;  // words per kind in a hand-over area: arrivals | ready flags
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 // the MFMA of a group behind which part p (1..4) of the next fragment's dequantisation goes
 constexpr int wide_slot(int MT, int p) { return p < MT ? p : MT - 1; }
 constexpr size_t wide_lds(int MT) { return (size_t)2 * MT * 32 * kWideXS * 2; }
 
-template <int MT, int CT, bool LORA>
-__device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* smem, int bx, int by, int bz) {
+template <int MT, int CT>
+__device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* smem, int bx, int slice, int bz) {
   constexpr int TS = kWideTS, XS = kWideXS, ROWS = MT * 32, KW = 8 / CT, TPW = TS / KW;
   static_assert(KW * CT == 8 && TPW >= 1, "8 waves, at least one k-tile of a step each");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ct = wave % CT, kw = wave / CT;
   const int h = lane >> 5, nl = lane & 31;
   const int KT = a.K >> 6;
-  const int slice = LORA ? (bx - a.n_main_blocks) + a.lora_blocks_per_split * by : by;
-  const int per = LORA ? a.kt_per_lora_split : a.kt_per_split;
+  const int per = a.kt_per_split;
   const int kb0 = slice * per;
   const int kb1 = (kb0 + per < KT) ? kb0 + per : KT;
   const int nsteps = (kb1 - kb0) / TS, last_step = nsteps - 1;  // host: whole steps
@@ -32,16 +33,13 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
   const int row0 = bz * ROWS;
   const int rows = a.M - row0 < ROWS ? a.M - row0 : ROWS;  // host: >= 1
   const int gs = __builtin_ctz(a.G >> 6), KG = a.K / a.G;
-  const int NT = LORA ? (a.Rpad >> 5) : (a.N >> 5);
-  const int nb = LORA ? ct : bx * CT + ct;
+  const int NT = a.N >> 5, nb = bx * CT + ct;
   const bool tile_ok = nb < NT;  // waves past the last tile only help with the slab
 
-  const __amdgpu_buffer_rsrc_t rw =
-      LORA ? make_rsrc(a.a_t, (uint32_t)KT * NT * 4096u) : make_rsrc(a.qw, (uint32_t)NT * KT * 1024u);
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.scales, LORA ? 0u : (uint32_t)NT * KG * 64u);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.qw, (uint32_t)NT * KT * 1024u);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.scales, (uint32_t)NT * KG * 64u);
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x + (size_t)row0 * a.ldx, (uint32_t)rows * a.ldx * 2u);
-  const int wv = LORA ? nb * 4096 + lane * 16 : (nb * KT * 64 + lane) * 16;
-  const int wstep = LORA ? NT * 4096 : 1024;  // bytes between consecutive k-tiles
+  const int wv = (nb * KT * 64 + lane) * 16;
   const int sv = (nb * KG * 32 + nl) * 2;
   // slab transfer: MT loads per wave and step; load i moves rows 4 wave + 32 i .. + 3 (16 lanes
   // each), lane l delivering chunk (l % 16) ^ (row % 16) of the step to slot l % 16
@@ -57,17 +55,15 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
-  constexpr int WPT = LORA ? 4 : 1;  // 16-byte words per lane and tile
-  u32x4_t wring[TPW][WPT];
+  u32x4_t wring[TPW];
   uint16_t sring[TPW];
 
   auto load_w_tile = [&](int step, auto jc) __attribute__((always_inline)) {
     constexpr int j = decltype(jc)::value;
     step = step < last_step ? step : last_step;
     const int kt = kb0 + step * TS + kw * TPW + j;
-#pragma unroll
-    for (int t = 0; t < WPT; ++t) wring[j][t] = __builtin_amdgcn_raw_buffer_load_b128(rw, wv + t * 1024, kt * wstep, 0);
-    if (!LORA) sring[j] = __builtin_amdgcn_raw_buffer_load_b16(rs, sv, (kt >> gs) * 64, 0);
+    wring[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, wv, kt * 1024, 0);
+    sring[j] = __builtin_amdgcn_raw_buffer_load_b16(rs, sv, (kt >> gs) * 64, 0);
   };
   auto dma_x = [&](int step, int buf) __attribute__((always_inline)) {
     step = step < last_step ? step : last_step;
@@ -81,13 +77,12 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
   // weight fragment a quarter at a time, so the matrix pipe waits neither for LDS nor for the
   // VALU, also when both waves of a SIMD run in phase after a barrier.  The order is pinned.
   auto step_math = [&](int step, int buf) __attribute__((always_inline)) {
-    u32x4_t wc[TPW][WPT];
+    u32x4_t wc[TPW];
     float s_c[TPW], m8s[TPW];
     static_for<TPW>([&](auto jc) __attribute__((always_inline)) {
       constexpr int j = decltype(jc)::value;
-#pragma unroll
-      for (int t = 0; t < WPT; ++t) wc[j][t] = wring[j][t];
-      s_c[j] = LORA ? 0.f : bf2f(sring[j]);
+      wc[j] = wring[j];
+      s_c[j] = bf2f(sring[j]);
       m8s[j] = -8.f * s_c[j];
       load_w_tile(step + 1, jc);  // registers consumed: refill them one step ahead
     });
@@ -95,7 +90,7 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
     const int c0 = 8 * TPW * kw + h;  // this wave's first chunk of a slab row
     auto word_of = [&](auto gc) __attribute__((always_inline)) {
       constexpr int g = decltype(gc)::value, j = g / 4, t = g % 4;
-      return t == 0 ? wc[j][0].x : (t == 1 ? wc[j][0].y : (t == 2 ? wc[j][0].z : wc[j][0].w));
+      return t == 0 ? wc[j].x : (t == 1 ? wc[j].y : (t == 2 ? wc[j].z : wc[j].w));
     };
     bf16x8_t xq[2][MT];
     u32x4_t bq[2];
@@ -103,14 +98,13 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
       const int slot = (c0 ^ (nl & 15)) * 8;
 #pragma unroll
       for (int m = 0; m < MT; ++m) xq[0][m] = *reinterpret_cast<const bf16x8_t*>(xb + m * 32 * XS + slot);
-      if (LORA) bq[0] = wc[0][0];
-      else bq[0] = __builtin_bit_cast(u32x4_t, dequant_word(word_of(IC<0>{}), s_c[0], m8s[0]));
+      bq[0] = __builtin_bit_cast(u32x4_t, dequant_word(word_of(IC<0>{}), s_c[0], m8s[0]));
     }
     __builtin_amdgcn_sched_barrier(0);
     static_for<4 * TPW>([&](auto gc) __attribute__((always_inline)) {
       constexpr int g = decltype(gc)::value, cur = g & 1, nxt = cur ^ 1;
       constexpr bool more = g + 1 < 4 * TPW;
-      constexpr int jn = (g + 1) / 4 % TPW, tn = (g + 1) % 4;
+      constexpr int jn = (g + 1) / 4 % TPW;
       const int slot = ((c0 + 2 * (g + 1)) ^ (nl & 15)) * 8;
       uint32_t lo = 0, hi = 0;
       static_for<MT>([&](auto mc) __attribute__((always_inline)) {
@@ -119,22 +113,18 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
                                                          0, 0, 0);
         if constexpr (more) {
           xq[nxt][m] = *reinterpret_cast<const bf16x8_t*>(xb + m * 32 * XS + slot);
-          if (LORA) {
-            if (m == 0) bq[nxt] = wc[jn][tn % WPT];
-          } else {
-            if (m == 0) dequant_masks(word_of(IC<g + 1>{}), lo, hi);
-            if (m == wide_slot(MT, 1)) bq[nxt].x = dequant_part<0>(lo, hi, s_c[jn], m8s[jn]);
-            if (m == wide_slot(MT, 2)) bq[nxt].y = dequant_part<1>(lo, hi, s_c[jn], m8s[jn]);
-            if (m == wide_slot(MT, 3)) bq[nxt].z = dequant_part<2>(lo, hi, s_c[jn], m8s[jn]);
-            if (m == wide_slot(MT, 4)) bq[nxt].w = dequant_part<3>(lo, hi, s_c[jn], m8s[jn]);
-          }
+          if (m == 0) dequant_masks(word_of(IC<g + 1>{}), lo, hi);
+          if (m == wide_slot(MT, 1)) bq[nxt].x = dequant_part<0>(lo, hi, s_c[jn], m8s[jn]);
+          if (m == wide_slot(MT, 2)) bq[nxt].y = dequant_part<1>(lo, hi, s_c[jn], m8s[jn]);
+          if (m == wide_slot(MT, 3)) bq[nxt].z = dequant_part<2>(lo, hi, s_c[jn], m8s[jn]);
+          if (m == wide_slot(MT, 4)) bq[nxt].w = dequant_part<3>(lo, hi, s_c[jn], m8s[jn]);
           __builtin_amdgcn_sched_barrier(0);
         }
       });
     });
   };
   // loads of a step younger than its slab transfer (in-order counter)
-  constexpr int kYounger = TPW * (LORA ? 4 : 2);
+  constexpr int kYounger = TPW * 2;
   auto wait_slab = [&]() __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
     if (tile_ok) __builtin_amdgcn_s_waitcnt(0x0F70 | (kYounger & 15) | ((kYounger >> 4) << 14));
@@ -180,9 +170,31 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
         }
     }
   }
+  bool t_ready = true;
+  if (a.t16) {
+    // t of this block's rows comes from the LoRA workgroups of the launch: wait (a bounded number of polls) for the
+    // flags of its row tiles
+    __shared__ uint32_t s_late;
+    if (tid == 0) s_late = 0u;
+    __syncthreads();
+    if (tid < MT && row0 + tid * 32 < a.M) {
+      uint32_t* flag = a.sync + kWideTiles32 + (row0 >> 5) + tid;
+      uint32_t ok = 0;
+      for (int spin = 0; spin < (1 << 20); ++spin) {
+        if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) { ok = 1; break; }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      if (!ok) {
+        s_late = 1u;
+        if (a.sync_status) __hip_atomic_store(a.sync_status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __syncthreads();
+    t_ready = s_late == 0u;  // false: t is taken as zero (the status word says so)
+  }
   if (!tile_ok) return;
   const int col = nb * 32 + nl;
-  if (!LORA && a.t16) {
+  if (a.t16) {
     // LoRA in the epilogue: delta tile [32 rows, 32 columns] = t16 rows . B columns, 16 ranks per
     // MFMA (t rows are the A operand, so the delta lands in the accumulator layout of acc[m]);
     // y = bf16(bf16(base) + bf16(bf16(delta) ls))
@@ -203,18 +215,21 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
       }
       bfr[kb] = u32x4_t{w[0], w[1], w[2], w[3]};
     }
+    const __amdgpu_buffer_rsrc_t rt = make_rsrc(a.t16, (uint32_t)a.M * a.ldt16 * 2u);
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const int trow = row0 + m * 32 + nl;
-      const uint16_t* tp = a.t16 + (size_t)(trow < a.M ? trow : a.M - 1) * a.ldt16 + tc0 + 8 * h;
+      const int tp = ((trow < a.M ? trow : a.M - 1) * a.ldt16 + tc0 + 8 * h) * 2;
       f32x16_t d;
 #pragma unroll
       for (int r = 0; r < 16; ++r) d[r] = 0.f;
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb)
         if (kb < nkb) {
-          const bf16x8_t tf = *reinterpret_cast<const bf16x8_t*>(tp + kb * 16);
-          d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tf, __builtin_bit_cast(bf16x8_t, bfr[kb]), d, 0, 0, 0);
+          // past this XCD's L2: the rows were written during this launch
+          u32x4_t tf = {0u, 0u, 0u, 0u};
+          if (t_ready) tf = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rt, tp + kb * 32, 0, 0x10));
+          d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, tf), __builtin_bit_cast(bf16x8_t, bfr[kb]), d, 0, 0, 0);
         }
 #pragma unroll
       for (int i = 0; i < NR; ++i) {
@@ -233,10 +248,121 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
       const int row = row0 + m * 32 + acc_row(rbase + i, lane);
       if (row >= a.M) continue;
       const float v = acc[m][i];
-      if (LORA) a.t_part[((size_t)slice * a.M + row) * a.ldt + col] = v;
-      else if (a.y_bf16) a.y_bf16[(size_t)row * a.ldy + col] = f2bf(v);
+      if (a.y_bf16) a.y_bf16[(size_t)row * a.ldy + col] = f2bf(v);
       else a.y_part[((size_t)slice * a.M + row) * a.N + col] = v;
     }
+}
+
+// t = x . A of one row tile (32 rows) over one K-slice.  The 8 waves are column tiles of A (1, 2 or 4) x k-parts; a wave
+// reads its x fragments straight from global memory (32 rows, 64 bytes each per pair of loads; the column tiles of a
+// k-part hit the same lines) two k-tiles ahead, the parts meet in LDS.  Every slice leaves its f32 plane; with a
+// hand-over area (a.sync) the last slice of the row tile to arrive adds the planes in slice order and writes the
+// rounded t: bf16 for the epilogues of this launch (a.t16, then its ready flag), f32 for a consumer behind it
+// (a.t_fin).  Stores are write-through and loads go past L2 (sc1), so no cache write-back happens inside the
+// launch.  These workgroups come first in dispatch order and wait for nobody.  What bounds them is latency: about 8 us
+// at 256 rows, hidden behind the main workgroups' loop, where a LoRA-only launch and a reduction launch in front of the
+// projection took 14 + 5 us (decode step of 256 sequences, 8 layers: 3.43 -> 3.25 ms).
+__device__ __forceinline__ void wide_lora_block(const QLinearArgs& a, float* red, int id) {
+  const int RT = (a.M + 31) >> 5, rt = id % RT, ks = id / RT;
+  if (ks >= a.n_lora_slices) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, nl = lane & 31;
+  const int KT = a.K >> 6, NT = a.Rpad >> 5, NP = NT > 2 ? 4 : NT, nk = 8 / NP;
+  const int ct = wave % NP, kp = wave / NP;
+  const int k0 = ks * a.kt_per_lora_split, k1 = min(k0 + a.kt_per_lora_split, KT);
+  if (a.sync_clear && ks == 0 && tid < 2) a.sync_clear[tid * kWideTiles32 + rt] = 0u;  // the next launch's area
+
+  f32x16_t acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  if (ct < NT) {
+    const int row = min(rt * 32 + nl, a.M - 1);
+    const u32x4_t* xp = reinterpret_cast<const u32x4_t*>(a.x + (size_t)row * a.ldx) + h;
+    const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + (size_t)ct * 256 + lane;
+    u32x4_t xr[2][4], ar[2][4];
+    auto load = [&](int kt, auto pc) __attribute__((always_inline)) {
+      constexpr int p = decltype(pc)::value;
+      kt = kt < k1 ? kt : k1 - 1;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        xr[p][t] = xp[kt * 8 + 2 * t];
+        ar[p][t] = ap[((size_t)kt * NT) * 256 + t * 64];
+      }
+    };
+    auto math = [&](auto pc) __attribute__((always_inline)) {
+      constexpr int p = decltype(pc)::value;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, xr[p][t]),
+                                                      __builtin_bit_cast(bf16x8_t, ar[p][t]), acc, 0, 0, 0);
+    };
+    int kt = k0 + kp;
+    if (kt < k1) {
+      load(kt, IC<0>{});
+      load(kt + nk, IC<1>{});
+      for (; kt < k1; kt += 2 * nk) {
+        math(IC<0>{});
+        load(kt + 2 * nk, IC<0>{});
+        if (kt + nk < k1) math(IC<1>{});
+        load(kt + 3 * nk, IC<1>{});
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) red[(wave * 16 + r) * 64 + lane] = acc[r];
+  __syncthreads();
+  // thread: four adjacent columns of a row
+  const int quads = a.Rpad >> 2;
+  const __amdgpu_buffer_rsrc_t rp = make_rsrc(a.t_part, 0x7FFFFFFFu);
+  const bool final_here = a.sync != nullptr;
+  auto finish = [&](int row, int c, f32x4_t v) __attribute__((always_inline)) {
+    const uint32_t lo = pack_bf2(v[0], v[1]), hi = pack_bf2(v[2], v[3]);
+    if (a.t16)
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{lo, hi}, make_rsrc(a.t16, (uint32_t)a.M * a.ldt16 * 2u),
+                                            (row * a.ldt16 + c) * 2, 0, 0x10);
+    if (a.t_fin) *reinterpret_cast<f32x4_t*>(a.t_fin + (size_t)row * a.ldt + c) = f32x4_t{bf_lo(lo), bf_hi(lo), bf_lo(hi), bf_hi(hi)};
+  };
+  for (int e = tid; e < 32 * quads; e += 512) {
+    const int rl = e / quads, c = (e - rl * quads) * 4, row = rt * 32 + rl;
+    if (row >= a.M) continue;
+    const int r = (rl >> 3) * 4 + (rl & 3), ln = ((rl >> 2) & 1) * 32 + (c & 31);
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < nk; ++p) v += *reinterpret_cast<const f32x4_t*>(red + ((p * NP + (c >> 5)) * 16 + r) * 64 + ln);
+    if (final_here && a.n_lora_slices == 1) finish(row, c, v);
+    else if (!final_here) *reinterpret_cast<f32x4_t*>(a.t_part + ((size_t)ks * a.M + row) * a.ldt + c) = v;
+    else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), rp, (int)((((size_t)ks * a.M + row) * a.ldt + c) * 4), 0, 0x10);
+  }
+  if (!final_here) return;
+  __builtin_amdgcn_s_waitcnt(0);  // this thread's stores are in memory
+  __syncthreads();
+  if (a.n_lora_slices > 1) {
+    __shared__ uint32_t s_last;
+    if (tid == 0)
+      s_last = __hip_atomic_fetch_add(a.sync + rt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(a.n_lora_slices - 1);
+    __syncthreads();
+    if (!s_last) return;
+    for (int e = tid; e < 32 * quads; e += 512) {
+      const int rl = e / quads, c = (e - rl * quads) * 4, row = rt * 32 + rl;
+      if (row >= a.M) continue;
+      f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+      for (int p0 = 0; p0 < a.n_lora_slices; p0 += 8) {
+        u32x4_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int p = min(p0 + u, a.n_lora_slices - 1);
+          v[u] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rp, (int)((((size_t)p * a.M + row) * a.ldt + c) * 4), 0, 0x10));
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (p0 + u < a.n_lora_slices) t += __builtin_bit_cast(f32x4_t, v[u]);
+      }
+      finish(row, c, t);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  }
+  if (tid == 0) __hip_atomic_store(a.sync + kWideTiles32 + rt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (linear id % 8), each with its own L2.
@@ -247,7 +373,11 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
 template <int MT, int CT>
 __global__ __launch_bounds__(512, MT <= 4 && CT == 4 ? 4 : 1) void qlinear_mfma_wide_kernel(QLinearArgs a, int blocks, int row_blocks, int S) {
   extern __shared__ __align__(16) uint16_t smem[];
-  const int id = (int)blockIdx.x, xcd = id & 7, idx = id >> 3;
+  if ((int)blockIdx.x < a.lora_wgs) {
+    wide_lora_block(a, reinterpret_cast<float*>(smem), (int)blockIdx.x);
+    return;
+  }
+  const int id = (int)blockIdx.x - a.lora_wgs, xcd = id & 7, idx = id >> 3;  // host: lora_wgs % 8 == 0
   const int per_rb = blocks * a.nsplit;
   const int p = xcd / S + (8 / S) * idx;
   // an XCD with an even number of row blocks takes them two at a time, the same column block on both in
@@ -257,43 +387,24 @@ __global__ __launch_bounds__(512, MT <= 4 && CT == 4 ? 4 : 1) void qlinear_mfma_
   const int bz = xcd % S + S * (blk * Gr + within % Gr);
   if (bz >= row_blocks) return;
   const int cb = within / Gr, bx = cb % blocks, by = cb / blocks;
-  if (bx >= a.n_main_blocks) gemm_block_wide<MT, CT, true>(a, smem, bx, by, bz);
-  else gemm_block_wide<MT, CT, false>(a, smem, bx, by, bz);
-}
-
-// t16[m][c] = bf16(sum of the planes' values) for c < cols, 0 up to the row stride ldt
-__global__ __launch_bounds__(256) void lora_t_reduce_kernel(const float* t_part, int nsplit, int M, int ldt,
-                                                            uint16_t* t16, int cols) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= M * ldt) return;
-  const int m = i / ldt, c = i - m * ldt;
-  float t = 0.f;
-  if (c < cols)
-    for (int sp = 0; sp < nsplit; ++sp) t += t_part[((size_t)sp * M + m) * ldt + c];
-  t16[(size_t)m * ldt + c] = f2bf(t);
-}
-
-int lora_t_reduce(hipStream_t st, const float* t_part, int nsplit, int M, uint16_t* t16, int cols) {
-  hipLaunchKernelGGL(lora_t_reduce_kernel, dim3((M * TMX_MAX_RPAD + 255) / 256), dim3(256), 0, st, t_part, nsplit, M,
-                     TMX_MAX_RPAD, t16, cols);
-  return check_launch();
+  gemm_block_wide<MT, CT>(a, smem, bx, by, bz);
 }
 
 template <int MT, int CT>
-static int launch_wide(hipStream_t st, QLinearArgs a, int part) {
+static int launch_wide(hipStream_t st, QLinearArgs a) {
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void*>(&qlinear_mfma_wide_kernel<MT, CT>), hipFuncAttributeMaxDynamicSharedMemorySize,
       (int)wide_lds(MT));
   if (attr != hipSuccess) return TMX_ERR_LAUNCH;
-  a.n_main_blocks = part == 1 ? 0 : (a.N + CT * 32 - 1) / (CT * 32);
-  const int blocks = a.n_main_blocks + ((a.a_t && part != 2) ? a.lora_blocks_per_split : 0);
+  const int blocks = (a.N + CT * 32 - 1) / (CT * 32);
+  a.lora_wgs = a.a_t ? ((a.M + 31) / 32 * a.n_lora_slices + 7) / 8 * 8 : 0;
   const int row_blocks = (a.M + MT * 32 - 1) / (MT * 32);
   int S = 8;
   while (row_blocks % S) S >>= 1;  // gcd(row_blocks, 8)
   // ids cover 8 / S XCDs x (row_blocks / S) row blocks x blocks x nsplit per residue, rounded up to 8
   const long total = (long)blocks * a.nsplit * row_blocks;
   const int ids = (int)((total + 7) / 8 * 8);
-  hipLaunchKernelGGL((qlinear_mfma_wide_kernel<MT, CT>), dim3(ids), dim3(512), wide_lds(MT), st, a, blocks, row_blocks, S);
+  hipLaunchKernelGGL((qlinear_mfma_wide_kernel<MT, CT>), dim3(a.lora_wgs + ids), dim3(512), wide_lds(MT), st, a, blocks, row_blocks, S);
   return check_launch();
 }
 
@@ -326,11 +437,11 @@ WidePlan wide_plan(int M, int N, int K, int nsplit) {
   return best;
 }
 
-// part: 0 = main blocks and LoRA blocks in one launch, 1 = LoRA blocks only, 2 = main blocks only
-int qwide_launch(hipStream_t st, const QLinearArgs& a, int part) {
-  const WidePlan p = part == 1 ? WidePlan{8, 8, 1} : wide_plan(a.M, a.N, a.K, a.nsplit);
+int qwide_launch(hipStream_t st, const QLinearArgs& a) {
+  if (a.sync && a.M > TMX_MAX_FILL_ROWS) return TMX_ERR_SHAPE;  // the hand-over area has a word per row tile
+  const WidePlan p = wide_plan(a.M, a.N, a.K, a.nsplit);
 #define TMX_WIDE_CASE(MM, CC) \
-  if (p.mt == MM && p.ct == CC) return launch_wide<MM, CC>(st, a, part);
+  if (p.mt == MM && p.ct == CC) return launch_wide<MM, CC>(st, a);
   TMX_WIDE_CASE(2, 4)
   TMX_WIDE_CASE(3, 4)
   TMX_WIDE_CASE(4, 4)

@@ -27,9 +27,9 @@ struct QLinearArgs {
   const uint16_t* lora_b;  // [lora_r][N] bf16
   int lora_r;
   float lora_ls;
-  // LoRA inside the epilogue of the many-rows kernel: t16 = bf16(x . A) [M][ldt16] computed beforehand;
+  // LoRA inside the epilogue of the many-rows kernel: t16 = bf16(x . A) [M][ldt16], made by its LoRA workgroups;
   // a column below seg_end[s] (and not below seg_end[s - 1]) uses t columns s lora_r .. s lora_r + lora_r - 1
-  const uint16_t* t16;
+  uint16_t* t16;
   int ldt16;
   int seg_end[3];
   // LoRA projection computed once per launch by extra workgroups and handed over through memory
@@ -45,6 +45,11 @@ struct QLinearArgs {
   // to the rounded sum of the planes instead of multiplying by B itself
   uint16_t* delta;
   int n_lora_slices;       // slices that hold k-tiles (the launch may have a few more LoRA blocks)
+  // many-rows kernel: LoRA workgroups in front of the launch; the hand-over area of the next launch, which they
+  // clear; the finished t in f32 for a consumer behind the launch [M][ldt]
+  int lora_wgs;
+  uint32_t* sync_clear;
+  float* t_fin;
 };
 
 // What qlinear_base needs to let the LoRA blocks produce the delta (all or nothing).
@@ -315,15 +320,25 @@ inline bool slices_ok(int KT, int s) { return (KT + slice_len(KT, s) - 1) / slic
 // Projections of more than 128 rows (qwide.hip): mt row tiles x ct column tiles per workgroup, K in nsplit slices
 struct WidePlan { int mt, ct, nsplit; };
 WidePlan wide_plan(int M, int N, int K, int nsplit);  // nsplit 0: its choice
-int qwide_launch(hipStream_t st, const QLinearArgs& a, int part);
-int lora_t_reduce(hipStream_t st, const float* t_part, int nsplit, int M, uint16_t* t16, int cols);
-// Many rows (M > 128), unsplit: y_bf16 = bf16(bf16(x . W) + bf16(bf16(t . B) ls)) in one pass, t = bf16(x . A)
-// computed by a LoRA-only launch of the same kernel and a small reduction (t_part: f32 planes, t16: bf16
-// [M][TMX_MAX_RPAD] scratch).  seg_end: column ends of the fused matrices (q | k | v, gate | up), unused
-// entries = N.  TMX_ERR_UNSUPPORTED when the shape needs K-slices or the rank is not a multiple of 8.
-int qlinear_wide_lora(hipStream_t st, const void* x, int ldx, const void* qw, const void* scales, const void* a_t,
-                      const void* lora_b, int r, float ls, const int* seg_end, void* y_bf16, float* t_part,
-                      uint16_t* t16, int M, int K, int N, int G, int Rpad);
+int qwide_launch(hipStream_t st, const QLinearArgs& a);
+// What the LoRA half of a many-rows projection hands over inside its launch.  Two areas of wide_sync_words() words take
+// turns: a launch uses one, which has to be zero, and clears the other.
+struct WideLora {
+  float* t_part;       // [TMX_MAX_LORA_SPLITS][M][TMX_MAX_RPAD] f32 planes
+  uint16_t* t16;       // [M][TMX_MAX_RPAD] bf16
+  float* t_fin;        // [M][TMX_MAX_RPAD] f32
+  uint32_t* sync;      // this launch's area
+  uint32_t* sync_clear;
+  uint32_t* status;    // set to 1 when a wait runs out (may be null)
+};
+inline size_t wide_sync_words() { return 2 * (TMX_MAX_FILL_ROWS / 32); }
+// Many rows (M > 128), LoRA included: t = bf16(x . A) by the LoRA workgroups of the launch.  With nsplit == 1 and
+// r % 8 == 0 also y_bf16 = bf16(bf16(x . W) + bf16(bf16(t . B) ls)) (returns with *fused = true); else the f32 planes
+// y_part (bf16 y_bf16 with one slice) and, with LoRA, t in w.t_fin for the consumer.  seg_end: column ends of the fused
+// matrices (q | k | v, gate | up), unused entries = N.
+int qlinear_wide(hipStream_t st, const void* x, int ldx, const void* qw, const void* scales, const void* a_t,
+                 const void* lora_b, int r, float ls, const int* seg_end, void* y_bf16, float* y_part, const WideLora& w,
+                 int M, int K, int N, int G, int Rpad, int nsplit, bool* fused);
 int qlinear_base(hipStream_t st, const void* x, int ldx, const void* qw, const void* scales,
                  const void* a_t, void* y_bf16, float* y_part, float* t_part, int ldt, int M, int K,
                  int N, int G, int Rpad, int nsplit, const LoraDelta* ld = nullptr);
