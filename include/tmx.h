@@ -426,6 +426,16 @@ size_t tmx_decode_workspace_bytes(const tmx_model_desc* model, int batch, int ca
 int tmx_decode_steps(const tmx_model_desc* model, const tmx_decode_state* state, void* stream,
                      int n_steps, int sample);
 
+/* One cache-fill pass that leaves out the padding in front of left-padded prompts: the columns *step .. *step + width - 1
+ * of every sequence, of sequence s only those from first_col[s] on (device array, [batch]), as n_rows rows in all
+ * (n_rows = the caller's count of them, <= TMX_MAX_FILL_ROWS and whatever bounds the rows of tmx_decode_steps; a
+ * workspace of tmx_decode_workspace_bytes(model, n_rows, cache_size)).  *step advances by width.  The reference computes
+ * the padding and masks it (tunix/generate/utils.py:35-59): no later token looks at the cache slots left out, which stay
+ * as they are.  state->tokens_per_pass is ignored.  TMX_ERR_UNSUPPORTED for head shapes the block attention does not
+ * serve (head_dim 64 with 8 query heads per kv head, and others). */
+int tmx_fill_ragged(const tmx_model_desc* model, const tmx_decode_state* state, void* stream, const int32_t* first_col,
+                    int width, int n_rows);
+
 /* Some decode kernels hand data from one group of workgroups to another inside a launch (the
  * fused gate | up projection computes its LoRA projection once and passes it on).  The
  * receiving side waits a bounded number of polls; if a wait ever runs out the kernel carries

@@ -733,3 +733,39 @@ def test_hf_checkpoint_loader_to_gpu_logits_match_oracle(tmp_path, family):
     assert np.abs(want).max() > 0.1  # the comparison is not between two all-zero tensors
     tok = ref['state'].token_buffer[:, 12 + step]
     st['token_buffer'][:, 12 + step] = torch.from_numpy(tok).to(st['token_buffer'].device)  # teacher forcing
+
+
+# prompt lengths of a left-padded batch: nothing to leave out, one token, more padding than a pass is wide, rows on both
+# sides of the many-rows kernels' threshold, more sequences than one round of the row planner
+@pytest.mark.parametrize('lengths', [(9, 9, 9), (1, 40, 2, 33), (5, 40), (40, 7, 39, 40, 28, 40, 1, 16), tuple(1 + i % 3 for i in range(1500))])
+def test_cache_fill_leaves_out_padding(lengths):
+  """The ragged cache fill writes the cache rows of the real tokens that a walk one token at a time writes, and the
+  next step's logits agree (tunix/generate/utils.py:35-59 masks the padding)."""
+  cfg = C.TOY
+  model = C.product_model(cfg, C.make_state(cfg, 43, 8, norm_jitter=0.05), 64, 16.0)
+  rng = np.random.default_rng(len(lengths))
+  b, p = len(lengths), max(lengths)
+  ids = np.zeros((b, p), np.int32)
+  for i, n in enumerate(lengths):
+    ids[i, p - n:] = rng.integers(3, cfg.vocab_size, n)
+  s = _sampler(model, cfg, p + 8)
+  s.share_prompt_kv = False
+  s.eos_ids = np.array([-1])
+  new = lambda: s.init_sample_state(ids, p + 4, True, None, 0.0, None, None, 0, include_logprobs=True)
+  st = new()
+  for _ in range(p - 1):
+    s.run_steps(st, 1, sample=False)
+  want = st['cache'].float().cpu().numpy().copy()
+  s.run_steps(st, 1)
+  want_logits = st['logits'].cpu().numpy().copy()
+  for limit in ([4096] if b > 1000 else [4096, 64]):  # one pass, or several
+    s.MAX_ROWS = s.MAX_FILL_ROWS = limit
+    st = new()
+    s.walk(st, p - 1)
+    assert int(st['step'].item()) == p - 1
+    got = st['cache'].float().cpu().numpy().copy()
+    s.run_steps(st, 1)
+    for i, n in enumerate(lengths):
+      d = np.abs(got[:, :, i, p - n:p - 1] - want[:, :, i, p - n:p - 1])
+      assert not d.size or d.max() <= 2.0 ** -6 * max(1.0, np.abs(want).max())
+    assert np.abs(st['logits'].cpu().numpy() - want_logits).max() <= LOGIT_TOL

@@ -583,17 +583,26 @@ __global__ __launch_bounds__(256) void gqa_fill_kernel(AttnArgs a) {
   constexpr int HT = H / 32;        // hidden tiles of the output
   constexpr int TPW = 32 / G, TQ = 4 * TPW;  // tokens per wave / workgroup
   __shared__ __align__(16) uint16_t kt[2][32 * H], vt[2][32 * H];
-  const int kvh = blockIdx.x, seq = blockIdx.y, tblk = blockIdx.z;
+  const int kvh = blockIdx.x, tblk = blockIdx.z;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = lane >> 5, qi = lane & 31;
-  const int T = a.tpp, step0 = max(min(*a.step, min(a.C, a.buf_len) - T), 0);  // clamped: every slot read lies in the cache
+  int seq = blockIdx.y, row_base = blockIdx.y * a.tpp, T = a.tpp, col0 = a.seg ? 0 : *a.step;
+  if (a.seg) {  // ragged pass: the sequence's own rows
+    const int4 g = a.seg[blockIdx.y];
+    seq = __builtin_amdgcn_readfirstlane(g.x);
+    row_base = __builtin_amdgcn_readfirstlane(g.y);
+    T = __builtin_amdgcn_readfirstlane(g.z);
+    col0 = __builtin_amdgcn_readfirstlane(g.w);
+    if (tblk * TQ >= T) return;
+  }
+  const int step0 = max(min(col0, min(a.C, a.buf_len) - T), 0);  // clamped: every slot read lies in the cache
   const int tok = tblk * TQ + wave * TPW + qi / G, g = qi % G;
   const int tok_l = tok < T ? tok : T - 1;
   const int limit = step0 + tok_l;  // newest slot this query sees
   const int last_tok = tblk * TQ + TQ - 1 < T - 1 ? tblk * TQ + TQ - 1 : T - 1;
   const int nblk = (step0 + last_tok + 32) >> 5;  // blocks of 32 positions up to the newest slot of the block
 
-  const size_t qoff = ((size_t)(seq * T + tok_l) * a.N + kvh * G + g) * H;
+  const size_t qoff = ((size_t)(row_base + tok_l) * a.N + kvh * G + g) * H;
   u32x4_t qf[KS];
 #pragma unroll
   for (int t = 0; t < KS; ++t) qf[t] = *reinterpret_cast<const u32x4_t*>(a.q + qoff + (H / 2) * h + 8 * t);
@@ -731,8 +740,9 @@ __global__ __launch_bounds__(256) void gqa_fill_kernel(AttnArgs a) {
 
 template <int H, int G>
 static int launch_fill(hipStream_t st, const AttnArgs& a) {
-  const int nseq = a.B / a.tpp, tq = 4 * (32 / G);
-  hipLaunchKernelGGL((gqa_fill_kernel<H, G>), dim3(a.Kh, nseq, (a.tpp + tq - 1) / tq), dim3(256), 0, st, a);
+  const int tq = 4 * (32 / G);
+  const int nseq = a.seg ? a.n_seg : a.B / a.tpp, width = a.seg ? a.seg_width : a.tpp;
+  hipLaunchKernelGGL((gqa_fill_kernel<H, G>), dim3(a.Kh, nseq, (width + tq - 1) / tq), dim3(256), 0, st, a);
   return check_launch();
 }
 
@@ -853,10 +863,15 @@ static int launch_tile(hipStream_t st, const AttnArgs& a, bool rows_on_tile) {
   return check_launch();
 }
 
+bool attn_fill_ok(int N, int Kh, int H, int C) {
+  const int G = Kh > 0 && N % Kh == 0 ? N / Kh : 0;
+  return (H == 64 || H == 128) && (G == 1 || G == 2 || G == 4 || (G == 8 && H == 128)) && (size_t)C * Kh * H * 2 < (1u << 31);
+}
+
 int gqa_decode(hipStream_t st, AttnArgs a, int H) {
   const int G = a.N / a.Kh;
   if (a.N % a.Kh) return TMX_ERR_SHAPE;
-  if (a.tpp <= 1) {
+  if (a.tpp <= 1 && !a.seg) {
     const AttnPlan p = plan_attention(a.B, a.N, a.Kh, H, a.C, a.share_gs, a.share_len);
     if (p.tile || p.shared) {
       a.nsplit = p.nsplit;
@@ -880,7 +895,7 @@ int gqa_decode(hipStream_t st, AttnArgs a, int H) {
   a.share_gs = a.share_len = a.psplits = 0;
   if (a.nsplit > 1 && !a.partial) return TMX_ERR_ARG;
   // several tokens per sequence: one walk over the cache for a block of them (MFMA kernel)
-  if (a.tpp >= kFillMinTokens && a.B % a.tpp == 0 && (size_t)a.C * a.Kh * H * 2 < (1u << 31)) {
+  if ((a.seg || (a.tpp >= kFillMinTokens && a.B % a.tpp == 0)) && (size_t)a.C * a.Kh * H * 2 < (1u << 31)) {
 #define TMX_FILL_CASE(HH, GG) \
   if (H == HH && G == GG) return launch_fill<HH, GG>(st, a);
     TMX_FILL_CASE(64, 1)
@@ -892,6 +907,7 @@ int gqa_decode(hipStream_t st, AttnArgs a, int H) {
     TMX_FILL_CASE(128, 8)
 #undef TMX_FILL_CASE
   }
+  if (a.seg) return TMX_ERR_UNSUPPORTED;
 #define TMX_ATTN_CASE(HH, GG) \
   if (H == HH && G == GG) return launch_attn<HH, GG>(st, a);
   TMX_ATTN_CASE(64, 1)

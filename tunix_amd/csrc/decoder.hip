@@ -34,6 +34,8 @@ struct Workspace {
   int32_t* expert_of;
   float* weight_of;
   uint16_t *pair_act, *pair_y;
+  int2* row_map;  // ragged pass: row -> (sequence, column), and the sequences' runs of rows
+  int4* seg;
   size_t total;
 };
 
@@ -133,6 +135,8 @@ static Workspace carve(const tmx_model_desc* m, int B, int C, char* base) {
   w.weight_of = (float*)take(P * 4);
   w.pair_act = (uint16_t*)take(P * F * 2);
   w.pair_y = (uint16_t*)take(P * D * 2);
+  w.row_map = (int2*)take((size_t)B * 8);
+  w.seg = (int4*)take((size_t)B * 16);
   w.total = off;
   return w;
 }
@@ -166,8 +170,15 @@ extern "C" size_t tmx_decode_workspace_bytes(const tmx_model_desc* m, int batch,
   return carve(m, batch, cache_size, nullptr).total;
 }
 
+// A cache-fill pass that leaves out the padding in front of the prompts: `width` columns of every sequence, of each
+// only those from first_col on, n_rows rows in all.
+struct Ragged {
+  const int32_t* first_col;
+  int width, n_rows;
+};
+
 static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s, void* stream,
-                             int n_steps, int sample, Prof* prof) {
+                             int n_steps, int sample, Prof* prof, const Ragged* rg = nullptr) {
   if (!m || !s || !m->layers || !m->embed || !m->final_norm_w || !m->head) return TMX_ERR_ARG;
   if (!s->token_buffer || !s->positions || !s->input_mask || !s->done || !s->step || !s->kv_cache ||
       !s->workspace)
@@ -175,14 +186,14 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
   const bool moe = m->num_experts > 0;
   // rows of a pass: one per sequence, or tokens_per_pass consecutive tokens of every sequence
   // (cache fill and scoring only: sampling needs the previous token)
-  const int NSEQ = s->batch, T = s->tokens_per_pass > 1 ? s->tokens_per_pass : 1;
-  if (NSEQ <= 0 || NSEQ > TMX_MAX_FILL_ROWS || T > 128) return TMX_ERR_SHAPE;
+  const int NSEQ = s->batch, T = rg ? rg->width : (s->tokens_per_pass > 1 ? s->tokens_per_pass : 1);
+  if (NSEQ <= 0 || NSEQ > TMX_MAX_FILL_ROWS || (!rg && T > TMX_MAX_FILL_ROWS / NSEQ)) return TMX_ERR_SHAPE;
   if (T > 1 && sample && s->sampling_mode != TMX_SAMPLE_SCORE) return TMX_ERR_ARG;
-  const int B = NSEQ * T, C = s->cache_size, L = s->buf_len;
+  const int B = rg ? rg->n_rows : NSEQ * T, C = s->cache_size, L = s->buf_len;
   // a pass takes up to TMX_MAX_FILL_ROWS rows; above 128 rows the projections multiply in 256-row
   // blocks (every K % 128 == 0), the head takes its rows 64 at a time or in 256 x 256 blocks; MoE models
   // are bounded by the routed pairs per pass (checked below)
-  if (B > TMX_MAX_FILL_ROWS || C <= 0 || L <= 0 || L > C) return TMX_ERR_SHAPE;
+  if (B <= 0 || B > TMX_MAX_FILL_ROWS || C <= 0 || L <= 0 || L > C) return TMX_ERR_SHAPE;
   if (moe && (m->experts_per_tok <= 0 || m->experts_per_tok > m->num_experts ||
               (size_t)B * m->experts_per_tok > TMX_MAX_MOE_PAIRS))
     return TMX_ERR_SHAPE;
@@ -216,7 +227,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
   }
 
   const Splits sp = plan_splits(m, B);
-  const bool small = small_batch_ok(m, B, T);
+  const bool small = !rg && small_batch_ok(m, B, T);
   auto lora_of = [&](const tmx_qlinear_desc& l, int) {
     LoraIn li = {};
     if (l.lora_a_t) {
@@ -266,12 +277,16 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
     if (rc != TMX_OK) return rc;
   }
   // samples of one prompt in consecutive rows: decode attention reads the prompt slots once per group
-  const bool share_walk = T == 1 && !small && w.attn_partial && attn_share_ok(B, N, Kh, H, C, s->share_group, s->share_len);
+  const bool share_walk = T == 1 && !rg && !small && w.attn_partial && attn_share_ok(B, N, Kh, H, C, s->share_group, s->share_len);
   for (int it = 0; it < n_steps; ++it) {
     if (w.wide_sync) {  // both areas start a step at zero, whichever the last launch of the step before used
       rc = zero_words(st, w.wide_sync, 2 * (int)wide_sync_words());
       if (rc != TMX_OK) return rc;
       wide_turn = 0;
+    }
+    if (rg) {
+      rc = plan_rows(st, rg->first_col, s->step, NSEQ, rg->width, B, L, w.row_map, w.seg);
+      if (rc != TMX_OK) return rc;
     }
     {  // embedding gather + first input norm + this step's RoPE table
       RowNormArgs a = {};
@@ -281,6 +296,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       a.step = s->step;
       a.buf_len = L;
       a.tpp = T;
+      if (rg) a.row_map = w.row_map;
       a.positions = s->positions;
       a.rope_tab = w.rope_tab;
       a.half = H / 2;
@@ -396,6 +412,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
         a.q_norm_w = (const uint16_t*)l.q_norm_w;
         a.k_norm_w = (const uint16_t*)l.k_norm_w;
         a.positions = s->positions; a.step = s->step; a.buf_len = L; a.tpp = T;
+        if (rg) a.row_map = w.row_map;
         a.rope_tab = w.rope_tab;
         a.q_out = w.q; a.kcache = kc; a.vcache = vc;
         a.N = N; a.Kh = Kh; a.H = H; a.C = C;
@@ -406,6 +423,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
         AttnArgs a = {};
         a.q = w.q; a.kcache = kc; a.vcache = vc;
         a.input_mask = s->input_mask; a.step = s->step; a.buf_len = L; a.tpp = T;
+        if (rg) { a.seg = w.seg; a.n_seg = NSEQ < B ? NSEQ : B; a.seg_width = T; }
         a.out = w.attn; a.partial = w.attn_partial;
         a.B = B; a.N = N; a.Kh = Kh; a.C = C;
         a.scale = 1.0f / sqrtf((float)H);
@@ -588,6 +606,15 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
 extern "C" int tmx_decode_steps(const tmx_model_desc* m, const tmx_decode_state* s, void* stream,
                                 int n_steps, int sample) {
   return decode_steps_impl(m, s, stream, n_steps, sample, nullptr);
+}
+
+extern "C" int tmx_fill_ragged(const tmx_model_desc* m, const tmx_decode_state* s, void* stream, const int32_t* first_col,
+                               int width, int n_rows) {
+  if (!m || !s || !first_col) return TMX_ERR_ARG;
+  if (width <= 0 || n_rows <= 0 || s->batch <= 0 || (long)n_rows > (long)width * s->batch) return TMX_ERR_SHAPE;
+  if (m->num_kv_heads <= 0 || !attn_fill_ok(m->num_heads, m->num_kv_heads, m->head_dim, s->cache_size)) return TMX_ERR_UNSUPPORTED;
+  const Ragged rg = {first_col, width, n_rows};
+  return decode_steps_impl(m, s, stream, 1, 0, nullptr, &rg);
 }
 
 extern "C" int tmx_decode_status(const tmx_model_desc* m, const tmx_decode_state* s, void* stream) {

@@ -181,7 +181,8 @@ __global__ __launch_bounds__(512) void row_norm_kernel(RowNormArgs a) {
     const int tpp = a.tpp > 0 ? a.tpp : 1;
     // column and id are clamped into range like the reference's gathers (jnp indexing clamps), so a
     // caller that oversteps the buffer or feeds an id outside the vocabulary reads a valid row
-    const int seq = m / tpp, step = min(*a.step + m % tpp, a.buf_len - 1);
+    const int2 at = a.row_map ? a.row_map[m] : make_int2(m / tpp, *a.step + m % tpp);
+    const int seq = at.x, step = min(at.y, a.buf_len - 1);
     int tok = a.token_buffer[(size_t)seq * a.buf_len + step];
     if (a.vocab > 0) tok = min(max(tok, 0), a.vocab - 1);
     src = a.embed + (size_t)tok * a.D;
@@ -381,7 +382,8 @@ __global__ __launch_bounds__(64) void rope_kvwrite_kernel(RopeArgs a) {
   const int head = blockIdx.x, b = blockIdx.y, B = gridDim.y, lane = threadIdx.x;
   const int half = a.H >> 1;
   const int tpp = a.tpp > 0 ? a.tpp : 1;
-  const int seq = b / tpp, step = min(*a.step + b % tpp, a.buf_len - 1);  // b: row of this pass (column clamped into the buffer)
+  const int2 at = a.row_map ? a.row_map[b] : make_int2(b / tpp, *a.step + b % tpp);  // b: row of this pass
+  const int seq = at.x, step = min(at.y, a.buf_len - 1);  // (column clamped into the buffer)
   const bool active = lane < half;
   const int ntot = (a.N + 2 * a.Kh) * a.H;
   const int kind = head < a.N ? 0 : (head < a.N + a.Kh ? 1 : 2);  // q, k, v
@@ -593,6 +595,63 @@ __global__ void advance_step_kernel(int32_t* step, int by) { *step += by; }
 
 int advance_step(hipStream_t st, int32_t* step, int by) {
   hipLaunchKernelGGL(advance_step_kernel, dim3(1), dim3(1), 0, st, step, by);
+  return check_launch();
+}
+
+// One workgroup: the sequences' row counts, their running sum (1024 sequences at a time), then the rows themselves by
+// binary search.  A few microseconds per pass of thousands of rows, instead of a copy from the host.
+constexpr int kPlanThreads = 1024;
+__global__ __launch_bounds__(kPlanThreads) void plan_rows_kernel(const int32_t* first_col, const int32_t* step, int batch,
+                                                                 int width, int n_rows, int buf_len, int2* row_map,
+                                                                 int4* seg, int n_seg) {
+  __shared__ int wave_n[16], wave_e[16];
+  __shared__ int e_row[TMX_MAX_FILL_ROWS];   // first row of every entry
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int c0 = min(max(*step, 0), buf_len - 1), c1 = min(c0 + width, buf_len);
+  int rows = 0, entries = 0;
+  for (int s0 = 0; s0 < batch; s0 += kPlanThreads) {
+    const int s = s0 + tid;
+    const int first = s < batch ? max(first_col[s], c0) : c1;
+    const int n = max(c1 - first, 0);
+    int pn = n, pe = n > 0 ? 1 : 0;  // inclusive sums over the wave
+    for (int o = 1; o < 64; o <<= 1) {
+      const int an = __shfl_up(pn, o, 64), ae = __shfl_up(pe, o, 64);
+      if (lane >= o) { pn += an; pe += ae; }
+    }
+    if (lane == 63) { wave_n[wave] = pn; wave_e[wave] = pe; }
+    __syncthreads();
+    int row0 = rows + pn - n, e = entries + pe - 1;
+    for (int w = 0; w < wave; ++w) { row0 += wave_n[w]; e += wave_e[w]; }
+    // (a caller whose n_rows is short of the real count gets its first rows)
+    if (n > 0 && row0 < n_rows && e < n_seg) {
+      seg[e] = make_int4(s, row0, min(n, n_rows - row0), first);
+      e_row[e] = row0;
+    }
+    for (int w = 0; w < 16; ++w) { rows += wave_n[w]; entries += wave_e[w]; }
+    __syncthreads();
+  }
+  entries = min(entries, n_seg);
+  for (int e = entries + tid; e < n_seg; e += kPlanThreads) seg[e] = make_int4(0, 0, 0, 0);
+  __threadfence_block();
+  __syncthreads();
+  for (int m = tid; m < n_rows; m += kPlanThreads) {
+    if (entries == 0) { row_map[m] = make_int2(0, c0); continue; }
+    int lo = 0, hi = entries;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (m >= e_row[mid]) lo = mid;
+      else hi = mid;
+    }
+    const int4 g = seg[lo];
+    row_map[m] = make_int2(g.x, g.w + min(m - g.y, g.z - 1));  // rows past the count repeat the last one
+  }
+}
+
+int plan_rows(hipStream_t st, const int32_t* first_col, const int32_t* step, int batch, int width, int n_rows,
+              int buf_len, int2* row_map, int4* seg) {
+  if (batch <= 0 || width <= 0 || n_rows <= 0 || n_rows > TMX_MAX_FILL_ROWS || buf_len <= 0) return TMX_ERR_SHAPE;
+  hipLaunchKernelGGL(plan_rows_kernel, dim3(1), dim3(kPlanThreads), 0, st, first_col, step, batch, width, n_rows, buf_len,
+                     row_map, seg, batch < n_rows ? batch : n_rows);
   return check_launch();
 }
 

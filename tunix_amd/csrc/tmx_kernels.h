@@ -105,6 +105,7 @@ struct RowNormArgs {
   const int32_t* step;          // device scalar: column of token_buffer to read
   int buf_len;
   int tpp;                      // tokens per pass: row m is sequence m / tpp at column *step + m % tpp (0: 1)
+  const int2* row_map;          // ragged pass: (sequence, column) of row m, replaces step and tpp (null: none)
   const int32_t* positions;     // [B, L] (embedding mode: fills rope_tab)
   float* rope_tab;              // [B][half][2] sin, cos of this step (may be null)
   int half;
@@ -138,6 +139,7 @@ struct RopeArgs {
   const int32_t* step;
   int buf_len;
   int tpp;                   // tokens per pass (0: 1): row m is sequence m / tpp at slot *step + m % tpp
+  const int2* row_map;       // ragged pass: (sequence, column) of row m, replaces step and tpp (null: none)
   const float* rope_tab;     // [B][H/2][2] or null (then sin/cos are computed here)
   uint16_t* q_out;           // [B, N * H]
   uint16_t* kcache;          // [B, C, Kh, H]
@@ -168,6 +170,10 @@ struct AttnArgs {
   int B, N, Kh, C, nsplit, chunk;
   float scale;
   int tpp;  // tokens per pass (0: 1): query row m belongs to sequence m / tpp and sees slots <= *step + m % tpp
+  // Ragged pass (null: none): entry e = (sequence, first row, rows, first column): rows first .. first + rows - 1 are
+  // consecutive tokens of the sequence.  n_seg entries (empty ones have 0 rows), none of more than seg_width rows.
+  const int4* seg;
+  int n_seg, seg_width;
   // Shared prompt slots (G samples of one prompt in consecutive rows): share_gs > 1 says that the sequences
   // come in consecutive groups of share_gs whose cache slots [0, share_len) and input_mask entries are
   // identical.  Those slots are then walked once per group (gqa_prefix_kernel, psplits splits, from the
@@ -284,8 +290,13 @@ int row_norm(hipStream_t st, const RowNormArgs& a, int M);
 int rope_kvwrite(hipStream_t st, const RopeArgs& a, int B);
 int swiglu(hipStream_t st, const SwigluArgs& a, int M);
 int advance_step(hipStream_t st, int32_t* step, int by);
+// Rows of a ragged pass over columns *step .. *step + width - 1: those from first_col[s] on, sequence by sequence.
+// row_map [n_rows], seg [min(batch, n_rows)] (see AttnArgs); n_rows is the caller's count of those rows.
+int plan_rows(hipStream_t st, const int32_t* first_col, const int32_t* step, int batch, int width, int n_rows,
+              int buf_len, int2* row_map, int4* seg);
 int empty_launch(hipStream_t st);  // measurement aid: a kernel that does nothing
 int gqa_decode(hipStream_t st, AttnArgs a, int H);
+bool attn_fill_ok(int N, int Kh, int H, int C);  // shapes of the kernel that serves ragged passes
 size_t attn_partial_bytes(int B, int N, int Kh, int H, int C);
 // the same when the rows may share prompt slots (AttnArgs::share_gs > 1): room for the prefix partials too
 size_t attn_shared_partial_bytes(int B, int N, int Kh, int H, int C);
