@@ -356,6 +356,58 @@ __global__ __launch_bounds__(512) void row_norm_kernel(RowNormArgs a) {
   }
 }
 
+// The same for a row that is finished (bf16, no LoRA left, no planes): what is bound by memory then, and the kernel above
+// holds the registers of its other sources (2 workgroups per CU).  256 threads, up to 16 chunks of 8 per row and thread
+// pair, 8 workgroups per CU: 4096 rows of 4096 values (134 MB in and out) 44 -> 29 us.
+template <int CPT>  // 8-element chunks per thread, D <= 2048 * CPT
+__global__ __launch_bounds__(256) void row_norm_plain_kernel(RowNormArgs a) {
+  __shared__ float smem[4];
+  const size_t base = (size_t)blockIdx.x * a.D;
+  const int nchunks = a.D >> 3;
+  uint4 y4[CPT], r4[CPT], w4[CPT];
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int c = threadIdx.x + 256 * i, n0 = (c < nchunks ? c : 0) * 8;
+    y4[i] = *reinterpret_cast<const uint4*>(a.y_bf16 + base + n0);
+    if (a.residual) r4[i] = *reinterpret_cast<const uint4*>(a.residual + base + n0);
+    if (a.norm_w) w4[i] = *reinterpret_cast<const uint4*>(a.norm_w + n0);
+  }
+  float v[CPT][8], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    unpack8(y4[i], v[i]);
+    if (a.residual) {
+      float r8[8];
+      unpack8(r4[i], r8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] = rbf(v[i][e] + r8[e]);
+    }
+    if (c < nchunks) {
+      if (a.x_out) *reinterpret_cast<uint4*>(a.x_out + base + c * 8) = pack8(v[i]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss += v[i][e] * v[i][e];
+    }
+  }
+  if (!a.norm_w) return;
+  ss = block_sum<4>(ss, smem);
+  const float rms = sqrtf(ss / (float)a.D + a.eps);
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    if (c < nchunks) {
+      float w[8], o[8];
+      unpack8(w4[i], w);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (a.family == TMX_FAMILY_LLAMA3) o[e] = rbf(w[e] * v[i][e]) / rms;
+        else o[e] = w[e] * (v[i][e] / rms);
+      }
+      *reinterpret_cast<uint4*>(a.xn_out + base + c * 8) = pack8(o);
+    }
+  }
+}
+
 int row_norm(hipStream_t st, const RowNormArgs& a, int M) {
   if (a.D <= 0 || a.D % 8 || a.D > 4096 * 4) return TMX_ERR_SHAPE;
   if (a.lora.t_part && a.lora.r > TMX_MAX_RPAD) return TMX_ERR_SHAPE;
@@ -367,6 +419,13 @@ int row_norm(hipStream_t st, const RowNormArgs& a, int M) {
     if (r.E <= 0 || r.E % 8 || r.top_k <= 0 || r.top_k > 64 || r.top_k > r.E) return TMX_ERR_SHAPE;
     lds = moe_router_lds_floats(a.D, r.E) * sizeof(float);
     if (lds > 60000) return TMX_ERR_SHAPE;
+  }
+  // (few rows leave most CUs one workgroup each: the wider one finishes sooner)
+  if (M > 128 && a.y_bf16 && !a.embed && !a.lora.t_part && !a.delta && !a.moe_y && !a.router.w && a.D <= 8192) {
+    if (a.D <= 2048) hipLaunchKernelGGL(row_norm_plain_kernel<1>, dim3(M), dim3(256), 0, st, a);
+    else if (a.D <= 4096) hipLaunchKernelGGL(row_norm_plain_kernel<2>, dim3(M), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(row_norm_plain_kernel<4>, dim3(M), dim3(256), 0, st, a);
+    return check_launch();
   }
   const int cpt = (a.D / 8 + 511) / 512;
   if (cpt <= 1) hipLaunchKernelGGL(row_norm_kernel<1>, dim3(M), dim3(512), lds, st, a);
@@ -460,9 +519,145 @@ __global__ __launch_bounds__(64) void rope_kvwrite_kernel(RopeArgs a) {
   }
 }
 
+// The same for head_dim 64 and 128 with 16-byte pieces of a head instead of single elements: H / 8 lanes own a head, a
+// lane the elements 4 i .. 4 i + 3 and their partners H / 2 further on; a workgroup of 256 takes 2048 / H heads of a
+// row.  One wave per head made a launch of (N + 2 Kh) B workgroups with 2-byte loads: 256 rows of 48 heads 13.4 us, 64
+// rows 6.2 us, of which the dispatch of the workgroups was most.  Every value is made by the same operations in the
+// same order.
+__device__ __forceinline__ void unpack4(const uint2& v, float* o) {
+  o[0] = bf_lo(v.x); o[1] = bf_hi(v.x); o[2] = bf_lo(v.y); o[3] = bf_hi(v.y);
+}
+template <int H>
+__global__ __launch_bounds__(256) void rope_heads_kernel(RopeArgs a) {
+  constexpr int LPH = H / 8, HPW = 256 / LPH, half = H / 2;
+  __shared__ float t_s[TMX_MAX_RPAD];
+  __shared__ float t_stage[TMX_MAX_LORA_SPLITS * 64];
+  const int b = blockIdx.y, B = gridDim.y;
+  const int lane = threadIdx.x & (LPH - 1), nheads = a.N + 2 * a.Kh;
+  const int head = blockIdx.x * HPW + threadIdx.x / LPH, hd = min(head, nheads - 1);
+  const int tpp = a.tpp > 0 ? a.tpp : 1;
+  const int2 at = a.row_map ? a.row_map[b] : make_int2(b / tpp, *a.step + b % tpp);
+  const int seq = at.x, step = min(at.y, a.buf_len - 1);
+  const int ntot = nheads * H;
+  const int kind = hd < a.N ? 0 : (hd < a.N + a.Kh ? 1 : 2);  // q, k, v
+  const int c1 = hd * H + lane * 4, c2 = c1 + half;
+  const bool lora = a.lora.t_part != nullptr;
+  float x1[4], x2[4];
+  if (a.qkv_bf16) {
+    unpack4(*reinterpret_cast<const uint2*>(a.qkv_bf16 + (size_t)b * ntot + c1), x1);
+    unpack4(*reinterpret_cast<const uint2*>(a.qkv_bf16 + (size_t)b * ntot + c2), x2);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x1[e] = x2[e] = 0.f;
+    const float* p = a.qkv_part + (size_t)b * ntot;
+    const size_t stride = (size_t)B * ntot;
+    for (int s0 = 0; s0 < a.nsplit; s0 += 4) {  // four planes in flight, added in ascending order
+      float4 u[4], w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float* q = p + (size_t)min(s0 + i, a.nsplit - 1) * stride;
+        u[i] = *reinterpret_cast<const float4*>(q + c1);
+        w[i] = *reinterpret_cast<const float4*>(q + c2);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (s0 + i < a.nsplit) {
+          x1[0] += u[i].x; x1[1] += u[i].y; x1[2] += u[i].z; x1[3] += u[i].w;
+          x2[0] += w[i].x; x2[1] += w[i].y; x2[2] += w[i].z; x2[3] += w[i].w;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { x1[e] = rbf(x1[e]); x2[e] = rbf(x2[e]); }
+  }
+  if (lora) {
+    // t of all three segments (a workgroup's heads may lie in several)
+    if (3 * a.lora.r * a.lora.nsplit <= TMX_MAX_LORA_SPLITS * 64) {
+      stage_t_block(t_s, t_stage, a.lora, b, B, 0, 3 * a.lora.r);
+    } else {
+      stage_t(t_s, a.lora, b, B, 0, 3 * a.lora.r);
+      __syncthreads();
+    }
+    float d1[4] = {0.f, 0.f, 0.f, 0.f}, d2[4] = {0.f, 0.f, 0.f, 0.f};
+    const float* t = t_s + kind * a.lora.r;
+#pragma unroll 8
+    for (int rr = 0; rr < a.lora.r; ++rr) {
+      float w1[4], w2[4];
+      unpack4(*reinterpret_cast<const uint2*>(a.lora.b + (size_t)rr * ntot + c1), w1);
+      unpack4(*reinterpret_cast<const uint2*>(a.lora.b + (size_t)rr * ntot + c2), w2);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        d1[e] = fmaf(t[rr], w1[e], d1[e]);
+        d2[e] = fmaf(t[rr], w2[e], d2[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x1[e] = rbf(x1[e] + rbf(rbf(d1[e]) * a.lora.ls));
+      x2[e] = rbf(x2[e] + rbf(rbf(d2[e]) * a.lora.ls));
+    }
+  }
+  const uint16_t* nw = kind == 0 ? a.q_norm_w : a.k_norm_w;
+  if (nw && a.q_norm_w && a.k_norm_w) {  // Qwen3 per-head RMSNorm, f32 with one cast (v lanes compute and drop it)
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss += x1[e] * x1[e] + x2[e] * x2[e];
+#pragma unroll
+    for (int o = 1; o < LPH; o <<= 1) ss += __shfl_xor(ss, o, 64);
+    const float rms = sqrtf(ss / (float)H + a.eps);
+    if (kind != 2) {
+      float n1[4], n2[4];
+      unpack4(*reinterpret_cast<const uint2*>(nw + lane * 4), n1);
+      unpack4(*reinterpret_cast<const uint2*>(nw + half + lane * 4), n2);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x1[e] = rbf(n1[e] * (x1[e] / rms));
+        x2[e] = rbf(n2[e] * (x2[e] / rms));
+      }
+    }
+  }
+  if (head >= nheads) return;
+  const int slot = step % a.C;
+  if (kind != 2) {
+    const float4* tab = reinterpret_cast<const float4*>(a.rope_tab + ((size_t)b * half + lane * 4) * 2);
+    const float4 t0 = tab[0], t1 = tab[1];
+    float sn[4] = {t0.x, t0.z, t1.x, t1.z}, cs[4] = {t0.y, t0.w, t1.y, t1.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float o1, o2;
+      if (a.family == TMX_FAMILY_LLAMA3) {
+        o1 = x1[e] * cs[e] - x2[e] * sn[e];
+        o2 = x2[e] * cs[e] + x1[e] * sn[e];
+      } else {
+        const float s = rbf(sn[e]), c = rbf(cs[e]);
+        o1 = rbf(x1[e] * c) - rbf(x2[e] * s);
+        o2 = rbf(x2[e] * c) + rbf(x1[e] * s);
+      }
+      x1[e] = o1;
+      x2[e] = o2;
+    }
+  }
+  uint16_t* dst;
+  if (kind == 0) dst = a.q_out + (size_t)b * a.N * H + head * H;
+  else if (kind == 1) dst = a.kcache + (((size_t)seq * a.C + slot) * a.Kh + (head - a.N)) * H;
+  else dst = a.vcache + (((size_t)seq * a.C + slot) * a.Kh + (head - a.N - a.Kh)) * H;
+  uint2 p;
+  p.x = pack_bf2(x1[0], x1[1]); p.y = pack_bf2(x1[2], x1[3]);
+  *reinterpret_cast<uint2*>(dst + lane * 4) = p;
+  p.x = pack_bf2(x2[0], x2[1]); p.y = pack_bf2(x2[2], x2[3]);
+  *reinterpret_cast<uint2*>(dst + half + lane * 4) = p;
+}
+
 int rope_kvwrite(hipStream_t st, const RopeArgs& a, int B) {
   if (a.H > 128 || a.H % 2) return TMX_ERR_SHAPE;
   if (a.lora.t_part && a.lora.r > 64) return TMX_ERR_SHAPE;
+  // the table comes from the row kernel of the pass; both head norms or none; t of the three segments in one row
+  if (a.rope_tab && (a.H == 64 || a.H == 128) && !a.q_norm_w == !a.k_norm_w && (!a.lora.t_part || 3 * a.lora.r <= TMX_MAX_RPAD)) {
+    const int hpw = 2048 / a.H;
+    const dim3 grid((a.N + 2 * a.Kh + hpw - 1) / hpw, B);
+    if (a.H == 128) hipLaunchKernelGGL(rope_heads_kernel<128>, grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(rope_heads_kernel<64>, grid, dim3(256), 0, st, a);
+    return check_launch();
+  }
   hipLaunchKernelGGL(rope_kvwrite_kernel, dim3(a.N + 2 * a.Kh, B), dim3(64), 0, st, a);
   return check_launch();
 }
@@ -513,7 +708,7 @@ __global__ __launch_bounds__(256) void swiglu_rows_kernel(SwigluArgs a, int M) {
   const int rows = M - m0 < kSwigluRows ? M - m0 : kSwigluRows;
   const int f0 = (blockIdx.x * 256 + threadIdx.x) * 8;
   const bool mine = f0 < a.F;
-  const int r = a.lora.t_part ? a.lora.r : 0;
+  const int r = a.lora.r;
   uint32_t pg[8][8], pu[8][8];  // [rank pair][column]: (B[2p][c], B[2p + 1][c])
   if (mine && r) {
 #pragma unroll
@@ -578,9 +773,30 @@ __global__ __launch_bounds__(256) void swiglu_rows_kernel(SwigluArgs a, int M) {
   }
 }
 
+// Finished gate | up rows (bf16, no LoRA left): elementwise, 8 hidden units per thread over all rows.
+__global__ __launch_bounds__(256) void swiglu_plain_kernel(SwigluArgs a, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x, per = a.F >> 3;
+  if (i >= n) return;
+  const int m = i / per, f0 = (i - m * per) * 8;
+  float g[8], u[8], o[8];
+  unpack8(*reinterpret_cast<const uint4*>(a.gu_bf16 + (size_t)m * 2 * a.F + f0), g);
+  unpack8(*reinterpret_cast<const uint4*>(a.gu_bf16 + (size_t)m * 2 * a.F + a.F + f0), u);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float sg = rbf(1.f / (1.f + expf(-g[e])));
+    o[e] = rbf(g[e] * sg) * u[e];
+  }
+  *reinterpret_cast<uint4*>(a.act + (size_t)m * a.F + f0) = pack8(o);
+}
+
 int swiglu(hipStream_t st, const SwigluArgs& a, int M) {
   if (a.F % 8 || (a.lora.t_part && 2 * a.lora.r > TMX_MAX_RPAD)) return TMX_ERR_SHAPE;
-  if (M > 128 && a.gu_bf16 && (!a.lora.t_part || a.lora.r <= 16)) {
+  if (a.gu_bf16 && !a.lora.t_part && (size_t)M * (a.F / 8) < (1u << 31)) {
+    const int n = M * (a.F / 8);
+    hipLaunchKernelGGL(swiglu_plain_kernel, dim3((n + 255) / 256), dim3(256), 0, st, a, n);
+    return check_launch();
+  }
+  if (M > 128 && a.gu_bf16 && a.lora.r <= 16) {
     hipLaunchKernelGGL(swiglu_rows_kernel, dim3((a.F + 2047) / 2048, (M + kSwigluRows - 1) / kSwigluRows), dim3(256),
                        0, st, a, M);
     return check_launch();
