@@ -988,6 +988,14 @@ def test_small_linear_matches_oracle(M, K, N, group, r, mode):
     G.assert_bf16_close(got, want, ulps=1.0, extra=extra, min_exact=0.99, what=f'small {mode} {M}x{K}x{N}')
 
 
+# 16 columns per workgroup: one pair of k-tiles for eight waves, waves without a pair, a ninth pair per wave, odd ranks
+@pytest.mark.parametrize('M,K,N,group,r,mode', [
+    (1, 128, 32, 64, 0, 'plain'), (4, 128, 96, 128, 5, 'residual'), (2, 1152, 64, 64, 1, 'norm'), (3, 1152, 32, 128, 32, 'plain'),
+    (3, 8320, 64, 64, 16, 'residual'), (1, 9216, 32, 256, 7, 'norm_qwen'), (4, 4096, 160, 64, 32, 'norm')])
+def test_small_linear_sixteen_columns(M, K, N, group, r, mode):
+  test_small_linear_matches_oracle(M, K, N, group, r, mode)
+
+
 def test_small_linear_rejects_what_it_cannot_take():
   lib = _lib.lib()
   one = torch.zeros(64, dtype=torch.uint8, device=G.DEV)

@@ -19,7 +19,8 @@
 // wave), every tile load of a wave is issued before the first use, dequantisation is the same
 // bit-exact bf16((u - 8) * s), and the product runs on v_mfma_f32_32x32x16_bf16 with the rows
 // beyond the batch ignored: at one row the VALU dequantisation, not the matrix pipe, is what a
-// tile costs.  A workgroup is 8 waves = column tiles x K-slices; the K-slices meet in LDS.
+// tile costs.  A workgroup is 8 waves = column tiles x K-slices; the K-slices meet in LDS.  (The projections without
+// SwiGLU take 16 columns per workgroup instead: sb_linear16_kernel.)
 #include "tmx_kernels.h"
 
 namespace tmx {
@@ -36,6 +37,206 @@ enum { SB_EPI_PLAIN = 0, SB_EPI_RESIDUAL = 1, SB_EPI_SWIGLU = 2 };
 __host__ __device__ inline size_t sb_x_bytes(int M, int K) { return ((size_t)M * (K + 8) * 2 + 15) & ~(size_t)15; }
 constexpr size_t kSbTailFloats = kSbWaves * kSbMaxRows * 32 + kSbWaves * kSbMaxRows * 64 + kSbMaxRows * 64 +
                                  kSbMaxRows * 32 + 4 + kSbWaves * 4;
+
+// t handed over as parts by the launch before: a thread adds a run of parts of four adjacent columns of a row (columns
+// 0 .. 4 nq - 1), in up to 32 runs; the runs meet in red_t [run][m][4 nq] and are added in run order.
+struct SbParts {
+  int nq, lanes, groups;  // groups 0: nothing handed over
+  f32x4_t pv[8];
+  __device__ __forceinline__ void load(const SbLinearArgs& a, int pb) {
+    const int rest = (int)threadIdx.x % lanes, m = rest / nq, c = (rest - m * nq) * 4;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      pv[u] = *reinterpret_cast<const f32x4_t*>(a.t_parts + ((size_t)min(pb + u, a.t_nparts - 1) * a.M + m) * 32 + c);
+  }
+  __device__ __forceinline__ void request(const SbLinearArgs& a) {
+    groups = 0;
+    if (!a.t_parts) return;
+    nq = (a.lora_r + 3) >> 2;
+    lanes = nq * a.M;
+    groups = min(kSbThreads / lanes, 32);
+    const int grp = (int)threadIdx.x / lanes;
+    if (grp < groups) load(a, grp * ((a.t_nparts + groups - 1) / groups));
+  }
+  __device__ __forceinline__ void finish(const SbLinearArgs& a, float* red_t) {
+    if (!groups) return;
+    const int grp = (int)threadIdx.x / lanes, rest = (int)threadIdx.x - grp * lanes;
+    if (grp >= groups) return;
+    const int run = (a.t_nparts + groups - 1) / groups;
+    const int b0 = grp * run, b1 = min(b0 + run, a.t_nparts);
+    f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+    for (int pb = b0; pb < b1; pb += 8) {
+      if (pb > b0) load(a, pb);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (pb + u < b1) t += pv[u];
+    }
+    *reinterpret_cast<f32x4_t*>(red_t + (grp * lanes + rest) * 4) = t;
+  }
+};
+__device__ __forceinline__ float sb_parts_total(const SbParts& p, const float* red_t, int m, int cc) {
+  if (cc >= p.nq * 4) return 0.f;
+  float t = 0.f;
+  for (int g = 0; g < p.groups; ++g) t += red_t[(g * p.lanes + m * p.nq) * 4 + cc];
+  return t;
+}
+__device__ __forceinline__ float sb_rms(const SbLinearArgs& a, const float* rms_s, int m) {
+  float t = 0.f;
+#pragma unroll
+  for (int w = 0; w < kSbWaves; ++w) t += rms_s[4 + w * 4 + m];
+  return sqrtf(t / (float)a.K + a.eps);
+}
+
+// The prologues: the activations of every row into LDS [M][XS] bf16, in two halves: request() before anything of the
+// launch is waited for, finish() afterwards.  Loads return in order, so a load requested behind a wait costs a whole
+// further round trip to memory.
+
+// merge of the context splits of the attention kernel: out = sum_s o_s exp(m_s - m) / sum_s l_s exp(m_s - m); a thread
+// owns four adjacent values of a head at a time, of up to 8 splits
+struct SbMerge {
+  f32x4_t po[8];
+  f32x2_t pm[8];
+  __device__ __forceinline__ void load(const SbLinearArgs& a, int e) {
+    const int H = a.attn_h, ns = a.attn_ns, G = a.attn_g, heads = a.attn_kh * G, per_row = heads * H / 4;
+    const float* ml = a.attn_part + (size_t)a.M * heads * ns * H;  // (max, sum) behind the outputs
+    if (e >= a.M * per_row) return;
+    const int m = e / per_row, rest = (e - m * per_row) * 4, head = rest / H, d = rest - head * H;
+    const size_t first = ((size_t)(m * a.attn_kh + head / G) * ns) * G + head % G;  // split 0 of this head; + G per split
+#pragma unroll
+    for (int sp = 0; sp < 8; ++sp)
+      if (sp < ns) {
+        const size_t i = first + (size_t)sp * G;
+        po[sp] = *reinterpret_cast<const f32x4_t*>(a.attn_part + i * H + d);
+        pm[sp] = *reinterpret_cast<const f32x2_t*>(ml + i * 2);
+      }
+  }
+  __device__ __forceinline__ void store(const SbLinearArgs& a, int e, uint16_t* xs, int XS) const {
+    const int ns = a.attn_ns, per_row = a.attn_kh * a.attn_g * a.attn_h / 4;
+    if (e >= a.M * per_row) return;
+    float mm = -1e30f;
+#pragma unroll
+    for (int sp = 0; sp < 8; ++sp)
+      if (sp < ns) mm = fmaxf(mm, pm[sp].x);
+    float ls = 0.f;
+    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int sp = 0; sp < 8; ++sp)
+      if (sp < ns) {
+        const float w = __expf(pm[sp].x - mm);
+        ls += pm[sp].y * w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] += po[sp][i] * w;
+      }
+    uint2 p = {0u, 0u};
+    if (ls > 0.f) {
+      p.x = pack_bf2(o[0] / ls, o[1] / ls);
+      p.y = pack_bf2(o[2] / ls, o[3] / ls);
+    }
+    const int m = e / per_row;
+    *reinterpret_cast<uint2*>(xs + m * XS + (e - m * per_row) * 4) = p;
+  }
+  __device__ __forceinline__ void request(const SbLinearArgs& a) { load(a, threadIdx.x); }
+  __device__ __forceinline__ void finish(const SbLinearArgs& a, uint16_t* xs, int XS, float*) {
+    const int items = a.M * a.attn_kh * a.attn_g * a.attn_h / 4;
+    store(a, threadIdx.x, xs, XS);
+    for (int e = (int)threadIdx.x + kSbThreads; e < items; e += 2 * kSbThreads) {  // more rows: two at a time
+      SbMerge second;
+      load(a, e);
+      second.load(a, e + kSbThreads);
+      store(a, e, xs, XS);
+      second.store(a, e + kSbThreads, xs, XS);
+    }
+  }
+};
+
+struct SbCopy {
+  uint4 v[8];  // host: at most 8 chunks per thread
+  __device__ __forceinline__ void request(const SbLinearArgs& a) {
+    const int cpr = a.K >> 3, nchunks = a.M * cpr;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int ch = (int)threadIdx.x + kSbThreads * i, m = ch / cpr;
+      if (ch < nchunks) v[i] = *reinterpret_cast<const uint4*>(a.x + (size_t)m * a.ldx + (ch - m * cpr) * 8);
+    }
+  }
+  __device__ __forceinline__ void finish(const SbLinearArgs& a, uint16_t* xs, int XS, float*) {
+    const int cpr = a.K >> 3, nchunks = a.M * cpr;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int ch = (int)threadIdx.x + kSbThreads * i, m = ch / cpr;
+      if (ch < nchunks) *reinterpret_cast<uint4*>(xs + m * XS + (ch - m * cpr) * 8) = v[i];
+    }
+  }
+};
+
+// RMSNorm of every row: up to 4 chunks of 8 elements per thread (M K <= 16384); rms_s: [4] + per-wave sums [8][4]
+struct SbNorm {
+  uint4 xq[4], wq[4];
+  __device__ __forceinline__ void request(const SbLinearArgs& a) {
+    const int cpr = a.K >> 3, nchunks = a.M * cpr;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ch = (int)threadIdx.x + kSbThreads * i, m = ch / cpr, cc = ch - m * cpr;
+      if (ch < nchunks) {
+        xq[i] = *reinterpret_cast<const uint4*>(a.x + (size_t)m * a.ldx + cc * 8);
+        wq[i] = *reinterpret_cast<const uint4*>(a.norm_w + cc * 8);
+      }
+    }
+  }
+  __device__ __forceinline__ void finish(const SbLinearArgs& a, uint16_t* xs, int XS, float* rms_s) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int cpr = a.K >> 3, nchunks = a.M * cpr;
+    auto unpack = [](const uint4& q, float (&v)[8]) __attribute__((always_inline)) {
+      v[0] = bf_lo(q.x); v[1] = bf_hi(q.x); v[2] = bf_lo(q.y); v[3] = bf_hi(q.y);
+      v[4] = bf_lo(q.z); v[5] = bf_hi(q.z); v[6] = bf_lo(q.w); v[7] = bf_hi(q.w);
+    };
+    float ss[kSbMaxRows] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ch = tid + kSbThreads * i;
+      if (ch < nchunks) {
+        const int m = ch / cpr;
+        float v[8], sq = 0.f;
+        unpack(xq[i], v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sq += v[e] * v[e];
+#pragma unroll
+        for (int r = 0; r < kSbMaxRows; ++r) ss[r] += (m == r) ? sq : 0.f;
+      }
+    }
+    // sum of squares of each row over the workgroup, in a fixed order
+#pragma unroll
+    for (int r = 0; r < kSbMaxRows; ++r)
+      if (r < a.M) ss[r] = wave_sum(ss[r]);
+    if (lane == 0) {
+#pragma unroll
+      for (int r = 0; r < kSbMaxRows; ++r) rms_s[4 + wave * 4 + r] = ss[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ch = tid + kSbThreads * i;
+      if (ch < nchunks) {
+        const int m = ch / cpr, cc = ch - m * cpr;
+        const float rms = sb_rms(a, rms_s, m);
+        float v[8], w[8], o[8];
+        unpack(xq[i], v);
+        unpack(wq[i], w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          o[e] = a.family == TMX_FAMILY_LLAMA3 ? rbf(w[e] * v[e]) / rms : w[e] * (v[e] / rms);
+        uint4 pk;
+        pk.x = pack_bf2(o[0], o[1]); pk.y = pack_bf2(o[2], o[3]);
+        pk.z = pack_bf2(o[4], o[5]); pk.w = pack_bf2(o[6], o[7]);
+        *reinterpret_cast<uint4*>(xs + m * XS + cc * 8) = pk;
+      }
+    }
+  }
+};
+
+template <int PRO> struct SbPrologue { using type = SbMerge; };
+template <> struct SbPrologue<SB_PRO_PLAIN> { using type = SbCopy; };
+template <> struct SbPrologue<SB_PRO_NORM> { using type = SbNorm; };
 
 template <int PRO, int EPI>
 __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
@@ -102,115 +303,15 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
       }
     }
   }
-  // t handed over by the previous launch as parts (down projection): thread (group, row, column) adds a
-  // contiguous run of parts, 16 loads in flight; the runs meet in LDS in run order
-  if (a.t_parts) {
-    const int lanes_per = 32 * M, groups = kSbThreads / lanes_per;
-    const int grp = tid / lanes_per, rest = tid - grp * lanes_per;
-    if (grp < groups) {
-      const int run = (a.t_nparts + groups - 1) / groups;
-      const int p0 = grp * run, p1 = min(p0 + run, a.t_nparts);
-      float t = 0.f;
-      for (int pb = p0; pb < p1; pb += 16) {
-        float pv[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) pv[u] = a.t_parts[(size_t)min(pb + u, a.t_nparts - 1) * lanes_per + rest];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) t += (pb + u < p1) ? pv[u] : 0.f;
-      }
-      red_t[grp * lanes_per + rest] = t;  // [group][m][32]
-    }
-  }
+  // parts of t and the rows: requested behind the weights (which come from farther), before anything is waited for
+  SbParts parts;
+  parts.request(a);  // handed over for single matrices only (down projection)
+  typename SbPrologue<PRO>::type pro;
+  pro.request(a);
 
   // ---- prologue: the activations of every row into LDS ----
-  if constexpr (PRO == SB_PRO_ATTN) {
-    // merge of the context splits of the attention kernel: out = sum_s o_s exp(m_s - m) / sum_s l_s exp(m_s - m)
-    const int NH = a.attn_kh * a.attn_g * a.attn_h;  // == K
-    for (int e = tid; e < M * NH; e += kSbThreads) {
-      const int m = e / NH, rest = e - m * NH, head = rest / a.attn_h, d = rest - head * a.attn_h;
-      const int kvh = head / a.attn_g, g = head - kvh * a.attn_g;
-      const float* pr = a.attn_part + ((((size_t)m * a.attn_kh + kvh) * a.attn_ns) * a.attn_g + g) * (a.attn_h + 2);
-      const size_t sstride = (size_t)a.attn_g * (a.attn_h + 2);
-      float pm[8], pl[8], po[8];  // up to 8 splits, every load requested before the first use
-#pragma unroll
-      for (int sp = 0; sp < 8; ++sp) {
-        const size_t o = (size_t)min(sp, a.attn_ns - 1) * sstride;
-        pm[sp] = pr[o + a.attn_h];
-        pl[sp] = pr[o + a.attn_h + 1];
-        po[sp] = pr[o + d];
-      }
-      float mm = -1e30f;
-#pragma unroll
-      for (int sp = 0; sp < 8; ++sp) mm = fmaxf(mm, sp < a.attn_ns ? pm[sp] : -1e30f);
-      float ls = 0.f, o = 0.f;
-#pragma unroll
-      for (int sp = 0; sp < 8; ++sp) {
-        const float w = sp < a.attn_ns ? __expf(pm[sp] - mm) : 0.f;
-        ls += pl[sp] * w;
-        o += po[sp] * w;
-      }
-      xs[m * XS + rest] = f2bf(ls > 0.f ? o / ls : 0.f);
-    }
-  } else if constexpr (PRO == SB_PRO_PLAIN) {
-    const int nchunks = M * (K >> 3), cpr = K >> 3;
-    for (int ch = tid; ch < nchunks; ch += kSbThreads) {
-      const int m = ch / cpr, cc = ch - m * cpr;
-      *reinterpret_cast<uint4*>(xs + m * XS + cc * 8) = *reinterpret_cast<const uint4*>(a.x + (size_t)m * a.ldx + cc * 8);
-    }
-  } else {
-    // RMSNorm of every row: up to 4 chunks of 8 elements per thread (M K <= 16384)
-    const int nchunks = M * (K >> 3), cpr = K >> 3;
-    float v[4][8];
-    float ss[kSbMaxRows] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ch = tid + kSbThreads * i;
-      if (ch < nchunks) {
-        const int m = ch / cpr, cc = ch - m * cpr;
-        const uint4 q = *reinterpret_cast<const uint4*>(a.x + (size_t)m * a.ldx + cc * 8);
-        v[i][0] = bf_lo(q.x); v[i][1] = bf_hi(q.x); v[i][2] = bf_lo(q.y); v[i][3] = bf_hi(q.y);
-        v[i][4] = bf_lo(q.z); v[i][5] = bf_hi(q.z); v[i][6] = bf_lo(q.w); v[i][7] = bf_hi(q.w);
-        float sq = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sq += v[i][e] * v[i][e];
-#pragma unroll
-        for (int r = 0; r < kSbMaxRows; ++r) ss[r] += (m == r) ? sq : 0.f;
-      }
-    }
-    // sum of squares of each row over the workgroup, in a fixed order
-#pragma unroll
-    for (int r = 0; r < kSbMaxRows; ++r) ss[r] = wave_sum(ss[r]);
-    if (lane == 0) {
-#pragma unroll
-      for (int r = 0; r < kSbMaxRows; ++r) rms_s[4 + wave * 4 + r] = ss[r];
-    }
-    __syncthreads();
-    if (tid < kSbMaxRows) {
-      float t = 0.f;
-      for (int w = 0; w < kSbWaves; ++w) t += rms_s[4 + w * 4 + tid];
-      rms_s[tid] = sqrtf(t / (float)K + a.eps);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ch = tid + kSbThreads * i;
-      if (ch < nchunks) {
-        const int m = ch / cpr, cc = ch - m * cpr;
-        const float rms = rms_s[m];
-        const uint4 wq = *reinterpret_cast<const uint4*>(a.norm_w + cc * 8);
-        const float w[8] = {bf_lo(wq.x), bf_hi(wq.x), bf_lo(wq.y), bf_hi(wq.y),
-                            bf_lo(wq.z), bf_hi(wq.z), bf_lo(wq.w), bf_hi(wq.w)};
-        float o[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          o[e] = a.family == TMX_FAMILY_LLAMA3 ? rbf(w[e] * v[i][e]) / rms : w[e] * (v[i][e] / rms);
-        uint4 pk;
-        pk.x = pack_bf2(o[0], o[1]); pk.y = pack_bf2(o[2], o[3]);
-        pk.z = pack_bf2(o[4], o[5]); pk.w = pack_bf2(o[6], o[7]);
-        *reinterpret_cast<uint4*>(xs + m * XS + cc * 8) = pk;
-      }
-    }
-  }
+  parts.finish(a, red_t);
+  pro.finish(a, xs, XS, rms_s);
   __syncthreads();
 
   // ---- the K-slice of this wave: its column tile, and its share of x . A ----
@@ -299,9 +400,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
     float t = 0.f;
     if (m < M) {
       if (a.t_parts) {
-        const int lanes_per = 32 * M, groups = kSbThreads / lanes_per;
-        if (cc < 32)
-          for (int g = 0; g < groups; ++g) t += red_t[g * lanes_per + m * 32 + cc];
+        t = sb_parts_total(parts, red_t, m, cc);
       } else if (lora_here) {
         for (int w = 0; w < kSbWaves; ++w) t += red_t[(w * kSbMaxRows + m) * 64 + cc];
       }
@@ -367,6 +466,191 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The projections without SwiGLU (q|k|v, o, down) with 16 columns per workgroup.  At one row such a launch is bound by
+// the bytes it has in flight and by its chain of round trips, not by HBM: 32 columns of a 2048-wide matrix were 64
+// workgroups on 256 CUs, each pulling a 128 KB column stream of the down projection (1B shape) at what one CU can keep
+// in flight.  16 columns are twice as many workgroups with half the stream each, and every load a wave makes (its whole
+// K-slice of weights, its tiles of A, its share of the handed-over results) is requested before the first is used.
+// The 16 x 16 x 32 MFMA takes them: lane (n = l % 16, q = l / 16) holds column n of k-tile 2 p + q / 2, half q % 2, so a
+// wave's load is two half tiles, and word t of the four lanes of a column is 32 consecutive steps of the contraction
+// (the x operand reads the same k).  Measured on the 1B shape at one row / three rows (trace, us per launch):
+// q|k|v 10.1 -> 8.1 / 9.2, o 9.7 / 15.9 -> 7.7 / 10.1, down 11.9 / 14.6 -> 10.1 / 13.3.
+constexpr int kSbPairs = 8;  // k-tile pairs per wave requested at once
+
+// LDS: x [M][K + 8] bf16 | red [8 waves][4][16] f32 | red_t [8][4][64] f32 | t [4][64] f32 | row scratch [4 + 8 * 4] f32
+constexpr size_t kSb16TailFloats = kSbWaves * kSbMaxRows * 16 + kSbWaves * kSbMaxRows * 64 + kSbMaxRows * 64 + 4 + kSbWaves * 4;
+
+template <int PRO, int EPI>
+__global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a) {
+  extern __shared__ __align__(16) unsigned char sb_smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n16 = lane & 15, q = lane >> 4, h = q & 1, par = q >> 1;
+  const int M = a.M, K = a.K, KT = K >> 6, KP = KT >> 1, XS = K + 8;
+  uint16_t* xs = reinterpret_cast<uint16_t*>(sb_smem);
+  float* red = reinterpret_cast<float*>(sb_smem + sb_x_bytes(M, K));
+  float* red_t = red + kSbWaves * kSbMaxRows * 16;
+  float* t_s = red_t + kSbWaves * kSbMaxRows * 64;
+  float* rms_s = t_s + kSbMaxRows * 64;  // [4] + per-wave sums [8][4]
+
+  // weights and scales of this wave's pairs
+  const int nb = (int)blockIdx.x >> 1, half16 = ((int)blockIdx.x & 1) * 16;
+  const int per = (KP + kSbWaves - 1) / kSbWaves, p0 = wave * per, p1 = min(p0 + per, KP);
+  const int gs = __builtin_ctz(a.G >> 6), KG = K / a.G;
+  const u32x4_t* wsrc = reinterpret_cast<const u32x4_t*>(a.qw) + ((size_t)nb * KT + par) * 64 + 32 * h + half16 + n16;
+  const uint16_t* ssrc = a.scales + (size_t)nb * KG * 32 + half16 + n16;
+  u32x4_t wr[kSbPairs];
+  uint16_t sr[kSbPairs];
+  auto load_w = [&](int p, int slot) __attribute__((always_inline)) {
+    p = min(p, KP - 1);
+    wr[slot] = __builtin_nontemporal_load(wsrc + (size_t)p * 128);
+    sr[slot] = ssrc[(size_t)((2 * p + par) >> gs) * 32];
+  };
+#pragma unroll
+  for (int i = 0; i < kSbPairs; ++i)
+    if (i < per) load_w(p0 + i, i);
+
+  // x . A of this wave's eighth of K (32 x 32 x 16 MFMAs: A's fragment order), for the 32-column tiles of A that hold
+  // this workgroup's segment; up to four (k-tile, tile) items at a time, the first four requested now
+  const int lrow = lane & 31, lh = lane >> 5;
+  const bool lora_here = a.a_t != nullptr;
+  int q0 = 0, q1 = -1;
+  if (lora_here) {
+    const int n0 = (int)blockIdx.x * 16;
+    const int seg = n0 >= a.seg_end[0] ? (n0 >= a.seg_end[1] ? 2 : 1) : 0;
+    q0 = (seg * a.lora_r) >> 5;
+    q1 = min(((seg + 1) * a.lora_r - 1) >> 5, (a.Rpad >> 5) - 1);
+  }
+  const int RT = a.Rpad >> 5, nq = q1 - q0 + 1;
+  const int lper = (KT + kSbWaves - 1) / kSbWaves, l0 = wave * lper, l1 = min(l0 + lper, KT);
+  const int items = lora_here ? max(l1 - l0, 0) * nq : 0;
+  u32x4_t ab[4][4];
+  auto load_a = [&](int it, auto ic) __attribute__((always_inline)) {
+    constexpr int i = decltype(ic)::value;
+    if (it < items) {
+      const int kt = l0 + (nq == 2 ? it >> 1 : it), qq = q0 + (nq == 2 ? it & 1 : 0);
+      const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + ((size_t)(kt * RT + qq) * 4) * 64 + lane;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) ab[i][t] = ap[t * 64];
+    }
+  };
+  static_for<4>([&](auto ic) __attribute__((always_inline)) { load_a(decltype(ic)::value, ic); });
+
+  // what the epilogue needs and no other launch makes
+  const bool epi_thread = tid < kSbMaxRows * 16 && (tid >> 4) < M;
+  const int em = tid >> 4, n = (int)blockIdx.x * 16 + (tid & 15);
+  uint16_t breg[16], res_v = 0;
+  if (epi_thread) {
+    if (a.lora_b) {
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) breg[rr] = a.lora_b[(size_t)min(rr, a.lora_r - 1) * a.N + n];
+    }
+    if constexpr (EPI == SB_EPI_RESIDUAL) res_v = a.residual[(size_t)em * a.ldy + n];
+  }
+
+  // parts of t and the rows: requested behind the weights (which come from farther), before anything is waited for
+  SbParts parts;
+  parts.request(a);  // handed over for single matrices only (down projection)
+  typename SbPrologue<PRO>::type pro;
+  pro.request(a);
+
+  // ---- prologue: the activations of every row into LDS ----
+  parts.finish(a, red_t);
+  pro.finish(a, xs, XS, rms_s);
+  __syncthreads();
+
+  // ---- this wave's pairs of k-tiles ----
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  const uint16_t* xb = xs + min(n16, M - 1) * XS + par * 64 + h * 8;  // rows beyond the batch repeat the last one
+  for (int base = 0; base < per; base += kSbPairs) {
+    static_for<kSbPairs>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int i = decltype(ic)::value;
+      const int p = p0 + base + i;
+      if (p < p1) {
+        bf16x8_t xa[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) xa[t] = *reinterpret_cast<const bf16x8_t*>(xb + p * 128 + t * 16);
+        const float sc = bf2f(sr[i]), m8s = -8.f * sc;
+        const uint32_t wd[4] = {wr[i].x, wr[i].y, wr[i].z, wr[i].w};
+        if (base + i + kSbPairs < per) load_w(p + kSbPairs, i);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[t], dequant_word<true>(wd[t], sc, m8s), acc, 0, 0, 0);
+      }
+    });
+  }
+  if (lora_here) {
+    f32x16_t tacc[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) tacc[u][r] = 0.f;
+    const uint16_t* lb = xs + min(lrow, M - 1) * XS + lh * 8;
+    for (int it0 = 0; it0 < items; it0 += 4) {
+      static_for<4>([&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        if (it0 + i < items) {
+          const int kt = l0 + (nq == 2 ? (it0 + i) >> 1 : it0 + i);
+          const bool second = nq == 2 && (i & 1);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const bf16x8_t xa = *reinterpret_cast<const bf16x8_t*>(lb + kt * 64 + t * 16), bb = __builtin_bit_cast(bf16x8_t, ab[i][t]);
+            if (second) tacc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, bb, tacc[1], 0, 0, 0);
+            else tacc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, bb, tacc[0], 0, 0, 0);
+          }
+          load_a(it0 + i + 4, ic);
+        }
+      });
+    }
+    if (lh == 0) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (u < nq) {
+#pragma unroll
+          for (int r = 0; r < kSbMaxRows; ++r) red_t[(wave * kSbMaxRows + r) * 64 + (q0 + u) * 32 + lrow] = tacc[u][r];
+        }
+    }
+  }
+  if (q == 0) {  // rows 0..3 of the 16 x 16 tile: registers 0..3 of lanes 0..15
+#pragma unroll
+    for (int r = 0; r < kSbMaxRows; ++r) red[(wave * kSbMaxRows + r) * 16 + n16] = acc[r];
+  }
+  __syncthreads();
+  // t = bf16(sum over the waves, in wave order), or bf16(sum of the runs, in run order)
+  if (tid < kSbMaxRows * 64) {
+    const int m = tid >> 6, cc = tid & 63;
+    float t = 0.f;
+    if (m < M) {
+      if (a.t_parts) {
+        t = sb_parts_total(parts, red_t, m, cc);
+      } else if (lora_here && (cc >> 5) >= q0 && (cc >> 5) <= q1) {
+#pragma unroll
+        for (int w = 0; w < kSbWaves; ++w) t += red_t[(w * kSbMaxRows + m) * 64 + cc];
+      }
+    }
+    t_s[m * 64 + cc] = rbf(t);
+  }
+  __syncthreads();
+  if (epi_thread) {
+    float b = 0.f;
+#pragma unroll
+    for (int w = 0; w < kSbWaves; ++w) b += red[(w * kSbMaxRows + em) * 16 + (tid & 15)];
+    b = rbf(b);
+    if (a.lora_b) {
+      const int seg = n >= a.seg_end[0] ? (n >= a.seg_end[1] ? 2 : 1) : 0;
+      const float* tp = t_s + em * 64 + seg * a.lora_r;
+      float d = 0.f;
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) d = fmaf(rr < a.lora_r ? tp[rr] : 0.f, bf2f(breg[rr]), d);
+      for (int rr = 16; rr < a.lora_r; ++rr) d = fmaf(tp[rr], bf2f(a.lora_b[(size_t)rr * a.N + n]), d);
+      b = rbf(b + rbf(rbf(d) * a.lora_ls));
+    }
+    if constexpr (EPI == SB_EPI_RESIDUAL) b = rbf(b + bf2f(res_v));
+    a.y[(size_t)em * a.ldy + n] = f2bf(b);
+  }
+}
+
 size_t sb_linear_lds(int M, int K) { return sb_x_bytes(M, K) + kSbTailFloats * 4; }
 
 template <int PRO, int EPI>
@@ -375,6 +659,17 @@ static int launch_sb(hipStream_t st, const SbLinearArgs& a, int blocks) {
       reinterpret_cast<const void*>(&sb_linear_kernel<PRO, EPI>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
   if (attr != hipSuccess) return TMX_ERR_LAUNCH;
   hipLaunchKernelGGL((sb_linear_kernel<PRO, EPI>), dim3(blocks), dim3(kSbThreads), sb_linear_lds(a.M, a.K), st, a);
+  return check_launch();
+}
+
+size_t sb_linear16_lds(int M, int K) { return sb_x_bytes(M, K) + kSb16TailFloats * 4; }
+
+template <int PRO, int EPI>
+static int launch_sb16(hipStream_t st, const SbLinearArgs& a) {
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(&sb_linear16_kernel<PRO, EPI>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+  if (attr != hipSuccess) return TMX_ERR_LAUNCH;
+  hipLaunchKernelGGL((sb_linear16_kernel<PRO, EPI>), dim3(a.N / 16), dim3(kSbThreads), sb_linear16_lds(a.M, a.K), st, a);
   return check_launch();
 }
 
@@ -391,6 +686,13 @@ int sb_linear(hipStream_t st, const SbLinearArgs& a, int pro, int epi) {
   if (epi == SB_EPI_SWIGLU) {
     if (pro != SB_PRO_NORM || a.N % 64) return TMX_ERR_UNSUPPORTED;
     return launch_sb<SB_PRO_NORM, SB_EPI_SWIGLU>(st, a, a.N / 64);
+  }
+  // whole pairs of k-tiles and segment ends on 16 columns: 16 columns per workgroup
+  if (a.K % 128 == 0 && a.seg_end[0] % 16 == 0 && a.seg_end[1] % 16 == 0) {
+    if (pro == SB_PRO_NORM && epi == SB_EPI_PLAIN) return launch_sb16<SB_PRO_NORM, SB_EPI_PLAIN>(st, a);
+    if (pro == SB_PRO_ATTN && epi == SB_EPI_RESIDUAL) return launch_sb16<SB_PRO_ATTN, SB_EPI_RESIDUAL>(st, a);
+    if (pro == SB_PRO_PLAIN && epi == SB_EPI_RESIDUAL) return launch_sb16<SB_PRO_PLAIN, SB_EPI_RESIDUAL>(st, a);
+    if (pro == SB_PRO_PLAIN && epi == SB_EPI_PLAIN) return launch_sb16<SB_PRO_PLAIN, SB_EPI_PLAIN>(st, a);
   }
   const int blocks = a.N / 32;
   if (pro == SB_PRO_NORM && epi == SB_EPI_PLAIN) return launch_sb<SB_PRO_NORM, SB_EPI_PLAIN>(st, a, blocks);
@@ -572,12 +874,9 @@ __global__ __launch_bounds__(256) void sb_attn_kernel(SbAttnArgs a) {
       ls += s_l[i][g] * w;
       o += s_acc[i][g][d] * w;
     }
-    float* pr = a.partial + ((((size_t)b * a.Kh + kvh) * a.nsplit + split) * G + g) * (H + 2);
-    pr[d] = o;
-    if (d == 0) {
-      pr[H] = mm;
-      pr[H + 1] = ls;
-    }
+    const size_t i = (((size_t)b * a.Kh + kvh) * a.nsplit + split) * G + g;
+    a.partial[i * H + d] = o;
+    if (d == 0) *reinterpret_cast<f32x2_t*>(a.partial + (size_t)a.B * a.Kh * a.nsplit * G * H + i * 2) = f32x2_t{mm, ls};
   }
 }
 

@@ -241,7 +241,7 @@ struct SbLinearArgs {
   const uint16_t* norm_w;   // [K] (norm prologue)
   float eps;
   int family;
-  const float* attn_part;   // attention prologue: [M][kh][ns][g][h + 2] split results (output | max | sum)
+  const float* attn_part;   // attention prologue: split results, outputs [M][kh][ns][g][h], then (max, sum) [M][kh][ns][g][2]
   int attn_kh, attn_g, attn_h, attn_ns;
   const uint4* qw;
   const uint16_t* scales;
@@ -270,7 +270,7 @@ struct SbAttnArgs {
   const uint8_t* input_mask;
   const int32_t* step;
   int buf_len;
-  float* partial;           // [B][Kh][nsplit][G][H + 2]
+  float* partial;           // outputs [B][Kh][nsplit][G][H], then (max, sum) [B][Kh][nsplit][G][2]
   int B, N, Kh, C, nsplit;
   float scale;
   const uint16_t* q_norm_w;  // [H] per-head RMSNorm of q and k before the rotation (Qwen3), or null
