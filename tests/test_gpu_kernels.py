@@ -554,6 +554,23 @@ def test_head_from_tiles_equals_head_from_rows_bit_for_bit(M, D, V):
       np.testing.assert_array_equal(a, b)
 
 
+# one k-tile, whole and partial ring turns, row counts at the edges of the 128- and 256-row forms, a second chunk,
+# vocabularies whose last workgroup has one to three tiles
+@pytest.mark.parametrize('M,D,V', [(65, 64, 1056), (128, 320, 1024), (129, 448, 2080), (200, 128, 1088), (256, 4096, 1120),
+                                   (330, 192, 1056)])
+def test_head_of_many_rows_from_tiles_equals_head_from_rows(M, D, V):
+  """Tokens, done flags and logits bit for bit; the log-softmax sum is taken in another order."""
+  global HEAD_LAYOUT
+  x, w = _head_inputs(M, D, V, 3 * M + V)
+  for mode, temp, key in ((0, 1.0, (0, 0)), (1, 0.7, prng.prng_key(4))):
+    outs = {}
+    for HEAD_LAYOUT in ('rows', 'tiles'):
+      outs[HEAD_LAYOUT] = _run_head(x, w, mode, temp, key, 2)
+    HEAD_LAYOUT = 'rows'
+    for i, (a, b) in enumerate(zip(outs['rows'], outs['tiles'])):
+      np.testing.assert_allclose(a, b, rtol=0, atol=3e-6 if i == 1 else 0)
+
+
 @pytest.mark.parametrize('M,D,V', [(1, 256, 1024), (5, 512, 4096), (64, 256, 1056), (100, 128, 2048)])
 def test_head_greedy(M, D, V, head_layout):
   T = G.Keep()

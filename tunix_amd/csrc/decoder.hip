@@ -549,27 +549,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       }
       if (prof) TMX_TRY(TMX_K_EMPTY, empty_launch(st));
     }
-    if (sample && !nucleus && B > 64 && !s->logits_out && s->n_forbidden == 0 && D % 128 == 0) {
-      // more than 64 rows: the head in 256 x 256 blocks, one pass over the head matrix (the 64-row kernel
-      // would take one pass per 64 rows)
-      HeadArgs a = {};
-      a.x = w.xn;
-      a.w = (const uint16_t*)m->head;
-      a.M = B; a.D = D; a.V = m->vocab_size;
-      a.mode = s->sampling_mode;
-      a.temperature = s->temperature;
-      a.k0 = s->seed_hi; a.k1 = s->seed_lo;
-      a.step = s->step;
-      a.part_f = (float*)w.head_partial;
-      a.part_i = (int32_t*)((float*)w.head_partial + (size_t)B * ((m->vocab_size + 255) / 256) * 4);
-      a.token_buffer = s->token_buffer;
-      a.logprobs = s->logprobs;
-      a.done = s->done;
-      a.eos = s->eos_ids; a.n_eos = s->n_eos;
-      a.buf_len = L;
-      a.tpp = T;
-      TMX_TRY(TMX_K_HEAD, head_wide(st, a));
-    } else if (sample) {
+    if (sample) {
       HeadArgs a = {};
       a.x = w.xn;
       a.w = (const uint16_t*)m->head;
@@ -581,7 +561,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       a.step = s->step;
       a.forbidden = s->forbidden; a.n_forbidden = s->n_forbidden;
       a.logits_out = s->logits_out;
-      const size_t nwg = (m->vocab_size + 127) / 128;
+      const size_t nwg = (m->vocab_size + 127) / 128;  // the wide kernel uses half of it
       a.part_f = (float*)w.head_partial;
       a.part_i = (int32_t*)((float*)w.head_partial + (size_t)B * nwg * 4);
       a.token_buffer = s->token_buffer;
@@ -593,6 +573,8 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       if (nucleus) {
         TMX_TRY(TMX_K_HEAD, head_sample_nucleus(st, a, s->top_p, s->top_k, s->nucleus_workspace,
                                                 s->nucleus_workspace_bytes));
+      } else if (head_wide_ok(a)) {
+        TMX_TRY(TMX_K_HEAD, head_wide(st, a));
       } else {
         TMX_TRY(TMX_K_HEAD, head_sample(st, a));
       }

@@ -34,6 +34,93 @@ __device__ __forceinline__ float score_clip(float z) {
   return z != z ? -1e9f : fminf(fmaxf(z, -1e9f), 1e9f);
 }
 
+// Running statistics of one sequence row: max and sum of exp over the vocabulary rows seen, best candidate by key.
+struct RowStat {
+  float mx = kNegBig, se = 0.f;
+  Best best = {-INFINITY, -INFINITY, 0x7FFFFFFF};
+};
+
+// Adds the 16 vocabulary rows of an accumulator tile (first row v0) to the statistics of sequence row `row`.
+__device__ __forceinline__ void head_tile_stats(const HeadArgs& a, const f32x16_t& acc, int v0, int row, int lane, int target,
+                                                uint32_t key0, uint32_t key1, RowStat& st) {
+  const bool score = a.mode == TMX_SAMPLE_SCORE;
+  uint64_t packed = 0;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int v = v0 + acc_row(r, lane);
+    float logit = rbf(acc[r]);
+    if (a.logits_out) a.logits_out[(size_t)row * a.V + v] = logit;
+    for (int f = 0; f < a.n_forbidden; ++f)
+      if (a.forbidden[f] == v) logit = -INFINITY;
+    float z = logit, key = logit;
+    if (score) {
+      // the "best" candidate is the given next token: its z is what the log-prob needs
+      z = score_clip(rbf(logit / a.temperature));  // bf16 logits divided in place stay bf16 (rl/common.py:591-592)
+      key = (v == target) ? 0.f : -INFINITY;
+    } else if (a.mode == TMX_SAMPLE_TOP_P) {
+      z = logit / a.temperature;
+      if (a.sort_keys) {
+        // 16-bit key whose ascending order is the descending order of the logit (= of z, T > 0;
+        // -0 counts as +0): non-negative values count down from 0x7FFF, negative ones up from 0x8000
+        const uint32_t zb = __float_as_uint(logit + 0.0f) >> 16;
+        // registers 4 q .. 4 q + 3 hold four consecutive vocabulary rows: one 8-byte store
+        packed |= (uint64_t)((zb & 0x8000u) ? zb : (~zb & 0x7FFFu)) << (16 * (r & 3));
+        if ((r & 3) == 3) {
+          *reinterpret_cast<uint64_t*>(a.sort_keys + (size_t)row * a.V + v - 3) = packed;
+          packed = 0;
+        }
+        key = z;
+      } else {
+        uint32_t o0, o1;
+        threefry2x32(key0, key1, 0u, (uint32_t)(a.row_off + row) * (uint32_t)a.V + (uint32_t)v, o0, o1);
+        key = z + gumbel_from_bits(o0 ^ o1);
+      }
+    }
+    if (z > st.mx) {
+      st.se = st.se * expf(st.mx - z) + 1.f;
+      st.mx = z;
+    } else {
+      st.se += expf(z - st.mx);
+    }
+    Best c = {key, z, v};
+    best_merge(st.best, c);
+  }
+}
+
+// The given next token of sequence row `row` of this launch (scoring), or -1.
+__device__ __forceinline__ int head_target(const HeadArgs& a, int row) {
+  if (a.mode != TMX_SAMPLE_SCORE || row >= a.M) return -1;
+  const int tpp = a.tpp > 0 ? a.tpp : 1, prow = a.row_base + row;  // row of the pass
+  return a.token_buffer[(size_t)(prow / tpp) * a.buf_len + min(*a.step + prow % tpp + 1, a.buf_len - 1)];
+}
+
+// The other half-wave holds the other 16 vocabulary rows of the same sequence; one half stores the result.
+__device__ __forceinline__ void head_stat_to_lds(RowStat st, int h, float* f, int* idx) {
+  const float mx2 = __shfl_xor(st.mx, 32, 64), se2 = __shfl_xor(st.se, 32, 64);
+  Best o = {__shfl_xor(st.best.key, 32, 64), __shfl_xor(st.best.z, 32, 64), __shfl_xor(st.best.idx, 32, 64)};
+  lse_merge(st.mx, st.se, mx2, se2);
+  best_merge(st.best, o);
+  if (h == 0) {
+    f[0] = st.mx; f[1] = st.se; f[2] = st.best.key; f[3] = st.best.z;
+    *idx = st.best.idx;
+  }
+}
+
+// Partials of this workgroup for row `row`: the `n` waves' statistics at f + 4 * stride * w, idx + stride * w.
+__device__ __forceinline__ void head_store_partial(const HeadArgs& a, int row, int wg, const float* f, const int* idx, int n, int stride) {
+  float mx = f[0], se = f[1];
+  Best best = {f[2], f[3], idx[0]};
+  for (int w = 1; w < n; ++w) {
+    const float* g = f + (size_t)4 * stride * w;
+    lse_merge(mx, se, g[0], g[1]);
+    Best o = {g[2], g[3], idx[stride * w]};
+    best_merge(best, o);
+  }
+  float* pf = a.part_f + ((size_t)row * a.nwg + wg) * 4;
+  pf[0] = mx; pf[1] = se; pf[2] = best.key; pf[3] = best.z;
+  a.part_i[(size_t)row * a.nwg + wg] = best.idx;
+}
+
 // Workgroup = 4 waves x 32 vocabulary rows.  The hidden-state k-tile x[0:M, 64 kb : 64 kb + 64]
 // is fetched once per workgroup, double-buffered in LDS and shared by the waves (MFMA B
 // fragments); head rows stream HBM -> registers through a ring of 4 k-tiles per wave.  Lane
@@ -141,95 +228,135 @@ __global__ __launch_bounds__(256, MT == 4 ? 1 : 2) void head_kernel(HeadArgs a) 
   // per-step key = fold_in(seed, step)
   uint32_t key0 = 0, key1 = 0;
   if (a.mode == TMX_SAMPLE_TOP_P) threefry2x32(a.k0, a.k1, 0u, (uint32_t)*a.step, key0, key1);
-  const bool score = a.mode == TMX_SAMPLE_SCORE;
-
-  int target[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     const int row = m * 32 + nl;
-    const int tpp = a.tpp > 0 ? a.tpp : 1;
-    const int prow = a.row_base + row;  // row of the pass
-    target[m] = (score && row < a.M)
-                    ? a.token_buffer[(size_t)(prow / tpp) * a.buf_len + min(*a.step + prow % tpp + 1, a.buf_len - 1)] : -1;
-  }
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int row = m * 32 + nl;
-    float mx = kNegBig, se = 0.f;
-    Best best = {-INFINITY, -INFINITY, 0x7FFFFFFF};
-    if (live && row < a.M) {
-      uint64_t packed = 0;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int v = v0 + acc_row(r, lane);
-        float logit = rbf(acc[m][r]);
-        if (a.logits_out) a.logits_out[(size_t)row * a.V + v] = logit;
-        for (int f = 0; f < a.n_forbidden; ++f)
-          if (a.forbidden[f] == v) logit = -INFINITY;
-        float z = logit, key = logit;
-        if (score) {
-          // the "best" candidate is the given next token: its z is what the log-prob needs
-          z = score_clip(rbf(logit / a.temperature));  // bf16 logits divided in place stay bf16 (rl/common.py:591-592)
-          key = (v == target[m]) ? 0.f : -INFINITY;
-        } else if (a.mode == TMX_SAMPLE_TOP_P) {
-          z = logit / a.temperature;
-          if (a.sort_keys) {
-            // 16-bit key whose ascending order is the descending order of the logit (= of z, T > 0;
-            // -0 counts as +0): non-negative values count down from 0x7FFF, negative ones up from 0x8000
-            const uint32_t zb = __float_as_uint(logit + 0.0f) >> 16;
-            // registers 4 q .. 4 q + 3 hold four consecutive vocabulary rows: one 8-byte store
-            packed |= (uint64_t)((zb & 0x8000u) ? zb : (~zb & 0x7FFFu)) << (16 * (r & 3));
-            if ((r & 3) == 3) {
-              *reinterpret_cast<uint64_t*>(a.sort_keys + (size_t)row * a.V + v - 3) = packed;
-              packed = 0;
-            }
-            key = z;
-          } else {
-            uint32_t o0, o1;
-            threefry2x32(key0, key1, 0u, (uint32_t)(a.row_off + row) * (uint32_t)a.V + (uint32_t)v, o0, o1);
-            key = z + gumbel_from_bits(o0 ^ o1);
-          }
-        }
-        if (z > mx) {
-          se = se * expf(mx - z) + 1.f;
-          mx = z;
-        } else {
-          se += expf(z - mx);
-        }
-        Best c = {key, z, v};
-        best_merge(best, c);
-      }
-    }
-    // the other half-wave holds the other 16 vocabulary rows of the same sequence
-    {
-      const float mx2 = __shfl_xor(mx, 32, 64), se2 = __shfl_xor(se, 32, 64);
-      Best o = {__shfl_xor(best.key, 32, 64), __shfl_xor(best.z, 32, 64), __shfl_xor(best.idx, 32, 64)};
-      lse_merge(mx, se, mx2, se2);
-      best_merge(best, o);
-    }
-    if (h == 0) {
-      s_f[wave][row][0] = mx;
-      s_f[wave][row][1] = se;
-      s_f[wave][row][2] = best.key;
-      s_f[wave][row][3] = best.z;
-      s_i[wave][row] = best.idx;
-    }
+    RowStat st;
+    if (live && row < a.M) head_tile_stats(a, acc[m], v0, row, lane, head_target(a, row), key0, key1, st);
+    head_stat_to_lds(st, h, s_f[wave][row], &s_i[wave][row]);
   }
   __syncthreads();
-  for (int row = threadIdx.x; row < MT * 32; row += 256) {
-    if (row >= a.M) continue;
-    float mx = s_f[0][row][0], se = s_f[0][row][1];
-    Best best = {s_f[0][row][2], s_f[0][row][3], s_i[0][row]};
+  for (int row = threadIdx.x; row < MT * 32; row += 256)
+    if (row < a.M) head_store_partial(a, row, blockIdx.x, s_f[0][row], &s_i[0][row], 4, MT * 32);
+}
+
+// 65 to 256 rows: the matrix still has to stream once, but a wave multiplies up to 256 sequence rows (MT = 4 or 8 tiles),
+// so the hidden states go to LDS by direct transfers (no registers) and the weights, from the tile copy, straight to
+// registers as MFMA A operands, P steps ahead.  NW waves of 32 vocabulary rows each; slabs of 64 columns in 64 KiB of LDS:
+// rows of 128 bytes, 16-byte chunk c of row r at slot c ^ (r / 2 % 8), which spreads a fragment read over all banks.
+// Two workgroups share a CU, so that one's epilogue (20 threefry rounds a value when sampling) runs under the other's
+// loads.  On the 1.05 GB head, greedy / sampling: 128 rows 218 / 253 us, bound by the stream (64 rows: 193 / 198); 256 rows
+// 327 / 396 us, bound by LDS (a fragment read per MFMA) and, sampling, by the epilogue's VALU work.  The 256 x 256 blocks
+// of head_wide_kernel take 440 us for either.  For 256 rows also measured: two waves of 64 vocabulary rows on each 128
+// rows (half the LDS reads, every weight read twice) 351 / 418; one workgroup of 8 waves per CU 316 / 412.
+template <int MT, int NW, int P>
+__global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void head_mid_kernel(HeadArgs a) {
+  constexpr int ROWS = MT * 32, R = 512 / ROWS, DX = ROWS / (8 * NW);
+  static_assert(P % R == 0 && NW % 4 == 0, "a ring turn covers whole turns of the slabs; 128 vocabulary rows per partial");
+  extern __shared__ __align__(16) uint16_t smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, nl = lane & 31;
+  const int KT = a.D >> 6, klast = KT - 1, vtiles = a.V >> 5;
+  const int tile = blockIdx.x * NW + wave;
+  const bool live = tile < vtiles;  // waves past the end repeat the last tile (dropped)
+  const int v0 = (live ? tile : vtiles - 1) * 32;
+  const u32x4_t* wsrc = reinterpret_cast<const u32x4_t*>(a.w_tiles + (size_t)v0 * a.D) + lane;
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x, (uint32_t)a.M * a.D * 2u);
+  int xoff[DX];  // transfer i of a wave: rows 8 (wave + NW i) .. + 7, 8 lanes each
 #pragma unroll
-    for (int w = 1; w < 4; ++w) {
-      lse_merge(mx, se, s_f[w][row][0], s_f[w][row][1]);
-      Best o = {s_f[w][row][2], s_f[w][row][3], s_i[w][row]};
-      best_merge(best, o);
-    }
-    float* pf = a.part_f + ((size_t)row * a.nwg + blockIdx.x) * 4;
-    pf[0] = mx; pf[1] = se; pf[2] = best.key; pf[3] = best.z;
-    a.part_i[(size_t)row * a.nwg + blockIdx.x] = best.idx;
+  for (int i = 0; i < DX; ++i) {
+    const int r = 8 * (wave + NW * i) + (lane >> 3);
+    xoff[i] = (r < a.M ? r : a.M - 1) * a.D * 2 + (((lane & 7) ^ ((r >> 1) & 7)) * 16);
   }
+  f32x16_t acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
+  u32x4_t wring[P][4];
+
+  auto load_w = [&](int kb, auto pc, auto tc) __attribute__((always_inline)) {
+    constexpr int p = decltype(pc)::value, t = decltype(tc)::value;
+    kb = kb < klast ? kb : klast;
+    wring[p][t] = __builtin_nontemporal_load(wsrc + (size_t)kb * 256 + t * 64);
+  };
+  auto dma_x = [&](int kb, int buf) __attribute__((always_inline)) {
+    kb = kb < klast ? kb : klast;
+    uint16_t* base = smem + (size_t)buf * ROWS * 64 + wave * 512;
+#pragma unroll
+    for (int i = 0; i < DX; ++i) load_row_to_lds(rx, base + i * (NW * 512), xoff[i], kb * 128);
+  };
+  // in-order counter: waiting for the slab of the next step leaves its step's weights and R - 2 whole steps outstanding
+  constexpr int kYounger = 4 + (R - 2) * (DX + 4);
+  auto step = [&](int kb, auto pc) __attribute__((always_inline)) {
+    constexpr int p = decltype(pc)::value;
+    dma_x(kb + R - 1, (p + R - 1) % R);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint16_t* xb = smem + (size_t)(p % R) * ROWS * 64 + nl * 64;
+    static_for<4>([&](auto tc) __attribute__((always_inline)) {
+      constexpr int t = decltype(tc)::value;
+      const int slot = ((4 * h + t) ^ ((nl >> 1) & 7)) * 8;
+      bf16x8_t xf[MT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) xf[m] = *reinterpret_cast<const bf16x8_t*>(xb + m * 32 * 64 + slot);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wring[p][t]), xf[m], acc[m], 0, 0, 0);
+      load_w(kb + P, pc, tc);  // consumed: refill
+    });
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (kYounger & 15) | ((kYounger >> 4) << 14));
+    __syncthreads();
+  };
+  static_for<P>([&](auto pc) __attribute__((always_inline)) {
+    static_for<4>([&](auto tc) __attribute__((always_inline)) { load_w(decltype(pc)::value, pc, tc); });
+  });
+#pragma unroll
+  for (int r = 0; r < R - 1; ++r) dma_x(r, r);
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __syncthreads();
+  int kb = 0;
+  for (; kb + P <= KT; kb += P)
+    static_for<P>([&](auto pc) __attribute__((always_inline)) { step(kb + decltype(pc)::value, pc); });
+  static_for<P - 1>([&](auto pc) __attribute__((always_inline)) {
+    if (kb + decltype(pc)::value < KT) step(kb + decltype(pc)::value, pc);
+  });
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // the surplus transfers of the last steps have landed, the slabs are free
+  __syncthreads();
+  uint32_t key0 = 0, key1 = 0;
+  if (a.mode == TMX_SAMPLE_TOP_P) threefry2x32(a.k0, a.k1, 0u, (uint32_t)*a.step, key0, key1);
+  float* s_f = reinterpret_cast<float*>(smem);             // [NW][ROWS][4]
+  int* s_i = reinterpret_cast<int*>(s_f + NW * ROWS * 4);  // [NW][ROWS]
+  // One copy of the epilogue's code for all tiles (unrolled over them it would not fit the instruction cache): a
+  // wave-uniform index picks the accumulators.
+#pragma unroll 1
+  for (int m = 0; m < MT; ++m) {
+    const int row = m * 32 + nl;
+    RowStat st;
+    f32x16_t cur = acc[0];
+    static_for<MT>([&](auto qc) __attribute__((always_inline)) {
+      if (m == decltype(qc)::value) cur = acc[decltype(qc)::value];
+    });
+    if (live && row < a.M) head_tile_stats(a, cur, v0, row, lane, head_target(a, row), key0, key1, st);
+    head_stat_to_lds(st, h, s_f + (wave * ROWS + row) * 4, s_i + wave * ROWS + row);
+  }
+  __syncthreads();
+  for (int e = tid; e < NW / 4 * ROWS; e += NW * 64) {  // a partial per four waves
+    const int row = e % ROWS, q = e / ROWS, wg = blockIdx.x * (NW / 4) + q;
+    if (row < a.M && wg < a.nwg) head_store_partial(a, row, wg, s_f + (q * 4 * ROWS + row) * 4, s_i + q * 4 * ROWS + row, 4, ROWS);
+  }
+}
+
+constexpr size_t kHeadMidLds = 65536;
+
+template <int MT, int NW, int P>
+static int launch_head_mid(hipStream_t st, const HeadArgs& a) {
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(&head_mid_kernel<MT, NW, P>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kHeadMidLds);
+  if (attr != hipSuccess) return TMX_ERR_LAUNCH;
+  hipLaunchKernelGGL((head_mid_kernel<MT, NW, P>), dim3((a.nwg + NW / 4 - 1) / (NW / 4)), dim3(NW * 64), kHeadMidLds, st, a);
+  return TMX_OK;
 }
 
 // The tile copy of the head matrix: row tile vt (32 vocabulary rows) x k-tile kt (64 columns) is 4 KiB at
@@ -491,8 +618,10 @@ static int launch_head_wide(hipStream_t st, const HeadArgs& a, int tok_blocks, i
   return TMX_OK;
 }
 
+// With a tile copy, up to 256 rows are faster from it (head_logits): both read the matrix once, and the 256 x 256 blocks
+// spend 432 us on the 1.05 GB head where the stream needs half of that at 128 rows.
 bool head_wide_ok(const HeadArgs& a) {
-  return a.D % 128 == 0 && a.M > 0 && (size_t)a.M * a.D * 2 < (1u << 31) && (size_t)256 * a.D * 2 < (1u << 31) &&
+  return (a.M > 256 || (a.M > 64 && !a.w_tiles)) && a.D % 128 == 0 && a.M > 0 && (size_t)a.M * a.D * 2 < (1u << 31) && (size_t)256 * a.D * 2 < (1u << 31) &&
          a.n_forbidden == 0 && !a.logits_out;
 }
 
@@ -520,13 +649,12 @@ int head_wide(hipStream_t st, HeadArgs a) {
 int head_logits(hipStream_t st, HeadArgs& a) {
   if (a.V % 32 || a.D % 64 || a.M <= 0 || a.M > TMX_MAX_FILL_ROWS) return TMX_ERR_SHAPE;
   a.nwg = (a.V + 127) / 128;
-  // Rows go through the 32- or 64-row kernel in chunks of 64: one pass over the head matrix per chunk.
-  // (A 128-row instantiation ran 0.87 ms on a 1 GB head against 2 x 0.27 ms: one workgroup per CU, its
-  // x tile and weight ring no longer hide the latencies.)  The partials of every chunk sit where one
-  // finalize launch over all rows expects them.
-  for (int r0 = 0; r0 < a.M; r0 += 64) {
+  // One pass over the head matrix per chunk of rows: up to 256 from the tile copy, 64 from the rows themselves.  The
+  // partials of every chunk sit where one finalize launch over all rows expects them.
+  const int chunk = a.w_tiles ? 256 : 64;
+  for (int r0 = 0; r0 < a.M; r0 += chunk) {
     HeadArgs c = a;
-    c.M = a.M - r0 < 64 ? a.M - r0 : 64;
+    c.M = a.M - r0 < chunk ? a.M - r0 : chunk;
     c.x = a.x + (size_t)r0 * a.D;
     c.row_base = a.row_base + r0;
     c.row_off = a.row_off + r0;
@@ -534,13 +662,16 @@ int head_logits(hipStream_t st, HeadArgs& a) {
     if (a.sort_keys) c.sort_keys = a.sort_keys + (size_t)r0 * a.V;
     c.part_f = a.part_f + (size_t)r0 * a.nwg * 4;
     c.part_i = a.part_i + (size_t)r0 * a.nwg;
+    int rc = TMX_OK;
     if (c.w_tiles) {
       if (c.M <= 32) hipLaunchKernelGGL((head_kernel<1, true>), dim3(a.nwg), dim3(256), 0, st, c);
-      else hipLaunchKernelGGL((head_kernel<2, true>), dim3(a.nwg), dim3(256), 0, st, c);
+      else if (c.M <= 64) hipLaunchKernelGGL((head_kernel<2, true>), dim3(a.nwg), dim3(256), 0, st, c);
+      else rc = c.M <= 128 ? launch_head_mid<4, 4, 4>(st, c) : launch_head_mid<8, 4, 4>(st, c);
     } else {
       if (c.M <= 32) hipLaunchKernelGGL((head_kernel<1, false>), dim3(a.nwg), dim3(256), 0, st, c);
       else hipLaunchKernelGGL((head_kernel<2, false>), dim3(a.nwg), dim3(256), 0, st, c);
     }
+    if (rc != TMX_OK) return rc;
   }
   return check_launch();
 }
