@@ -233,6 +233,8 @@ int tmx_qlora_gate_up_swiglu_handover(void* stream, const void* x, const void* q
 /* out[B, N H] = softmax(q . K^T / sqrt(H) over positions j <= *step with
  * input_mask[b, j]) . V, caches bf16 [B, C, Kh, H].  tunix/models/llama3/model.py:379-396,
  * tunix/models/qwen3/model.py:776-793 with the mask of tunix/generate/utils.py:35-59.
+ * Every slot of the caches has to be finite: masked slots, and slots behind *step that share a block of 32 with it, are
+ * read and weighed with a probability of 0 (the reference's softmax over the whole cache does the same).
  * workspace: tmx_gqa_decode_workspace_bytes() bytes (may be 0 -> NULL allowed). */
 size_t tmx_gqa_decode_workspace_bytes(int B, int N, int Kh, int H, int C);
 int tmx_gqa_decode_attention(void* stream, const void* q, const void* kcache, const void* vcache,
@@ -379,7 +381,9 @@ typedef struct {
   float* logprobs;       /* [B, buf_len] or NULL */
   uint8_t* done;         /* [B] */
   int32_t* step;         /* device scalar: decoding_step */
-  void* kv_cache;        /* bf16 [layers][2 (k, v)][B][C][Kh][H] */
+  void* kv_cache;        /* bf16 [layers][2 (k, v)][B][C][Kh][H].  Every slot has to hold finite values before the first
+                            step (zero-fill it, also between unrelated batches): slots that are masked or lie behind
+                            the newest one are read and weighed with a probability of 0, and 0 x NaN is NaN */
   int sampling_mode;     /* TMX_SAMPLE_* */
   float temperature, top_p;
   int top_k;
@@ -430,8 +434,9 @@ int tmx_decode_steps(const tmx_model_desc* model, const tmx_decode_state* state,
  * of every sequence, of sequence s only those from first_col[s] on (device array, [batch]), as n_rows rows in all
  * (n_rows = the caller's count of them, <= TMX_MAX_FILL_ROWS and whatever bounds the rows of tmx_decode_steps; a
  * workspace of tmx_decode_workspace_bytes(model, n_rows, cache_size)).  *step advances by width.  The reference computes
- * the padding and masks it (tunix/generate/utils.py:35-59): no later token looks at the cache slots left out, which stay
- * as they are.  state->tokens_per_pass is ignored.  TMX_ERR_UNSUPPORTED for head shapes the block attention does not
+ * the padding and masks it (tunix/generate/utils.py:35-59).  The cache slots left out stay as they are; input_mask keeps
+ * them out of every later softmax, but they are read and have to be finite (see kv_cache).  state->tokens_per_pass is
+ * ignored.  TMX_ERR_UNSUPPORTED for head shapes the block attention does not
  * serve (head_dim 64 with 8 query heads per kv head, and others). */
 int tmx_fill_ragged(const tmx_model_desc* model, const tmx_decode_state* state, void* stream, const int32_t* first_col,
                     int width, int n_rows);

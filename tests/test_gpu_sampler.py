@@ -769,3 +769,27 @@ def test_cache_fill_leaves_out_padding(lengths):
       d = np.abs(got[:, :, i, p - n:p - 1] - want[:, :, i, p - n:p - 1])
       assert not d.size or d.max() <= 2.0 ** -6 * max(1.0, np.abs(want).max())
     assert np.abs(st['logits'].cpu().numpy() - want_logits).max() <= LOGIT_TOL
+
+
+@pytest.mark.parametrize('lengths', [(70, 61, 66), (70, 70, 70)])  # padding in front of two prompts; none, and a last block of 32 slots written in part
+def test_earlier_rollout_of_nans_leaves_nothing_in_the_caches(lengths):
+  """After a rollout whose K / V rows were NaN (a diverged adapter), the next one gives what a fresh sampler gives,
+  bit for bit: no slot that a walk leaves out, in front of a prompt or behind its newest token, keeps the old value."""
+  cfg = OM.Config('llama3', 2, 512, 256, 512, 8, 64, 2, norm_eps=1e-5)
+  model = C.product_model(cfg, C.make_state(cfg, 31, 8), 64, 16.0)
+  rng = np.random.default_rng(11)
+  base = [rng.integers(3, 512, n) for n in lengths]
+  for per_prompt in (4, 1):  # the prompt walked once per group, in a cache of its own, and every row by itself
+    kw = dict(prompt_token_ids=[q for q in base for _ in range(per_prompt)], max_generation_steps=6, max_prompt_length=70,
+              eos_tokens=[-1], return_logprobs=True, temperature=1.0, top_p=1.0, seed=5)
+    want = _sampler(model, cfg, 96)(**kw)
+    s = _sampler(model, cfg, 96)
+    s(**kw)
+    assert (getattr(s, '_lead_cache', None) is not None) == (per_prompt > 1)
+    for cache in [s._cache] + ([s._lead_cache] if per_prompt > 1 else []):
+      cache.fill_(float('nan'))
+    s._workspace[256:].fill_(255)  # (NaN as bf16 and as f32)
+    got = s(**kw)
+    assert np.isfinite(np.array(got.logprobs)).all()
+    np.testing.assert_array_equal(np.stack(got.tokens), np.stack(want.tokens))
+    np.testing.assert_array_equal(np.array(got.logprobs), np.array(want.logprobs))

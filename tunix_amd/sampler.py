@@ -405,6 +405,10 @@ class Sampler:
     if getattr(self, '_lead_cache', None) is None or tuple(self._lead_cache.shape) != need:
       self._lead_cache = None
       self._lead_cache = self._transformer.init_cache(b // g, self.cache_config.cache_size)
+    else:
+      # attention multiplies the slots it masks by 0: slots that this walk does not write (padding, what lies behind
+      # the newest one) must not keep a NaN or infinity of an earlier rollout
+      self._lead_cache.zero_()
     sub = dict(st)
     sub.update({
         'token_buffer': st['token_buffer'][lead].contiguous(), 'positions': st['positions'][lead].contiguous(),
