@@ -448,8 +448,8 @@ int tmx_fill_ragged(const tmx_model_desc* model, const tmx_decode_state* state, 
  * that word, clears it, and returns TMX_ERR_DEVICE_WAIT if it was set (the tokens produced
  * since the previous check are then not to be trusted), else TMX_OK.  The word lives in the
  * first 256 bytes of state->workspace, which the decode calls never clear: zero-fill them
- * once before the workspace's first use.  No counterpart in the reference (XLA has no such
- * failure mode). */
+ * once before the workspace's first use, and copy them when another workspace takes its place
+ * before the check.  No counterpart in the reference (XLA has no such failure mode). */
 int tmx_decode_status(const tmx_model_desc* model, const tmx_decode_state* state, void* stream);
 
 /* The same steps with one of them recorded into a HIP graph and replayed n_steps - 1 times

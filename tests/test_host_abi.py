@@ -130,6 +130,30 @@ def test_sampler_row_limits_are_checked_on_the_host():
     odd._c_state({'token_buffer': torch.zeros(130, 16, dtype=torch.int32)})
 
 
+def test_status_word_survives_a_larger_workspace():
+  """Passes of one call differ in rows and with them in the workspace they need: the word that a kernel sets when a
+  bounded wait runs out moves along, and a first workspace starts at zero."""
+  import types
+  import torch
+  from tunix_amd.model import ModelDesc
+  s = _sampler(16)
+  s._transformer.desc = ModelDesc
+  sizes = {1: 1024, 2: 4096, 3: 512}  # bytes by rows of the pass: not monotone
+  s._lib = types.SimpleNamespace(tmx_decode_workspace_bytes=lambda desc, rows, cache_size: sizes[rows])
+  i32 = lambda *shape: torch.zeros(*shape, dtype=torch.int32)
+  st = {'token_buffer': i32(1, 16), 'positions': i32(1, 16), 'input_mask': i32(1, 16), 'done': i32(1), 'step': i32(1),
+        'logprobs': None, 'cache': i32(1), 'sampling_mode': 'greedy', 'temperature': 0.0, 'top_p': None, 'top_k': None,
+        'seed': (0, 0), 'eos': i32(1), 'forbidden': None, 'logits': None}
+  s._c_state(st, 1, 1)
+  assert s._workspace.numel() == 1024 and not s._workspace.any()
+  s._workspace[:4] = torch.tensor([1, 0, 0, 0], dtype=torch.uint8)  # what a kernel of the first pass does
+  s._workspace[256:] = 7
+  for rows in (2, 3):
+    c = s._c_state(st, 1, rows)
+    assert s._workspace.numel() == c.workspace_bytes == 4096 and c.workspace == s._workspace.data_ptr()
+    assert s._workspace[0] == 1 and not s._workspace[1:].any()
+
+
 def test_sampler_tokenize_and_surface():
   s = _sampler(16)
   np.testing.assert_array_equal(s.tokenize('5 6 7'), [1, 5, 6, 7])  # bos prepended

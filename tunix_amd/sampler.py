@@ -262,8 +262,13 @@ class Sampler:
     ws_bytes = self._lib.tmx_decode_workspace_bytes(
         ctypes.byref(self._transformer.desc()), rows, self.cache_config.cache_size)
     if self._workspace is None or self._workspace.numel() < ws_bytes:
-      # zero-filled: the first 256 bytes hold the status word tmx_decode_status reads
+      # zero-filled: the first 256 bytes hold the status word tmx_decode_status reads.  A larger workspace takes over the
+      # old one's: passes of one call differ in rows, and a wait that ran out in an earlier one still has to be reported
+      status = None if self._workspace is None else self._workspace[:256].clone()
+      self._workspace = None
       self._workspace = torch.zeros(ws_bytes, dtype=torch.uint8, device=self._transformer.device)
+      if status is not None:
+        self._workspace[:256].copy_(status)
     s = DecodeState()
     s.tokens_per_pass = tokens_per_pass
     s.share_group, s.share_len = st.get('share_group', 1), st.get('share_len', 0)
