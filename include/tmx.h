@@ -84,7 +84,8 @@ int tmx_int4_dequant(void* stream, const void* qweight, const void* scales, void
  *              at ((((kb * (r_pad/32) + ct) * 4 + t) * 64 + 32 h + c) * 8 + j)
  *   lora_b   : bf16 [r, N]
  *   residual : bf16 [M, N] or NULL; added after the LoRA delta, in bf16
- *   workspace: tmx_qlora_linear_workspace_bytes(M, K, N) bytes (f32 K-slice planes) */
+ *   workspace: tmx_qlora_linear_workspace_bytes(M, K, N) bytes (f32 K-slice planes)
+ * The launches of a call are ordered by the stream alone: no kernel of it waits for another one's data. */
 size_t tmx_qlora_linear_workspace_bytes(int M, int K, int N);
 int tmx_qlora_linear(void* stream, const void* x, const void* qweight, const void* scales,
                      const void* lora_a_t, const void* lora_b, const void* residual, void* y,

@@ -401,3 +401,58 @@ def test_shared_prompt_groups_are_found_on_the_host():
   m[3, 10] = False                                                          # one row masks a column: not the same prompt any more
   assert groups(ids, m)[1] < 32 or groups(ids, m)[0] != 8
   assert groups(ids[:, :16], ones(ids[:, :16])) == (1, 0, 0)               # too short to be worth a launch of its own
+
+
+# Stands for the part of the HIP runtime that a launch goes through, so that a call's launches can be counted without a
+# GPU: loaded before libtmx.so, whose undefined symbols resolve to it first.
+_LAUNCH_RECORDER = r"""
+#include <stddef.h>
+typedef struct { unsigned x, y, z; } dim3;
+static dim3 grid_, block_;
+static size_t shmem_;
+int launches = 0;
+unsigned grid_x[64];
+int __hipPushCallConfiguration(dim3 g, dim3 b, size_t s, void* st) { (void)st; grid_ = g; block_ = b; shmem_ = s; return 0; }
+int __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, void** st) { *g = grid_; *b = block_; *s = shmem_; *st = 0; return 0; }
+int hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t s, void* st) {
+  (void)f; (void)b; (void)args; (void)s; (void)st;
+  if (launches < 64) grid_x[launches] = g.x;
+  ++launches;
+  return 0;
+}
+int hipFuncSetAttribute(const void* f, int attr, int v) { (void)f; (void)attr; (void)v; return 0; }
+int hipGetLastError(void) { return 0; }
+"""
+
+
+@pytest.mark.parametrize('M,K,N,r', [(129, 256, 96, 8), (300, 4096, 12288, 16), (1000, 4224, 4096, 24)])
+def test_many_row_linear_makes_its_lora_projection_in_a_launch_before(tmp_path, M, K, N, r):
+  """tmx_qlora_linear has no word in which a kernel could report a wait that ran out, so t = x . A of more than 128 rows
+  comes from a launch of its own: cleared counts, the LoRA workgroups alone, the projection without them."""
+  import shutil
+  import subprocess
+  if shutil.which('gcc') is None:
+    pytest.skip('gcc is not installed')
+  src, so = tmp_path / 'recorder.c', tmp_path / 'recorder.so'
+  src.write_text(_LAUNCH_RECORDER)
+  subprocess.run(['gcc', '-shared', '-fPIC', '-o', str(so), str(src)], check=True)
+  child = f"""
+import ctypes, sys
+rec = ctypes.CDLL({str(so)!r}, mode=ctypes.RTLD_GLOBAL)
+sys.path.insert(0, {ROOT!r})
+from tunix_amd import _lib
+lib = _lib.lib()
+count = ctypes.c_int.in_dll(rec, 'launches')
+grids = (ctypes.c_uint * 64).in_dll(rec, 'grid_x')
+assert lib.tmx_qlora_linear_num_splits({M}, {K}, {N}) == 1
+for a in (None, 16):
+  count.value = 0
+  rc = lib.tmx_qlora_linear(None, 16, 16, 16, a, a, None, 16, 1 << 20, {M}, {K}, {N}, 64, {r}, {(r + 31) // 32 * 32}, 2.0)
+  print(rc, *grids[:count.value])
+"""
+  res = subprocess.run([sys.executable, '-c', child], capture_output=True, text=True)
+  assert res.returncode == 0, res.stderr
+  plain, lora = [[int(v) for v in line.split()] for line in res.stdout.splitlines()]
+  assert plain[0] == lora[0] == 0 and len(plain) == 2
+  row_tiles = (M + 31) // 32
+  assert len(lora) == 4 and lora[2] >= row_tiles and lora[3] == plain[1]

@@ -1779,7 +1779,9 @@ int qlinear_wide(hipStream_t st, const void* x, int ldx, const void* qw, const v
                  int M, int K, int N, int G, int Rpad, int nsplit, bool* fused) {
   if (!x || !qw || !scales || (nsplit == 1 ? !y_bf16 : !y_part)) return TMX_ERR_ARG;
   *fused = nsplit == 1 && (!a_t || r % 8 == 0);
-  if (a_t && (!lora_b || !w.t_part || !(*fused ? (void*)w.t16 : (void*)w.t_fin) || !w.sync || !w.sync_clear || r <= 0))
+  // a wait that runs out drops the LoRA term: somebody has to be told (status), or nothing may wait (ordered)
+  if (a_t && (!lora_b || !w.t_part || !(*fused ? (void*)w.t16 : (void*)w.t_fin) || !w.sync || r <= 0 ||
+              (!w.ordered && (!w.sync_clear || !w.status))))
     return TMX_ERR_ARG;
   if (M <= 128 || K % 128 || N % 32 || G % 64 || (G & (G - 1)) || K % G || ldx % 8) return TMX_ERR_SHAPE;
   if (a_t && (r > 64 || Rpad <= 0 || Rpad % 32 || Rpad > TMX_MAX_RPAD)) return TMX_ERR_SHAPE;
@@ -1808,7 +1810,7 @@ int qlinear_wide(hipStream_t st, const void* x, int ldx, const void* qw, const v
     a.kt_per_lora_split = (KT + n - 1) / n;
     a.n_lora_slices = (KT + a.kt_per_lora_split - 1) / a.kt_per_lora_split;
     a.sync = w.sync;
-    a.sync_clear = w.sync_clear;
+    a.sync_clear = w.ordered ? nullptr : w.sync_clear;
     a.sync_status = w.status;
     if (*fused) {
       a.t16 = w.t16;
@@ -1819,6 +1821,12 @@ int qlinear_wide(hipStream_t st, const void* x, int ldx, const void* qw, const v
       for (int i = 0; i < 3; ++i) a.seg_end[i] = seg_end ? seg_end[i] : N;
     } else {
       a.t_fin = w.t_fin;
+    }
+    if (w.ordered) {
+      const int rc = qwide_lora_launch(st, a);
+      if (rc != TMX_OK) return rc;
+      a.a_t = nullptr;  // t is there: no LoRA workgroups in the projection's launch, and no flags to wait for
+      a.sync = nullptr;
     }
   }
   return qwide_launch(st, a);
@@ -1894,9 +1902,9 @@ extern "C" int tmx_int4_dequant(void* stream, const void* qweight, const void* s
 
 extern "C" size_t tmx_qlora_linear_workspace_bytes(int M, int K, int N) {
   const size_t s = qlinear_num_splits(K, N, M);
-  // f32 K-slice planes, f32 LoRA planes; many rows: bf16 LoRA projection and its hand-over areas
+  // f32 K-slice planes, f32 LoRA planes; many rows: bf16 LoRA projection and the arrival counts of its slices
   return (s * (size_t)M * N + (size_t)TMX_MAX_LORA_SPLITS * M * TMX_MAX_RPAD) * sizeof(float) +
-         (M > 128 ? (size_t)M * TMX_MAX_RPAD * 2 + 2 * wide_sync_words() * 4 : 0);
+         (M > 128 ? (size_t)M * TMX_MAX_RPAD * 2 + wide_sync_words() * 4 : 0);
 }
 
 extern "C" int tmx_qlora_linear_num_splits(int M, int K, int N) { return qlinear_num_splits(K, N, M); }
@@ -1961,13 +1969,14 @@ extern "C" int tmx_qlora_linear(void* stream, const void* x, const void* qweight
   float* y_part = (float*)workspace;
   float* t_part = y_part + (size_t)ns * M * N;
   if (M > 128 && M <= TMX_MAX_FILL_ROWS && !residual && ns == 1 && (!lora || (r % 8 == 0 && r <= 64))) {
-    // many rows, unsplit: LoRA in the projection's epilogue
+    // Many rows, unsplit: LoRA in the projection's epilogue.  t by a launch of its own: a caller that sees TMX_OK relies
+    // on y, and has no word to ask whether a wait inside a launch ran out.
     WideLora w = {};
+    w.ordered = true;
     w.t_part = t_part;
     w.t16 = (uint16_t*)(t_part + (size_t)TMX_MAX_LORA_SPLITS * M * TMX_MAX_RPAD);
     if (lora) {
       w.sync = (uint32_t*)(w.t16 + (size_t)M * TMX_MAX_RPAD);
-      w.sync_clear = w.sync + wide_sync_words();
       const int zrc = zero_words(st, w.sync, (int)wide_sync_words());
       if (zrc != TMX_OK) return zrc;
     }

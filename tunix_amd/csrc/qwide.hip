@@ -171,8 +171,8 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
     }
   }
   bool t_ready = true;
-  if (a.t16) {
-    // t of this block's rows comes from the LoRA workgroups of the launch: wait (a bounded number of polls) for the
+  if (a.t16 && a.sync) {
+    // t of this block's rows comes from the LoRA workgroups of the launch (without a.sync: of a launch before): wait (a bounded number of polls) for the
     // flags of its row tiles
     __shared__ uint32_t s_late;
     if (tid == 0) s_late = 0u;
@@ -259,7 +259,7 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
 // hand-over area (a.sync) the last slice of the row tile to arrive adds the planes in slice order and writes the
 // rounded t: bf16 for the epilogues of this launch (a.t16, then its ready flag), f32 for a consumer behind it
 // (a.t_fin).  Stores are write-through and loads go past L2 (sc1), so no cache write-back happens inside the
-// launch.  These workgroups come first in dispatch order and wait for nobody.  What bounds them is latency: about 8 us
+// launch.  In the projection's launch these workgroups come first in dispatch order and wait for nobody.  What bounds them is latency: about 8 us
 // at 256 rows, hidden behind the main workgroups' loop, where a LoRA-only launch and a reduction launch in front of the
 // projection took 14 + 5 us (decode step of 256 sequences, 8 layers: 3.43 -> 3.25 ms).
 __device__ __forceinline__ void wide_lora_block(const QLinearArgs& a, float* red, int id) {
@@ -435,6 +435,17 @@ WidePlan wide_plan(int M, int N, int K, int nsplit) {
     }
   }
   return best;
+}
+
+// t in a launch of its own, ordered in front of the projection, for callers that have no word to ask whether a wait ran
+// out (tmx_qlora_linear).  It costs the launch, 2 to 7 us: 300 x 4096 x 12288 with rank 16 takes 63 us against 57 with
+// the LoRA workgroups inside, 4096 x 4096 x 28672 841 against 840.
+int qwide_lora_launch(hipStream_t st, QLinearArgs a) {
+  static_assert(wide_lds(2) >= 8 * 16 * 64 * 4, "the accumulators of the 8 waves meet in LDS");
+  if (!a.a_t || !a.sync || a.M > TMX_MAX_FILL_ROWS) return TMX_ERR_ARG;
+  a.lora_wgs = ((a.M + 31) / 32 * a.n_lora_slices + 7) / 8 * 8;
+  hipLaunchKernelGGL((qlinear_mfma_wide_kernel<2, 4>), dim3(a.lora_wgs), dim3(512), wide_lds(2), st, a, 1, 1, 1);
+  return check_launch();
 }
 
 int qwide_launch(hipStream_t st, const QLinearArgs& a) {

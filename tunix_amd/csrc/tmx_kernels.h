@@ -332,6 +332,7 @@ inline bool slices_ok(int KT, int s) { return (KT + slice_len(KT, s) - 1) / slic
 struct WidePlan { int mt, ct, nsplit; };
 WidePlan wide_plan(int M, int N, int K, int nsplit);  // nsplit 0: its choice
 int qwide_launch(hipStream_t st, const QLinearArgs& a);
+int qwide_lora_launch(hipStream_t st, QLinearArgs a);  // the LoRA workgroups of such a launch by themselves
 // What the LoRA half of a many-rows projection hands over inside its launch.  Two areas of wide_sync_words() words take
 // turns: a launch uses one, which has to be zero, and clears the other.
 struct WideLora {
@@ -340,7 +341,8 @@ struct WideLora {
   float* t_fin;        // [M][TMX_MAX_RPAD] f32
   uint32_t* sync;      // this launch's area
   uint32_t* sync_clear;
-  uint32_t* status;    // set to 1 when a wait runs out (may be null)
+  uint32_t* status;    // set to 1 when a wait runs out
+  bool ordered;        // t in a launch of its own in front: nothing waits, sync_clear and status are not used
 };
 inline size_t wide_sync_words() { return 2 * (TMX_MAX_FILL_ROWS / 32); }
 // Many rows (M > 128), LoRA included: t = bf16(x . A) by the LoRA workgroups of the launch.  With nsplit == 1 and
