@@ -64,9 +64,12 @@ extern "C" {
                               :207-226 selective_log_softmax) */
 
 const char* tmx_status_string(int status);
-/* Bumped whenever a struct of this header grows or an entry point changes: 7 = tmx_model_desc.head_tiles and the
- * tmx_decode_state.share_* fields are present.  A caller that fills the structs checks it once after loading. */
-#define TMX_ABI_VERSION 7
+/* Bumped whenever a struct of this header grows or an entry point is added or changes.  A caller checks it once after
+ * loading, before it looks up anything else.
+ *   7: tmx_model_desc.head_tiles and the tmx_decode_state.share_* fields
+ *   8: tmx_lora_pack and tmx_fill_ragged; tokens_per_pass up to TMX_MAX_FILL_ROWS / batch (128 before);
+ *      tmx_qlora_linear needs a larger workspace for more than 128 rows */
+#define TMX_ABI_VERSION 8
 int tmx_abi_version(void);
 
 /* w_out[K, N] bf16 = bf16(q) * scale evaluated in bf16, bit-exact.

@@ -51,9 +51,9 @@ def test_header_is_plain_c_and_cxx():
 
 def test_status_strings_and_version():
   lib = _lib.lib()
-  assert lib.tmx_abi_version() == 7 == _lib.ABI_VERSION
+  assert lib.tmx_abi_version() == 8 == _lib.ABI_VERSION
   header = open(os.path.join(os.path.dirname(os.path.abspath(__file__)), '..', 'include', 'tmx.h')).read()
-  assert '#define TMX_ABI_VERSION 7' in header
+  assert '#define TMX_ABI_VERSION 8' in header
   assert lib.tmx_status_string(0) == b'ok'
   for code in (-1, -2, -3, -4):
     assert len(lib.tmx_status_string(code)) > 5
@@ -183,6 +183,19 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
   monkeypatch.setattr(_lib, '_lib', None)
   monkeypatch.setattr(_lib, 'LIB_PATH', str(tmp_path / 'nope.so'))
   with pytest.raises(_lib.TmxError, match='no CPU fallback'):
+    _lib.lib()
+
+
+@pytest.mark.parametrize('version', [None, 7, 9])
+def test_library_of_another_version_is_refused_before_its_symbols_are_looked_up(monkeypatch, version):
+  """An older library lacks entry points of this package: what the caller sees is the version, not the missing symbol."""
+  class Library:  # as ctypes.CDLL answers: AttributeError for what is not exported
+    def __init__(self, path):
+      if version is not None:
+        self.tmx_abi_version = lambda: version
+  monkeypatch.setattr(_lib, '_lib', None)
+  monkeypatch.setattr(_lib.ctypes, 'CDLL', Library)
+  with pytest.raises(_lib.TmxError, match=f'ABI version {version}, this package expects {_lib.ABI_VERSION}'):
     _lib.lib()
 
 
