@@ -127,6 +127,31 @@ def test_rmsnorm(family, M, D):
   G.assert_bf16_close(G.host(y), ref, ulps=1.0, min_exact=0.99, what='rmsnorm')
 
 
+# finished rows of a pass of more than 128: one, two and four chunks per thread (D up to 2048, 4096, 8192) with and
+# without a ragged last one, and the first D behind them
+@pytest.mark.parametrize('family', [0, 1])
+@pytest.mark.parametrize('M,D', [(129, 256), (200, 2040), (129, 2048), (131, 2056), (300, 4096), (129, 4104), (130, 8192), (129, 8200)])
+def test_row_norm_of_many_finished_rows(family, M, D):
+  T = G.Keep()
+  rng = np.random.default_rng(D + family)
+  y = bf16_round(rng.standard_normal((M, D)).astype(np.float32) * 3)
+  res = bf16_round(rng.standard_normal((M, D)).astype(np.float32))
+  w = bf16_round(rng.uniform(0.5, 1.5, D).astype(np.float32))
+  norm = L.rmsnorm_llama3 if family == 0 else L.rmsnorm_qwen3
+  for use_res, use_norm in ((False, True), (True, True), (True, False)):
+    h = bf16_round(y + res) if use_res else y
+    x = G.bf(res)  # the residual stream, updated in place
+    xn = torch.full((M, D), 7.0, dtype=torch.bfloat16, device=G.DEV)
+    G.call('tmx_lora_residual_rmsnorm', S(), T.bf(y), None, 0, None, 0, 0, None, 0, 0.0, G.p(x) if use_res else None, G.p(x),
+           T.bf(w) if use_norm else None, G.p(xn), M, D, 1e-6, family)
+    G.sync()
+    np.testing.assert_array_equal(G.host(x), h)
+    if use_norm:  # the sum of squares in another order: a last bit of the rounded result
+      G.assert_bf16_close(G.host(xn), norm(h, w, 1e-6, BF16), ulps=1.0, min_exact=0.99, what=f'norm {M}x{D}')
+    else:
+      assert torch.all(xn == 7.0)
+
+
 @pytest.mark.parametrize('family', [0, 1])
 def test_lora_residual_rmsnorm_planes(family):
   T = G.Keep()

@@ -5,17 +5,19 @@ import numpy as np
 import pytest
 import torch
 
+from oracle import layers as OL
 from oracle import masks as OMK
 from oracle import model as OM
 from oracle import prng
 from oracle import sampler as OSAM
 from oracle import sampling as OS
-from oracle.bf16 import bf16_round
+from oracle.bf16 import BF16, bf16_round
 from tunix_amd.configs import CacheConfig, RolloutConfig
 from tunix_amd.rollout import TmxRollout
 from tunix_amd.sampler import Sampler
 
 import common as C
+import gpu_util as G
 
 pytestmark = pytest.mark.gpu
 
@@ -793,3 +795,69 @@ def test_earlier_rollout_of_nans_leaves_nothing_in_the_caches(lengths):
     assert np.isfinite(np.array(got.logprobs)).all()
     np.testing.assert_array_equal(np.stack(got.tokens), np.stack(want.tokens))
     np.testing.assert_array_equal(np.array(got.logprobs), np.array(want.logprobs))
+
+
+# head dimension, embedding width (K-slices of the projection), sequences, tokens of each per pass, rank: one token with
+# f32 planes (one plane, several, more planes of t than LDS holds, more heads than a workgroup takes), passes of many
+# finished rows and of planes, one whose rank leaves LoRA to the rotation, and passes with a row map
+@pytest.mark.parametrize('family', ['llama3', 'qwen3'])
+@pytest.mark.parametrize('H,D,n_seq,T,rank,ragged', [
+    (64, 256, 5, 1, 8, False), (128, 2048, 7, 1, 8, False), (128, 8192, 6, 1, 40, False), (64, 2048, 9, 3, 0, False),
+    (128, 256, 9, 17, 16, False), (64, 2048, 9, 17, 16, False),
+    (64, 256, 10, 13, 12, False), (128, 2048, 4, 20, 8, True), (64, 256, 11, 29, 16, True)])
+def test_rotated_heads_of_whole_passes_match_oracle(family, H, D, n_seq, T, rank, ragged):
+  """q, k and v of the first layer as a pass leaves them: LoRA, Qwen3's head norms, the rotation at each row's position,
+  the cache slot of each row's column.  q is read where the pass keeps it in its workspace."""
+  N, Kh = (16, 4) if H == 128 else (8, 2)
+  cfg = OM.Config(family, 1, 512, D, 256, N, H, Kh, rope_theta=1_000_000, norm_eps=1e-6)
+  st0 = C.make_state(cfg, 3 + T, rank, targets=('q_proj', 'k_proj', 'v_proj'), norm_jitter=0.05)
+  lw = C.oracle_weights(cfg, st0, 64, 16.0, rank)['layers'][0]
+  model = C.product_model(cfg, st0, 64, 16.0)
+  rng = np.random.default_rng(n_seq)
+  ids = rng.integers(3, 512, (n_seq, T)).astype(np.int32)
+  for i in range(n_seq if ragged else 0):
+    ids[i, :(i * 5) % T] = 0  # left padding
+  s = _sampler(model, cfg, T + 8)
+  s.share_prompt_kv = False
+  s.eos_ids = np.array([-1])
+  st = s.init_sample_state(ids, T + 4, False, None, 0.0, None, None, 0)
+  if ragged:
+    s.walk(st, T)
+    rows = [(i, t) for i in range(n_seq) for t in range(st['first_col_host'][i], T)]
+  else:
+    s.run_steps(st, 1, sample=False, tokens_per_pass=T)
+    rows = [(i, t) for i in range(n_seq) for t in range(T)]
+  align = lambda n: (n + 255) // 256 * 256
+  q_at = 256 + 2 * align(len(rows) * D * 2)  # workspace: status word, residual stream, normed rows, q
+  got_q = s._workspace[q_at:q_at + len(rows) * N * H * 2].view(torch.bfloat16).float().cpu().numpy().reshape(-1, N, H)
+  cache = st['cache'][0].float().cpu().numpy()  # [k | v][sequence][slot][Kh][H]
+  seq, col = np.array(rows).T
+  # the normed rows by the row kernel itself (a last bit of theirs moves small sums by more than a bit), which takes up to
+  # 128 finished rows for what the pass does
+  x = st0['embedder.input_embedding'][ids[seq, col]]
+  xn = []
+  for part in np.array_split(x, -(-len(x) // 128)):
+    xt, yt = G.bf(part), torch.empty(part.shape, dtype=torch.bfloat16, device=G.DEV)
+    G.call('tmx_rmsnorm', None, G.p(xt), G.p(model.layers[0]['norm1']), G.p(yt), len(part), D, 1e-6, int(family == 'qwen3'))
+    xn.append(G.host(yt))
+  xn = np.concatenate(xn)
+  q, k, v = (lw[n](xn, BF16).reshape(len(rows), 1, -1, H) for n in 'qkv')
+  pos = st['positions_host'][seq, col][:, None]
+  if family == 'qwen3':
+    q, k = OL.rmsnorm_qwen3(q, lw['q_norm'], 1e-6, BF16), OL.rmsnorm_qwen3(k, lw['k_norm'], 1e-6, BF16)
+    rope = lambda u: OL.rope_qwen3(u, pos, cfg.rope_theta, BF16)[:, 0]
+  else:
+    rope = lambda u: OL.rope_llama3(u, pos, 1_000_000, BF16)[:, 0]
+
+  def close(got, want, what):
+    # a last bit of the two elements that the rotation mixes (of the projection, of its LoRA delta, of the sum of both,
+    # of the head norm): the two elements together are as large as after the rotation
+    pair = np.sqrt(want[..., :H // 2] ** 2 + want[..., H // 2:] ** 2)
+    G.assert_bf16_close(got, want, ulps=1.0, extra=4.0 * G.ulp_bf16(np.concatenate([pair, pair], axis=-1)), min_exact=0.97,
+                        what=what)
+  close(got_q, rope(q), 'q')
+  close(cache[0][seq, col], rope(k), 'k rows')
+  close(cache[1][seq, col], v[:, 0], 'v rows')
+  rest = np.ones(cache.shape[1:3], bool)
+  rest[seq, col] = False
+  assert not cache[:, rest].any()  # no other slot is written

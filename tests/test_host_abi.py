@@ -282,6 +282,43 @@ def test_update_params_accepts_nested_states_and_keeps_the_reference_errors():
     s.transformer_state = {'layers.0.attn.q_proj.w_lora_a': a}  # the setter wants the whole LoRA state
 
 
+@pytest.mark.parametrize('device', ['cpu', pytest.param('cuda', marks=pytest.mark.gpu)])
+def test_adapter_sync_takes_any_subset_layout_and_dtype(device):
+  """merge_lora: some of the adapters and none, transposed and 3-D tensors, other dtypes, host arrays for a model on the
+  GPU; the others keep their values, and a state that is refused changes nothing."""
+  import torch
+  from tunix_amd.model import QLoRAModel
+  m = QLoRAModel.random_init(ModelConfig.toy(), seed=3, lora_rank=8, lora_alpha=16.0, device=device)
+  want = {k: v.clone() for k, v in m.lora_state().items()}
+  g = torch.Generator().manual_seed(5)
+  new = lambda name, dtype=torch.float32: torch.randn(*want[name].shape, generator=g).to(dtype)
+  p, q = 'layers.0.', 'layers.1.'
+  wide = new(p + 'attn.q_proj.w_lora_a')
+  sent = {p + 'attn.q_proj.w_lora_a': torch.cat([wide, wide], dim=1)[:, :8],                       # a slice
+          p + 'attn.v_proj.w_lora_b': new(p + 'attn.v_proj.w_lora_b').t().contiguous().t(),          # transposed
+          p + 'mlp.up_proj.kernel_lora_a': new(p + 'mlp.up_proj.kernel_lora_a', torch.float64),
+          p + 'mlp.down_proj.kernel_lora_b': new(p + 'mlp.down_proj.kernel_lora_b', torch.float16).requires_grad_(),
+          q + 'attn.k_proj.w_lora_b': new(q + 'attn.k_proj.w_lora_b', torch.bfloat16).reshape(8, 4, 64),
+          q + 'attn.o_proj.w_lora_a': new(q + 'attn.o_proj.w_lora_a').reshape(4, 64, 8).numpy()}
+  on_device = {p + 'attn.q_proj.w_lora_a', p + 'attn.v_proj.w_lora_b', q + 'attn.k_proj.w_lora_b'}
+  for name, v in sent.items():
+    want[name] = torch.as_tensor(v).detach().to(torch.bfloat16).reshape(want[name].shape).to(device)
+
+  def same():
+    got = m.lora_state()
+    return set(got) == set(want) and all(torch.equal(got[k], want[k]) for k in want)
+  m.merge_lora({k: v.to(device) if k in on_device else v for k, v in sent.items()})
+  assert same()
+  m.merge_lora({})
+  assert same()
+  good = {p + 'attn.q_proj.w_lora_a': torch.zeros(256, 8)}
+  with pytest.raises(ValueError, match='same structure'):
+    m.merge_lora({**good, p + 'attn.z_proj.w_lora_a': torch.zeros(256, 8)})
+  with pytest.raises(ValueError, match='same shape'):
+    m.merge_lora({**good, q + 'attn.q_proj.w_lora_a': torch.zeros(256, 4)})
+  assert same()
+
+
 def test_seed_words_follow_prngkey_without_x64():
   from oracle import prng
   from tunix_amd.sampler import _seed_key
