@@ -861,3 +861,24 @@ def test_rotated_heads_of_whole_passes_match_oracle(family, H, D, n_seq, T, rank
   rest = np.ones(cache.shape[1:3], bool)
   rest[seq, col] = False
   assert not cache[:, rest].any()  # no other slot is written
+
+
+# one pass and several, up to and over 128 rows, fewer tokens than a block of the attention, a last pass of one column
+@pytest.mark.parametrize('n_seq,p,limit', [(4, 33, 4096), (1, 5, 4096), (7, 60, 4096), (5, 61, 150), (3, 4, 4096), (40, 13, 160)])
+def test_cache_fill_without_padding_equals_the_ragged_pass(n_seq, p, limit):
+  """Nothing to leave out: the pass over all columns leaves the cache of the pass that plans its rows, bit for bit."""
+  cfg = C.TOY
+  model = C.product_model(cfg, C.make_state(cfg, 43, 8, norm_jitter=0.05), 64, 16.0)
+  ids = np.random.default_rng(p).integers(3, cfg.vocab_size, (n_seq, p)).astype(np.int32)
+  caches = []
+  for min_tokens in (Sampler.MIN_BLOCK_TOKENS, 1 << 30):
+    s = _sampler(model, cfg, p + 8)
+    s.MAX_ROWS = s.MAX_FILL_ROWS = limit
+    s.MIN_BLOCK_TOKENS = min_tokens
+    s.share_prompt_kv = False
+    s.eos_ids = np.array([-1])
+    st = s.init_sample_state(ids, p + 4, False, None, 0.0, None, None, 0)
+    s.walk(st, p - 1)
+    assert int(st['step'].item()) == p - 1 and (st['first_col'] is None) == (min_tokens == 4 and p - 1 >= 4)
+    caches.append(st['cache'].clone())
+  assert caches[0].any() and torch.equal(caches[0], caches[1])

@@ -249,8 +249,8 @@ class Sampler:
     dev = self._transformer.device
     st['input_mask_host'] = mask
     st['input_mask'] = torch.from_numpy(mask.astype(np.uint8)).to(dev)
-    first = np.where(mask.any(axis=1), mask.argmax(axis=1), mask.shape[1]).astype(np.int32)
-    st['first_col_host'], st['first_col'] = first, torch.from_numpy(first).to(dev)
+    st['first_col_host'] = np.where(mask.any(axis=1), mask.argmax(axis=1), mask.shape[1]).astype(np.int32)
+    st['first_col'] = None  # on the device once a pass asks for it
 
   def _c_state(self, st, tokens_per_pass=1, rows=None):
     b, total = st['token_buffer'].shape
@@ -301,6 +301,7 @@ class Sampler:
   MAX_FILL_ROWS = 4096  # rows of one cache-fill or scoring pass of a dense model (256-row projection blocks)
 
   MAX_MOE_PAIRS = 8192  # routed (token, expert) pairs of one pass of a MoE model
+  MIN_BLOCK_TOKENS = 4  # tokens per sequence from which a pass over all columns runs the attention that ragged passes run
   MAX_PASSES_IN_FLIGHT = 64  # passes a walk enqueues before it waits for the stream
 
   def _max_rows(self):
@@ -373,8 +374,11 @@ class Sampler:
     end = col + n_tokens
     rows_upto = lambda c: int(np.maximum(c - np.maximum(first, col), 0).sum())
     total, limit = rows_upto(end), self._fill_rows()
-    passes = max(1, -(-total // limit))
-    target = min(limit, -(-total // passes // 256) * 256) if passes > 1 else limit
+    if total <= limit:
+      yield n_tokens, total
+      return
+    passes = -(-total // limit)
+    target = min(limit, -(-total // passes // 256) * 256)
     while col < end:
       lo, hi = col + 1, end  # the last column that keeps the pass within `target` rows
       while lo < hi:
@@ -391,6 +395,12 @@ class Sampler:
     if rows == 0:
       st['step'].add_(width)
       return
+    if rows == width * st['token_buffer'].shape[0] and width >= self.MIN_BLOCK_TOKENS:
+      # nothing to leave out: the same rows and kernels without the plan of the rows and its copy to the device
+      self.run_steps(st, 1, sample=False, tokens_per_pass=width)
+      return
+    if st['first_col'] is None:
+      st['first_col'] = torch.from_numpy(st['first_col_host']).to(self._transformer.device)
     cs = self._c_state(st, 1, rows)
     rc = self._lib.tmx_fill_ragged(ctypes.byref(self._transformer.desc()), ctypes.byref(cs), _lib.stream(),
                                    st['first_col'].data_ptr(), width, rows)
@@ -417,8 +427,8 @@ class Sampler:
     sub = dict(st)
     sub.update({
         'token_buffer': st['token_buffer'][lead].contiguous(), 'positions': st['positions'][lead].contiguous(),
-        'input_mask': st['input_mask'][lead].contiguous(), 'first_col': st['first_col'][lead].contiguous(),
-        'first_col_host': st['first_col_host'][::g], 'done': torch.zeros(b // g, dtype=torch.uint8, device=dev),
+        'input_mask': st['input_mask'][lead].contiguous(), 'first_col': None,
+        'first_col_host': np.ascontiguousarray(st['first_col_host'][::g]), 'done': torch.zeros(b // g, dtype=torch.uint8, device=dev),
         'logprobs': None, 'logits': None, 'step': torch.zeros(1, dtype=torch.int32, device=dev),
         'cache': self._lead_cache, 'share_group': 1, 'share_len': 0, 'share_common': 0, 'fresh': True})
     self.walk(sub, n)
