@@ -797,14 +797,16 @@ def test_earlier_rollout_of_nans_leaves_nothing_in_the_caches(lengths):
     np.testing.assert_array_equal(np.array(got.logprobs), np.array(want.logprobs))
 
 
-# head dimension, embedding width (K-slices of the projection), sequences, tokens of each per pass, rank: one token with
-# f32 planes (one plane, several, more planes of t than LDS holds, more heads than a workgroup takes), passes of many
-# finished rows and of planes, one whose rank leaves LoRA to the rotation, and passes with a row map
+# head dimension, embedding width (K-slices of the projection), sequences, tokens of each per pass, rank.  Up to 128 rows,
+# a wave per head: one token with f32 planes (one plane, several, many planes of t), several tokens, a row map.  More rows,
+# several heads per wave (8 and 24 of 16 or 32 per workgroup): finished rows, planes, a rank that leaves LoRA to the rotation,
+# without and with a row map
 @pytest.mark.parametrize('family', ['llama3', 'qwen3'])
 @pytest.mark.parametrize('H,D,n_seq,T,rank,ragged', [
     (64, 256, 5, 1, 8, False), (128, 2048, 7, 1, 8, False), (128, 8192, 6, 1, 40, False), (64, 2048, 9, 3, 0, False),
     (128, 256, 9, 17, 16, False), (64, 2048, 9, 17, 16, False),
-    (64, 256, 10, 13, 12, False), (128, 2048, 4, 20, 8, True), (64, 256, 11, 29, 16, True)])
+    (64, 256, 10, 13, 12, False), (128, 2048, 9, 17, 40, False), (64, 256, 129, 1, 0, False),
+    (128, 2048, 4, 20, 8, True), (64, 256, 11, 29, 16, True), (128, 512, 12, 20, 12, True)])
 def test_rotated_heads_of_whole_passes_match_oracle(family, H, D, n_seq, T, rank, ragged):
   """q, k and v of the first layer as a pass leaves them: LoRA, Qwen3's head norms, the rotation at each row's position,
   the cache slot of each row's column.  q is read where the pass keeps it in its workspace."""

@@ -519,11 +519,15 @@ __global__ __launch_bounds__(64) void rope_kvwrite_kernel(RopeArgs a) {
   }
 }
 
-// The same for head_dim 64 and 128 with 16-byte pieces of a head instead of single elements: H / 8 lanes own a head, a
-// lane the elements 4 i .. 4 i + 3 and their partners H / 2 further on; a workgroup of 256 takes 2048 / H heads of a
-// row.  One wave per head made a launch of (N + 2 Kh) B workgroups with 2-byte loads: 256 rows of 48 heads 13.4 us, 64
-// rows 6.2 us, of which the dispatch of the workgroups was most.  Every value is made by the same operations in the
-// same order.
+// The same for head_dim 64 and 128 and more than 128 rows, with 8-byte pieces of a head instead of single elements: H / 8
+// lanes own a head, a lane the elements 4 i .. 4 i + 3 and their partners H / 2 further on; a workgroup of 256 takes
+// 2048 / H heads of a row.  One wave per head is a launch of (N + 2 Kh) B workgroups with 2-byte loads, whose dispatch
+// bounds it at many rows; at few rows its workgroups, without a barrier between them, finish sooner.  Measured (trace, us,
+// one wave per head / this kernel), 48 heads of 128: 32 rows 5.0 / 5.8, 64 rows 5.7 / 6.3, 128 rows 7.3 / 8.0, 160 rows
+// 9.8 / 8.1, 256 rows 11.5 / 9.0, 1024 rows (40 heads) 31 / 10.6; with Qwen3's head norms 64 rows 6.8 / 8.1, 128 rows
+// 9.3 / 10.9, 160 rows 12.4 / 10.6.  Both round at the same points; last bits may differ, since the sum of squares of a head
+// norm takes four pairs per lane and then H / 8 lanes here, one pair per lane and then all of them there, and which
+// products are fused with a sum is the compiler's choice in each.
 __device__ __forceinline__ void unpack4(const uint2& v, float* o) {
   o[0] = bf_lo(v.x); o[1] = bf_hi(v.x); o[2] = bf_lo(v.y); o[3] = bf_hi(v.y);
 }
@@ -531,7 +535,6 @@ template <int H>
 __global__ __launch_bounds__(256) void rope_heads_kernel(RopeArgs a) {
   constexpr int LPH = H / 8, HPW = 256 / LPH, half = H / 2;
   __shared__ float t_s[TMX_MAX_RPAD];
-  __shared__ float t_stage[TMX_MAX_LORA_SPLITS * 64];
   const int b = blockIdx.y, B = gridDim.y;
   const int lane = threadIdx.x & (LPH - 1), nheads = a.N + 2 * a.Kh;
   const int head = blockIdx.x * HPW + threadIdx.x / LPH, hd = min(head, nheads - 1);
@@ -570,13 +573,8 @@ __global__ __launch_bounds__(256) void rope_heads_kernel(RopeArgs a) {
     for (int e = 0; e < 4; ++e) { x1[e] = rbf(x1[e]); x2[e] = rbf(x2[e]); }
   }
   if (lora) {
-    // t of all three segments (a workgroup's heads may lie in several)
-    if (3 * a.lora.r * a.lora.nsplit <= TMX_MAX_LORA_SPLITS * 64) {
-      stage_t_block(t_s, t_stage, a.lora, b, B, 0, 3 * a.lora.r);
-    } else {
-      stage_t(t_s, a.lora, b, B, 0, 3 * a.lora.r);
-      __syncthreads();
-    }
+    stage_t(t_s, a.lora, b, B, 0, 3 * a.lora.r);  // t of all three segments (a workgroup's heads may lie in several)
+    __syncthreads();
     float d1[4] = {0.f, 0.f, 0.f, 0.f}, d2[4] = {0.f, 0.f, 0.f, 0.f};
     const float* t = t_s + kind * a.lora.r;
 #pragma unroll 8
@@ -651,7 +649,7 @@ int rope_kvwrite(hipStream_t st, const RopeArgs& a, int B) {
   if (a.H > 128 || a.H % 2) return TMX_ERR_SHAPE;
   if (a.lora.t_part && a.lora.r > 64) return TMX_ERR_SHAPE;
   // the table comes from the row kernel of the pass; both head norms or none; t of the three segments in one row
-  if (a.rope_tab && (a.H == 64 || a.H == 128) && !a.q_norm_w == !a.k_norm_w && (!a.lora.t_part || 3 * a.lora.r <= TMX_MAX_RPAD)) {
+  if (B > 128 && a.rope_tab && (a.H == 64 || a.H == 128) && !a.q_norm_w == !a.k_norm_w && (!a.lora.t_part || 3 * a.lora.r <= TMX_MAX_RPAD)) {
     const int hpw = 2048 / a.H;
     const dim3 grid((a.N + 2 * a.Kh + hpw - 1) / hpw, B);
     if (a.H == 128) hipLaunchKernelGGL(rope_heads_kernel<128>, grid, dim3(256), 0, st, a);
