@@ -503,8 +503,8 @@ __global__ __launch_bounds__(64) void rope_kvwrite_kernel(RopeArgs a) {
     }
     float o1, o2;
     if (a.family == TMX_FAMILY_LLAMA3) {
-      o1 = x1 * cs - x2 * sn;
-      o2 = x2 * cs + x1 * sn;
+      o1 = fmaf(x1, cs, -(x2 * sn));  // which product is fused is said, so that every row count rotates alike
+      o2 = fmaf(x2, cs, x1 * sn);
     } else {
       sn = rbf(sn);
       cs = rbf(cs);
@@ -525,9 +525,8 @@ __global__ __launch_bounds__(64) void rope_kvwrite_kernel(RopeArgs a) {
 // bounds it at many rows; at few rows its workgroups, without a barrier between them, finish sooner.  Measured (trace, us,
 // one wave per head / this kernel), 48 heads of 128: 32 rows 5.0 / 5.8, 64 rows 5.7 / 6.3, 128 rows 7.3 / 8.0, 160 rows
 // 9.8 / 8.1, 256 rows 11.5 / 9.0, 1024 rows (40 heads) 31 / 10.6; with Qwen3's head norms 64 rows 6.8 / 8.1, 128 rows
-// 9.3 / 10.9, 160 rows 12.4 / 10.6.  Both round at the same points; last bits may differ, since the sum of squares of a head
-// norm takes four pairs per lane and then H / 8 lanes here, one pair per lane and then all of them there, and which
-// products are fused with a sum is the compiler's choice in each.
+// 9.3 / 10.9, 160 rows 12.4 / 10.6.  Every value is made by the same operations in the same order, but for the sum of
+// squares of a head norm: four pairs per lane and then H / 8 lanes here, one pair per lane and then all of them there.
 __device__ __forceinline__ void unpack4(const uint2& v, float* o) {
   o[0] = bf_lo(v.x); o[1] = bf_hi(v.x); o[2] = bf_lo(v.y); o[3] = bf_hi(v.y);
 }
@@ -623,8 +622,8 @@ __global__ __launch_bounds__(256) void rope_heads_kernel(RopeArgs a) {
     for (int e = 0; e < 4; ++e) {
       float o1, o2;
       if (a.family == TMX_FAMILY_LLAMA3) {
-        o1 = x1[e] * cs[e] - x2[e] * sn[e];
-        o2 = x2[e] * cs[e] + x1[e] * sn[e];
+        o1 = fmaf(x1[e], cs[e], -(x2[e] * sn[e]));
+        o2 = fmaf(x2[e], cs[e], x1[e] * sn[e]);
       } else {
         const float s = rbf(sn[e]), c = rbf(cs[e]);
         o1 = rbf(x1[e] * c) - rbf(x2[e] * s);
