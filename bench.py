@@ -215,7 +215,7 @@ def main():
         'data': 'synthetic (random-init weights, uniform-random token ids)',
         'config': {'workload': args.workload, 'shape': name, 'sequences': batch, 'prompt_len': prompt,
                    'scored_tokens': new, 'quant': f'int4 group {group}', 'lora_rank': rank,
-                   'rows_per_pass': min(sampler._fill_rows() // batch, 128) * batch},
+                   'rows_per_pass': -(-new // -(-new // max(1, sampler._fill_rows() // batch))) * batch},
     }))
     return
 
@@ -413,8 +413,8 @@ def main():
         return f'tmx::qlinear_mfma_dma_kernel<{mt}>'
       return f'tmx::qlinear_mfma_kernel<{mt}, 2>'
     if batch > 128 and not cfg.num_experts:
-      # more than 128 sequences (--sequences): every projection runs the 256-row kernel, the head in
-      # 256 x 256 blocks (the byte-based fractions below then understate these MFMA-bound kernels)
+      # more than 128 sequences (--sequences): every projection runs the many-rows kernel, in tiles chosen by
+      # shape (the byte-based fractions below then understate these MFMA-bound kernels)
       symbols = {'tmx::qlinear_mfma_wide_kernel': ['qkv_linear', 'o_linear', 'gate_up_linear', 'down_linear']}
       dense = []
     for cls_name, key in dense:
@@ -435,11 +435,11 @@ def main():
     on_tile = g_heads in (4, 8) and batch * cfg.num_kv_heads <= 3 * cus
     symbols.update({} if small else {
         f"tmx::gqa_{'tile' if on_tile else 'decode'}_kernel<{cfg.head_dim}, {g_heads}>": ['attention']})
-    symbols.update({
-        # more than 64 rows: the head in 256 x 256 blocks (template argument: the sampling mode, 1 = top-p branch);
-        # with top_p < 1 the class also holds the three selection launches of nucleus.hip
-        ('tmx::head_wide_kernel<1>' if batch > 64 else f'tmx::head_kernel<{min(mt, 2)}, true>'): ['head_sample'],
-    })
+    # the head from its tile copy, 65 to 256 rows by head_mid_kernel, more in 256 x 256 blocks (template argument 1:
+    # sampling); with top_p < 1 the class also holds the three selection launches of nucleus.hip
+    head_symbol = (f'head_kernel<{min(mt, 2)}, true>' if batch <= 64 else 'head_mid_kernel<4, 4, 4>' if batch <= 128 else
+                   'head_mid_kernel<8, 4, 4>' if batch <= 256 else 'head_wide_kernel<1>')
+    symbols.update({f'tmx::{head_symbol}': ['head_sample']})
     idx = {n: i for i, n in enumerate(CLASS_NAMES)}
     # An event pair around a launch also times the packet processing on both sides of it, so it
     # reads a few microseconds above rocprofv3's kernel trace (which brackets the dispatch
@@ -489,11 +489,11 @@ def main():
         result['roofline_all'][n] = {'avg_launch_ms': avg, 'achieved_GBps': alg[n] / (avg * 1e-3) / 1e9,
                                      'frac': alg[n] / (avg * 1e-3) / 8e12}
 
-  if not args.no_profile and not cfg.num_experts and sampler._fill_rows() > 128:
+  rows = min(sampler._fill_rows(), batch * (start - 1))  # of a full pass of the walk without sharing
+  if not args.no_profile and not cfg.num_experts and rows > 128:
     # Cache fill (outside the headline metric): the prompt walk above, and the projection kernel that
-    # carries it (256-row blocks, MFMA-bound) timed alone on the gate|up shape at the rows of one pass.
+    # carries it (MFMA-bound) timed alone on the gate|up shape at the rows of one pass.
     lib = _lib.lib()
-    rows = min(sampler._fill_rows() // batch, 128, start - 1) * batch
     pl = model.layers[0]['gate_up']
     xs = torch.randn(rows, pl.k, device='cuda').to(torch.bfloat16)
     ns = lib.tmx_qlora_linear_num_splits(rows, pl.k, pl.n)

@@ -79,7 +79,7 @@ int tmx_int4_dequant(void* stream, const void* qweight, const void* scales, void
                      int G);
 
 /* y[M, N] = bf16(x[M, K] . dequant(qweight)) (+ LoRA delta) (+ residual).  Up to 128 rows run
- * the decode kernels (K % 64 == 0); more rows run in 256-row blocks and need K % 128 == 0.
+ * the decode kernels (K % 64 == 0); more rows run in tiles of 64 to 256 rows and need K % 128 == 0.
  * Replaces the qwix-wrapped Einsum / nnx.Linear call: tunix/models/llama3/model.py:216-218,
  * :489-496; tunix/models/qwen3/model.py:389-393, :1199-1208.
  *   lora_a_t : A in MFMA fragment order, bf16 [K/64][r_pad/32][4][64][8], r_pad % 32 == 0,

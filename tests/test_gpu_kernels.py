@@ -46,7 +46,7 @@ def test_int4_dequant_bit_exact_exhaustive():
 @pytest.mark.parametrize('M,K,N,group,r', [
     (1, 256, 96, 64, 0), (4, 256, 256, 64, 8), (7, 512, 96, 64, 8), (33, 1024, 160, 128, 16),
     (64, 2048, 1024, 64, 16), (100, 512, 256, 64, 32), (128, 4096, 512, 128, 32), (64, 14336, 256, 64, 16),
-    # more than 128 rows: 256-row blocks (one partial, several, a ragged tail), with and without K-slices
+    # more than 128 rows: the many-rows kernel (one partial row block, several, a ragged tail), with and without K-slices
     (129, 256, 96, 64, 8), (256, 512, 160, 64, 16), (300, 1024, 256, 128, 16), (700, 4096, 512, 64, 32),
     (1024, 2048, 384, 64, 0), (520, 1152, 4096, 128, 16),
     # unsplit at many rows: LoRA inside the projection's epilogue (ranks 8, 16 and 32, ragged rows)

@@ -300,13 +300,15 @@ def test_temperature_sampling_follows_the_threefry_schedule():
   assert all((a == b).all() for a, b in zip(out.tokens, out3.tokens))
 
 
-def test_batches_over_128_sequences():
-  """More than 128 sequences per step: the projections run in 256-row blocks, the head takes the
-  rows 64 at a time.  Greedy rows spread over the batch against the oracle (a sequence does not
+@pytest.mark.parametrize('stream_head', [True, False])
+def test_batches_over_128_sequences(stream_head):
+  """More than 128 sequences per step: many-rows projections, the head from its tile copy or, without one, in
+  256 x 256 blocks (row by row where logits are asked for).  Greedy rows spread over the batch against the oracle (a sequence does not
   depend on its neighbours), temperature sampling against the threefry schedule over all rows
   (the noise counter is row * V + v), top-p through the sorting branch."""
   cfg = C.TOY
   oracle, model = _pair(cfg, seed=11, targets=('q_proj', 'k_proj', 'v_proj', 'o_proj', 'gate_proj', 'up_proj', 'down_proj'))
+  model.stream_head = stream_head
   rng = np.random.default_rng(6)
   nb = 150
   prompts = [rng.integers(3, cfg.vocab_size, 3 + (i * 7) % 10) for i in range(nb)]
@@ -337,21 +339,25 @@ def test_batches_over_128_sequences():
     want_lp = OS.log_softmax(z)[np.arange(nb), got]
     np.testing.assert_allclose([out.logprobs[b][step] for b in range(nb)], want_lp, atol=3e-5)
   assert agree >= total - 8
-  # without the logits output the 256 x 256 head kernel samples: same seed, same noise, logits equal up to
-  # the f32 summation order, so the tokens agree except at near-ties (after which a row goes its own way)
+  # without the logits output (another head kernel where there is no tile copy): same seed, same noise, logits equal up
+  # to the f32 summation order, so the tokens agree except at near-ties (after which a row goes its own way)
   out_w = s(prompt_token_ids=prompts8, max_generation_steps=4, return_logprobs=True, eos_tokens=[-1],
             temperature=0.9, top_p=1.0, seed=7)
   same = sum(int((np.asarray(out_w.tokens[b]) == np.asarray(out.tokens[b])).all()) for b in range(nb))
   assert same >= nb - 3, same
   first = np.array([out_w.logprobs[b][0] for b in range(nb)]) - np.array([out.logprobs[b][0] for b in range(nb)])
   assert np.abs(first).max() <= LOGPROB_TOL
-  # the sorting branch (top-p < 1): tokens come from the nucleus of the row's own logits
+  # the sorting branch (top-p < 1): tokens come from the nucleus of the row's own logits, and the same ones without the
+  # logits output (up to near-ties)
   out = s(prompt_token_ids=prompts8, max_generation_steps=3, return_logits=True, eos_tokens=[-1],
           temperature=1.0, top_p=0.5, seed=3)
   for b in (0, 64, 128, 149):
     for step in range(3):
       members = OS.nucleus_members(np.asarray(out.logits[b][step], np.float32), 0.5)
       assert out.tokens[b][step] in members, (b, step)
+  out_w = s(prompt_token_ids=prompts8, max_generation_steps=3, eos_tokens=[-1], temperature=1.0, top_p=0.5, seed=3)
+  same = sum(int((np.asarray(out_w.tokens[b]) == np.asarray(out.tokens[b])).all()) for b in range(nb))
+  assert same >= nb - 3, same
 
 
 def test_top_p_and_top_k_sampling_follow_the_reference_rule():
@@ -514,8 +520,8 @@ def test_graph_replay_matches_plain_launches_on_every_replay(nseq, top_p, group)
   program's own eager work (a plain step, host reads) and synchronisation between them; every
   call's tokens, logprobs, KV cache and step counter equal the plain launches'.  4 sequences: the
   small-batch launches; 150: the many-rows kernels; top_p < 1: the selection launches of the
-  top-p branch (6 sequences behind the 64-row head and the gate|up hand-over, 70 behind the head in
-  256 x 256 blocks) are recorded and replayed.  group > 1: four rows per 40-token prompt on a model with
+  top-p branch (6 sequences behind the 64-row head and the gate|up hand-over, 70 behind the head of
+  65 to 256 rows) are recorded and replayed.  group > 1: four rows per 40-token prompt on a model with
   that many query heads per KV head, so the recorded attention launches are the ones that read the common
   prompt slots once per group of rows (vector walk plus merge for 4 heads per KV head, the walk on the
   matrix pipe for 8)."""
@@ -590,11 +596,12 @@ def test_per_token_logps_match_oracle_and_the_rollout_logprobs():
     s.per_token_logps(np.zeros((2, 0), np.int32), comp[:2])
 
 
-def test_scoring_clip_reaches_the_many_rows_head():
+@pytest.mark.parametrize('stream_head', [True, False])
+def test_scoring_clip_reaches_the_many_rows_head(stream_head):
   """A head scaled by 1e30 puts every logit beyond the reference's clip at +-1e9
   (tunix/rl/common.py:217-221): a target with a positive logit then scores 1e9 - (1e9 + log n) = 0
-  in f32, one with a negative logit -2e9.  8 sequences x 22 tokens = 176 rows per pass: the
-  256 x 256 head kernel."""
+  in f32, one with a negative logit -2e9.  8 sequences x 12 tokens = 96 rows in the scored pass: the
+  head of 65 to 256 rows from the tile copy, or without one the 256 x 256 head kernel."""
   from oracle import scoring
   cfg = C.TOY
   st = C.make_state(cfg, 31, 8, norm_jitter=0.05)
@@ -602,6 +609,7 @@ def test_scoring_clip_reaches_the_many_rows_head():
   st['lm_head.w'] = bf16_round(st['lm_head.w'] * np.float32(1e30))
   oracle = OM.Decoder(cfg, C.oracle_weights(cfg, st, 64, 16.0, 8))
   model = C.product_model(cfg, st, 64, 16.0)
+  model.stream_head = stream_head
   s = _sampler(model, cfg, 48)
   rng = np.random.default_rng(4)
   prompt = rng.integers(3, cfg.vocab_size, (8, 10)).astype(np.int32)
@@ -638,7 +646,7 @@ def test_multi_token_passes_equal_one_token_passes(family):
   s = _sampler(model, cfg, 64)
   s.eos_ids = np.array([-1])
   rng = np.random.default_rng(3)
-  # 8 sequences, so that 40 tokens per pass are 320 rows (256-row projection blocks; MoE: 640 routed pairs)
+  # 8 sequences, so that 40 tokens per pass are 320 rows (many-rows projections; MoE: 640 routed pairs)
   ids = rng.integers(3, cfg.vocab_size, (8, 41)).astype(np.int32)
   ids[1, :7] = 0   # left padding
   ids[2, :1] = 0

@@ -190,9 +190,9 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
   if (NSEQ <= 0 || NSEQ > TMX_MAX_FILL_ROWS || (!rg && T > TMX_MAX_FILL_ROWS / NSEQ)) return TMX_ERR_SHAPE;
   if (T > 1 && sample && s->sampling_mode != TMX_SAMPLE_SCORE) return TMX_ERR_ARG;
   const int B = rg ? rg->n_rows : NSEQ * T, C = s->cache_size, L = s->buf_len;
-  // a pass takes up to TMX_MAX_FILL_ROWS rows; above 128 rows the projections multiply in 256-row
-  // blocks (every K % 128 == 0), the head takes its rows 64 at a time or in 256 x 256 blocks; MoE models
-  // are bounded by the routed pairs per pass (checked below)
+  // a pass takes up to TMX_MAX_FILL_ROWS rows; above 128 rows the projections run the many-rows kernel
+  // (every K % 128 == 0), above 256 the head 256 x 256 blocks where it can; MoE models are bounded by the
+  // routed pairs per pass (checked below)
   if (B <= 0 || B > TMX_MAX_FILL_ROWS || C <= 0 || L <= 0 || L > C) return TMX_ERR_SHAPE;
   if (moe && (m->experts_per_tok <= 0 || m->experts_per_tok > m->num_experts ||
               (size_t)B * m->experts_per_tok > TMX_MAX_MOE_PAIRS))

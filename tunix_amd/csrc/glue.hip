@@ -357,8 +357,11 @@ __global__ __launch_bounds__(512) void row_norm_kernel(RowNormArgs a) {
 }
 
 // The same for a row that is finished (bf16, no LoRA left, no planes): what is bound by memory then, and the kernel above
-// holds the registers of its other sources (2 workgroups per CU).  256 threads, up to 16 chunks of 8 per row and thread
-// pair, 8 workgroups per CU: 4096 rows of 4096 values (134 MB in and out) 44 -> 29 us.
+// holds the registers of its other sources (2 workgroups per CU).  256 threads, up to 4 chunks of 8 values each, 8
+// workgroups per CU.  Measured (trace, back to back, us, the kernel above / this one), 4096 values a row: 129 rows 4.1 /
+// 4.0, 512 rows 7.3 / 5.6, 4096 rows 41.5 / 21.3; 2048 values: 129 rows 4.1 / 3.4, 4096 rows 39.4 / 11.9.  Above 2048
+// values a row a thread's chunks are others than in the kernel above: the sum of squares is taken in another order and a
+// last bit of the norm may differ between the two.
 template <int CPT>  // 8-element chunks per thread, D <= 2048 * CPT
 __global__ __launch_bounds__(256) void row_norm_plain_kernel(RowNormArgs a) {
   __shared__ float smem[4];

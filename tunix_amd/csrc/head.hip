@@ -245,10 +245,11 @@ __global__ __launch_bounds__(256, MT == 4 ? 1 : 2) void head_kernel(HeadArgs a) 
 // registers as MFMA A operands, P steps ahead.  NW waves of 32 vocabulary rows each; slabs of 64 columns in 64 KiB of LDS:
 // rows of 128 bytes, 16-byte chunk c of row r at slot c ^ (r / 2 % 8), which spreads a fragment read over all banks.
 // Two workgroups share a CU, so that one's epilogue (20 threefry rounds a value when sampling) runs under the other's
-// loads.  On the 1.05 GB head, greedy / sampling: 128 rows 218 / 253 us, bound by the stream (64 rows: 193 / 198); 256 rows
-// 327 / 396 us, bound by LDS (a fragment read per MFMA) and, sampling, by the epilogue's VALU work.  The 256 x 256 blocks
-// of head_wide_kernel take 440 us for either.  For 256 rows also measured: two waves of 64 vocabulary rows on each 128
-// rows (half the LDS reads, every weight read twice) 351 / 418; one workgroup of 8 waves per CU 316 / 412.
+// loads.  On the 1.05 GB head, greedy / sampling (trace): 96 rows 196 / 221 us, 128 rows 214 / 245, bound by the stream (64
+// rows: 182 / 187); 160 rows 277 / 321, 256 rows 309 / 383, bound by LDS (a fragment read per MFMA) and, sampling, by the
+// epilogue's VALU work.  The 256 x 256 blocks of head_wide_kernel take 280 / 372, 301 / 402 (160 rows) and 334 / 429 (256).
+// For 256 rows also measured, where this form took 327 / 396: two waves of 64 vocabulary rows on each 128 rows (half the
+// LDS reads, every weight read twice) 351 / 418; one workgroup of 8 waves per CU 316 / 412.
 template <int MT, int NW, int P>
 __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void head_mid_kernel(HeadArgs a) {
   constexpr int ROWS = MT * 32, R = 512 / ROWS, DX = ROWS / (8 * NW);
@@ -618,8 +619,9 @@ static int launch_head_wide(hipStream_t st, const HeadArgs& a, int tok_blocks, i
   return TMX_OK;
 }
 
-// With a tile copy, up to 256 rows are faster from it (head_logits): both read the matrix once, and the 256 x 256 blocks
-// spend 432 us on the 1.05 GB head where the stream needs half of that at 128 rows.
+// With a tile copy, up to 256 rows are faster from it (head_logits): both read the matrix once, and on the 1.05 GB head the
+// 256 x 256 blocks take 280 us at 96 rows and 334 at 256, greedy, where the stream takes 196 and 309 (sampling 372 and 429
+// against 221 and 383).  More rows would be several passes over the tile copy.
 bool head_wide_ok(const HeadArgs& a) {
   return (a.M > 256 || (a.M > 64 && !a.w_tiles)) && a.D % 128 == 0 && a.M > 0 && (size_t)a.M * a.D * 2 < (1u << 31) && (size_t)256 * a.D * 2 < (1u << 31) &&
          a.n_forbidden == 0 && !a.logits_out;

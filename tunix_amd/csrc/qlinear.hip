@@ -1753,7 +1753,7 @@ int qlinear_base(hipStream_t st, const void* x, int ldx, const void* qw, const v
     a.n_lora_slices = (KT + a.kt_per_lora_split - 1) / a.kt_per_lora_split;  // slices that hold k-tiles
   }
   if (M > 128) {
-    // more than 128 rows: the 256-row block (whole 2-tile steps, 32-bit byte offsets per row block)
+    // more than 128 rows: the many-rows kernel (whole 2-tile steps, 32-bit byte offsets per row block of up to 256)
     if (K % 128 || a.kt_per_split % 2 || (size_t)256 * ldx * 2 >= (1u << 31) ||
         (size_t)K * N / 2 >= (1u << 31) || (size_t)K * Rpad * 2 >= (1u << 31))
       return TMX_ERR_SHAPE;

@@ -409,13 +409,17 @@ static int launch_wide(hipStream_t st, QLinearArgs a) {
 }
 
 // Which tile and how many K-slices.  A launch of at most one workgroup per CU takes (steps of a slice) x (time of a
-// step) + a fixed part; a step is 0.24 us + 0.05 us per column tile and row tile (measured, 8B and 1B shapes, 160 to
-// 4096 rows: 0.64 us for 2 x 4 tiles, 1.04 for 4 x 4, 1.76 for 8 x 4, 3.37 for 8 x 8), the fixed part 8 us (first slab
-// and weights from cold caches, exchange, stores).  More workgroups run in rounds, except that two workgroups of up to
+// step) + a fixed part; a step is priced at 0.24 us + 0.05 us per column tile and row tile, the fixed part at 8 us (first
+// slab and weights from cold caches, exchange, stores).  Measured at K = 4096, fixed part taken off: 0.58 us a step for
+// 2 x 4 tiles, 0.95 for 4 x 4, 1.75 for 8 x 4, 3.0 for 8 x 8.  More workgroups run in rounds, except that two workgroups of up to
 // 4 x 4 tiles share a CU and hide each other's fixed part.  K-slices cost their f32 planes twice, written here and
-// read by the consumer.  So the tile is as large as still gives every CU one workgroup: at 256 rows of the 8B shape
-// q|k|v runs 4 x 4 tiles in 2 slices (25.6 us with its planes; 8 x 8 in 8 slices 34.3), o 2 x 4 in 2 (19.2; 30.6),
-// gate|up 8 x 4 unsplit (65.7; 72.3), down 4 x 4 in 4 (40.7; 50.7); from 4096 rows on 8 x 8 wins everywhere.
+// read by the consumer.  So the tile is as large as still gives every CU one workgroup: at 256 rows of the 8B shape (us,
+// without LoRA and without the consumer's read) q|k|v runs 4 x 4 tiles in 2 slices, 24.3 (8 x 8 in 8: 25.9 and four times
+// the planes), o 2 x 4 in 2, 19.0 (8 x 8 in 8: 25.0), gate|up 8 x 4 unsplit, 64.0 (8 x 8 unsplit: 88.3), down 4 x 4 in 4,
+// 38.0 (8 x 8 in 8: 47.9); 4096 rows of gate|up 8 x 8, 771 (4 x 4: 888).  Every tile and slice count timed for ten
+// matrices of the 8B, 1B and Qwen3-8B shapes at 13 row counts from 135 to 4096: the choice is 1.4 % slower than the best
+// in the mean, more than 5 % in 18 of 130, 13 % at worst (768 rows of 4096 x 28672: 3 x 4 tiles 184, 6 x 8 162).  What it
+// prices wrong is several rounds of large tiles, about 10 % too high (2048 rows there: 4 x 4 448, 8 x 8 418).
 static const int kWideTiles[][2] = {{2, 4}, {3, 4}, {4, 4}, {5, 4}, {6, 4}, {7, 4}, {8, 4}, {4, 8}, {5, 8}, {6, 8}, {7, 8}, {8, 8}};
 
 WidePlan wide_plan(int M, int N, int K, int nsplit) {

@@ -474,8 +474,8 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
 // K-slice of weights, its tiles of A, its share of the handed-over results) is requested before the first is used.
 // The 16 x 16 x 32 MFMA takes them: lane (n = l % 16, q = l / 16) holds column n of k-tile 2 p + q / 2, half q % 2, so a
 // wave's load is two half tiles, and word t of the four lanes of a column is 32 consecutive steps of the contraction
-// (the x operand reads the same k).  Measured on the 1B shape at one row / three rows (trace, us per launch):
-// q|k|v 10.1 -> 8.1 / 9.2, o 9.7 / 15.9 -> 7.7 / 10.1, down 11.9 / 14.6 -> 10.1 / 13.3.
+// (the x operand reads the same k).  Measured on the 1B shape at one row / three rows (trace, us per launch,
+// 32 columns -> 16): q|k|v 8.0 / 9.1 -> 8.0 / 9.0, o 9.3 / 15.6 -> 7.4 / 9.6, down 11.8 / 14.4 -> 9.8 / 13.0.
 constexpr int kSbPairs = 8;  // k-tile pairs per wave requested at once
 
 // LDS: x [M][K + 8] bf16 | red [8 waves][4][16] f32 | red_t [8][4][64] f32 | t [4][64] f32 | row scratch [4 + 8 * 4] f32

@@ -298,14 +298,14 @@ class Sampler:
     return s
 
   MAX_ROWS = 128        # rows of one pass that chooses tokens (sequences x tokens per pass)
-  MAX_FILL_ROWS = 4096  # rows of one cache-fill or scoring pass of a dense model (256-row projection blocks)
+  MAX_FILL_ROWS = 4096  # rows of one cache-fill or scoring pass of a dense model (many-rows projections)
 
   MAX_MOE_PAIRS = 8192  # routed (token, expert) pairs of one pass of a MoE model
   MIN_BLOCK_TOKENS = 4  # tokens per sequence from which a pass over all columns runs the attention that ragged passes run
   MAX_PASSES_IN_FLIGHT = 64  # passes a walk enqueues before it waits for the stream
 
   def _max_rows(self):
-    """Rows one pass can take: more than 128 need the 256-row projection blocks (every attention /
+    """Rows one pass can take: more than 128 need the many-rows projections (every attention /
     dense-MLP projection with K % 128 == 0); MoE models are bounded by the routed pairs per pass."""
     cfg = self._transformer.config
     ks = [cfg.embed_dim, cfg.num_heads * cfg.head_dim] + ([] if cfg.num_experts else [cfg.hidden_dim])
