@@ -424,8 +424,8 @@ def main():
     if small:
       # 1..4 rows: five launches per layer, norm / LoRA / residual / SwiGLU inside the projections
       # (template arguments: prologue 0 plain, 1 norm, 2 attention merge; epilogue 0 plain, 1 residual, 2 SwiGLU)
-      symbols = {'tmx::sb_linear_kernel<1, 0>': ['qkv_linear'], 'tmx::sb_linear_kernel<2, 1>': ['o_linear'],
-                 'tmx::sb_linear_kernel<1, 2>': ['gate_up_linear'], 'tmx::sb_linear_kernel<0, 1>': ['down_linear'],
+      symbols = {'tmx::sb_linear16_kernel<1, 0>': ['qkv_linear'], 'tmx::sb_linear16_kernel<2, 1>': ['o_linear'],
+                 'tmx::sb_linear_kernel<1, 2>': ['gate_up_linear'], 'tmx::sb_linear16_kernel<0, 1>': ['down_linear'],
                  f'tmx::sb_attn_kernel<{cfg.head_dim}, {cfg.num_heads // cfg.num_kv_heads}>': ['attention']}
     # the walk of the run without shared slots: on the matrix pipe for 4 or 8 query heads per kv head while three
     # workgroups per CU hold every (sequence, kv head) pair at once (+ gqa_combine_kernel where a row is split),
