@@ -429,7 +429,7 @@ class QLoRAModel:
     d.rope_theta, d.norm_eps = float(c.rope_theta), float(c.norm_eps)
     d.embed, d.final_norm_w, d.head = self.embed.data_ptr(), self.final_norm.data_ptr(), self.head.data_ptr()
     if self.stream_head and c.vocab_size % 32 == 0 and c.embed_dim % 64 == 0 and c.vocab_size <= 32 * 65535:
-      # one more copy of the head (V * D * 2 bytes) that one-token steps of up to 64 sequences stream
+      # one more copy of the head (V * D * 2 bytes) that passes whose head takes up to 256 rows stream
       if self.head_tiles is None:
         self.head_tiles = torch.empty_like(self.head)
         _lib.check(_lib.lib().tmx_head_tiles_pack(_lib.stream(), _lib.ptr(self.head), _lib.ptr(self.head_tiles),
