@@ -892,3 +892,21 @@ def test_cache_fill_without_padding_equals_the_ragged_pass(n_seq, p, limit):
     assert int(st['step'].item()) == p - 1 and (st['first_col'] is None) == (min_tokens == 4 and p - 1 >= 4)
     caches.append(st['cache'].clone())
   assert caches[0].any() and torch.equal(caches[0], caches[1])
+
+
+def test_scoring_shares_no_prompt_between_rows_whose_token_masks_differ():
+  """Rows with the same ids but another token_mask have other positions and look at other slots (tunix/rl/common.py:257-330):
+  their log-probs are those of a walk of every row by itself."""
+  cfg = C.TOY
+  model = C.product_model(cfg, C.make_state(cfg, 47, 8, norm_jitter=0.05), 64, 16.0)
+  rng = np.random.default_rng(8)
+  prompt = np.repeat(rng.integers(3, cfg.vocab_size, (2, 48)), 2, axis=0).astype(np.int32)
+  comp = rng.integers(3, cfg.vocab_size, (4, 9)).astype(np.int32)
+  mask = np.ones((4, 57), bool)
+  mask[1, :20] = mask[3, 30:40] = False
+  got = {}
+  for share in (True, False):
+    s = _sampler(model, cfg, 64)
+    s.share_prompt_kv = share
+    got[share] = s.per_token_logps(prompt, comp, pad_id=0, token_mask=mask)
+  assert np.abs(got[True] - got[False]).max() <= LOGPROB_TOL

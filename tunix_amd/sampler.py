@@ -488,6 +488,9 @@ class Sampler:
                                 1.0, None, 0, include_logprobs=True)
     dev = self._transformer.device
     self._set_mask(st, valid)
+    if token_mask is not None:  # rows of the same ids share a prompt only where they are masked alike
+      share = shared_prompt_groups(ids, valid) if self.share_prompt_kv else (1, 0, 0)
+      st['share_group'], st['share_len'], st['share_common'] = share
     st['positions'] = torch.from_numpy(utils.build_positions_from_mask(valid).astype(np.int32)).to(dev)
     st['sampling_mode'] = 'score'
     self.walk(st, p - 1)
