@@ -172,8 +172,8 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
   }
   bool t_ready = true;
   if (a.t16 && a.sync) {
-    // t of this block's rows comes from the LoRA workgroups of the launch (without a.sync: of a launch before): wait (a bounded number of polls) for the
-    // flags of its row tiles
+    // t of this block's rows comes from the LoRA workgroups of the launch (without a.sync: of a launch before): wait (a
+    // bounded number of polls) for the flags of its row tiles
     __shared__ uint32_t s_late;
     if (tid == 0) s_late = 0u;
     __syncthreads();
@@ -259,9 +259,9 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
 // hand-over area (a.sync) the last slice of the row tile to arrive adds the planes in slice order and writes the
 // rounded t: bf16 for the epilogues of this launch (a.t16, then its ready flag), f32 for a consumer behind it
 // (a.t_fin).  Stores are write-through and loads go past L2 (sc1), so no cache write-back happens inside the
-// launch.  In the projection's launch these workgroups come first in dispatch order and wait for nobody.  What bounds them is latency: about 8 us
-// at 256 rows, hidden behind the main workgroups' loop, where a LoRA-only launch and a reduction launch in front of the
-// projection took 14 + 5 us (decode step of 256 sequences, 8 layers: 3.43 -> 3.25 ms).
+// launch.  In the projection's launch these workgroups come first in dispatch order and wait for nobody.  What bounds
+// them is latency: about 8 us at 256 rows, hidden behind the main workgroups' loop, where a LoRA-only launch and a
+// reduction launch in front of the projection took 14 + 5 us (decode step of 256 sequences, 8 layers: 3.43 -> 3.25 ms).
 __device__ __forceinline__ void wide_lora_block(const QLinearArgs& a, float* red, int id) {
   const int RT = (a.M + 31) >> 5, rt = id % RT, ks = id / RT;
   if (ks >= a.n_lora_slices) return;
