@@ -1105,6 +1105,16 @@ def test_many_rows_projection_tiles(M, K, N):
   assert (got - want).norm() <= 1e-5 * want.norm() and (got - want).abs().max() <= 1e-4 * want.abs().max()
 
 
+# every row and column tile again with one step of 128 k, with an odd number of steps and with fewer than there are slab
+# buffers, rows that end inside a tile of 16, column tiles that end inside a workgroup
+@pytest.mark.parametrize('M,K,N', [
+    (129, 128, 96), (131, 256, 96), (145, 640, 32), (200, 128, 8224), (200, 128, 28704), (450, 384, 8224), (161, 640, 28704),
+    (200, 640, 28704), (700, 1024, 8224), (383, 128, 16416), (129, 128, 32800), (161, 128, 57344), (200, 128, 57344),
+    (700, 128, 16416)])
+def test_many_rows_projection_steps(M, K, N):
+  test_many_rows_projection_tiles(M, K, N)
+
+
 # one and several K-slices of x . A, one to four column tiles of A, a ragged last row tile
 @pytest.mark.parametrize('M,K,N,r', [(129, 256, 96, 8), (300, 4096, 12288, 16), (161, 5120, 28672, 32), (416, 2048, 16384, 64),
                                      (1000, 4224, 4096, 24)])

@@ -5,25 +5,50 @@
 
 namespace tmx {
 
-// A workgroup is 8 waves = CT column tiles x KW = 8 / CT k-parts over MT row tiles of 32.  A wave multiplies its column
-// tile against all MT row tiles (16 MT accumulator registers), so a dequantised weight fragment feeds MT MFMAs.
-// Weights come by buffer loads one step ahead, the activation slab of a step (2 k-tiles) by direct-to-LDS loads into
-// two buffers: slab rows are 256 bytes (four per 1 KiB transfer), their 16-byte chunks XOR-swizzled by row % 16.  With
-// KW = 2 a wave takes one k-tile of every step, and the two halves of a column tile meet through LDS at the end.
+// A workgroup is 8 waves = CT column tiles of 32 x KW = 8 / CT k-parts over MT row tiles of 32.  A wave multiplies its
+// column tile against all row tiles (16 MT accumulator registers) on the 16 x 16 x 32 MFMA with the weights as A operand,
+// so a lane ends up with four consecutive columns of a row, and a dequantised weight fragment feeds 2 MT MFMAs.
+// What bounds it: at a thousand rows and more the power of the chip.  With every CU at work the clock falls from 2.39 to
+// 1.8 GHz (4096 x 4096 x 28672), and the same launch with zeros for x runs 1.27 times as fast.  Registers only and on
+// random bf16 the 16 x 16 x 32 MFMA sustains 2.02 PFLOP/s and the 32 x 32 x 16 one 1.77, so the former, although it takes
+// twice the issue slots.  In one round of workgroups it is the schedule: the loop below takes 2.18 us a step of 8 x 8 tiles
+// where its MFMAs alone are 1.71 (2.75 us with 32 x 32 x 16, the barrier between two steps and the transfers in one
+// burst behind it).
+// A q4t word holds 8 k of a column; lane (h, n) of a tile has those of column n, k-chunk 2 t + h in word t.  Two lane
+// swaps of the words of a group leave lane group q of 16 lanes with chunk q of column n % 16 in one and of 16 + n % 16 in
+// the other.  In that order of the chunks the MFMA rounds like two 32 x 32 x 16 ones, bit for bit.
+// Weights come by buffer loads, the activation slab of a step (2 k-tiles) by direct-to-LDS loads into NB buffers: slab
+// rows are 256 bytes (four per 1 KiB transfer), their 16-byte chunks XOR-swizzled by row % 16.  With KW = 2 a wave takes
+// one k-tile of every step, and the two halves of a column tile meet through LDS at the end.
+// NB is 4 for the smallest tile (256 x 4096 x 4096 in 2 slices: 19.1 -> 15.9 us; a step of it is shorter than a load takes), 2 for
+// the others (3 x 4 in 3 buffers measured the same).
 constexpr int kWideTS = 2, kWideXS = 128;
 constexpr int kWideTiles32 = TMX_MAX_FILL_ROWS / 32;  // words per kind in a hand-over area: arrivals | ready flags
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-// the MFMA of a group behind which part p (1..4) of the next fragment's dequantisation goes
-constexpr int wide_slot(int MT, int p) { return p < MT ? p : MT - 1; }
-constexpr size_t wide_lds(int MT) { return (size_t)2 * MT * 32 * kWideXS * 2; }
+constexpr int wide_bufs(int mt) { return mt == 2 ? 4 : 2; }
+constexpr size_t wide_lds(int mt) { return (size_t)wide_bufs(mt) * mt * 32 * kWideXS * 2; }
+
+// A copy the compiler does not see through: it happens here, so the registers of v are free for the load that follows
+// (otherwise the copy moves to the end of the loop, behind that load, and waits for it).
+__device__ __forceinline__ uint32_t moved(uint32_t v) {
+  uint32_t r;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+__device__ __forceinline__ u32x4_t moved(u32x4_t v) { return u32x4_t{moved(v.x), moved(v.y), moved(v.z), moved(v.w)}; }
 
 template <int MT, int CT>
 __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* smem, int bx, int slice, int bz) {
   constexpr int TS = kWideTS, XS = kWideXS, ROWS = MT * 32, KW = 8 / CT, TPW = TS / KW;
+  constexpr int NB = wide_bufs(MT), WB = NB > 2 ? NB : 1;  // slab buffers; weight registers (steps on the way)
+  constexpr int G = 2 * TPW, RF = 2 * MT;                  // groups of 32 k a step, x fragments (16 rows) of a group
+  constexpr int RING = RF <= 4 ? RF : RF / 2;              // x fragments in registers
+  constexpr int MEET = RF - RING + 2;                      // the fragment of the last group in front of which the waves meet
+  constexpr int DS = (G - 1) * RF / MT < 2 ? 1 : 2;        // fragments between two slab transfers
   static_assert(KW * CT == 8 && TPW >= 1, "8 waves, at least one k-tile of a step each");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ct = wave % CT, kw = wave / CT;
-  const int h = lane >> 5, nl = lane & 31;
+  const int q = lane >> 4, nl = lane & 15;
   const int KT = a.K >> 6;
   const int per = a.kt_per_split;
   const int kb0 = slice * per;
@@ -40,217 +65,271 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.scales, (uint32_t)NT * KG * 64u);
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x + (size_t)row0 * a.ldx, (uint32_t)rows * a.ldx * 2u);
   const int wv = (nb * KT * 64 + lane) * 16;
-  const int sv = (nb * KG * 32 + nl) * 2;
-  // slab transfer: MT loads per wave and step; load i moves rows 4 wave + 32 i .. + 3 (16 lanes
-  // each), lane l delivering chunk (l % 16) ^ (row % 16) of the step to slot l % 16
-  int xoff[MT];  // per-lane byte offset in the row block (rows past the end repeat the last)
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const int row_l = 4 * wave + 32 * i + (lane >> 4);
-    xoff[i] = (row_l < rows ? row_l : rows - 1) * a.ldx * 2 + (((lane & 15) ^ (row_l & 15)) * 16) + kb0 * 128;
-  }
+  const int sv = (nb * KG * 32 + (lane & 31)) * 2;
+  // slab transfer: MT loads per wave and step; load i moves rows 4 wave + 32 i .. + 3 (16 lanes each), lane l
+  // delivering chunk (l % 16) ^ (row % 16) of the step to slot l % 16.  Rows past the end lie past the descriptor's: zeros.
+  const int row_l = 4 * wave + (lane >> 4);
+  const int xoff = row_l * a.ldx * 2 + (((lane & 15) ^ (row_l & 15)) * 16) + kb0 * 128;
 
-  f32x16_t acc[MT];
+  f32x4_t acc[2][RF];  // columns 0..15 and 16..31 of the tile
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
-  u32x4_t wring[TPW];
-  uint16_t sring[TPW];
+  for (int r = 0; r < RF; ++r) acc[0][r] = acc[1][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  u32x4_t wring[WB][TPW], wc[TPW];
+  uint16_t sring[WB][TPW];
+  NibbleScale sc[TPW][2];
 
-  auto load_w_tile = [&](int step, auto jc) __attribute__((always_inline)) {
-    constexpr int j = decltype(jc)::value;
+  auto load_w = [&](int step, auto bc) __attribute__((always_inline)) {
+    constexpr int b = decltype(bc)::value;
     step = step < last_step ? step : last_step;
-    const int kt = kb0 + step * TS + kw * TPW + j;
-    wring[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, wv, kt * 1024, 0);
-    sring[j] = __builtin_amdgcn_raw_buffer_load_b16(rs, sv, (kt >> gs) * 64, 0);
-  };
-  auto dma_x = [&](int step, int buf) __attribute__((always_inline)) {
-    step = step < last_step ? step : last_step;
-    uint16_t* base = smem + (size_t)buf * ROWS * XS + wave * 4 * XS;
-#pragma unroll
-    for (int i = 0; i < MT; ++i) load_row_to_lds(rx, base + i * 32 * XS, xoff[i], step * (TS * 128));
-  };
-  // One step: 4 TPW fragment groups g = 4 j + t (k-tile j, 16-wide k-block t) of MT MFMAs, one per row
-  // tile.  Between the MFMAs of group g the wave reads the x fragments of group g + 1 (one LDS
-  // read per MFMA; chunk 2 g + h of its part of a row sits at that slot ^ (row % 16)) and dequantises its
-  // weight fragment a quarter at a time, so the matrix pipe waits neither for LDS nor for the
-  // VALU, also when both waves of a SIMD run in phase after a barrier.  The order is pinned.
-  auto step_math = [&](int step, int buf) __attribute__((always_inline)) {
-    u32x4_t wc[TPW];
-    float s_c[TPW], m8s[TPW];
     static_for<TPW>([&](auto jc) __attribute__((always_inline)) {
       constexpr int j = decltype(jc)::value;
-      wc[j] = wring[j];
-      s_c[j] = bf2f(sring[j]);
-      m8s[j] = -8.f * s_c[j];
-      load_w_tile(step + 1, jc);  // registers consumed: refill them one step ahead
+      const int kt = kb0 + step * TS + kw * TPW + j;
+      wring[b][j] = __builtin_amdgcn_raw_buffer_load_b128(rw, wv, kt * 1024, 0);
+      sring[b][j] = __builtin_amdgcn_raw_buffer_load_b16(rs, sv, (kt >> gs) * 64, 0);
     });
-    const uint16_t* xb = smem + (size_t)buf * ROWS * XS + nl * XS;
-    const int c0 = 8 * TPW * kw + h;  // this wave's first chunk of a slab row
-    auto word_of = [&](auto gc) __attribute__((always_inline)) {
-      constexpr int g = decltype(gc)::value, j = g / 4, t = g % 4;
-      return t == 0 ? wc[j].x : (t == 1 ? wc[j].y : (t == 2 ? wc[j].z : wc[j].w));
-    };
-    bf16x8_t xq[2][MT];
-    u32x4_t bq[2];
-    {
-      const int slot = (c0 ^ (nl & 15)) * 8;
-#pragma unroll
-      for (int m = 0; m < MT; ++m) xq[0][m] = *reinterpret_cast<const bf16x8_t*>(xb + m * 32 * XS + slot);
-      bq[0] = __builtin_bit_cast(u32x4_t, dequant_word(word_of(IC<0>{}), s_c[0], m8s[0]));
-    }
+  };
+  auto take_w = [&](auto bc) __attribute__((always_inline)) {
+    constexpr int b = decltype(bc)::value;
+    static_for<TPW>([&](auto jc) __attribute__((always_inline)) {
+      constexpr int j = decltype(jc)::value;
+      wc[j] = WB == 1 ? moved(wring[b][j]) : wring[b][j];
+      const uint32_t both = WB == 1 ? moved((uint32_t)sring[b][j]) : (uint32_t)sring[b][j];
+      const auto s = __builtin_amdgcn_permlane16_swap(both, both, false, false);
+      sc[j][0] = nibble_scale(bf2f((uint16_t)s[0]));
+      sc[j][1] = nibble_scale(bf2f((uint16_t)s[1]));
+    });
+  };
+  auto dma_x = [&](int step, int buf, int i) __attribute__((always_inline)) {
+    step = step < last_step ? step : last_step;
+    uint16_t* base = smem + (size_t)buf * ROWS * XS + wave * 4 * XS;
+    load_row_to_lds(rx, base + i * 32 * XS, xoff + i * 64 * a.ldx, step * (TS * 128));
+  };
+  // all but the youngest loads of this wave have arrived and its LDS reads are done; then all waves
+  auto meet = [&](auto younger) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-    static_for<4 * TPW>([&](auto gc) __attribute__((always_inline)) {
-      constexpr int g = decltype(gc)::value, cur = g & 1, nxt = cur ^ 1;
-      constexpr bool more = g + 1 < 4 * TPW;
-      constexpr int jn = (g + 1) / 4 % TPW;
-      const int slot = ((c0 + 2 * (g + 1)) ^ (nl & 15)) * 8;
-      uint32_t lo = 0, hi = 0;
-      static_for<MT>([&](auto mc) __attribute__((always_inline)) {
-        constexpr int m = decltype(mc)::value;
-        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xq[cur][m], __builtin_bit_cast(bf16x8_t, bq[cur]), acc[m],
-                                                         0, 0, 0);
-        if constexpr (more) {
-          xq[nxt][m] = *reinterpret_cast<const bf16x8_t*>(xb + m * 32 * XS + slot);
-          if (m == 0) dequant_masks(word_of(IC<g + 1>{}), lo, hi);
-          if (m == wide_slot(MT, 1)) bq[nxt].x = dequant_part<0>(lo, hi, s_c[jn], m8s[jn]);
-          if (m == wide_slot(MT, 2)) bq[nxt].y = dequant_part<1>(lo, hi, s_c[jn], m8s[jn]);
-          if (m == wide_slot(MT, 3)) bq[nxt].z = dequant_part<2>(lo, hi, s_c[jn], m8s[jn]);
-          if (m == wide_slot(MT, 4)) bq[nxt].w = dequant_part<3>(lo, hi, s_c[jn], m8s[jn]);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(decltype(younger)::value) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  bf16x8_t xq[RING];
+  u32x4_t bq[2][2];  // weight fragments of two groups
+  uint32_t words[2];
+  const int c0 = 8 * TPW * kw + q;  // this lane's first chunk of a slab row
+  const uint16_t* xlane = smem + nl * XS;
+  auto read_x = [&](const uint16_t* xb, auto rc) __attribute__((always_inline)) {
+    constexpr int r = decltype(rc)::value;
+    xq[r % RING] = *reinterpret_cast<const bf16x8_t*>(xb + r * 16 * XS);
+  };
+  // an eighth of the weight fragments of group g
+  auto dequant = [&](auto gc, auto pc) __attribute__((always_inline)) {
+    constexpr int g = decltype(gc)::value, p = decltype(pc)::value, j = g / 2;
+    if constexpr (p == 0) {
+      const auto x = __builtin_amdgcn_permlane32_swap(wc[j][g % 2 * 2], wc[j][g % 2 * 2 + 1], false, false);
+      const auto w = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+      words[0] = w[0]; words[1] = w[1];
+    }
+    bq[g & 1][p / 4][p % 4] = dequant_part<p % 4>(words[p / 4], sc[j][p / 4]);
+  };
+  // A step is G groups of RF fragments of two MFMAs.  Behind the MFMAs of a fragment its register is refilled with the
+  // one RING further on, and the weight fragments of the next group are dequantised an eighth at a time, so the matrix pipe
+  // waits neither for LDS nor for the VALU; the transfers of a slab are spread over the first fragments of a step
+  // (in one burst they hold up all waves: a step 12 % longer).  The order is pinned.
+  // The barrier that hands over the next slab stands inside the last group, where no fragment of this slab is left to
+  // read and those in registers keep the pipe busy; the first ones of the next step are read behind it.
+  // The wave that is behind goes first (s_setprio falls with the groups done): otherwise the older of the two waves of a
+  // SIMD runs ahead and then waits at the barrier, and the other cannot fill the pipe by itself (717 us against 750 at
+  // 4096 x 4096 x 28672).
+  // buf: the slab's buffer, step % NB; bc: the same as a constant where WB > 1
+  auto step_math = [&](int step, int buf, auto bc) __attribute__((always_inline)) {
+    constexpr int b = decltype(bc)::value;
+    const int next = buf + 1 == NB ? 0 : buf + 1, prev = buf == 0 ? NB - 1 : buf - 1;
+    const uint16_t* xs = xlane + (size_t)buf * ROWS * XS;
+    const uint16_t* xn = xlane + (size_t)next * ROWS * XS + (c0 ^ nl) * 8;
+    static_for<G>([&](auto gc) __attribute__((always_inline)) {
+      constexpr int g = decltype(gc)::value;
+      constexpr bool last = g == G - 1;
+      __builtin_amdgcn_s_setprio(G - 1 - g);
+      if constexpr (last) take_w(IC<(b + 1) % WB>{});
+      const uint16_t* xb = xs + ((c0 + 4 * g) ^ nl) * 8;
+      const uint16_t* xb1 = last ? xn : xs + ((c0 + 4 * (g + 1)) ^ nl) * 8;
+      static_for<RF>([&](auto rc) __attribute__((always_inline)) {
+        constexpr int r = decltype(rc)::value, f = g * RF + r;
+        if constexpr (last && r == MEET) {
+          // the next slab was requested NB - 2 slabs and weight loads ago (at least one of the latter in the first steps)
+          meet(IC<(NB - 2) * MT + (NB > 2 ? 2 * TPW : 0)>{});
+          load_w(step + 1 + WB, IC<(b + 1) % WB>{});
           __builtin_amdgcn_sched_barrier(0);
         }
+        static_for<2>([&](auto uc) __attribute__((always_inline)) {
+          constexpr int u = decltype(uc)::value;
+          acc[u][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, bq[g & 1][u]), xq[r % RING], acc[u][r], 0, 0, 0);
+          static_for<8>([&](auto pc) __attribute__((always_inline)) {
+            if constexpr (decltype(pc)::value * RF / 4 == 2 * r + u) dequant(IC<last ? 0 : g + 1>{}, pc);
+          });
+          if constexpr (u == 0) __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (f % DS == 0 && f / DS < MT) dma_x(step + NB - 1, prev, f / DS);
+        if constexpr (r + RING < RF) {
+          read_x(xb, IC<r + RING>{});
+        } else if constexpr (!last) {
+          read_x(xb1, IC<r + RING - RF>{});
+        } else if constexpr (r >= MEET) {  // two at a time until the two left out in front of the barrier are caught up
+          constexpr int n = r - MEET, t0 = n < 2 ? 2 * n : n + 2, t1 = r + 1 == RF ? RING : n < 1 ? 2 : n + 3;
+          static_for<t1 - t0>([&](auto nc) __attribute__((always_inline)) { read_x(xb1, IC<t0 + decltype(nc)::value>{}); });
+        }
+        __builtin_amdgcn_sched_barrier(0);
       });
     });
   };
-  // loads of a step younger than its slab transfer (in-order counter)
-  constexpr int kYounger = TPW * 2;
-  auto wait_slab = [&]() __attribute__((always_inline)) {
-    __builtin_amdgcn_sched_barrier(0);
-    if (tile_ok) __builtin_amdgcn_s_waitcnt(0x0F70 | (kYounger & 15) | ((kYounger >> 4) << 14));
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-  };
 
-  dma_x(0, 0);
-  if (tile_ok) static_for<TPW>([&](auto jc) __attribute__((always_inline)) { load_w_tile(0, jc); });
-  wait_slab();
-  for (int step = 0; step < nsteps; ++step) {
-    const int buf = step & 1;
-    dma_x(step + 1, buf ^ 1);
-    __builtin_amdgcn_sched_barrier(0);
-    if (tile_ok) step_math(step, buf);
-    wait_slab();
+  static_for<WB>([&](auto bc) __attribute__((always_inline)) { load_w(decltype(bc)::value, bc); });
+#pragma unroll
+  for (int i = 0; i < (NB - 1) * MT; ++i) dma_x(i / MT, i / MT, i % MT);
+  meet(IC<(NB - 2) * MT>{});
+  take_w(IC<0>{});
+  load_w(WB, IC<0>{});
+  if (tile_ok) {
+    static_for<RING>([&](auto rc) __attribute__((always_inline)) { read_x(xlane + (c0 ^ nl) * 8, rc); });
+    static_for<8>([&](auto pc) __attribute__((always_inline)) { dequant(IC<0>{}, pc); });
+    if constexpr (WB == 1) {
+      for (int step = 0; step < nsteps; ++step) step_math(step, step & 1, IC<0>{});
+    } else {
+      for (int step = 0; step < nsteps; step += NB)
+        static_for<NB>([&](auto bc) __attribute__((always_inline)) {
+          if (step + decltype(bc)::value < nsteps) step_math(step + decltype(bc)::value, decltype(bc)::value, bc);
+        });
+    }
+  } else {
+    for (int step = 0; step < nsteps; ++step) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) dma_x(step + NB - 1, (step + NB - 1) % NB, i);
+      meet(IC<(NB - 2) * MT>{});
+    }
   }
-  // Two k-parts of a tile swap halves of their accumulators (the slab is free: the last step ended with a barrier,
-  // and its surplus transfer, a repeat of the last step, has landed): the first finishes registers 0..7, the
-  // second 8..15.
-  constexpr int NR = 16 / KW;  // accumulator registers this wave finishes
-  const int rbase = kw * NR;
+  __builtin_amdgcn_s_setprio(0);
+  // Two k-parts of a tile swap halves of their accumulators (the slab is free once the surplus transfers, repeats of
+  // the last step, have landed): the first finishes the first half of the rows, the second the other.
+  constexpr int NR = RF / KW;  // row tiles of 16 this wave finishes
   if constexpr (KW == 2) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);
+    meet(IC<0>{});
+    f32x4_t* hb = reinterpret_cast<f32x4_t*>(smem) + (size_t)ct * RF * 2 * 64 + lane;  // [CT][2 parts][2][NR][64]
+    if (tile_ok)
+#pragma unroll
+      for (int i = 0; i < RF; ++i) {
+        f32x4_t(&v)[RF] = acc[i / NR];
+        hb[(i + (kw ? 0 : RF)) * 64] = kw ? v[i % NR] : v[i % NR + NR];
+      }
     __syncthreads();
-    float* hb = reinterpret_cast<float*>(smem);  // [CT][MT][16][64]
-    if (tile_ok) {
+    if (tile_ok)
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int r8 = 0; r8 < 8; ++r8)
-          hb[(((ct * MT + m) * 16 + (kw ? r8 : r8 + 8)) << 6) + lane] = kw ? acc[m][r8] : acc[m][r8 + 8];
-    }
-    __syncthreads();
-    if (tile_ok) {
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int r8 = 0; r8 < 8; ++r8) {
-          const float mine = kw ? acc[m][r8 + 8] : acc[m][r8];
-          const float other = hb[(((ct * MT + m) * 16 + (kw ? r8 + 8 : r8)) << 6) + lane];
-          acc[m][r8] = kw ? other + mine : mine + other;  // first half + second half
-        }
-    }
+      for (int i = 0; i < RF; ++i) {
+        f32x4_t(&v)[RF] = acc[i / NR];
+        const f32x4_t mine = kw ? v[i % NR + NR] : v[i % NR], other = hb[(i + (kw ? RF : 0)) * 64];
+        v[i % NR] = kw ? other + mine : mine + other;  // first half + second half
+      }
   }
-  bool t_ready = true;
-  if (a.t16 && a.sync) {
-    // t of this block's rows comes from the LoRA workgroups of the launch (without a.sync: of a launch before): wait (a
-    // bounded number of polls) for the flags of its row tiles
-    __shared__ uint32_t s_late;
-    if (tid == 0) s_late = 0u;
-    __syncthreads();
-    if (tid < MT && row0 + tid * 32 < a.M) {
-      uint32_t* flag = a.sync + kWideTiles32 + (row0 >> 5) + tid;
-      uint32_t ok = 0;
-      for (int spin = 0; spin < (1 << 20); ++spin) {
-        if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) { ok = 1; break; }
-        __builtin_amdgcn_s_sleep(1);
-      }
-      if (!ok) {
-        s_late = 1u;
-        if (a.sync_status) __hip_atomic_store(a.sync_status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-    __syncthreads();
-    t_ready = s_late == 0u;  // false: t is taken as zero (the status word says so)
-  }
-  if (!tile_ok) return;
-  const int col = nb * 32 + nl;
-  if (a.t16) {
-    // LoRA in the epilogue: delta tile [32 rows, 32 columns] = t16 rows . B columns, 16 ranks per
-    // MFMA (t rows are the A operand, so the delta lands in the accumulator layout of acc[m]);
-    // y = bf16(bf16(base) + bf16(bf16(delta) ls))
-    const int seg = nb * 32 >= a.seg_end[0] ? (nb * 32 >= a.seg_end[1] ? 2 : 1) : 0;
-    const int tc0 = seg * a.lora_r;
-    const int nkb = (a.lora_r + 15) >> 4;  // host: <= 4
-    u32x4_t bfr[4];
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      uint32_t w[4] = {0, 0, 0, 0};
-      if (kb < nkb) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int rr = kb * 16 + 8 * h + j;
-          const uint32_t e = rr < a.lora_r ? a.lora_b[(size_t)rr * a.N + col] : 0u;
-          w[j >> 1] |= e << (16 * (j & 1));
-        }
-      }
-      bfr[kb] = u32x4_t{w[0], w[1], w[2], w[3]};
-    }
-    const __amdgpu_buffer_rsrc_t rt = make_rsrc(a.t16, (uint32_t)a.M * a.ldt16 * 2u);
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const int trow = row0 + m * 32 + nl;
-      const int tp = ((trow < a.M ? trow : a.M - 1) * a.ldt16 + tc0 + 8 * h) * 2;
-      f32x16_t d;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) d[r] = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-        if (kb < nkb) {
-          // past this XCD's L2: the rows were written during this launch
-          u32x4_t tf = {0u, 0u, 0u, 0u};
-          if (t_ready) tf = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rt, tp + kb * 32, 0, 0x10));
-          d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, tf), __builtin_bit_cast(bf16x8_t, bfr[kb]), d, 0, 0, 0);
-        }
+  const int wrow0 = row0 + kw * NR * 16 + nl;  // this lane's row of the first row tile
+  const int tile0 = nb * 32, col0 = tile0 + 4 * q;  // its four columns of the first half of the tile, + 16 of the second
+  if (!a.t16) {
+    if (tile_ok)
 #pragma unroll
       for (int i = 0; i < NR; ++i) {
-        const int row = row0 + m * 32 + acc_row(rbase + i, lane);
+        const int row = wrow0 + i * 16;
         if (row >= a.M) continue;
-        const float dv = KW == 2 ? (kw ? d[(i + 8) & 15] : d[i]) : d[i];
-        a.y_bf16[(size_t)row * a.ldy + col] = f2bf(rbf(acc[m][i]) + rbf(rbf(dv) * a.lora_ls));
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const f32x4_t v = acc[u][i];
+          if (a.y_bf16) *reinterpret_cast<u32x2_t*>(a.y_bf16 + (size_t)row * a.ldy + col0 + 16 * u) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+          else *reinterpret_cast<f32x4_t*>(a.y_part + ((size_t)slice * a.M + row) * a.N + col0 + 16 * u) = v;
+        }
       }
-    }
     return;
   }
+  // LoRA in the epilogue: delta tile [16 columns, 16 rows] = B columns . t16 rows, 32 ranks per MFMA (in the
+  // orientation of acc); y = bf16(bf16(base) + bf16(bf16(delta) ls)).  What it costs is round trips to memory, so the
+  // columns of B are requested in front of the wait for t, and the rows of t four row tiles ahead.
+  auto lora = [&](auto nkbc) __attribute__((always_inline)) {
+    constexpr int NKB = decltype(nkbc)::value, BT = 4, NBT = (NR + BT - 1) / BT;
+    const int seg = tile0 >= a.seg_end[0] ? (tile0 >= a.seg_end[1] ? 2 : 1) : 0;
+    uint16_t be[2][NKB][8];
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int row = row0 + m * 32 + acc_row(rbase + i, lane);
-      if (row >= a.M) continue;
-      const float v = acc[m][i];
-      if (a.y_bf16) a.y_bf16[(size_t)row * a.ldy + col] = f2bf(v);
-      else a.y_part[((size_t)slice * a.M + row) * a.N + col] = v;
+    for (int i = 0; i < 2 * NKB * 8; ++i) {
+      const int u = i / (8 * NKB), kb = i / 8 % NKB, rr = kb * 32 + 8 * q + i % 8;
+      be[u][kb][i % 8] = tile_ok && rr < a.lora_r ? a.lora_b[(size_t)rr * a.N + tile0 + u * 16 + nl] : (uint16_t)0;
     }
+    bool t_ready = true;
+    if (a.sync) {
+      // t of this block's rows comes from the LoRA workgroups of the launch (without a.sync: of a launch before): wait (a
+      // bounded number of polls) for the flags of its row tiles
+      __shared__ uint32_t s_late;
+      if (tid == 0) s_late = 0u;
+      __syncthreads();
+      if (tid < MT && row0 + tid * 32 < a.M) {
+        uint32_t* flag = a.sync + kWideTiles32 + (row0 >> 5) + tid;
+        uint32_t ok = 0;
+        for (int spin = 0; spin < (1 << 20); ++spin) {
+          if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) { ok = 1; break; }
+          __builtin_amdgcn_s_sleep(1);
+        }
+        if (!ok) {
+          s_late = 1u;
+          if (a.sync_status) __hip_atomic_store(a.sync_status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+      __syncthreads();
+      t_ready = s_late == 0u;  // false: t is taken as zero (the status word says so)
+    }
+    if (!tile_ok) return;
+    u32x4_t bfr[2][NKB];
+#pragma unroll
+    for (int i = 0; i < 2 * NKB; ++i) __builtin_memcpy(&bfr[i / NKB][i % NKB], be[i / NKB][i % NKB], 16);
+    const __amdgpu_buffer_rsrc_t rt = make_rsrc(a.t16, (uint32_t)a.M * a.ldt16 * 2u);
+    u32x4_t tf[2][BT][NKB];
+    auto load_t = [&](auto bc) __attribute__((always_inline)) {
+      constexpr int bt = decltype(bc)::value;
+#pragma unroll
+      for (int i = 0; i < BT; ++i) {
+        const int row = wrow0 + (bt * BT + i) * 16;
+        const int tp = ((row < a.M ? row : a.M - 1) * a.ldt16 + seg * a.lora_r + 8 * q) * 2;
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) {
+          // past this XCD's L2: the rows were written during this launch
+          tf[bt & 1][i][kb] = u32x4_t{0u, 0u, 0u, 0u};
+          if (bt * BT + i < NR && t_ready && kb * 32 + 8 * q < a.lora_r)
+            tf[bt & 1][i][kb] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rt, tp + kb * 64, 0, 0x10));
+        }
+      }
+    };
+    load_t(IC<0>{});
+    static_for<NBT>([&](auto bc) __attribute__((always_inline)) {
+      constexpr int bt = decltype(bc)::value;
+      if constexpr (bt + 1 < NBT) load_t(IC<bt + 1>{});
+#pragma unroll
+      for (int ii = 0; ii < BT; ++ii) {
+        const int i = bt * BT + ii, row = wrow0 + i * 16;
+        if (i >= NR) break;
+        f32x4_t d[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          d[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kb = 0; kb < NKB; ++kb)
+            d[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, bfr[u][kb]), __builtin_bit_cast(bf16x8_t, tf[bt & 1][ii][kb]), d[u], 0, 0, 0);
+        }
+        if (row >= a.M) continue;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          f32x4_t v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = rbf(acc[u][i][e]) + rbf(rbf(d[u][e]) * a.lora_ls);
+          *reinterpret_cast<u32x2_t*>(a.y_bf16 + (size_t)row * a.ldy + col0 + 16 * u) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+        }
+      }
+    });
+  };
+  if (a.lora_r <= 32) lora(IC<1>{});
+  else lora(IC<2>{});
 }
 
 // t = x . A of one row tile (32 rows) over one K-slice.  The 8 waves are column tiles of A (1, 2 or 4) x k-parts; a wave
@@ -408,36 +487,49 @@ static int launch_wide(hipStream_t st, QLinearArgs a) {
   return check_launch();
 }
 
-// Which tile and how many K-slices.  A launch of at most one workgroup per CU takes (steps of a slice) x (time of a
-// step) + a fixed part; a step is priced at 0.24 us + 0.05 us per column tile and row tile, the fixed part at 8 us (first
-// slab and weights from cold caches, exchange, stores).  Measured at K = 4096, fixed part taken off: 0.58 us a step for
-// 2 x 4 tiles, 0.95 for 4 x 4, 1.75 for 8 x 4, 3.0 for 8 x 8.  More workgroups run in rounds, except that two workgroups of up to
-// 4 x 4 tiles share a CU and hide each other's fixed part.  K-slices cost their f32 planes twice, written here and
-// read by the consumer.  So the tile is as large as still gives every CU one workgroup: at 256 rows of the 8B shape (us,
-// without LoRA and without the consumer's read) q|k|v runs 4 x 4 tiles in 2 slices, 24.3 (8 x 8 in 8: 25.9 and four times
-// the planes), o 2 x 4 in 2, 19.0 (8 x 8 in 8: 25.0), gate|up 8 x 4 unsplit, 64.0 (8 x 8 unsplit: 88.3), down 4 x 4 in 4,
-// 38.0 (8 x 8 in 8: 47.9); 4096 rows of gate|up 8 x 8, 771 (4 x 4: 888).  Every tile and slice count timed for ten
-// matrices of the 8B, 1B and Qwen3-8B shapes at 13 row counts from 135 to 4096: the choice is 1.4 % slower than the best
-// in the mean, more than 5 % in 18 of 130, 13 % at worst (768 rows of 4096 x 28672: 3 x 4 tiles 184, 6 x 8 162).  What it
-// prices wrong is several rounds of large tiles, about 10 % too high (2048 rows there: 4 x 4 448, 8 x 8 418).
+// Which tile and how many K-slices.  The order in which a sum runs over K is set by the slices and by CT (one or two
+// k-parts); it follows prices of its own that stay as they are, so that a call gives the same bits whatever
+// becomes of the kernel (a greedy rollout goes another way where the two best logits are one bf16 step apart): a fixed part
+// of 8 us and steps of 0.24 us + 0.05 us per column tile and row tile.  The row tiles follow what the kernel takes now: a
+// fixed part (first slab and weights from cold caches, exchange, stores) and a time per step, both linear in the tile;
+// fitted to every tile and slice count of twelve matrices of the 8B, 1B, Qwen3-8B and 30B-A3B shapes at 13 row counts from 135 to
+// 4096, they are 6 % off in the mean.  More workgroups than CUs run in rounds, whose steps are 1.12 times as long (the clock falls
+// with every CU at work) and which hide half of the fixed part; two workgroups of up to 4 x 4 tiles share a CU and hide
+// all of it.  K-slices cost their f32 planes, written here and read by the consumer.  At 256 rows of the 8B shape (us,
+// without LoRA and without the consumer's read) q|k|v runs 4 x 4 tiles in 2 slices, 20.6 (8 x 4 in 4: 21.6 and
+// twice the planes), gate|up 8 x 4 unsplit, 55 (4 x 4: 59, 8 x 8: 81), down 4 x 4 in 4, 33 (8 x 4 in 4: 43); 4096 rows of
+// gate|up 8 x 8, 715 (4 x 4: 840).
 static const int kWideTiles[][2] = {{2, 4}, {3, 4}, {4, 4}, {5, 4}, {6, 4}, {7, 4}, {8, 4}, {4, 8}, {5, 8}, {6, 8}, {7, 8}, {8, 8}};
+
+// What a tile in s slices costs, us; `order`: by the prices that fix the order of the sums.
+static float wide_price(int M, int N, int KT, int mt, int ct, int s, int cus, bool order) {
+  const long tiles = (long)((M + 32 * mt - 1) / (32 * mt)) * ((N + 32 * ct - 1) / (32 * ct));
+  const long n = (tiles * s + cus - 1) / cus;  // workgroups of a CU
+  const bool pairs = mt <= 4 && ct == 4;
+  const float steps = (float)(slice_len(KT, s) / kWideTS), planes = s > 1 ? 0.3e-6f * s * (float)M * N * 4.f : 0.f;
+  if (order) {
+    const float loop = steps * (0.24f + 0.05f * mt * ct);
+    return (pairs ? 8.f + (n == 1 ? 1.f : 0.92f) * n * loop : n * (8.f + loop)) + planes;
+  }
+  const float fixed = ct == 4 ? 3.7f + 0.78f * mt : 5.8f + 0.62f * mt, loop = steps * ((ct == 4 ? 0.4f : 0.56f) + 0.024f * mt * ct);
+  return (pairs || n == 1 ? fixed + n * loop : fixed + 1.12f * n * loop + 0.5f * (n - 1) * fixed) + planes;
+}
 
 WidePlan wide_plan(int M, int N, int K, int nsplit) {
   const int cus = device_cus(), KT = K >> 6;
   WidePlan best = {8, 8, nsplit > 0 ? nsplit : 1};
   float best_cost = 1e30f;
-  for (const auto& t : kWideTiles) {
-    const int mt = t[0], ct = t[1];
-    const long tiles = (long)((M + 32 * mt - 1) / (32 * mt)) * ((N + 32 * ct - 1) / (32 * ct));
-    for (int s = nsplit > 0 ? nsplit : 1; s <= (nsplit > 0 ? nsplit : TMX_MAX_SPLITS); ++s) {
-      if (!slices_ok(KT, s)) continue;
-      const float loop = (slice_len(KT, s) / kWideTS) * (0.24f + 0.05f * mt * ct);
-      const long n = (tiles * s + cus - 1) / cus;  // workgroups of a CU
-      const float t_us = mt <= 4 && ct == 4 ? 8.f + (n == 1 ? 1.f : 0.92f) * n * loop : n * (8.f + loop);
-      const float cost = t_us + (s > 1 ? 0.3e-6f * s * (float)M * N * 4.f : 0.f);
-      if (cost < best_cost) { best_cost = cost; best = {mt, ct, s}; }
-    }
-  }
+  auto offer = [&](int mt, int ct, int s, bool order) {
+    const float cost = wide_price(M, N, KT, mt, ct, s, cus, order);
+    if (cost < best_cost) { best_cost = cost; best = {mt, ct, s}; }
+  };
+  for (const auto& t : kWideTiles)
+    for (int s = nsplit > 0 ? nsplit : 1; s <= (nsplit > 0 ? nsplit : TMX_MAX_SPLITS); ++s)
+      if (slices_ok(KT, s)) offer(t[0], t[1], s, true);
+  const int ct = best.ct, s = best.nsplit;
+  best_cost = 1e30f;
+  for (const auto& t : kWideTiles)
+    if (t[1] == ct) offer(t[0], ct, s, false);
   return best;
 }
 
