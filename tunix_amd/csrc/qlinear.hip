@@ -8,9 +8,8 @@
 // Mapping to CDNA4: weights are the B operand of v_mfma_f32_32x32x16_bf16.  The
 // packed tile format stores, for every 64(k) x 32(n) tile, the 32 nibbles a lane
 // needs as ONE 128-bit word, so a wave fetches a tile with a single coalesced
-// 1 KiB load and never touches LDS for weights.  Nibbles are widened with
-// v_cvt_f32_ubyteN (or two at a time with v_cvt_pk_f32_fp8: dequant_word in tmx_common.h),
-// scaled with one fma ((u - 8) * s is exact in f32) and
+// 1 KiB load and never touches LDS for weights.  Nibbles are widened and
+// scaled with one v_fma_mix_f32 (dequant_word in tmx_common.h; (u - 8) * s is exact in f32) and
 // rounded pairwise to bf16 by the hardware converter, which reproduces the
 // reference's bf16 dequantised weight bit for bit before it enters the MFMA.
 #include <atomic>
@@ -159,15 +158,14 @@ __device__ __forceinline__ void gemm_block4(const QLinearArgs& a, uint16_t (*xs)
     u32x4_t wc[WPT];
 #pragma unroll
     for (int t = 0; t < WPT; ++t) wc[t] = wring[d][kt][t];
-    const float s_c = LORA ? 0.f : bf2f(sring[d][kt]);
+    const NibbleScale sc = nibble_scale(LORA ? 0.f : bf2f(sring[d][kt]));
     load_w_tile(step + DW, dc, kc);  // slot consumed: refill it DW steps ahead
-    const float m8s = -8.f * s_c;
     const uint32_t wd[4] = {wc[0].x, wc[0].y, wc[0].z, wc[0].w};
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       bf16x8_t b;
       if (LORA) b = __builtin_bit_cast(bf16x8_t, wc[t % WPT]);
-      else b = dequant_word(wd[t], s_c, m8s);
+      else b = dequant_word(wd[t], sc);
 #pragma unroll
       for (int m = 0; m < MT; ++m)
         acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[m][t], b, acc[m], 0, 0, 0);
@@ -448,12 +446,12 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(MoeArgs m) {
           else load_w(u + 1, kt + kMoeRing - KT, sc);
 #pragma unroll
           for (int c = 0; c < TPU; ++c) {
-            const float m8s = -8.f * s_c[c];
+            const NibbleScale sc = nibble_scale(s_c[c]);
             const uint32_t wd[4] = {wc[c].x, wc[c].y, wc[c].z, wc[c].w};
 #pragma unroll
             for (int t = 0; t < 4; ++t)
               acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, xq[sl & 1][t]),
-                                                               dequant_word<true>(wd[t], s_c[c], m8s), acc[c], 0, 0, 0);
+                                                               dequant_word(wd[t], sc), acc[c], 0, 0, 0);
           }
         });
       }
@@ -689,16 +687,15 @@ __device__ __forceinline__ void gemm_block(const QLinearArgs& a, uint16_t* smem)
     u32x4_t wc[WPT];
 #pragma unroll
     for (int t = 0; t < WPT; ++t) wc[t] = wring[d][j][t];
-    const float s_c = LORA ? 0.f : bf2f(sring[d][j]);
+    const NibbleScale sc = nibble_scale(LORA ? 0.f : bf2f(sring[d][j]));
     load_w_tile(step + DW, dc, jc);  // slot consumed: refill it DW steps ahead
     if (step * KS + kw * TPW + j > last_tile) return;  // past the slice (ragged last step)
-    const float m8s = -8.f * s_c;
     const uint32_t wd[4] = {wc[0].x, wc[0].y, wc[0].z, wc[0].w};
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       bf16x8_t b;
       if (LORA) b = __builtin_bit_cast(bf16x8_t, wc[t % WPT]);
-      else b = dequant_word(wd[t], s_c, m8s);
+      else b = dequant_word(wd[t], sc);
 #pragma unroll
       for (int m = 0; m < MT; ++m)
         acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[m][t], b, acc[m], 0, 0, 0);
@@ -991,13 +988,12 @@ __global__ __launch_bounds__(512, 1) void qlinear_gate_up8_kernel(QLinearArgs a)
     if constexpr (j + 1 < TPW) read_x(buf, IC<j + 1>{});
     auto& xa = xq[j & 1];
     const u32x4_t wc = wring[j];
-    const float s_c = bf2f(sring[j]);
+    const NibbleScale sc = nibble_scale(bf2f(sring[j]));
     load_w_tile(step + 1, jc);  // slot consumed: refill it for the next step
-    const float m8s = -8.f * s_c;
     const uint32_t wd[4] = {wc.x, wc.y, wc.z, wc.w};
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const bf16x8_t b = dequant_word<true>(wd[t], s_c, m8s);
+      const bf16x8_t b = dequant_word(wd[t], sc);
 #pragma unroll
       for (int m = 0; m < MT; ++m)
         acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[m][t], b, acc[m], 0, 0, 0);
@@ -1422,15 +1418,14 @@ __device__ __forceinline__ void gemm_block_dma(const QLinearArgs& a, uint16_t* s
     u32x4_t wc[WPT];
 #pragma unroll
     for (int t = 0; t < WPT; ++t) wc[t] = wring[d][j][t];
-    const float s_c = LORA ? 0.f : bf2f(sring[d][j]);
+    const NibbleScale sc = nibble_scale(LORA ? 0.f : bf2f(sring[d][j]));
     load_w_tile(step + DW, dc, jc);  // slot consumed: refill it DW steps ahead
-    const float m8s = -8.f * s_c;
     const uint32_t wd[4] = {wc[0].x, wc[0].y, wc[0].z, wc[0].w};
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       bf16x8_t b;
       if (LORA) b = __builtin_bit_cast(bf16x8_t, wc[t % WPT]);
-      else b = dequant_word(wd[t], s_c, m8s);
+      else b = dequant_word(wd[t], sc);
 #pragma unroll
       for (int m = 0; m < MT; ++m)
         acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[m][t], b, acc[m], 0, 0, 0);
@@ -1848,7 +1843,7 @@ __global__ __launch_bounds__(256) void int4_dequant_kernel(const uint4* qw, cons
   const uint32_t wd[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    const bf16x8_t b = dequant_word<true>(wd[t], s, -8.f * s);
+    const bf16x8_t b = dequant_word_any_scale(wd[t], s, -8.f * s);
     uint16_t e[8];
     __builtin_memcpy(e, &b, 16);
 #pragma unroll

@@ -12,16 +12,16 @@ namespace tmx {
 // 1.8 GHz (4096 x 4096 x 28672), and the same launch with zeros for x runs 1.27 times as fast.  Registers only and on
 // random bf16 the 16 x 16 x 32 MFMA sustains 2.02 PFLOP/s and the 32 x 32 x 16 one 1.77, so the former, although it takes
 // twice the issue slots.  In one round of workgroups it is the schedule: the loop below takes 2.18 us a step of 8 x 8 tiles
-// where its MFMAs alone are 1.71 (2.75 us with 32 x 32 x 16, the barrier between two steps and the transfers in one
-// burst behind it).
+// where its MFMAs alone are 1.71.  Before (32 x 32 x 16, the barrier between two steps, the transfers of a slab in one
+// burst behind it), us: 4096 x 4096 x 28672 800 -> 715, 4096 x 14336 x 4096 385 -> 338, 256 x 4096 x 28672 64 -> 55.
 // A q4t word holds 8 k of a column; lane (h, n) of a tile has those of column n, k-chunk 2 t + h in word t.  Two lane
 // swaps of the words of a group leave lane group q of 16 lanes with chunk q of column n % 16 in one and of 16 + n % 16 in
 // the other.  In that order of the chunks the MFMA rounds like two 32 x 32 x 16 ones, bit for bit.
 // Weights come by buffer loads, the activation slab of a step (2 k-tiles) by direct-to-LDS loads into NB buffers: slab
 // rows are 256 bytes (four per 1 KiB transfer), their 16-byte chunks XOR-swizzled by row % 16.  With KW = 2 a wave takes
 // one k-tile of every step, and the two halves of a column tile meet through LDS at the end.
-// NB is 4 for the smallest tile (256 x 4096 x 4096 in 2 slices: 19.1 -> 15.9 us; a step of it is shorter than a load takes), 2 for
-// the others (3 x 4 in 3 buffers measured the same).
+// NB is 4 for the smallest tile, whose step is shorter than a load takes (256 x 4096 x 4096 in 2 slices: 19.1 -> 15.9 us), 2
+// for the others (3 x 4 in 3 buffers measured the same).
 constexpr int kWideTS = 2, kWideXS = 128;
 constexpr int kWideTiles32 = TMX_MAX_FILL_ROWS / 32;  // words per kind in a hand-over area: arrivals | ready flags
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
@@ -134,7 +134,7 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
   // A step is G groups of RF fragments of two MFMAs.  Behind the MFMAs of a fragment its register is refilled with the
   // one RING further on, and the weight fragments of the next group are dequantised an eighth at a time, so the matrix pipe
   // waits neither for LDS nor for the VALU; the transfers of a slab are spread over the first fragments of a step
-  // (in one burst they hold up all waves: a step 12 % longer).  The order is pinned.
+  // (in one burst behind the barrier they hold up all waves: 256 x 14336 x 4096 in 8 x 8 tiles 310 -> 268 us).  The order is pinned.
   // The barrier that hands over the next slab stands inside the last group, where no fragment of this slab is left to
   // read and those in registers keep the pipe busy; the first ones of the next step are read behind it.
   // The wave that is behind goes first (s_setprio falls with the groups done): otherwise the older of the two waves of a
