@@ -1080,6 +1080,43 @@ def test_adapter_sync_writes_both_operands(K, r, widths, dtype):
     assert torch.equal(ga, want_a) and torch.equal(gb, want_b)
 
 
+# experts with no row, with one, and with as many as end and begin a row tile of 16 and a chunk; column blocks whose last waves
+# have no columns; the reference is the f32 product with the dequantised matrices
+@pytest.mark.parametrize('down,K,N', [(0, 256, 640), (0, 512, 128), (1, 256, 384), (1, 768, 128)])
+def test_moe_experts_row_counts(down, K, N):
+  from tunix_amd import quant
+  counts = [0, 1, 15, 16, 17, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 257, 300]
+  E, k, group = len(counts), 2, 64
+  g = torch.Generator(device=G.DEV).manual_seed(K + N)
+  idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+  P = idx.numel() // k * k
+  assert 1024 < P <= 8192
+  idx = idx[torch.randperm(idx.numel(), generator=torch.Generator().manual_seed(3))][:P].to(torch.int32).to(G.DEV)
+  w = (torch.randn(K, E * N, generator=g, device=G.DEV) * 0.05).to(torch.bfloat16)
+  pl = quant.PackedLinear.from_dense([w], group, G.DEV)
+  dense = torch.empty(K, E * N, dtype=torch.bfloat16, device=G.DEV)
+  G.call('tmx_int4_dequant', S(), G.p(pl.qweight), G.p(pl.scales), G.p(dense), K, E * N, group)
+  x = torch.randn(P if down else P // k, K, generator=g, device=G.DEV).to(torch.bfloat16)
+  cols = N if down else N // 2
+  out = torch.full((P + 1, cols), 7.0, dtype=torch.bfloat16, device=G.DEV)  # the last row stays
+  G.call('tmx_moe_experts', S(), G.p(x), K, G.p(pl.qweight), G.p(pl.scales), G.p(idx), P, k, E, K, N, group, down, G.p(out), cols)
+  rows = x.float() if down else x.float().repeat_interleave(k, 0)
+  want = torch.empty(P, cols, device=G.DEV)
+  rb = lambda t: t.to(torch.bfloat16).float()
+  for e in range(E):
+    mine = (idx == e).nonzero().flatten()
+    y = rows[mine] @ dense[:, e * N:(e + 1) * N].float()
+    if not down:
+      gate, up = rb(y[:, :cols]), rb(y[:, cols:])
+      y = rb(gate * rb(torch.sigmoid(gate))) * up
+    want[mine] = y
+  assert (out[P] == 7.0).all()
+  got = out[:P].float()
+  # one rounding to bf16 of down, four of gate | up (a flip of one of them by a bf16 step now and then)
+  assert (got - want).norm() <= (2e-3 if down else 6e-3) * want.norm()
+  assert ((got - want).abs() > 2.0 ** -6 * want.abs() + 2.0 ** -8).sum() == 0
+
+
 # row tiles x column tiles of the many-rows kernel that these shapes take on 256 compute units (wide_plan), ragged in
 # rows and columns; the reference is the f32 product of the dequantised matrix
 @pytest.mark.parametrize('M,K,N', [

@@ -49,7 +49,7 @@ __device__ __forceinline__ void gemm_block4(const QLinearArgs& a, uint16_t (*xs)
   // K-slice of this block: main blocks follow blockIdx.y; the LoRA blocks of a launch cut K
   // into finer slices of their own so that none of them is the last to finish
   const int slice = LORA ? ((int)blockIdx.x - a.n_main_blocks) + a.lora_blocks_per_split * (int)blockIdx.y
-                         : (a.fixed_slice >= 0 ? a.fixed_slice : (int)blockIdx.y);
+                         : (int)blockIdx.y;
   const int per = LORA ? a.kt_per_lora_split : a.kt_per_split;
   const int kb0 = slice * per;
   const int kb1 = (kb0 + per < KT) ? kb0 + per : KT;
@@ -92,8 +92,7 @@ __device__ __forceinline__ void gemm_block4(const QLinearArgs& a, uint16_t (*xs)
     const int c = tid + 256 * i;
     const int row_l = c >> 5, col_l = (c & 31) * 8;
     xoff_l[i] = row_l * kXStride + col_l;
-    int row = row_l < a.M ? row_l : a.M - 1;
-    if (a.row_src) row = a.row_src[row];
+    const int row = row_l < a.M ? row_l : a.M - 1;
     xsrc[i] = a.x + (size_t)row * a.ldx + (size_t)kb0 * 64 + col_l;
   }
   constexpr int WPT = LORA ? 4 : 1;  // 16-byte words per lane and tile
@@ -297,8 +296,7 @@ __device__ __forceinline__ void gemm_block4(const QLinearArgs& a, uint16_t (*xs)
           if (row >= a.M) continue;
           const float g = acc[m][r], u = ex[(((wave * MT + m) * 16 + r) << 6) + lane];
           const float sg = rbf(1.f / (1.f + expf(-g)));
-          const int drow = a.row_dst ? a.row_dst[row] : row;
-          a.y_bf16[(size_t)drow * a.ldy + col] = f2bf(rbf(g * sg) * u);
+          a.y_bf16[(size_t)row * a.ldy + col] = f2bf(rbf(g * sg) * u);
         }
     }
     return;
@@ -312,9 +310,8 @@ __device__ __forceinline__ void gemm_block4(const QLinearArgs& a, uint16_t (*xs)
       for (int r = 0; r < 16; ++r) {
         const int row = m * 32 + acc_row(r, lane);
         if (row >= a.M) continue;
-        const int drow = (!LORA && a.row_dst) ? a.row_dst[row] : row;
         if (LORA) a.t_part[((size_t)slice * a.M + row) * a.ldt + col] = acc[m][r];
-        else if (a.y_bf16) a.y_bf16[(size_t)drow * a.ldy + col] = f2bf(acc[m][r]);
+        else if (a.y_bf16) a.y_bf16[(size_t)row * a.ldy + col] = f2bf(acc[m][r]);
         else a.y_part[((size_t)slice * a.M + row) * a.N + col] = acc[m][r];
       }
   }
@@ -357,11 +354,12 @@ static int launch_qlinear4(hipStream_t st, QLinearArgs a) {
 // on this part, a non-temporal one 6.3-7.0; the split projections and the 64-row head measured slower with it.
 constexpr int kNtLoad = 2;
 
+constexpr int kMoeStreamPairs = 1024;  // most pairs of a launch (more: moe_rows)
 constexpr int kMoeRing = 4;  // divides K / 64 (K % 256 == 0), so a ring slot is k-tile % 4 in every unit
 
 template <bool DOWN>
 __global__ __launch_bounds__(256, 2) void moe_stream_kernel(MoeArgs m) {
-  __shared__ int rows_s[TMX_MAX_MOE_PAIRS];
+  __shared__ int rows_s[kMoeStreamPairs];
   __shared__ int wave_cnt[4];
   __shared__ int n_s;
   constexpr int TPU = DOWN ? 1 : 2;  // tiles per unit: one column tile, or a gate tile and its up tile
@@ -474,77 +472,12 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(MoeArgs m) {
   }
 }
 
-// Many rows per expert (cache fill and scoring passes of a MoE model: thousands of routed pairs): the
-// stream kernel above would re-read the gathered activation rows in every wave, so here a workgroup
-// (column block, expert) runs the 4-wave block over the expert's rows in chunks of 32 with the
-// activation slab shared in LDS (gathered rows in, scattered rows out).  DOWN = false fuses SwiGLU: the
-// workgroup owns 64 gate columns and the matching 64 up columns.
-template <bool DOWN>
-__global__ __launch_bounds__(256, 2) void moe_block_kernel(MoeArgs m) {
-  __shared__ __align__(16) uint16_t xs[2][32][kXStride];
-  __shared__ int rows_s[TMX_MAX_MOE_PAIRS];
-  __shared__ int src_s[32], dst_s[32];
-  __shared__ int wave_cnt[4];
-  __shared__ int n_s;
-  const int e = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int base = 0;
-  int ev = tid < m.P ? m.expert_of[tid] : -1;
-  for (int p0 = 0; p0 < m.P; p0 += 256) {  // ordered compaction of { p : expert_of[p] == e }
-    const int p = p0 + tid;
-    const bool hit = ev == e;
-    ev = p + 256 < m.P ? m.expert_of[p + 256] : -1;  // the next round's entry travels during this one's barriers
-    const unsigned long long mask = __ballot(hit);
-    if (lane == 0) wave_cnt[wave] = __popcll(mask);
-    __syncthreads();
-    int off = base;
-    for (int w = 0; w < wave; ++w) off += wave_cnt[w];
-    if (hit) rows_s[off + __popcll(mask & ((1ull << lane) - 1ull))] = p;
-    base += wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
-    __syncthreads();
-  }
-  if (tid == 0) n_s = base;
-  __syncthreads();
-  const int n = n_s;
-  if (n == 0) return;
-  QLinearArgs a = {};
-  a.x = m.x;
-  a.ldx = m.ldx;
-  a.qw = m.qw + (size_t)e * m.qw_stride;
-  a.scales = m.scales + (size_t)e * m.sc_stride;
-  a.y_bf16 = m.out;
-  a.ldy = m.ldo;
-  a.K = m.K; a.N = m.N; a.G = m.G;
-  a.n_main_blocks = gridDim.x;
-  a.nsplit = 1;
-  a.kt_per_split = m.K >> 6;
-  a.fixed_slice = 0;
-  a.row_src = src_s;
-  a.row_dst = dst_s;
-  a.pair_off = DOWN ? 0 : (m.N >> 6);  // tiles in F = N / 2 columns
-  for (int c0 = 0; c0 < n; c0 += 32) {
-    if (tid < 32 && c0 + tid < n) {
-      const int p = rows_s[c0 + tid];
-      src_s[tid] = DOWN ? p : p / m.top_k;
-      dst_s[tid] = p;
-    }
-    __syncthreads();
-    a.M = n - c0 < 32 ? n - c0 : 32;
-    gemm_block4<1, false>(a, xs);
-    __syncthreads();
-  }
-}
-
-
 int moe_experts(hipStream_t st, const MoeArgs& a, int E, bool down) {
   if (!a.x || !a.qw || !a.scales || !a.expert_of || !a.out) return TMX_ERR_ARG;
   if (a.P <= 0 || a.P > TMX_MAX_MOE_PAIRS || a.top_k <= 0 || E <= 0) return TMX_ERR_SHAPE;
   if (a.K % 256 || a.G % 64 || (a.G & (a.G - 1)) || a.K % a.G || a.ldx % 8) return TMX_ERR_SHAPE;
   if (a.N % 128) return TMX_ERR_SHAPE;  // gate | up: F % 64 == 0
-  if (a.P > 1024) {  // many rows per expert: the block kernel with the activation slab in LDS
-    if (down) hipLaunchKernelGGL(moe_block_kernel<true>, dim3(a.N / 128, E), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(moe_block_kernel<false>, dim3(a.N / 128, E), dim3(256), 0, st, a);
-    return check_launch();
-  }
+  if (a.P > kMoeStreamPairs) return moe_rows(st, a, E, down);  // many rows per expert (qwide.hip)
   // decode: few rows per expert, a pure weight stream
   // column groups per expert: one gate | up pair (2 x K / 64 weight tiles) or two down tiles per wave
   // (measured on the 30B-A3B shapes: 6 groups for gate | up, 8 for down; fewer leave CUs short of
@@ -1627,7 +1560,6 @@ int qlinear_gate_up_swiglu(hipStream_t st, const void* x, int ldx, const void* q
     return TMX_ERR_SHAPE;
   if (a_t && (!lora_b || r <= 0 || 2 * r > 32)) return TMX_ERR_SHAPE;
   QLinearArgs a = {};
-  a.fixed_slice = -1;
   a.x = (const uint16_t*)x;
   a.ldx = ldx;
   a.qw = (const uint4*)qw;
@@ -1716,7 +1648,6 @@ int qlinear_base(hipStream_t st, const void* x, int ldx, const void* qw, const v
   const int KT = K / 64;
   if (!slices_ok(KT, nsplit)) return TMX_ERR_SHAPE;  // an empty K-slice
   QLinearArgs a = {};
-  a.fixed_slice = -1;
   a.ldy = N;
   a.x = (const uint16_t*)x;
   a.ldx = ldx;
@@ -1785,7 +1716,6 @@ int qlinear_wide(hipStream_t st, const void* x, int ldx, const void* qw, const v
   if ((size_t)256 * ldx * 2 >= (1u << 31) || (size_t)K * N / 2 >= (1u << 31) || (size_t)K * Rpad * 2 >= (1u << 31))
     return TMX_ERR_SHAPE;
   QLinearArgs a = {};
-  a.fixed_slice = -1;
   a.ldy = N;
   a.x = (const uint16_t*)x;
   a.ldx = ldx;

@@ -37,41 +37,22 @@ __device__ __forceinline__ uint32_t moved(uint32_t v) {
 }
 __device__ __forceinline__ u32x4_t moved(u32x4_t v) { return u32x4_t{moved(v.x), moved(v.y), moved(v.z), moved(v.w)}; }
 
-template <int MT, int CT>
-__device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* smem, int bx, int slice, int bz) {
-  constexpr int TS = kWideTS, XS = kWideXS, ROWS = MT * 32, KW = 8 / CT, TPW = TS / KW;
-  constexpr int NB = wide_bufs(MT), WB = NB > 2 ? NB : 1;  // slab buffers; weight registers (steps on the way)
+// The product itself: acc[u][r] = rows 16 r .. + 15 of x times columns 16 u .. + 15 of a wave's column tile, over nsteps steps
+// from k-tile kb0 on.  wv / sv: byte offsets of this lane's words and scale in the first k-tile (of the tile's columns
+// lane % 32; any 16 + 16 columns do); xo(i): of this lane's 16 bytes of the i-th slab transfer.  Every wave of the workgroup
+// takes part; one that is not `active` only helps with the slab.
+template <int MT, int KW, int NB, class XO>
+__device__ __forceinline__ void wide_core(uint16_t* smem, __amdgpu_buffer_rsrc_t rw, int wv, __amdgpu_buffer_rsrc_t rs, int sv,
+                                          int gs, __amdgpu_buffer_rsrc_t rx, XO xo, int kb0, int nsteps, int kw, bool active,
+                                          f32x4_t (&acc)[2][2 * MT]) {
+  constexpr int TS = kWideTS, XS = kWideXS, ROWS = MT * 32, TPW = TS / KW;
+  constexpr int WB = NB > 2 ? NB : 1;                      // weight registers (steps on the way)
   constexpr int G = 2 * TPW, RF = 2 * MT;                  // groups of 32 k a step, x fragments (16 rows) of a group
   constexpr int RING = RF <= 4 ? RF : RF / 2;              // x fragments in registers
-  constexpr int MEET = RF - RING + 2;                      // the fragment of the last group in front of which the waves meet
+  constexpr int MEET = RF - RING + 2 < RF ? RF - RING + 2 : RF - 1;  // the fragment of the last group in front of which the waves meet
   constexpr int DS = (G - 1) * RF / MT < 2 ? 1 : 2;        // fragments between two slab transfers
-  static_assert(KW * CT == 8 && TPW >= 1, "8 waves, at least one k-tile of a step each");
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ct = wave % CT, kw = wave / CT;
-  const int q = lane >> 4, nl = lane & 15;
-  const int KT = a.K >> 6;
-  const int per = a.kt_per_split;
-  const int kb0 = slice * per;
-  const int kb1 = (kb0 + per < KT) ? kb0 + per : KT;
-  const int nsteps = (kb1 - kb0) / TS, last_step = nsteps - 1;  // host: whole steps
-  if (nsteps <= 0) return;
-  const int row0 = bz * ROWS;
-  const int rows = a.M - row0 < ROWS ? a.M - row0 : ROWS;  // host: >= 1
-  const int gs = __builtin_ctz(a.G >> 6), KG = a.K / a.G;
-  const int NT = a.N >> 5, nb = bx * CT + ct;
-  const bool tile_ok = nb < NT;  // waves past the last tile only help with the slab
-
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.qw, (uint32_t)NT * KT * 1024u);
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.scales, (uint32_t)NT * KG * 64u);
-  const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x + (size_t)row0 * a.ldx, (uint32_t)rows * a.ldx * 2u);
-  const int wv = (nb * KT * 64 + lane) * 16;
-  const int sv = (nb * KG * 32 + (lane & 31)) * 2;
-  // slab transfer: MT loads per wave and step; load i moves rows 4 wave + 32 i .. + 3 (16 lanes each), lane l
-  // delivering chunk (l % 16) ^ (row % 16) of the step to slot l % 16.  Rows past the end lie past the descriptor's: zeros.
-  const int row_l = 4 * wave + (lane >> 4);
-  const int xoff = row_l * a.ldx * 2 + (((lane & 15) ^ (row_l & 15)) * 16) + kb0 * 128;
-
-  f32x4_t acc[2][RF];  // columns 0..15 and 16..31 of the tile
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int q = lane >> 4, nl = lane & 15, last_step = nsteps - 1;
 #pragma unroll
   for (int r = 0; r < RF; ++r) acc[0][r] = acc[1][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   u32x4_t wring[WB][TPW], wc[TPW];
@@ -102,7 +83,7 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
   auto dma_x = [&](int step, int buf, int i) __attribute__((always_inline)) {
     step = step < last_step ? step : last_step;
     uint16_t* base = smem + (size_t)buf * ROWS * XS + wave * 4 * XS;
-    load_row_to_lds(rx, base + i * 32 * XS, xoff + i * 64 * a.ldx, step * (TS * 128));
+    load_row_to_lds(rx, base + i * 32 * XS, xo(i), step * (TS * 128));
   };
   // all but the youngest loads of this wave have arrived and its LDS reads are done; then all waves
   auto meet = [&](auto younger) __attribute__((always_inline)) {
@@ -189,7 +170,7 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
   meet(IC<(NB - 2) * MT>{});
   take_w(IC<0>{});
   load_w(WB, IC<0>{});
-  if (tile_ok) {
+  if (active) {
     static_for<RING>([&](auto rc) __attribute__((always_inline)) { read_x(xlane + (c0 ^ nl) * 8, rc); });
     static_for<8>([&](auto pc) __attribute__((always_inline)) { dequant(IC<0>{}, pc); });
     if constexpr (WB == 1) {
@@ -208,11 +189,45 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
     }
   }
   __builtin_amdgcn_s_setprio(0);
+}
+
+template <int MT, int CT>
+__device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* smem, int bx, int slice, int bz) {
+  constexpr int ROWS = MT * 32, KW = 8 / CT, RF = 2 * MT;
+  static_assert(KW * CT == 8, "8 waves");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ct = wave % CT, kw = wave / CT;
+  const int q = lane >> 4, nl = lane & 15;
+  const int KT = a.K >> 6;
+  const int per = a.kt_per_split;
+  const int kb0 = slice * per;
+  const int kb1 = (kb0 + per < KT) ? kb0 + per : KT;
+  const int nsteps = (kb1 - kb0) / kWideTS;  // host: whole steps
+  if (nsteps <= 0) return;
+  const int row0 = bz * ROWS;
+  const int rows = a.M - row0 < ROWS ? a.M - row0 : ROWS;  // host: >= 1
+  const int gs = __builtin_ctz(a.G >> 6), KG = a.K / a.G;
+  const int NT = a.N >> 5, nb = bx * CT + ct;
+  const bool tile_ok = nb < NT;  // waves past the last tile only help with the slab
+
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.qw, (uint32_t)NT * KT * 1024u);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.scales, (uint32_t)NT * KG * 64u);
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x + (size_t)row0 * a.ldx, (uint32_t)rows * a.ldx * 2u);
+  const int wv = (nb * KT * 64 + lane) * 16;
+  const int sv = (nb * KG * 32 + (lane & 31)) * 2;
+  // slab transfer: MT loads per wave and step; load i moves rows 4 wave + 32 i .. + 3 (16 lanes each), lane l
+  // delivering chunk (l % 16) ^ (row % 16) of the step to slot l % 16.  Rows past the end lie past the descriptor's: zeros.
+  const int row_l = 4 * wave + (lane >> 4);
+  const int xoff = row_l * a.ldx * 2 + (((lane & 15) ^ (row_l & 15)) * 16) + kb0 * 128;
+
+  f32x4_t acc[2][RF];  // columns 0..15 and 16..31 of the tile
+  wide_core<MT, KW, wide_bufs(MT)>(smem, rw, wv, rs, sv, gs, rx, [&](int i) { return xoff + i * 64 * a.ldx; }, kb0, nsteps, kw, tile_ok, acc);
   // Two k-parts of a tile swap halves of their accumulators (the slab is free once the surplus transfers, repeats of
   // the last step, have landed): the first finishes the first half of the rows, the second the other.
   constexpr int NR = RF / KW;  // row tiles of 16 this wave finishes
   if constexpr (KW == 2) {
-    meet(IC<0>{});
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    __syncthreads();
     f32x4_t* hb = reinterpret_cast<f32x4_t*>(smem) + (size_t)ct * RF * 2 * 64 + lane;  // [CT][2 parts][2][NR][64]
     if (tile_ok)
 #pragma unroll
@@ -485,6 +500,107 @@ static int launch_wide(hipStream_t st, QLinearArgs a) {
   const int ids = (int)((total + 7) / 8 * 8);
   hipLaunchKernelGGL((qlinear_mfma_wide_kernel<MT, CT>), dim3(a.lora_wgs + ids), dim3(512), wide_lds(MT), st, a, blocks, row_blocks, S);
   return check_launch();
+}
+
+// Routed experts with many rows (cache fill and scoring passes of a MoE model): workgroup = (column block, expert), up to 128
+// of the expert's rows at a time through the many-rows product, gathered rows in and scattered rows out.  A wave has 32
+// columns: a tile of down, or 16 hidden units of gate | up as 16 gate and the matching 16 up columns, so that both meet in
+// a lane and SwiGLU needs no exchange.  Sums run over K in the order of moe_stream_kernel: the same bits.
+// What bounds it at the 64 rows an expert has in a pass of 1024 tokens (128 experts of 2048 x 768, top-8) is the
+// instructions of the dequantisation (32 us of issue) beside those of the MFMAs: 92 + 63 us per layer, in chunks of 32 rows that
+// dequantised every matrix two to three times 194 + 145 us.  In this form (134 to 150 registers, one workgroup per CU): held to 128
+// registers, two per CU, it spills and takes 121 us for gate | up; three or four slab buffers, 101 and 106; chunks
+// of 64 rows 125 (an expert with 65 rows streams its matrices twice).  The list of rows is read in one go by every
+// workgroup, consecutive pairs by consecutive lanes; 16 pairs per lane instead cost 23 us of down's 80.
+constexpr int kMoeRows = 128;  // rows of a chunk
+template <bool DOWN, int MT>
+__device__ __forceinline__ void moe_chunk(const MoeArgs& m, int e, int bx, const uint16_t* rows_s, int n, uint16_t* smem) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q = lane >> 4, nl = lane & 15, h = lane >> 5, sub = q & 1;
+  const int KT = m.K >> 6, KG = m.K / m.G, unit = bx * 8 + wave;
+  const bool active = unit * 32 < m.N;
+  // the tile and the 16 columns of it that this lane has words of
+  const int nb = DOWN ? unit : (unit >> 1) + sub * (m.N >> 6), half = DOWN ? sub : unit & 1;
+  const int wv = (nb * KT * 64 + 32 * h + 16 * half + nl) * 16, sv = (nb * KG * 32 + 16 * half + nl) * 2;
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(m.qw + (size_t)e * m.qw_stride, (uint32_t)m.K * m.N / 2u);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(m.scales + (size_t)e * m.sc_stride, (uint32_t)KG * m.N * 2u);
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(m.x, (uint32_t)(DOWN ? m.P : m.P / m.top_k) * m.ldx * 2u);
+  const int row_l = 4 * wave + q;
+  int xoff[MT];  // rows past the end: past the descriptor's end, zeros
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int r = row_l + 32 * i, p = rows_s[r < n ? r : 0];
+    xoff[i] = r < n ? (DOWN ? p : p / m.top_k) * m.ldx * 2 + ((nl ^ (row_l & 15)) * 16) : (int)0x7FFF0000;
+  }
+  f32x4_t acc[2][2 * MT];
+  wide_core<MT, 1, 2>(smem, rw, wv, rs, sv, __builtin_ctz(m.G >> 6), rx, [&](int i) { return xoff[i]; }, 0, m.K / (64 * kWideTS), 0,
+                      active, acc);
+  if (!active) return;
+#pragma unroll
+  for (int i = 0; i < 2 * MT; ++i) {
+    const int r = i * 16 + nl;
+    if (r >= n) continue;
+    uint16_t* out = m.out + (size_t)rows_s[r] * m.ldo + unit * (DOWN ? 32 : 16) + 4 * q;
+    if constexpr (DOWN) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        *reinterpret_cast<u32x2_t*>(out + 16 * u) = u32x2_t{pack_bf2(acc[u][i][0], acc[u][i][1]), pack_bf2(acc[u][i][2], acc[u][i][3])};
+    } else {
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float g = rbf(acc[0][i][k]), up = rbf(acc[1][i][k]);
+        v[k] = rbf(g * rbf(1.f / (1.f + expf(-g)))) * up;
+      }
+      *reinterpret_cast<u32x2_t*>(out) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+    }
+  }
+}
+
+template <bool DOWN>
+__global__ __launch_bounds__(512, 2) void moe_rows_kernel(MoeArgs m, int E, int blocks) {
+  extern __shared__ __align__(16) uint16_t smem[];
+  __shared__ uint16_t rows_s[TMX_MAX_MOE_PAIRS];
+  __shared__ int n_s;
+  // the column blocks of an expert on one XCD: its rows are fetched into one L2
+  const int xcd = blockIdx.x & 7, idx = (int)blockIdx.x >> 3, e = idx / blocks * 8 + xcd, bx = idx % blocks, tid = threadIdx.x;
+  if (e >= E) return;
+  if (tid == 0) n_s = 0;
+  __syncthreads();
+  {  // { p : expert_of[p] == e }, in any order: the rows of a product do not meet
+    constexpr int PT = TMX_MAX_MOE_PAIRS / 512;
+    int ex[PT];
+#pragma unroll
+    for (int u = 0; u < PT; ++u) ex[u] = tid + 512 * u < m.P ? m.expert_of[tid + 512 * u] : -1;
+#pragma unroll
+    for (int u = 0; u < PT; ++u)
+      if (ex[u] == e) rows_s[atomicAdd(&n_s, 1)] = (uint16_t)(tid + 512 * u);
+  }
+  __syncthreads();
+  const int n = n_s;
+  for (int c0 = 0; c0 < n; c0 += kMoeRows) {
+    const int left = n - c0;
+    if (left <= 32) moe_chunk<DOWN, 1>(m, e, bx, rows_s + c0, left, smem);
+    else if (left <= 64) moe_chunk<DOWN, 2>(m, e, bx, rows_s + c0, left, smem);
+    else if (left <= 96) moe_chunk<DOWN, 3>(m, e, bx, rows_s + c0, left, smem);
+    else moe_chunk<DOWN, 4>(m, e, bx, rows_s + c0, left < kMoeRows ? left : kMoeRows, smem);
+    __builtin_amdgcn_s_waitcnt(0x0070);  // the surplus transfers have landed before the slab is used again
+    __syncthreads();
+  }
+}
+
+template <bool DOWN>
+static int launch_moe_rows(hipStream_t st, const MoeArgs& a, int E) {
+  constexpr size_t lds = (size_t)2 * kMoeRows * kWideXS * 2;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_rows_kernel<DOWN>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (attr != hipSuccess) return TMX_ERR_LAUNCH;
+  const int blocks = (a.N + 255) / 256;
+  hipLaunchKernelGGL(moe_rows_kernel<DOWN>, dim3((E + 7) / 8 * 8 * blocks), dim3(512), lds, st, a, E, blocks);
+  return check_launch();
+}
+int moe_rows(hipStream_t st, const MoeArgs& a, int E, bool down) {
+  return down ? launch_moe_rows<true>(st, a, E) : launch_moe_rows<false>(st, a, E);
 }
 
 // Which tile and how many K-slices.  The order in which a sum runs over K is set by the slices and by CT (one or two

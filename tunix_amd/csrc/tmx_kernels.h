@@ -17,11 +17,7 @@ struct QLinearArgs {
   int M, K, N, G, Rpad;
   int n_main_blocks, nsplit, kt_per_split;
   int lora_blocks_per_split, kt_per_lora_split;  // finer K-slices of the LoRA projection
-  // routed-expert use of the 4-wave block (all zero / null / -1 for plain projections)
   int ldy;                 // row stride of y_bf16
-  int fixed_slice;         // K-slice index when blockIdx.y means something else (-1: blockIdx.y)
-  const int* row_src;      // activation row of tile row i (null: i)
-  const int* row_dst;      // output row of tile row i (null: i)
   int pair_off;            // != 0: gate | up pairing, tile distance between a gate tile and its up tile
   // LoRA inside the pair epilogue (fused gate | up kernel): a_t = [A_gate | A_up], Rpad == 32
   const uint16_t* lora_b;  // [lora_r][N] bf16
@@ -303,6 +299,7 @@ size_t attn_shared_partial_bytes(int B, int N, int Kh, int H, int C);
 bool attn_share_ok(int B, int N, int Kh, int H, int C, int share_gs, int share_len);
 int moe_route(hipStream_t st, const RouterArgs& a, int B);
 int moe_experts(hipStream_t st, const MoeArgs& a, int E, bool down);
+int moe_rows(hipStream_t st, const MoeArgs& a, int E, bool down);  // its form for many rows per expert
 int head_sample(hipStream_t st, HeadArgs a);
 // any number of rows in 256 x 256 blocks (greedy, sampling without the sorting branch, scoring); needs
 // D % 128 == 0, no forbidden ids, no logits output; part_f / part_i sized [M][ceil(V / 256)]
