@@ -1350,8 +1350,8 @@ __device__ __forceinline__ void gemm_block_dma(const QLinearArgs& a, uint16_t* s
       }
     u32x4_t wc[WPT];
 #pragma unroll
-    for (int t = 0; t < WPT; ++t) wc[t] = wring[d][j][t];
-    const NibbleScale sc = nibble_scale(LORA ? 0.f : bf2f(sring[d][j]));
+    for (int t = 0; t < WPT; ++t) wc[t] = moved(wring[d][j][t]);
+    const NibbleScale sc = nibble_scale(LORA ? 0.f : bf2f((uint16_t)moved((uint32_t)sring[d][j])));
     load_w_tile(step + DW, dc, jc);  // slot consumed: refill it DW steps ahead
     const uint32_t wd[4] = {wc[0].x, wc[0].y, wc[0].z, wc[0].w};
 #pragma unroll
@@ -1371,7 +1371,10 @@ __device__ __forceinline__ void gemm_block_dma(const QLinearArgs& a, uint16_t* s
     __builtin_amdgcn_sched_barrier(0);
     if (tile_ok) __builtin_amdgcn_s_waitcnt(0x0F70 | (kYounger & 15) | ((kYounger >> 4) << 14));
     else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
   };
   auto do_step = [&](int step, auto sc) __attribute__((always_inline)) {
     constexpr int sp = decltype(sc)::value;
@@ -1397,6 +1400,8 @@ __device__ __forceinline__ void gemm_block_dma(const QLinearArgs& a, uint16_t* s
 
   // the two k-halves of a tile swap halves of their accumulators through LDS (the slab is free:
   // the last step ended with a barrier): the first finishes registers 0..7, the second 8..15
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  __syncthreads();
   float* hb = reinterpret_cast<float*>(smem);  // [4 tiles][MT][16][64]
   if (tile_ok) {
 #pragma unroll

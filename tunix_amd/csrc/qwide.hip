@@ -28,15 +28,6 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 constexpr int wide_bufs(int mt) { return mt == 2 ? 4 : 2; }
 constexpr size_t wide_lds(int mt) { return (size_t)wide_bufs(mt) * mt * 32 * kWideXS * 2; }
 
-// A copy the compiler does not see through: it happens here, so the registers of v are free for the load that follows
-// (otherwise the copy moves to the end of the loop, behind that load, and waits for it).
-__device__ __forceinline__ uint32_t moved(uint32_t v) {
-  uint32_t r;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
-  return r;
-}
-__device__ __forceinline__ u32x4_t moved(u32x4_t v) { return u32x4_t{moved(v.x), moved(v.y), moved(v.z), moved(v.w)}; }
-
 // The product itself: acc[u][r] = rows 16 r .. + 15 of x times columns 16 u .. + 15 of a wave's column tile, over nsteps steps
 // from k-tile kb0 on.  wv / sv: byte offsets of this lane's words and scale in the first k-tile (of the tile's columns
 // lane % 32; any 16 + 16 columns do); xo(i): of this lane's 16 bytes of the i-th slab transfer.  Every wave of the workgroup

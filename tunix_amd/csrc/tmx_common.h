@@ -136,6 +136,15 @@ __device__ __forceinline__ bf16x8_t dequant_word(uint32_t d, const NibbleScale& 
   return r;
 }
 
+// A copy the compiler does not see through: it happens here, so the registers of v are free for the load that follows
+// (otherwise the copy moves to the end of the loop, behind that load, and waits for it).
+__device__ __forceinline__ uint32_t moved(uint32_t v) {
+  uint32_t r;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+__device__ __forceinline__ u32x4_t moved(u32x4_t v) { return u32x4_t{moved(v.x), moved(v.y), moved(v.z), moved(v.w)}; }
+
 template <int V>
 struct IC { static constexpr int value = V; };
 
