@@ -910,3 +910,31 @@ def test_scoring_shares_no_prompt_between_rows_whose_token_masks_differ():
     s.share_prompt_kv = share
     got[share] = s.per_token_logps(prompt, comp, pad_id=0, token_mask=mask)
   assert np.abs(got[True] - got[False]).max() <= LOGPROB_TOL
+
+
+@pytest.mark.parametrize('family', ['llama3', 'moe'])
+@pytest.mark.parametrize('b,p,t', [(5, 37, 20), (1, 2, 1), (3, 1, 6), (4, 65, 3)])
+def test_scoring_in_one_walk_equals_prompt_and_completion_walks(family, b, p, t):
+  """Prompt and completion in one pass, where padding in front of the prompts is walked too and scores of prompt columns are
+  left out: the log-probs are those of two walks.  Rows of other counts take other tiles and K-slices, so sums round
+  differently: the tolerance of the log-probs."""
+  cfg = C.TOY if family == 'llama3' else OM.Config('qwen3', 2, 1024, 256, 256, 4, 64, 2, rope_theta=1_000_000, norm_eps=1e-6,
+                                                   tied=False, num_experts=8, experts_per_tok=2)
+  model = C.product_model(cfg, C.make_state(cfg, 47, 8, norm_jitter=0.05), 64, 16.0)
+  rng = np.random.default_rng(p + t)
+  prompt = rng.integers(3, cfg.vocab_size, (b, p)).astype(np.int32)
+  comp = rng.integers(3, cfg.vocab_size, (b, t)).astype(np.int32)
+  for i in range(b):
+    prompt[i, :rng.integers(0, p)] = 0
+    comp[i, t - rng.integers(0, t):] = 0
+  if b > 2:
+    prompt[1] = 0  # nothing but padding in front of the completion
+  got, walks = [], []
+  for limit in (256, -1):
+    s = _sampler(model, cfg, 96)
+    s.ONE_WALK_ROWS = limit
+    walk = s.walk
+    s.walk = lambda st, n, sample=False, walk=walk: (walks.append((limit, n)), walk(st, n, sample))
+    got.append(s.per_token_logps(prompt, comp, pad_id=0))
+  assert walks == [(256, p + t - 1), (-1, p - 1), (-1, t)]
+  assert np.isfinite(got[0]).all() and np.abs(got[0] - got[1]).max() <= (2 if family == 'moe' else 1) * LOGPROB_TOL
