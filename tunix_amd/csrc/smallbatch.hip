@@ -499,7 +499,8 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
 // The 16 x 16 x 32 MFMA takes them: lane (n = l % 16, q = l / 16) holds column n of k-tile 2 p + q / 2, half q % 2, so a
 // wave's load is two half tiles, and word t of the four lanes of a column is 32 consecutive steps of the contraction
 // (the x operand reads the same k).  Measured on the 1B shape at one row / three rows (trace, us per launch,
-// 32 columns -> 16): q|k|v 8.0 / 9.1 -> 8.0 / 9.0, o 9.3 / 15.6 -> 7.4 / 9.6, down 11.8 / 14.4 -> 9.8 / 13.0.
+// 32 columns -> 16): q|k|v 8.0 / 9.1 -> 8.0 / 9.0, o 9.3 / 15.6 -> 7.4 / 9.6, down 11.8 / 14.4 -> 9.8 / 13.0 (less since, see
+// below and SbCopy).
 constexpr int kSbPairs = 8;  // k-tile pairs per wave requested at once
 
 // LDS: x [M][K + 8] bf16 | red [8 waves][4][16] f32 | red_t [8][4][64] f32 | t [4][64] f32 | row scratch [4 + 8 * 4] f32
@@ -535,28 +536,30 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
   for (int i = 0; i < kSbPairs; ++i)
     if (i < per) load_w(p0 + i, i);
 
-  // x . A of this wave's eighth of K (32 x 32 x 16 MFMAs: A's fragment order), for the 32-column tiles of A that hold
-  // this workgroup's segment; up to four (k-tile, tile) items at a time, the first four requested now
-  const int lrow = lane & 31, lh = lane >> 5;
+  // x . A of this wave's eighth of K, for the tiles of 16 columns of A that hold this workgroup's segment (of a rank of 16
+  // half of what lies in a tile of 32 is another segment's or padding: 64 KB instead of 128 KB of A per workgroup on the 1B
+  // shape, one row / three rows: q|k|v 8.0 / 9.1 -> 7.0 / 7.8 us, o 7.5 / 9.8 -> 6.4 / 8.7); up to four (k-tile, tile) items at a time, the first four requested now.
+  // The four lane groups of a load hold 32 consecutive steps of the contraction.
   const bool lora_here = a.a_t != nullptr;
-  int q0 = 0, q1 = -1;
+  int q0 = 0, nq = 0;
   if (lora_here) {
     const int n0 = (int)blockIdx.x * 16;
     const int seg = n0 >= a.seg_end[0] ? (n0 >= a.seg_end[1] ? 2 : 1) : 0;
-    q0 = (seg * a.lora_r) >> 5;
-    q1 = min(((seg + 1) * a.lora_r - 1) >> 5, (a.Rpad >> 5) - 1);
+    q0 = (seg * a.lora_r) >> 4;
+    nq = min(((seg + 1) * a.lora_r - 1) >> 4, (a.Rpad >> 4) - 1) - q0 + 1;  // 1 to 3: ranks up to 32
   }
-  const int RT = a.Rpad >> 5, nq = q1 - q0 + 1;
+  const int RT = a.Rpad >> 5;
   const int lper = (KT + kSbWaves - 1) / kSbWaves, l0 = wave * lper, l1 = min(l0 + lper, KT);
-  const int items = lora_here ? max(l1 - l0, 0) * nq : 0;
-  u32x4_t ab[4][4];
+  const int items = max(l1 - l0, 0) * nq;
+  u32x4_t ab[4][2];
   auto load_a = [&](int it, auto ic) __attribute__((always_inline)) {
     constexpr int i = decltype(ic)::value;
     if (it < items) {
-      const int kt = l0 + (nq == 2 ? it >> 1 : it), qq = q0 + (nq == 2 ? it & 1 : 0);
-      const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + ((size_t)(kt * RT + qq) * 4) * 64 + lane;
+      const int k = nq == 1 ? it : it / nq, qq = q0 + it - k * nq;
+      const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + ((size_t)((l0 + k) * RT + (qq >> 1)) * 4 + par) * 64 + 32 * h +
+                          (qq & 1) * 16 + n16;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) ab[i][t] = ap[t * 64];
+      for (int s = 0; s < 2; ++s) ab[i][s] = ap[s * 128];
     }
   };
   static_for<4>([&](auto ic) __attribute__((always_inline)) { load_a(decltype(ic)::value, ic); });
@@ -605,34 +608,30 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
     });
   }
   if (lora_here) {
-    f32x16_t tacc[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) tacc[u][r] = 0.f;
-    const uint16_t* lb = xs + min(lrow, M - 1) * XS + lh * 8;
+    f32x4_t tacc[3] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    const uint16_t* lb = xs + min(n16, M - 1) * XS + l0 * 64 + par * 16 + h * 8;
     for (int it0 = 0; it0 < items; it0 += 4) {
       static_for<4>([&](auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
         if (it0 + i < items) {
-          const int kt = l0 + (nq == 2 ? (it0 + i) >> 1 : it0 + i);
-          const bool second = nq == 2 && (i & 1);
+          const int k = nq == 1 ? it0 + i : (it0 + i) / nq, u = it0 + i - k * nq;
 #pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const bf16x8_t xa = *reinterpret_cast<const bf16x8_t*>(lb + kt * 64 + t * 16), bb = __builtin_bit_cast(bf16x8_t, ab[i][t]);
-            if (second) tacc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, bb, tacc[1], 0, 0, 0);
-            else tacc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, bb, tacc[0], 0, 0, 0);
+          for (int s = 0; s < 2; ++s) {
+            const bf16x8_t xa = *reinterpret_cast<const bf16x8_t*>(lb + k * 64 + s * 32), bb = __builtin_bit_cast(bf16x8_t, ab[i][s]);
+            if (u == 0) tacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, bb, tacc[0], 0, 0, 0);
+            else if (u == 1) tacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, bb, tacc[1], 0, 0, 0);
+            else tacc[2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, bb, tacc[2], 0, 0, 0);
           }
           load_a(it0 + i + 4, ic);
         }
       });
     }
-    if (lh == 0) {
+    if (q == 0) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < 3; ++u)
         if (u < nq) {
 #pragma unroll
-          for (int r = 0; r < kSbMaxRows; ++r) red_t[(wave * kSbMaxRows + r) * 64 + (q0 + u) * 32 + lrow] = tacc[u][r];
+          for (int r = 0; r < kSbMaxRows; ++r) red_t[(wave * kSbMaxRows + r) * 64 + (q0 + u) * 16 + n16] = tacc[u][r];
         }
     }
   }
@@ -648,7 +647,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
     if (m < M) {
       if (a.t_parts) {
         t = sb_parts_total(parts, red_t, m, cc);
-      } else if (lora_here && (cc >> 5) >= q0 && (cc >> 5) <= q1) {
+      } else if (lora_here && (cc >> 4) >= q0 && (cc >> 4) < q0 + nq) {
 #pragma unroll
         for (int w = 0; w < kSbWaves; ++w) t += red_t[(w * kSbMaxRows + m) * 64 + cc];
       }
