@@ -938,3 +938,19 @@ def test_scoring_in_one_walk_equals_prompt_and_completion_walks(family, b, p, t)
     got.append(s.per_token_logps(prompt, comp, pad_id=0))
   assert walks == [(256, p + t - 1), (-1, p - 1), (-1, t)]
   assert np.isfinite(got[0]).all() and np.abs(got[0] - got[1]).max() <= (2 if family == 'moe' else 1) * LOGPROB_TOL
+
+
+@pytest.mark.parametrize('rank', [4, 12, 16, 20, 21])
+@pytest.mark.parametrize('n_seq', [1, 4])
+def test_adapters_of_any_rank_in_steps_of_one_to_four_rows(rank, n_seq):
+  """q, k and v take the adapter's columns of their segment, in tiles of 16 that two segments may share: the log-probs of a
+  rollout are those of the scoring pass, whose projections of more than 128 rows know no such tiles."""
+  cfg = C.TOY
+  model = C.product_model(cfg, C.make_state(cfg, 5, rank, norm_jitter=0.05), 64, 8.0 * rank)
+  s = _sampler(model, cfg, 96)
+  rng = np.random.default_rng(rank)
+  prompts = [rng.integers(3, cfg.vocab_size, 40).astype(np.int32) for _ in range(n_seq)]
+  out = s(prompt_token_ids=prompts, max_generation_steps=6, temperature=0.0, eos_tokens=[-1], return_logprobs=True)
+  many = 8 // n_seq
+  scored = s.per_token_logps(np.tile(np.stack(prompts), (many, 1)), np.tile(np.stack(out.tokens), (many, 1)), pad_id=0)
+  assert np.abs(scored[:n_seq] - np.array(out.logprobs)).max() <= LOGPROB_TOL
