@@ -549,6 +549,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       }
       if (prof) TMX_TRY(TMX_K_EMPTY, empty_launch(st));
     }
+    bool advanced = false;  // by the last launch of the head
     if (sample) {
       HeadArgs a = {};
       a.x = w.xn;
@@ -570,6 +571,11 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       a.eos = s->eos_ids; a.n_eos = s->n_eos;
       a.buf_len = L;
       a.tpp = T;
+      if (w.dsync && !nucleus && !prof) {  // one word of the hand-over header, which starts a call at zero
+        a.advance = s->step;
+        a.arrived = (uint32_t*)w.dsync + 63;
+        advanced = true;
+      }
       if (nucleus) {
         TMX_TRY(TMX_K_HEAD, head_sample_nucleus(st, a, s->top_p, s->top_k, s->nucleus_workspace,
                                                 s->nucleus_workspace_bytes));
@@ -579,7 +585,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
         TMX_TRY(TMX_K_HEAD, head_sample(st, a));
       }
     }
-    TMX_TRY(TMX_K_ADVANCE, advance_step(st, s->step, T));
+    if (!advanced) TMX_TRY(TMX_K_ADVANCE, advance_step(st, s->step, T));
   }
 #undef TMX_TRY
   return TMX_OK;

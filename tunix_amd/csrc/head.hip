@@ -377,6 +377,18 @@ int head_tiles_pack(hipStream_t st, const uint16_t* w, uint16_t* tiles, int V, i
   return check_launch();
 }
 
+// The last workgroup of a launch to come here moves the step on (a launch of its own costs 1 to 4.6 us): all the others have
+// read it.  One thread per workgroup; the counter is left at zero.
+__device__ __forceinline__ void finalize_advance(const HeadArgs& a, int step) {
+  if (!a.advance) return;
+  if (gridDim.x > 1) {
+    __builtin_amdgcn_s_waitcnt(0);
+    if (__hip_atomic_fetch_add(a.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
+    __hip_atomic_store(a.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  *a.advance = step + (a.tpp > 0 ? a.tpp : 1);
+}
+
 // One workgroup per sequence: merge the vocabulary-tile partials, emit the token
 // and its log-probability into column step + 1, update `done`.
 __global__ __launch_bounds__(256) void head_finalize_kernel(HeadArgs a) {
@@ -416,12 +428,14 @@ __global__ __launch_bounds__(256) void head_finalize_kernel(HeadArgs a) {
       const int tpp = a.tpp > 0 ? a.tpp : 1;
       const int prow = a.row_base + row;
       // selective_log_softmax: logit - logsumexp, with logsumexp = max + log(sum exp(z - max))
-      const int scol = *a.step + prow % tpp + 1;
+      const int step = *a.step, scol = step + prow % tpp + 1;
       if (a.logprobs && scol < a.buf_len)
         a.logprobs[(size_t)(prow / tpp) * a.buf_len + scol] = best.z - (mx + logf(se));
+      finalize_advance(a, step);
       return;
     }
-    const int col = *a.step + 1;
+    const int step = *a.step, col = step + 1;
+    finalize_advance(a, step);
     if (col >= a.buf_len) return;  // a caller that steps past the buffer gets no write instead of a stray one
     const int tok = best.idx;
     a.token_buffer[(size_t)row * a.buf_len + col] = tok;
