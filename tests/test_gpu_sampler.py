@@ -954,3 +954,25 @@ def test_adapters_of_any_rank_in_steps_of_one_to_four_rows(rank, n_seq):
   many = 8 // n_seq
   scored = s.per_token_logps(np.tile(np.stack(prompts), (many, 1)), np.tile(np.stack(out.tokens), (many, 1)), pad_id=0)
   assert np.abs(scored[:n_seq] - np.array(out.logprobs)).max() <= LOGPROB_TOL
+
+
+@pytest.mark.parametrize('b,p,t', [(257, 2, 1), (29, 1, 10), (300, 3, 2)])
+def test_head_of_more_than_256_rows_equals_heads_of_fewer(b, p, t):
+  """Row counts that fill no block of 32: the last rows of the copy in fragment order.  Scored whole and in parts of at most 128
+  rows, greedy and sampled rollouts of as many sequences too."""
+  cfg = C.TOY
+  model = C.product_model(cfg, C.make_state(cfg, 11, 8, norm_jitter=0.05), 64, 16.0)
+  s = _sampler(model, cfg, 32)
+  rng = np.random.default_rng(b)
+  prompt = rng.integers(3, cfg.vocab_size, (b, p)).astype(np.int32)
+  part = 128 // t
+
+  def in_parts(comp):
+    return np.concatenate([s.per_token_logps(prompt[i:i + part], comp[i:i + part], pad_id=0) for i in range(0, b, part)])
+
+  comp = rng.integers(3, cfg.vocab_size, (b, t)).astype(np.int32)
+  assert np.abs(s.per_token_logps(prompt, comp, pad_id=0) - in_parts(comp)).max() <= LOGPROB_TOL
+  for temperature in (0.0, 1.0):
+    out = s(prompt_token_ids=list(prompt), max_generation_steps=t, temperature=temperature, eos_tokens=[-1],
+            return_logprobs=True, seed=3)
+    assert np.abs(np.array(out.logprobs) - in_parts(np.stack(out.tokens))).max() <= LOGPROB_TOL

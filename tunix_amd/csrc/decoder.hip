@@ -571,6 +571,11 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       a.eos = s->eos_ids; a.n_eos = s->n_eos;
       a.buf_len = L;
       a.tpp = T;
+      {  // the many-rows head reorders its rows into a buffer that is free by now
+        const size_t room = (size_t)(B + 31) / 32 * 32 * D;
+        if ((size_t)B * 2 * F >= room) a.x_tiles = w.y16;
+        else if (moe && (size_t)B * m->experts_per_tok * D >= room) a.x_tiles = w.pair_y;
+      }
       if (w.dsync && !nucleus && !prof) {  // one word of the hand-over header, which starts a call at zero
         a.advance = s->step;
         a.arrived = (uint32_t*)w.dsync + 63;

@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256, MT == 4 ? 1 : 2) void head_kernel(HeadArgs a) 
 // Two workgroups share a CU, so that one's epilogue (20 threefry rounds a value when sampling) runs under the other's
 // loads.  On the 1.05 GB head, greedy / sampling (trace): 96 rows 196 / 221 us, 128 rows 214 / 245, bound by the stream (64
 // rows: 182 / 187); 160 rows 277 / 321, 256 rows 309 / 383, bound by LDS (a fragment read per MFMA) and, sampling, by the
-// epilogue's VALU work.  The 256 x 256 blocks of head_wide_kernel take 280 / 372, 301 / 402 (160 rows) and 334 / 429 (256).
+// epilogue's VALU work.  The 256 x 256 blocks of head_wide_kernel take 266 / 369, 277 / 387 (160 rows) and 287 / 414 (256).
 // For 256 rows also measured, where this form took 327 / 396: two waves of 64 vocabulary rows on each 128 rows (half the
 // LDS reads, every weight read twice) 351 / 418; one workgroup of 8 waves per CU 316 / 412.
 template <int MT, int NW, int P>
@@ -449,24 +449,40 @@ __global__ __launch_bounds__(256) void head_finalize_kernel(HeadArgs a) {
 // ---------------------------------------------------------------------------
 // Many rows (scoring passes over whole sequences, decode steps of more than 128 sequences): the same
 // product as a matrix-pipe-bound kernel.  A workgroup multiplies 256 vocabulary rows by 256 sequence rows:
-// the vocabulary rows are the A operand and come through a double-buffered LDS slab filled by
-// direct-to-LDS loads (256-byte rows of a 128-wide k-step, chunks XOR-swizzled by row % 16);
+// the vocabulary rows are the A operand and come through four LDS slabs filled by
+// direct-to-LDS loads (128-byte rows of 64 k, 16-byte chunk c of row r at slot c ^ (r / 2 % 8));
 // wave w owns sequence rows 32 w .. 32 w + 31 as the B operand, read straight from global
-// memory, 64 contiguous bytes per lane and k-tile (lane (row, h) holds k = 32 h .. 32 h + 31 of
-// the tile, MFMA step t pairs k = 32 h + 8 t .. with the same k of the vocabulary rows).  A lane's
+// memory (lane (row, h) holds k = 32 h .. 32 h + 31 of a k-tile of 64, MFMA step t pairs k = 32 h + 8 t ..
+// with the same k of the vocabulary rows), from a copy of the rows in fragment order where there is room for one.  A lane's
 // 128 accumulator registers are 128 vocabulary rows of ONE sequence row, so max / sum-exp / the
 // target's z run down the registers.  LDS reads of fragment group g + 1 and the refill of the
-// B registers are pinned between the MFMAs of group g.  Consecutive workgroups take the
+// B registers are pinned between the MFMAs of group g.  The matrix comes from HBM, so its slabs are short (64 k) and
+// requested three ahead; the barrier that hands one over stands inside the last group of the one before, whose fragments
+// are in registers, and the wave that is behind goes first (see wide_core in qwide.hip).  Consecutive workgroups take the
 // sequence-row blocks of one vocabulary block, so the head matrix leaves HBM once.
+// Bound by the matrix pipe and, a tenth of the time, by the epilogue, which nothing runs beside.  Scoring, 4096 rows of the
+// 1.05 GB head: 4.67 ms with the rows read in place and two slabs of 128 k, 3.86 ms + 0.01 for the copy (1.11 PF/s); 630 rows
+// of the 0.53 GB head 592 -> 501 us.  The four slabs without the copy took 5.0 ms (the address unit, see below), without
+// wave priorities 5.2.  Taking the maximum of the accumulators first, then one exponential a value: 3.88 ms, nothing gained.
 struct HW {
-  static constexpr int MT = 8, ROWS = 256, TS = 2, XS = 128;
-  static constexpr size_t LDS = (size_t)2 * ROWS * XS * 2;  // 128 KiB
+  static constexpr int MT = 8, ROWS = 256, XS = 64, NB = 4;
+  static constexpr size_t LDS = (size_t)NB * ROWS * XS * 2;  // 128 KiB
 };
+
+// The rows of x in the order the wide kernel's B fragments take them: 32 rows x 16 k are 1 KiB, lane (row, h) of fragment
+// 4 j + t of a step holds k = 64 j + 32 h + 8 t .. + 7.  Read from the rows themselves neighbouring lanes are in different
+// rows, and the CU's address unit takes one of them at a time: 64 clocks a fragment, as much as the products of a step.
+__global__ __launch_bounds__(512) void head_x_tiles_kernel(const uint16_t* x, uint16_t* tiles, int M, int D) {
+  const int row = threadIdx.x >> 4, c = threadIdx.x & 15;  // 16 bytes of a row: k = 8 c of step blockIdx.x
+  const u32x4_t v = *reinterpret_cast<const u32x4_t*>(x + (size_t)min((int)blockIdx.y * 32 + row, M - 1) * D + blockIdx.x * 128 + c * 8);
+  const int g = (c >> 3) * 4 + (c & 3), h = (c >> 2) & 1;
+  reinterpret_cast<u32x4_t*>(tiles)[((size_t)blockIdx.y * (D >> 4) + blockIdx.x * 8 + g) * 64 + 32 * h + row] = v;
+}
 
 template <int MODE>  // TMX_SAMPLE_*: the epilogue is compiled per mode
 __global__ __launch_bounds__(512, 1) void head_wide_kernel(HeadArgs a, int tok_blocks, int voc_blocks) {
   extern __shared__ __align__(16) uint16_t smem[];
-  constexpr int MT = HW::MT, TS = HW::TS, XS = HW::XS, ROWS = HW::ROWS;
+  constexpr int MT = HW::MT, XS = HW::XS, ROWS = HW::ROWS, NB = HW::NB;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, nl = lane & 31;
@@ -476,82 +492,92 @@ __global__ __launch_bounds__(512, 1) void head_wide_kernel(HeadArgs a, int tok_b
   const int vrows = a.V - v0 < ROWS ? a.V - v0 : ROWS;
   const int tok = tb * 256 + wave * 32 + nl;       // sequence row of this lane's accumulator column
   const int tok_l = tok < a.M ? tok : a.M - 1;
-  const int nsteps = a.D >> 7, last_step = nsteps - 1;
+  const int nsteps = a.D >> 7, last_step = nsteps - 1;  // steps of two slabs
 
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.w + (size_t)v0 * a.D, (uint32_t)vrows * a.D * 2u);
-  const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x, (uint32_t)a.M * a.D * 2u);
-  constexpr int XR = ROWS / 32;
-  int woff[XR];  // slab transfer: load i moves vocabulary rows 4 wave + 32 i .. + 3, 16 lanes each
+  const __amdgpu_buffer_rsrc_t rx = a.x_tiles ? make_rsrc(a.x_tiles, (uint32_t)(a.M + 31) / 32 * 32 * a.D * 2u) : make_rsrc(a.x, (uint32_t)a.M * a.D * 2u);
+  constexpr int XR = ROWS / 64;
+  int woff[XR];  // slab transfer: load i moves vocabulary rows 8 wave + 64 i .. + 7, 8 lanes each
 #pragma unroll
   for (int i = 0; i < XR; ++i) {
-    const int row_l = 4 * wave + 32 * i + (lane >> 4);
-    woff[i] = (row_l < vrows ? row_l : vrows - 1) * a.D * 2 + (((lane & 15) ^ (row_l & 15)) * 16);
+    const int row_l = 8 * wave + 64 * i + (lane >> 3);
+    woff[i] = (row_l < vrows ? row_l : vrows - 1) * a.D * 2 + (((lane & 7) ^ ((row_l >> 1) & 7)) * 16);
   }
-  const int xv = tok_l * a.D * 2 + h * 64;
+  // B fragments: from the rows themselves, or 1 KiB each from their tile copy (head_x_tiles_kernel)
+  const bool tiled = a.x_tiles != nullptr;
+  const int xv = tiled ? (tb * 8 + wave) * (a.D >> 4) * 1024 + lane * 16 : tok_l * a.D * 2 + h * 64;
+  const int xt = tiled ? 1024 : 16, xj = tiled ? 4096 : 128;  // bytes between fragments and between k-tiles of 64
 
   f32x16_t acc[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
-  u32x4_t breg[4 * TS];  // B fragments of the 8 groups of a step, refilled for the next step after use
+  constexpr int G = 8;  // fragment groups of a step, 16 k each
+  u32x4_t breg[G];      // B fragments of a step, refilled for the next one after use
 
   auto load_b = [&](int step, auto gc) __attribute__((always_inline)) {
     constexpr int g = decltype(gc)::value;
     step = step < last_step ? step : last_step;
-    breg[g] = __builtin_amdgcn_raw_buffer_load_b128(rx, xv + (g & 3) * 16, (step * TS + (g >> 2)) * 128, 0);
+    breg[g] = __builtin_amdgcn_raw_buffer_load_b128(rx, xv, (step * 2 + (g >> 2)) * xj + (g & 3) * xt, 0);
   };
-  auto dma_w = [&](int step, int buf) __attribute__((always_inline)) {
-    step = step < last_step ? step : last_step;
-    uint16_t* base = smem + (size_t)buf * ROWS * XS + wave * 4 * XS;
-#pragma unroll
-    for (int i = 0; i < XR; ++i) load_row_to_lds_nt(rw, base + i * 32 * XS, woff[i], step * (TS * 128));
+  auto dma_w = [&](int slab, int i) __attribute__((always_inline)) {
+    uint16_t* base = smem + (size_t)(slab & (NB - 1)) * ROWS * XS + wave * 8 * XS;
+    load_row_to_lds_nt(rw, base + i * 64 * XS, woff[i], min(slab, 2 * nsteps - 1) * 128);
   };
-  constexpr int kYounger = 4 * TS;
-  auto wait_slab = [&]() __attribute__((always_inline)) {
+  // all but the youngest loads of this wave have arrived and its LDS reads are done; then all waves
+  auto meet = [&](auto younger) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (kYounger & 15) | ((kYounger >> 4) << 14));
-    __syncthreads();
-  };
-  auto step_math = [&](int step, int buf) __attribute__((always_inline)) {
-    const uint16_t* wb = smem + (size_t)buf * ROWS * XS + nl * XS;
-    bf16x8_t wq[2][MT];
-    {
-      // group g = 4 j + t needs k = 64 j + 32 h + 8 t ..: chunk 8 j + 4 h + t of the slab row
-      const int slot = ((4 * h) ^ (nl & 15)) * 8;
-#pragma unroll
-      for (int m = 0; m < MT; ++m) wq[0][m] = *reinterpret_cast<const bf16x8_t*>(wb + m * 32 * XS + slot);
-    }
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(decltype(younger)::value) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    static_for<4 * TS>([&](auto gc) __attribute__((always_inline)) {
+  };
+  constexpr int MEET = 2;  // the MFMA of a slab's last group in front of which the waves meet
+  // younger than a slab when the next one is handed over: the B fragments behind its transfer (4), a slab and its B
+  // fragments (XR + 4), and of the current one the transfer and three B fragments
+  constexpr int kYounger = 4 + XR + 4 + XR + 3;
+  bf16x8_t wq[2][MT];
+  const uint16_t* wlane = smem + nl * XS;
+  // group g = 4 j + t needs k = 64 j + 32 h + 8 t ..: chunk 4 h + t of slab j's row, at that slot ^ (row / 2 % 8)
+  auto slot_of = [&](int g) __attribute__((always_inline)) { return ((4 * h + (g & 3)) ^ ((nl >> 1) & 7)) * 8; };
+  auto step_math = [&](int step) __attribute__((always_inline)) {
+    static_for<G>([&](auto gc) __attribute__((always_inline)) {
       constexpr int g = decltype(gc)::value, cur = g & 1, nxt = cur ^ 1;
-      constexpr bool more = g + 1 < 4 * TS;
-      constexpr int gn = g + 1;
-      const int slot = ((8 * (gn >> 2) + 4 * h + (gn & 3)) ^ (nl & 15)) * 8;
+      constexpr bool last = g % 4 == 3;
+      const int slab = 2 * step + g / 4;
+      const uint16_t* wb = wlane + (size_t)((last ? slab + 1 : slab) & (NB - 1)) * ROWS * XS + slot_of(g + 1);
       const bf16x8_t b = __builtin_bit_cast(bf16x8_t, breg[g]);
+      __builtin_amdgcn_s_setprio(3 - g % 4);
       static_for<MT>([&](auto mc) __attribute__((always_inline)) {
         constexpr int m = decltype(mc)::value;
+        if constexpr (last && m == MEET) meet(IC<kYounger>{});
         acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wq[cur][m], b, acc[m], 0, 0, 0);
-        if constexpr (more) {
-          wq[nxt][m] = *reinterpret_cast<const bf16x8_t*>(wb + m * 32 * XS + slot);
-          __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!last) {
+          wq[nxt][m] = *reinterpret_cast<const bf16x8_t*>(wb + m * 32 * XS);
+        } else if constexpr (m >= MEET) {  // two at a time until the two left out in front of the barrier are caught up
+          constexpr int n = m - MEET, t0 = n < 2 ? 2 * n : n + 2, t1 = n < 1 ? 2 : n + 3;
+          static_for<t1 - t0>([&](auto nc) __attribute__((always_inline)) {
+            constexpr int r = t0 + decltype(nc)::value;
+            wq[nxt][r] = *reinterpret_cast<const bf16x8_t*>(wb + r * 32 * XS);
+          });
         }
+        if constexpr (g % 4 == 0 && m % 2 == 0 && m / 2 < XR) dma_w(slab + NB - 1, m / 2);
+        __builtin_amdgcn_sched_barrier(0);
       });
       load_b(step + 1, gc);  // fragment consumed: refill it for the next step
       __builtin_amdgcn_sched_barrier(0);
     });
   };
 
-  dma_w(0, 0);
-  static_for<4 * TS>([&](auto gc) __attribute__((always_inline)) { load_b(0, gc); });
-  wait_slab();
-  for (int step = 0; step < nsteps; ++step) {
-    const int buf = step & 1;
-    dma_w(step + 1, buf ^ 1);
-    __builtin_amdgcn_sched_barrier(0);
-    step_math(step, buf);
-    wait_slab();
-  }
+#pragma unroll
+  for (int i = 0; i < (NB - 1) * XR; ++i) dma_w(i / XR, i % XR);
+  static_for<G>([&](auto gc) __attribute__((always_inline)) { load_b(0, gc); });
+  meet(IC<(NB - 2) * XR + G>{});
+#pragma unroll
+  for (int m = 0; m < MT; ++m) wq[0][m] = *reinterpret_cast<const bf16x8_t*>(wlane + slot_of(0) + m * 32 * XS);
+  for (int step = 0; step < nsteps; ++step) step_math(step);
+  __builtin_amdgcn_s_setprio(0);
 
   // per sequence row: running max and sum of exp over this block's vocabulary rows and the best
   // candidate by key, as in head_kernel: greedy key = logit; sampling key = z + Gumbel noise of the
@@ -634,8 +660,9 @@ static int launch_head_wide(hipStream_t st, const HeadArgs& a, int tok_blocks, i
 }
 
 // With a tile copy, up to 256 rows are faster from it (head_logits): both read the matrix once, and on the 1.05 GB head the
-// 256 x 256 blocks take 280 us at 96 rows and 334 at 256, greedy, where the stream takes 196 and 309 (sampling 372 and 429
-// against 221 and 383).  More rows would be several passes over the tile copy.
+// 256 x 256 blocks take 266 us at 96 rows and 287 at 256, greedy, where the stream takes 196 and 309 (sampling 369 and 414
+// against 221 and 383; at 160 rows 277 each and 387 against 321): one line for all, although greedy alone it would lie at
+// 160.  More rows would be several passes over the tile copy.
 bool head_wide_ok(const HeadArgs& a) {
   return (a.M > 256 || (a.M > 64 && !a.w_tiles)) && a.D % 128 == 0 && a.M > 0 && (size_t)a.M * a.D * 2 < (1u << 31) && (size_t)256 * a.D * 2 < (1u << 31) &&
          a.n_forbidden == 0 && !a.logits_out;
@@ -645,6 +672,11 @@ bool head_wide_ok(const HeadArgs& a) {
 int head_wide_logits(hipStream_t st, HeadArgs& a) {
   if (!head_wide_ok(a)) return TMX_ERR_SHAPE;
   const int tok_blocks = (a.M + 255) / 256, voc_blocks = (a.V + HW::ROWS - 1) / HW::ROWS;
+  if (a.x_tiles) {
+    hipLaunchKernelGGL(head_x_tiles_kernel, dim3(a.D / 128, (a.M + 31) / 32), dim3(512), 0, st, a.x, a.x_tiles, a.M, a.D);
+    const int rc = check_launch();
+    if (rc != TMX_OK) return rc;
+  }
   a.nwg = voc_blocks;
   a.row_base = 0;
   int lrc;

@@ -180,6 +180,7 @@ struct AttnArgs {
 
 struct HeadArgs {
   const uint16_t* x;  // [M, D] final-normed hidden states
+  uint16_t* x_tiles;  // room for x again, rows rounded up to 32, in the wide kernel's order (null: it reads x itself)
   const uint16_t* w;  // [V, D]
   const uint16_t* w_tiles;  // the same matrix in the tile layout of head_tiles_kernel, or null
   int M, D, V;
