@@ -96,8 +96,8 @@ __device__ __forceinline__ int acc_row(int r, int lane) {
 }
 
 // Expand one 32-bit word (8 nibbles, element j = 2 (i % 4) + i / 4 for nibble i) into the 8 bf16 B-operand values of
-// one MFMA step: bf16((u - 8) * s), (4 + 8 significant bits) exact as a float and rounded once.  This form, for a checker
-// that takes every scale, widens a nibble per v_cvt_f32_ubyteN: 23 instructions per word.
+// one MFMA step: bf16((u - 8) * s), (4 + 8 significant bits) exact as a float and rounded once.  This form, for
+// int4_dequant_kernel, takes every scale and widens a nibble per v_cvt_f32_ubyteN: 23 instructions per word.
 __device__ __forceinline__ bf16x8_t dequant_word_any_scale(uint32_t d, float s, float m8s) {
   const uint32_t lo = d & 0x0F0F0F0Fu;         // nibbles 0,2,4,6 in bytes 0..3
   const uint32_t hi = (d >> 4) & 0x0F0F0F0Fu;  // nibbles 1,3,5,7 in bytes 0..3
