@@ -332,7 +332,8 @@ int tmx_moe_route(void* stream, const void* x, const void* router_w, int B, int 
  *   down == 0: x = hidden states [P / top_k, K = D] (row p / top_k), N = 2 F with columns
  *              gate | up; out[p, 0:F] = bf16(silu(gate) * up) (F % 64 == 0)
  *   down != 0: x = activations [P, K = F] (row p); out[p, 0:N] = bf16(x . W_e) (N % 128 == 0)
- * K % 256 == 0, P <= TMX_MAX_MOE_PAIRS. */
+ * K % 256 == 0, K * N < 2^33, P <= TMX_MAX_MOE_PAIRS (any: the last token may have fewer than top_k pairs); ldx % 8 == 0,
+ * rows of out at any element. */
 int tmx_moe_experts(void* stream, const void* x, int ldx, const void* qweight, const void* scales,
                     const int32_t* expert_of, int P, int top_k, int E, int K, int N, int G, int down,
                     void* out, int ldo);

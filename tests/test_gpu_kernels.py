@@ -1117,6 +1117,40 @@ def test_moe_experts_row_counts(down, K, N):
   assert ((got - want).abs() > 2.0 ** -6 * want.abs() + 2.0 ** -8).sum() == 0
 
 
+# A call of more than 1024 pairs is one launch of the many-rows kernel, a call of fewer the stream kernel: same bits, whatever the
+# distance of the rows (0: one row for all; 2^21 bytes apart: beyond 32-bit offsets), where rows of out begin, and also when the
+# last token has fewer pairs than top_k.
+@pytest.mark.parametrize('down', [0, 1])
+@pytest.mark.parametrize('P,k,ldx,ldo_pad,out0', [
+    (1032, 4, None, 0, 0), (1031, 4, None, 0, 0), (2049, 2, 264, 3, 1), (1030, 4, 0, 1, 3), (1025, 1, 1 << 20, 2, 2), (1026, 1, 1 << 20, 0, 0)])
+def test_moe_experts_one_call_equals_calls_of_fewer_pairs(down, P, k, ldx, ldo_pad, out0):
+  K, N, E, group = 256, 256, 5, 64
+  g = torch.Generator(device=G.DEV).manual_seed(P + down)
+  pl = quant.PackedLinear.from_dense([(torch.randn(K, E * N, generator=g, device=G.DEV) * 0.05).to(torch.bfloat16)], group, G.DEV)
+  idx = torch.randint(0, E, (P,), generator=g, device=G.DEV, dtype=torch.int32)
+  rows, cols = P if down else -(-P // k), N if down else N // 2
+  ldx = K if ldx is None else ldx
+  buf = torch.empty((rows - 1) * ldx + K, dtype=torch.bfloat16, device=G.DEV)
+  x = buf.as_strided((rows if ldx else 1, K), (ldx or K, 1))
+  x.copy_(torch.randn(x.shape, generator=g, device=G.DEV))
+  ldo = cols + ldo_pad
+
+  def run(runs):
+    out = torch.full((out0 + P * ldo,), 7.0, dtype=torch.bfloat16, device=G.DEV)
+    for p0, n in runs:
+      xp = buf.data_ptr() + 2 * ldx * (p0 if down else p0 // k)
+      G.call('tmx_moe_experts', S(), xp, ldx, G.p(pl.qweight), G.p(pl.scales), idx.data_ptr() + 4 * p0, n, k, E, K, N, group, down,
+             out.data_ptr() + 2 * (out0 + p0 * ldo), ldo)
+    return out
+
+  got, want = run([(0, P)]), run([(p0, min(1000, P - p0)) for p0 in range(0, P, 1000)])
+  G.sync()
+  assert torch.equal(got, want)
+  body = got[out0:].reshape(P, ldo)
+  assert (got[:out0] == 7.0).all() and (body[:, cols:] == 7.0).all() and (body[:, :cols].abs() != 7.0).all()
+  assert (body[:, :cols] != 0).float().mean(1).min() > 0.9
+
+
 # row tiles x column tiles of the many-rows kernel that these shapes take on 256 compute units (wide_plan), ragged in
 # rows and columns; the reference is the f32 product of the dequantised matrix
 @pytest.mark.parametrize('M,K,N', [

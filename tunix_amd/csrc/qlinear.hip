@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(MoeArgs m) {
     // A fragments: lane (row nl, h) reads x[src][64 kt + 16 t + 8 h ..]; absent rows stay zero
     const bool live = nl < rows;
     const int pr = live ? rows_s[c0 + nl] : 0;
-    const uint16_t* xrow = m.x + (size_t)(DOWN ? pr : pr / m.top_k) * m.ldx + 8 * h;
+    const uint16_t* xrow = m.x + (size_t)(DOWN ? pr : (m.pair0 + pr) / m.top_k) * m.ldx + 8 * h;
     u32x4_t wring[kMoeRing][TPU];
     uint16_t sring[kMoeRing][TPU];
     // tile (unit ui of this wave, k-tile kt) into ring slot sl; past the last unit: its last tile again
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(MoeArgs m) {
 #pragma unroll
       for (int c = 0; c < TPU; ++c) {
         const int nb = u0 + ui * ustride + c * units;  // the gate tile, or the up tile F / 32 further on
-        wring[sl][c] = __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, (nb * KT + kt) * 1024, kNtLoad);
+        wring[sl][c] = __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, (int)((uint32_t)(nb * KT + kt) * 1024u), kNtLoad);
         sring[sl][c] = __builtin_amdgcn_raw_buffer_load_b16(rs, nl * 2, (nb * KG + (kt >> gs)) * 64, 0);
       }
     };
@@ -476,8 +476,23 @@ int moe_experts(hipStream_t st, const MoeArgs& a, int E, bool down) {
   if (!a.x || !a.qw || !a.scales || !a.expert_of || !a.out) return TMX_ERR_ARG;
   if (a.P <= 0 || a.P > TMX_MAX_MOE_PAIRS || a.top_k <= 0 || E <= 0) return TMX_ERR_SHAPE;
   if (a.K % 256 || a.G % 64 || (a.G & (a.G - 1)) || a.K % a.G || a.ldx % 8) return TMX_ERR_SHAPE;
-  if (a.N % 128) return TMX_ERR_SHAPE;  // gate | up: F % 64 == 0
-  if (a.P > kMoeStreamPairs) return moe_rows(st, a, E, down);  // many rows per expert (qwide.hip)
+  if (a.N <= 0 || a.N % 128) return TMX_ERR_SHAPE;  // gate | up: F % 64 == 0
+  if ((size_t)a.K * a.N >= (1ull << 33)) return TMX_ERR_SHAPE;  // 32-bit offsets within an expert's matrix
+  if (a.P > kMoeStreamPairs) {
+    if (moe_x_bytes(a, down) <= kMoeRowsXBytes) return moe_rows(st, a, E, down);  // many rows per expert (qwide.hip)
+    // rows further apart than 32-bit offsets reach: runs of the stream kernel, which addresses them by pointers
+    for (int p0 = 0; p0 < a.P; p0 += kMoeStreamPairs) {
+      MoeArgs r = a;
+      r.expert_of = a.expert_of + p0;
+      r.P = a.P - p0 < kMoeStreamPairs ? a.P - p0 : kMoeStreamPairs;
+      r.out = a.out + (size_t)p0 * a.ldo;
+      if (down) r.x = a.x + (size_t)p0 * a.ldx;
+      else r.pair0 = p0;
+      const int rc = moe_experts(st, r, E, down);
+      if (rc != TMX_OK) return rc;
+    }
+    return TMX_OK;
+  }
   // decode: few rows per expert, a pure weight stream
   // column groups per expert: one gate | up pair (2 x K / 64 weight tiles) or two down tiles per wave
   // (measured on the 30B-A3B shapes: 6 groups for gate | up, 8 for down; fewer leave CUs short of

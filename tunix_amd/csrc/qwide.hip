@@ -25,6 +25,9 @@ namespace tmx {
 constexpr int kWideTS = 2, kWideXS = 128;
 constexpr int kWideTiles32 = TMX_MAX_FILL_ROWS / 32;  // words per kind in a hand-over area: arrivals | ready flags
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+// four bf16 of an output row in one store: rows may begin at any element (a caller's stride or view), and 8-byte stores take
+// every address
+__device__ __forceinline__ void store8(uint16_t* p, u32x2_t v) { __builtin_memcpy(p, &v, 8); }
 constexpr int wide_bufs(int mt) { return mt == 2 ? 4 : 2; }
 constexpr size_t wide_lds(int mt) { return (size_t)wide_bufs(mt) * mt * 32 * kWideXS * 2; }
 
@@ -246,7 +249,7 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const f32x4_t v = acc[u][i];
-          if (a.y_bf16) *reinterpret_cast<u32x2_t*>(a.y_bf16 + (size_t)row * a.ldy + col0 + 16 * u) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+          if (a.y_bf16) store8(a.y_bf16 + (size_t)row * a.ldy + col0 + 16 * u, u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])});
           else *reinterpret_cast<f32x4_t*>(a.y_part + ((size_t)slice * a.M + row) * a.N + col0 + 16 * u) = v;
         }
       }
@@ -329,7 +332,7 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
           f32x4_t v;
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = rbf(acc[u][i][e]) + rbf(rbf(d[u][e]) * a.lora_ls);
-          *reinterpret_cast<u32x2_t*>(a.y_bf16 + (size_t)row * a.ldy + col0 + 16 * u) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+          store8(a.y_bf16 + (size_t)row * a.ldy + col0 + 16 * u, u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])});
         }
       }
     });
@@ -510,18 +513,20 @@ __device__ __forceinline__ void moe_chunk(const MoeArgs& m, int e, int bx, const
   const int q = lane >> 4, nl = lane & 15, h = lane >> 5, sub = q & 1;
   const int KT = m.K >> 6, KG = m.K / m.G, unit = bx * 8 + wave;
   const bool active = unit * 32 < m.N;
-  // the tile and the 16 columns of it that this lane has words of
-  const int nb = DOWN ? unit : (unit >> 1) + sub * (m.N >> 6), half = DOWN ? sub : unit & 1;
-  const int wv = (nb * KT * 64 + 32 * h + 16 * half + nl) * 16, sv = (nb * KG * 32 + 16 * half + nl) * 2;
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(m.qw + (size_t)e * m.qw_stride, (uint32_t)m.K * m.N / 2u);
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(m.scales + (size_t)e * m.sc_stride, (uint32_t)KG * m.N * 2u);
-  const __amdgpu_buffer_rsrc_t rx = make_rsrc(m.x, (uint32_t)(DOWN ? m.P : m.P / m.top_k) * m.ldx * 2u);
+  // the tile and the 16 columns of it that this lane has words of; descriptors begin at the wave's first tile, so 32-bit
+  // offsets reach an up tile of every matrix that moe_experts takes
+  const int nb = DOWN ? unit : unit >> 1, up = DOWN ? 0 : sub * (m.N >> 6), half = DOWN ? sub : unit & 1;
+  const int wv = (up * KT * 64 + 32 * h + 16 * half + nl) * 16, sv = (up * KG * 32 + 16 * half + nl) * 2;
+  const uint32_t tiles = active ? (DOWN ? 1u : (uint32_t)(m.N >> 6) + 1u) : 0u;
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(m.qw + (size_t)e * m.qw_stride + (active ? (size_t)nb * KT * 64 : 0), tiles * KT * 1024u);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(m.scales + (size_t)e * m.sc_stride + (active ? (size_t)nb * KG * 32 : 0), tiles * KG * 64u);
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(m.x, (uint32_t)moe_x_bytes(m, DOWN));
   const int row_l = 4 * wave + q;
   int xoff[MT];  // rows past the end: past the descriptor's end, zeros
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int r = row_l + 32 * i, p = rows_s[r < n ? r : 0];
-    xoff[i] = r < n ? (DOWN ? p : p / m.top_k) * m.ldx * 2 + ((nl ^ (row_l & 15)) * 16) : (int)0x7FFF0000;
+    xoff[i] = r < n ? (DOWN ? p : p / m.top_k) * m.ldx * 2 + ((nl ^ (row_l & 15)) * 16) : (int)kMoeRowsXBytes;
   }
   f32x4_t acc[2][2 * MT];
   wide_core<MT, 1, 2>(smem, rw, wv, rs, sv, __builtin_ctz(m.G >> 6), rx, [&](int i) { return xoff[i]; }, 0, m.K / (64 * kWideTS), 0,
@@ -535,7 +540,7 @@ __device__ __forceinline__ void moe_chunk(const MoeArgs& m, int e, int bx, const
     if constexpr (DOWN) {
 #pragma unroll
       for (int u = 0; u < 2; ++u)
-        *reinterpret_cast<u32x2_t*>(out + 16 * u) = u32x2_t{pack_bf2(acc[u][i][0], acc[u][i][1]), pack_bf2(acc[u][i][2], acc[u][i][3])};
+        store8(out + 16 * u, u32x2_t{pack_bf2(acc[u][i][0], acc[u][i][1]), pack_bf2(acc[u][i][2], acc[u][i][3])});
     } else {
       float v[4];
 #pragma unroll
@@ -543,7 +548,7 @@ __device__ __forceinline__ void moe_chunk(const MoeArgs& m, int e, int bx, const
         const float g = rbf(acc[0][i][k]), up = rbf(acc[1][i][k]);
         v[k] = rbf(g * rbf(1.f / (1.f + expf(-g)))) * up;
       }
-      *reinterpret_cast<u32x2_t*>(out) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+      store8(out, u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])});
     }
   }
 }

@@ -74,7 +74,13 @@ struct MoeArgs {
   int K, N, G;             // per-expert matrix [K, N] (gate|up: N = 2 F)
   uint16_t* out;           // gate|up: act [P, F]; down: y [P, D]
   int ldo;
+  int pair0;               // gate|up in runs of pairs: the first pair of the run (x is the whole batch's)
 };
+// Bytes of x from its first to its last element, and how many of them the many-rows kernel's offsets reach.
+__host__ __device__ inline size_t moe_x_bytes(const MoeArgs& a, bool down) {
+  return ((size_t)(down ? a.P - 1 : (a.P - 1) / a.top_k) * a.ldx + a.K) * 2;
+}
+constexpr size_t kMoeRowsXBytes = 0x7FFF0000;
 
 struct RouterArgs {
   const uint16_t* x;       // [B, D] normed hidden states
