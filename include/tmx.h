@@ -86,7 +86,7 @@ int tmx_int4_dequant(void* stream, const void* qweight, const void* scales, void
  *              columns >= r zero (NULL: no LoRA): element A[64 kb + 16 t + 8 h + j][32 ct + c]
  *              at ((((kb * (r_pad/32) + ct) * 4 + t) * 64 + 32 h + c) * 8 + j)
  *   lora_b   : bf16 [r, N]
- *   scales   : bf16 [N/32][K/G][32], below 2^104 in magnitude (larger ones overflow inside the product)
+ *   scales   : bf16 [N/32][K/G][32]
  *   residual : bf16 [M, N] or NULL; added after the LoRA delta, in bf16
  *   workspace: tmx_qlora_linear_workspace_bytes(M, K, N) bytes (f32 K-slice planes)
  * The launches of a call are ordered by the stream alone: no kernel of it waits for another one's data. */

@@ -43,6 +43,68 @@ def test_int4_dequant_bit_exact_exhaustive():
     np.testing.assert_array_equal(G.host(out), int4.dequantize(q, s, group))
 
 
+# Scales up to 2^124 (from 2^125 on -8 s is infinite), with activations that keep the sums finite: every projection kernel against the f32
+# product with the matrix that tmx_int4_dequant makes of the same words, bit for bit bf16((u - 8) * s).
+def _huge_scales(K, N, group, seed):
+  g = torch.Generator(device=G.DEV).manual_seed(seed)
+  q = torch.randint(-8, 8, (K, N), generator=g, device=G.DEV, dtype=torch.int8)
+  e = torch.randint(100, 124, (K // group, N), generator=g, device=G.DEV).double()
+  s = (torch.rand(K // group, N, generator=g, device=G.DEV, dtype=torch.double) + 1).to(torch.bfloat16)
+  s = s.double() * torch.exp2(e)
+  pl = quant.PackedLinear.from_quantized([q], [s.to(torch.bfloat16)], group, G.DEV)
+  dense = torch.empty(K, N, dtype=torch.bfloat16, device=G.DEV)
+  G.call('tmx_int4_dequant', S(), G.p(pl.qweight), G.p(pl.scales), G.p(dense), K, N, group)
+  exact = (q.double() * s.repeat_interleave(group, 0)).to(torch.bfloat16)
+  assert torch.equal(dense, exact) and dense.isfinite().all()
+  x = lambda rows, cols=K: (torch.randn(rows, cols, generator=g, device=G.DEV) * 2.0 ** -110).to(torch.bfloat16)
+  return pl, dense, x
+
+
+def _assert_rel(got, want, tol):
+  assert got.isfinite().all() and (got.double() - want).norm() <= tol * want.norm()
+
+
+# 4-wave kernel, direct-to-LDS split kernel, k-way kernel, many rows; one to four rows in 16 and in 32 columns
+@pytest.mark.parametrize('M,K,N,group', [(7, 512, 96, 64), (100, 1024, 256, 128), (30, 4096, 2048, 64), (64, 4096, 2048, 64),
+                                         (100, 8192, 256, 64), (5, 320, 64, 64), (64, 1152, 256, 128), (130, 256, 96, 64),
+                                         (700, 1024, 8224, 64), (1, 1024, 96, 64), (3, 320, 64, 64)])
+def test_projection_of_the_largest_scales(M, K, N, group):
+  pl, dense, x = _huge_scales(K, N, group, M + K)
+  x = x(M)
+  y = torch.empty(M, N, dtype=torch.bfloat16, device=G.DEV)
+  if M <= 4:
+    G.call('tmx_small_linear', S(), G.p(x), None, 1e-5, 0, G.p(pl.qweight), G.p(pl.scales), None, None, None, G.p(y), M, K, N, group, 0, 0, 0.0, 0)
+  else:
+    ws = torch.empty(_lib.lib().tmx_qlora_linear_workspace_bytes(M, K, N), dtype=torch.uint8, device=G.DEV)
+    G.call('tmx_qlora_linear', S(), G.p(x), G.p(pl.qweight), G.p(pl.scales), None, None, None, G.p(y), G.p(ws), M, K, N, group, 0, 0, 0.0)
+  G.sync()
+  _assert_rel(y, x.double() @ dense.double(), 3e-3)
+
+
+@pytest.mark.parametrize('M,K,F', [(20, 512, 4096), (64, 512, 4096), (40, 768, 192)])
+def test_gate_up_of_the_largest_scales(M, K, F):
+  pl, dense, x = _huge_scales(K, 2 * F, 64, M + K)
+  x = x(M) * 2.0 ** -20
+  act = torch.empty(M, F, dtype=torch.bfloat16, device=G.DEV)
+  G.call('tmx_qlora_gate_up_swiglu', S(), G.p(x), G.p(pl.qweight), G.p(pl.scales), None, None, G.p(act), M, K, F, 64, 0, 0.0)
+  G.sync()
+  y = (x.double() @ dense.double()).to(torch.bfloat16).double()
+  _assert_rel(act, y[:, :F] * torch.sigmoid(y[:, :F]) * y[:, F:], 1e-2)
+
+
+@pytest.mark.parametrize('P', [300, 1100])
+def test_moe_experts_of_the_largest_scales(P):
+  K, N, E = 512, 256, 6
+  pl, dense, x = _huge_scales(K, E * N, 64, P)
+  x = x(P)
+  idx = torch.arange(P, device=G.DEV, dtype=torch.int32) % E
+  y = torch.empty(P, N, dtype=torch.bfloat16, device=G.DEV)
+  G.call('tmx_moe_experts', S(), G.p(x), K, G.p(pl.qweight), G.p(pl.scales), G.p(idx), P, 1, E, K, N, 64, 1, G.p(y), N)
+  G.sync()
+  for e in range(E):
+    _assert_rel(y[e::E], x[e::E].double() @ dense[:, e * N:(e + 1) * N].double(), 3e-3)
+
+
 @pytest.mark.parametrize('M,K,N,group,r', [
     (1, 256, 96, 64, 0), (4, 256, 256, 64, 8), (7, 512, 96, 64, 8), (33, 1024, 160, 128, 16),
     (64, 2048, 1024, 64, 16), (100, 512, 256, 64, 32), (128, 4096, 512, 128, 32), (64, 14336, 256, 64, 16),

@@ -8,8 +8,8 @@
 // Mapping to CDNA4: weights are the B operand of v_mfma_f32_32x32x16_bf16.  The
 // packed tile format stores, for every 64(k) x 32(n) tile, the 32 nibbles a lane
 // needs as ONE 128-bit word, so a wave fetches a tile with a single coalesced
-// 1 KiB load and never touches LDS for weights.  Nibbles are widened and
-// scaled with one v_fma_mix_f32 (dequant_word in tmx_common.h; (u - 8) * s is exact in f32) and
+// 1 KiB load and never touches LDS for weights.  Nibbles are widened two
+// at a time (dequant_word in tmx_common.h), scaled with one fma ((u - 8) * s is exact in f32) and
 // rounded pairwise to bf16 by the hardware converter, which reproduces the
 // reference's bf16 dequantised weight bit for bit before it enters the MFMA.
 #include <atomic>
@@ -1793,7 +1793,7 @@ __global__ __launch_bounds__(256) void int4_dequant_kernel(const uint4* qw, cons
   const uint32_t wd[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    const bf16x8_t b = dequant_word_any_scale(wd[t], s, -8.f * s);
+    const bf16x8_t b = dequant_word(wd[t], nibble_scale(s));
     uint16_t e[8];
     __builtin_memcpy(e, &b, 16);
 #pragma unroll

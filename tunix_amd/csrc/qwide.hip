@@ -90,6 +90,7 @@ __device__ __forceinline__ void wide_core(uint16_t* smem, __amdgpu_buffer_rsrc_t
   bf16x8_t xq[RING];
   u32x4_t bq[2][2];  // weight fragments of two groups
   uint32_t words[2];
+  NibblePairs pairs;
   const int c0 = 8 * TPW * kw + q;  // this lane's first chunk of a slab row
   const uint16_t* xlane = smem + nl * XS;
   auto read_x = [&](const uint16_t* xb, auto rc) __attribute__((always_inline)) {
@@ -104,7 +105,7 @@ __device__ __forceinline__ void wide_core(uint16_t* smem, __amdgpu_buffer_rsrc_t
       const auto w = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
       words[0] = w[0]; words[1] = w[1];
     }
-    bq[g & 1][p / 4][p % 4] = dequant_part<p % 4>(words[p / 4], sc[j][p / 4]);
+    dequant_part<p % 4>(words[p / 4], sc[j][p / 4], pairs, bq[g & 1][p / 4]);
   };
   // A step is G groups of RF fragments of two MFMAs.  Behind the MFMAs of a fragment its register is refilled with the
   // one RING further on, and the weight fragments of the next group are dequantised an eighth at a time, so the matrix pipe

@@ -32,28 +32,6 @@ constexpr int kSbMaxTiles = 8;   // k-tiles per wave requested at once
 enum { SB_PRO_PLAIN = 0, SB_PRO_NORM = 1, SB_PRO_ATTN = 2 };
 enum { SB_EPI_PLAIN = 0, SB_EPI_RESIDUAL = 1, SB_EPI_SWIGLU = 2 };
 
-// bf16((u - 8) * s) of the eight nibbles of a word, two widened per v_cvt_pk_f32_fp8: a byte 0x0U read as an fp8 number (E4M3,
-// bias 7) is U * 2^-9 for every U in 0..15 (below 8 subnormal, from 8 on with exponent field 1), and the factor 2^9 goes into
-// the scale, exactly.  The form of the other projections (dequant_word) has fewer instructions but a longer chain of
-// dependent ones, which shows where no MFMAs hide it: gate | up of the 1B shape at one row 11.8 against 12.3 us.
-template <bool HIGH>
-__device__ __forceinline__ f32x2_t nibble_pair_f32(uint32_t w) {
-  return __builtin_amdgcn_cvt_pk_f32_fp8((int)w, HIGH);
-}
-__device__ __forceinline__ bf16x8_t sb_dequant(uint32_t d, float s, float m8s) {
-  const uint32_t lo = d & 0x0F0F0F0Fu;         // nibbles 0,2,4,6 in bytes 0..3
-  const uint32_t hi = (d >> 4) & 0x0F0F0F0Fu;  // nibbles 1,3,5,7 in bytes 0..3
-  const float s9 = s * 512.f;
-  const f32x2_t a = nibble_pair_f32<false>(lo), b = nibble_pair_f32<true>(lo);  // nibbles (0, 2), (4, 6)
-  const f32x2_t c = nibble_pair_f32<false>(hi), e = nibble_pair_f32<true>(hi);  // nibbles (1, 3), (5, 7)
-  // register p holds elements j = 2p, 2p + 1  <->  nibbles p, p + 4
-  const uint32_t p[4] = {pack_bf2(fmaf(a.x, s9, m8s), fmaf(b.x, s9, m8s)), pack_bf2(fmaf(c.x, s9, m8s), fmaf(e.x, s9, m8s)),
-                         pack_bf2(fmaf(a.y, s9, m8s), fmaf(b.y, s9, m8s)), pack_bf2(fmaf(c.y, s9, m8s), fmaf(e.y, s9, m8s))};
-  bf16x8_t r;
-  __builtin_memcpy(&r, p, 16);
-  return r;
-}
-
 // LDS carve of sb_linear_kernel (bytes): x [M][K + 8] bf16 | red [8 waves][4][32] f32 |
 // red_t [8][4][64] f32 | t [4][64] f32 | act [4][32] f32 | row scratch [4 + 8 * 4] f32
 __host__ __device__ inline size_t sb_x_bytes(int M, int K) { return ((size_t)M * (K + 8) * 2 + 15) & ~(size_t)15; }
@@ -384,7 +362,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
         bf16x8_t xa[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) xa[t] = *reinterpret_cast<const bf16x8_t*>(xb + kt * 64 + t * 16);
-        const float sc = bf2f(sr[i]), m8s = -8.f * sc;
+        const NibbleScale sc = nibble_scale(bf2f(sr[i]));
         const uint32_t wd[4] = {wr[i].x, wr[i].y, wr[i].z, wr[i].w};
         if (base + i + kSbMaxTiles < per) {  // slot consumed: refill it for the tile 8 further on
           const int ktn = min(kt + kSbMaxTiles, KT - 1);
@@ -393,7 +371,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
         }
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[t], sb_dequant(wd[t], sc, m8s), acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[t], dequant_word(wd[t], sc), acc, 0, 0, 0);
         if (mine(base + i)) {
 #pragma unroll
           for (int q = 0; q < 2; ++q) {
@@ -598,12 +576,12 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
         bf16x8_t xa[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) xa[t] = *reinterpret_cast<const bf16x8_t*>(xb + p * 128 + t * 16);
-        const float sc = bf2f(sr[i]), m8s = -8.f * sc;
+        const NibbleScale sc = nibble_scale(bf2f(sr[i]));
         const uint32_t wd[4] = {wr[i].x, wr[i].y, wr[i].z, wr[i].w};
         if (base + i + kSbPairs < per) load_w(p + kSbPairs, i);
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[t], sb_dequant(wd[t], sc, m8s), acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[t], dequant_word(wd[t], sc), acc, 0, 0, 0);
       }
     });
   }

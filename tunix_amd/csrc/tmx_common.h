@@ -96,44 +96,38 @@ __device__ __forceinline__ int acc_row(int r, int lane) {
 }
 
 // Expand one 32-bit word (8 nibbles, element j = 2 (i % 4) + i / 4 for nibble i) into the 8 bf16 B-operand values of
-// one MFMA step: bf16((u - 8) * s), (4 + 8 significant bits) exact as a float and rounded once.  This form, for
-// int4_dequant_kernel, takes every scale and widens a nibble per v_cvt_f32_ubyteN: 23 instructions per word.
-__device__ __forceinline__ bf16x8_t dequant_word_any_scale(uint32_t d, float s, float m8s) {
-  const uint32_t lo = d & 0x0F0F0F0Fu;         // nibbles 0,2,4,6 in bytes 0..3
-  const uint32_t hi = (d >> 4) & 0x0F0F0F0Fu;  // nibbles 1,3,5,7 in bytes 0..3
-  // register p holds elements j = 2p, 2p + 1  <->  nibbles p, p + 4
-  uint32_t p[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t w = i & 1 ? hi : lo;
-    p[i] = pack_bf2(fmaf((float)((w >> (8 * (i / 2))) & 0xFF), s, m8s), fmaf((float)((w >> (8 * (i / 2) + 16)) & 0xFF), s, m8s));
-  }
-  bf16x8_t r;
-  __builtin_memcpy(&r, p, 16);
-  return r;
-}
-
-// The form of the projections: a masked word 0x000U000V or 0x00U000V0 is a pair of f16 subnormals, U * 2^-24 or U * 2^-20,
-// which v_fma_mix_f32 widens and multiplies in one instruction: 17 instructions per word, the same exact products.  Registers
-// only, two waves per SIMD, ns per word and wave beside two (eight) 32 x 32 x 16 MFMAs: 53.1 (155); with v_cvt_f32_ubyteN
-// 60.7 (162), with two nibbles per v_cvt_pk_f32_fp8 (19 instructions) 54.9 (156).
-// Exact for |s| < 2^104, beyond which s * 2^24 is no finite float.
-struct NibbleScale { float s24, s20, m8s; };  // s * 2^24, s * 2^20, -8 s
-__device__ __forceinline__ NibbleScale nibble_scale(float s) { return {s * 16777216.f, s * 1048576.f, -8.f * s}; }
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-// register P of the B operand (elements 2 P, 2 P + 1 = nibbles P, P + 4 of word d)
+// one MFMA step: bf16((u - 8) * s), (4 + 8 significant bits) exact as a float and rounded once, for every scale whose -8 s is
+// finite.  A byte 0x0U read as an fp8 number (E4M3, bias 7) is U * 2^-9 for every U in 0..15 (below 8 subnormal, from 8 on
+// with exponent field 1), so one v_cvt_scalef32_pk_f32_fp8 with the scale 2^9 widens two nibbles of a masked word: 19
+// instructions per word.  Widening and scaling masked nibbles as f16 subnormals by v_fma_mix_f32 takes 17, but needs s * 2^24
+// finite; it is 0.4 to 0.8 % of a decode step faster (64 rows of the 8B shape, 8 layers, 64 tokens: 74.6 against 75.0 ms, 23 rows 42.0
+// against 42.4), and a branch per tile for the scales it cannot take costs more than it gains (77.8, 43.6 ms).
+struct NibbleScale { float s, m8s; };  // s, -8 s
+__device__ __forceinline__ NibbleScale nibble_scale(float s) { return {s, -8.f * s}; }
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+// The four registers of the B operand (register p: elements 2 p, 2 p + 1 = nibbles p, p + 4 of word d) in four parts, for loops
+// that spread them between MFMAs: part 0 widens the even nibbles and makes register 0, part 1 register 2, part 2 widens the
+// odd ones and makes register 1, part 3 register 3.
+struct NibblePairs { f32x2_t a, b; };
 template <int P>
-__device__ __forceinline__ uint32_t dequant_part(uint32_t d, const NibbleScale& sc) {
-  const uint32_t w = (P >= 2 ? d >> 8 : d) & (P & 1 ? 0x00F000F0u : 0x000F000Fu);
-  const float s = P & 1 ? sc.s20 : sc.s24;
-  const f16x2_t v = __builtin_bit_cast(f16x2_t, w);
-  return pack_bf2(fmaf((float)v.x, s, sc.m8s), fmaf((float)v.y, s, sc.m8s));
+__device__ __forceinline__ void dequant_part(uint32_t d, const NibbleScale& sc, NibblePairs& n, u32x4_t& r) {
+  if constexpr (P % 2 == 0) {
+    const uint32_t w = (P ? d >> 4 : d) & 0x0F0F0F0Fu;
+    n.a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w, 512.f, false);
+    n.b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w, 512.f, true);
+    r[P / 2] = pack_bf2(fmaf(n.a.x, sc.s, sc.m8s), fmaf(n.b.x, sc.s, sc.m8s));
+  } else {
+    r[P / 2 + 2] = pack_bf2(fmaf(n.a.y, sc.s, sc.m8s), fmaf(n.b.y, sc.s, sc.m8s));
+  }
 }
 __device__ __forceinline__ bf16x8_t dequant_word(uint32_t d, const NibbleScale& sc) {
-  const uint32_t p[4] = {dequant_part<0>(d, sc), dequant_part<1>(d, sc), dequant_part<2>(d, sc), dequant_part<3>(d, sc)};
-  bf16x8_t r;
-  __builtin_memcpy(&r, p, 16);
-  return r;
+  NibblePairs n;
+  u32x4_t r;
+  dequant_part<0>(d, sc, n, r);
+  dequant_part<1>(d, sc, n, r);
+  dequant_part<2>(d, sc, n, r);
+  dequant_part<3>(d, sc, n, r);
+  return __builtin_bit_cast(bf16x8_t, r);
 }
 
 // A copy the compiler does not see through: it happens here, so the registers of v are free for the load that follows
