@@ -940,6 +940,27 @@ def test_scoring_in_one_walk_equals_prompt_and_completion_walks(family, b, p, t)
   assert np.isfinite(got[0]).all() and np.abs(got[0] - got[1]).max() <= (2 if family == 'moe' else 1) * LOGPROB_TOL
 
 
+def test_scoring_does_not_read_the_embedding_of_padding_in_front_of_prompts():
+  """Padding in front of a prompt is not walked, or walked as another token: whatever its embedding holds, the log-probs are the
+  same.  In one walk of prompt and completion and in two."""
+  cfg = C.TOY
+  model = C.product_model(cfg, C.make_state(cfg, 47, 8, norm_jitter=0.05), 64, 16.0)
+  rng = np.random.default_rng(9)
+  prompt = rng.integers(3, cfg.vocab_size, (5, 20)).astype(np.int32)
+  comp = rng.integers(3, cfg.vocab_size, (5, 7)).astype(np.int32)
+  for i, n in enumerate((0, 1, 7, 18, 19)):
+    prompt[i, :n] = 0
+  for limit in (256, -1):
+    s = _sampler(model, cfg, 64)
+    s.ONE_WALK_ROWS = limit
+    want = s.per_token_logps(prompt, comp, pad_id=0)
+    kept = model.embed[0].clone()
+    model.embed[0] = float('nan')
+    got = s.per_token_logps(prompt, comp, pad_id=0)
+    model.embed[0] = kept
+    assert np.isfinite(want).all() and np.abs(got - want).max() <= LOGPROB_TOL, limit
+
+
 @pytest.mark.parametrize('rank', [4, 12, 16, 20, 21])
 @pytest.mark.parametrize('n_seq', [1, 4])
 def test_adapters_of_any_rank_in_steps_of_one_to_four_rows(rank, n_seq):

@@ -497,7 +497,15 @@ class Sampler:
     st['positions'] = torch.from_numpy(utils.build_positions_from_mask(valid).astype(np.int32)).to(dev)
     st['sampling_mode'] = 'score'
     if st['share_group'] == 1 and b * (p - 1) <= self.ONE_WALK_ROWS and b * (total - 1) <= self._fill_rows():
-      self.walk(st, total - 1, sample=True)  # prompt columns are scored too, and their scores left out
+      # Prompt columns are scored too, and their scores left out.  Padding in front of a prompt is walked as well, here as
+      # the row's first real token: what its slots hold is multiplied by probabilities of 0, and the embedding of the padding
+      # id, which a walk of the prompts never reads, need not be finite.
+      first = st['first_col_host']
+      unread = np.arange(total) < np.minimum(first, p - 1)[:, None]
+      if unread.any():
+        real = np.take_along_axis(ids, np.minimum(first, total - 1)[:, None], axis=1)
+        st['token_buffer'].copy_(torch.from_numpy(np.where(unread, real, ids)))
+      self.walk(st, total - 1, sample=True)
     else:
       self.walk(st, p - 1)
       self.walk(st, t, sample=True)
