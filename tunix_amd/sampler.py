@@ -185,8 +185,9 @@ class Sampler:
   # -- state ----------------------------------------------------------------
   def init_sample_state(self, all_input_ids, total_sampling_steps, include_logits,
                         forbidden_token_ids, temperature, top_p, top_k, seed, beam_size=None,
-                        include_logprobs=False, prompt_lengths=None):
-    """Device-side _SamplingState (tunix/generate/sampler.py:402-509)."""
+                        include_logprobs=False, prompt_lengths=None, walked_ids=None):
+    """Device-side _SamplingState (tunix/generate/sampler.py:402-509).  walked_ids: what the token buffer holds in place of
+    the ids, which give the mask and the shared prompts."""
     if beam_size is not None:
       raise NotImplementedError('beam search is outside this decode path')
     dev = self._transformer.device
@@ -203,7 +204,7 @@ class Sampler:
     if not 0 <= pad < vocab:
       raise ValueError(f'pad_id {pad} is outside the vocabulary [0, {vocab})')
     token_buffer = np.full((b, total_sampling_steps), pad, dtype=np.int32)
-    token_buffer[:, :p] = ids
+    token_buffer[:, :p] = ids if walked_ids is None else walked_ids
     input_mask = np.ones((b, total_sampling_steps), dtype=bool)
     if prompt_lengths is not None:
       lens = np.asarray(prompt_lengths).reshape(-1, 1)
@@ -486,9 +487,13 @@ class Sampler:
     valid = (ids != pad) if token_mask is None else np.asarray(token_mask).astype(bool)
     if valid.shape != ids.shape:
       raise ValueError('token_mask must match the full prompt/completion shape')
+    # Padding in front of a prompt may be walked, as the row's first real token: what its slots hold is multiplied by
+    # probabilities of 0, so it has to be finite, and the embedding of the padding id need not be.
+    first = valid.argmax(axis=1)
+    walked = np.where(np.arange(total) < np.minimum(first, p - 1)[:, None], ids[np.arange(b), first][:, None], ids)
     self.eos_ids = np.array([-1])
     st = self.init_sample_state(ids, total, False, None, temperature if temperature not in (0.0, 1.0) else 1.0,
-                                1.0, None, 0, include_logprobs=True)
+                                1.0, None, 0, include_logprobs=True, walked_ids=walked)
     dev = self._transformer.device
     self._set_mask(st, valid)
     if token_mask is not None:  # rows of the same ids share a prompt only where they are masked alike
@@ -497,14 +502,7 @@ class Sampler:
     st['positions'] = torch.from_numpy(utils.build_positions_from_mask(valid).astype(np.int32)).to(dev)
     st['sampling_mode'] = 'score'
     if st['share_group'] == 1 and b * (p - 1) <= self.ONE_WALK_ROWS and b * (total - 1) <= self._fill_rows():
-      # Prompt columns are scored too, and their scores left out.  Padding in front of a prompt is walked as well, here as
-      # the row's first real token: what its slots hold is multiplied by probabilities of 0, and the embedding of the padding
-      # id, which a walk of the prompts never reads, need not be finite.
-      first = st['first_col_host']
-      unread = np.arange(total) < np.minimum(first, p - 1)[:, None]
-      if unread.any():
-        real = np.take_along_axis(ids, np.minimum(first, total - 1)[:, None], axis=1)
-        st['token_buffer'].copy_(torch.from_numpy(np.where(unread, real, ids)))
+      # prompt columns are scored too, and their scores left out
       self.walk(st, total - 1, sample=True)
     else:
       self.walk(st, p - 1)
