@@ -89,6 +89,26 @@ def _sampler(cache_size=5):
   return Sampler(_StubModel(), C.ToyTokenizer(), CacheConfig(cache_size, c.num_layers, c.num_kv_heads, c.head_dim))
 
 
+# Scoring of few rows in one walk or in two, each as it measured faster (us of one and of two walks beside it)
+@pytest.mark.parametrize('model,layers,b,p,t,one', [
+    ('toy', 2, 4, 65, 16, True),                 # 479, 547
+    ('llama3p2_1b', 16, 1, 257, 8, True),        # 2971, 3550
+    ('llama3p2_1b', 2, 1, 257, 8, False),        # 930, 767
+    ('llama3p2_1b', 2, 2, 65, 60, True),         # 766, 835
+    ('llama3p2_1b', 1, 4, 65, 16, False),        # 821, 632
+    ('llama3p1_8b', 8, 1, 129, 500, True),       # 4458, 4787
+    ('llama3p1_8b', 2, 1, 129, 500, False),      # 2007, 1875
+    ('qwen3_30b_a3b', 6, 1, 257, 8, True),       # 2073, 2401
+    ('qwen3_30b_a3b', 2, 1, 257, 8, False),      # 1140, 1055
+    ('llama3p2_1b', 16, 1, 258, 8, False),       # more prompt rows than were measured
+    ('llama3p2_1b', 16, 64, 5, 64, False)])      # more rows than a pass takes
+def test_scoring_walks_follow_depth_and_vocabulary(model, layers, b, p, t, one):
+  import dataclasses
+  s = _sampler()
+  s._transformer.config = dataclasses.replace(getattr(ModelConfig, model)(), num_layers=layers)
+  assert s._one_walk(b, p, t) is one
+
+
 def test_sampler_rejects_invalid_inputs_like_the_reference():
   s = _sampler(5)
   with pytest.raises(ValueError, match='exactly one'):

@@ -303,9 +303,7 @@ class Sampler:
 
   MAX_MOE_PAIRS = 8192  # routed (token, expert) pairs of one pass of a MoE model
   MIN_BLOCK_TOKENS = 4  # tokens per sequence from which a pass over all columns runs the attention that ragged passes run
-  # Scoring: prompt rows up to which prompt and completion are one pass.  A prompt row costs the head about 1 us there, a walk of
-  # its own 8 launches per layer that few rows do not fill (5 sequences of 37 + 90 tokens on the 1B shape 5.0 -> 3.8 ms).
-  ONE_WALK_ROWS = 256
+  ONE_WALK_ROWS = 256   # scoring: prompt rows up to which prompt and completion may be one pass (_one_walk)
   MAX_PASSES_IN_FLIGHT = 64  # passes a walk enqueues before it waits for the stream
 
   def _max_rows(self):
@@ -318,6 +316,24 @@ class Sampler:
     if cfg.num_experts:
       return max(128, min(4096, self.MAX_MOE_PAIRS // cfg.num_experts_per_tok))
     return 4096
+
+  def _one_walk(self, b, p, t):
+    """Whether scoring takes prompt and completion in one pass: the head then multiplies the prompt's rows too, and
+    a walk of their own, 8 launches per layer that few rows do not fill, is saved.  us, fitted to 11 models of 1 to 16 layers:
+    the head streams up to 256 rows, more in blocks of 256; a layer of the second walk costs 45, one with routed experts 100 (two
+    walks -> one: 1B shape of 16 layers, 5 x (37 + 90) tokens 5000 -> 3800; of 2 layers, 1 x (257 + 8) 767 -> 930, 2 x (65 + 60)
+    835 -> 766; 8B shape of 2 layers, 1 x (129 + 500) 1875 -> 2007, of 8 layers 4787 -> 4458)."""
+    if b * (p - 1) > self.ONE_WALK_ROWS or b * (p + t - 1) > self._fill_rows():
+      return False
+    c = self._transformer.config
+    streams = 256 if getattr(self._transformer, 'stream_head', True) else 64
+
+    def head(rows):
+      if rows <= streams:
+        return c.vocab_size * c.embed_dim * 3.5e-7 * (1 + 0.7 * rows / 256)
+      return -(-rows // 256) * c.vocab_size * (3.2e-7 * c.embed_dim + 6.5e-4)
+
+    return head(b * (p + t - 1)) - head(b * t) <= c.num_layers * (100 if c.num_experts else 45)
 
   def _many_rows_ok(self):
     return self._max_rows() > 128
@@ -501,7 +517,7 @@ class Sampler:
       st['share_group'], st['share_len'], st['share_common'] = share
     st['positions'] = torch.from_numpy(utils.build_positions_from_mask(valid).astype(np.int32)).to(dev)
     st['sampling_mode'] = 'score'
-    if st['share_group'] == 1 and b * (p - 1) <= self.ONE_WALK_ROWS and b * (total - 1) <= self._fill_rows():
+    if st['share_group'] == 1 and self._one_walk(b, p, t):
       # prompt columns are scored too, and their scores left out
       self.walk(st, total - 1, sample=True)
     else:
