@@ -827,6 +827,12 @@ def test_head_nucleus_matches_oracle(M, D, V, temp, top_p, top_k, sharp):
   assert np.all(tok[:, :step + 1] == -5) and np.all(tok[:, step + 2:] == -5)
 
 
+# the head's 256 x 256 blocks, whose copy of the rows lies in the nucleus workspace: rows and vocabularies that fill no block
+@pytest.mark.parametrize('M,D,V', [(65, 128, 1024), (100, 256, 2080), (257, 128, 2048)])
+def test_head_nucleus_of_many_rows(M, D, V):
+  test_head_nucleus_matches_oracle(M, D, V, 0.9, 0.8, None, 2.0)
+
+
 def test_head_nucleus_limits():
   x, w = _head_inputs(16, 128, 1024, 3)
   key = prng.prng_key(5)

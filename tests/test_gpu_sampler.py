@@ -981,7 +981,19 @@ def test_adapters_of_any_rank_in_steps_of_one_to_four_rows(rank, n_seq):
 def test_head_of_more_than_256_rows_equals_heads_of_fewer(b, p, t):
   """Row counts that fill no block of 32: the last rows of the copy in fragment order.  Scored whole and in parts of at most 128
   rows, greedy and sampled rollouts of as many sequences too."""
-  cfg = C.TOY
+  _check_head_of_many_rows(C.TOY, b, p, t, LOGPROB_TOL)
+
+
+# the copy of the rows in the activations of the experts (2 F < D; every expert is used, so that no rounding changes the
+# routing), and in room of its own (no buffer is as large)
+@pytest.mark.parametrize('cfg', [
+    OM.Config('qwen3', 2, 1024, 768, 256, 4, 64, 2, rope_theta=1_000_000, norm_eps=1e-6, num_experts=8, experts_per_tok=8),
+    OM.Config('llama3', 2, 1024, 512, 128, 4, 64, 2)], ids=['experts', 'narrow mlp'])
+def test_head_of_more_than_256_rows_finds_room_for_its_copy(cfg):
+  _check_head_of_many_rows(cfg, 300, 3, 2, (2 if cfg.num_experts else 1) * LOGPROB_TOL)
+
+
+def _check_head_of_many_rows(cfg, b, p, t, tol):
   model = C.product_model(cfg, C.make_state(cfg, 11, 8, norm_jitter=0.05), 64, 16.0)
   s = _sampler(model, cfg, 32)
   rng = np.random.default_rng(b)
@@ -989,11 +1001,12 @@ def test_head_of_more_than_256_rows_equals_heads_of_fewer(b, p, t):
   part = 128 // t
 
   def in_parts(comp):
-    return np.concatenate([s.per_token_logps(prompt[i:i + part], comp[i:i + part], pad_id=0) for i in range(0, b, part)])
+    every = np.ones((part, p + t), bool)  # a chosen token may be the padding id
+    return np.concatenate([s.per_token_logps(prompt[i:i + part], comp[i:i + part], token_mask=every[:b - i]) for i in range(0, b, part)])
 
   comp = rng.integers(3, cfg.vocab_size, (b, t)).astype(np.int32)
-  assert np.abs(s.per_token_logps(prompt, comp, pad_id=0) - in_parts(comp)).max() <= LOGPROB_TOL
+  assert np.abs(s.per_token_logps(prompt, comp, pad_id=0) - in_parts(comp)).max() <= tol
   for temperature in (0.0, 1.0):
     out = s(prompt_token_ids=list(prompt), max_generation_steps=t, temperature=temperature, eos_tokens=[-1],
             return_logprobs=True, seed=3)
-    assert np.abs(np.array(out.logprobs) - in_parts(np.stack(out.tokens))).max() <= LOGPROB_TOL
+    assert np.abs(np.array(out.logprobs) - in_parts(np.stack(out.tokens))).max() <= tol

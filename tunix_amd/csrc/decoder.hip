@@ -34,6 +34,7 @@ struct Workspace {
   int32_t* expert_of;
   float* weight_of;
   uint16_t *pair_act, *pair_y;
+  uint16_t* head_x;  // the many-rows head's copy of its rows: a buffer that is free by then where one is large enough
   int2* row_map;  // ragged pass: row -> (sequence, column), and the sequences' runs of rows
   int4* seg;
   size_t total;
@@ -135,6 +136,10 @@ static Workspace carve(const tmx_model_desc* m, int B, int C, char* base) {
   w.weight_of = (float*)take(P * 4);
   w.pair_act = (uint16_t*)take(P * F * 2);
   w.pair_y = (uint16_t*)take(P * D * 2);
+  {
+    const size_t room = head_x_tiles_bytes(B, (int)D);
+    w.head_x = (size_t)B * 2 * F * 2 >= room ? w.y16 : P * D * 2 >= room ? w.pair_y : (uint16_t*)take(room);
+  }
   w.row_map = (int2*)take((size_t)B * 8);
   w.seg = (int4*)take((size_t)B * 16);
   w.total = off;
@@ -571,11 +576,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       a.eos = s->eos_ids; a.n_eos = s->n_eos;
       a.buf_len = L;
       a.tpp = T;
-      {  // the many-rows head reorders its rows into a buffer that is free by now
-        const size_t room = (size_t)(B + 31) / 32 * 32 * D;
-        if ((size_t)B * 2 * F >= room) a.x_tiles = w.y16;
-        else if (moe && (size_t)B * m->experts_per_tok * D >= room) a.x_tiles = w.pair_y;
-      }
+      a.x_tiles = w.head_x;
       if (w.dsync && !nucleus && !prof) {  // one word of the hand-over header, which starts a call at zero
         a.advance = s->step;
         a.arrived = (uint32_t*)w.dsync + 63;

@@ -453,7 +453,7 @@ __global__ __launch_bounds__(256) void head_finalize_kernel(HeadArgs a) {
 // direct-to-LDS loads (128-byte rows of 64 k, 16-byte chunk c of row r at slot c ^ (r / 2 % 8));
 // wave w owns sequence rows 32 w .. 32 w + 31 as the B operand, read straight from global
 // memory (lane (row, h) holds k = 32 h .. 32 h + 31 of a k-tile of 64, MFMA step t pairs k = 32 h + 8 t ..
-// with the same k of the vocabulary rows), from a copy of the rows in fragment order where there is room for one.  A lane's
+// with the same k of the vocabulary rows), from a copy of the rows in fragment order.  A lane's
 // 128 accumulator registers are 128 vocabulary rows of ONE sequence row, so max / sum-exp / the
 // target's z run down the registers.  LDS reads of fragment group g + 1 and the refill of the
 // B registers are pinned between the MFMAs of group g.  The matrix comes from HBM, so its slabs are short (64 k) and
@@ -495,7 +495,7 @@ __global__ __launch_bounds__(512, 1) void head_wide_kernel(HeadArgs a, int tok_b
   const int nsteps = a.D >> 7, last_step = nsteps - 1;  // steps of two slabs
 
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.w + (size_t)v0 * a.D, (uint32_t)vrows * a.D * 2u);
-  const __amdgpu_buffer_rsrc_t rx = a.x_tiles ? make_rsrc(a.x_tiles, (uint32_t)(a.M + 31) / 32 * 32 * a.D * 2u) : make_rsrc(a.x, (uint32_t)a.M * a.D * 2u);
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x_tiles, (uint32_t)(a.M + 31) / 32 * 32 * a.D * 2u);
   constexpr int XR = ROWS / 64;
   int woff[XR];  // slab transfer: load i moves vocabulary rows 8 wave + 64 i .. + 7, 8 lanes each
 #pragma unroll
@@ -503,10 +503,7 @@ __global__ __launch_bounds__(512, 1) void head_wide_kernel(HeadArgs a, int tok_b
     const int row_l = 8 * wave + 64 * i + (lane >> 3);
     woff[i] = (row_l < vrows ? row_l : vrows - 1) * a.D * 2 + (((lane & 7) ^ ((row_l >> 1) & 7)) * 16);
   }
-  // B fragments: from the rows themselves, or 1 KiB each from their tile copy (head_x_tiles_kernel)
-  const bool tiled = a.x_tiles != nullptr;
-  const int xv = tiled ? (tb * 8 + wave) * (a.D >> 4) * 1024 + lane * 16 : tok_l * a.D * 2 + h * 64;
-  const int xt = tiled ? 1024 : 16, xj = tiled ? 4096 : 128;  // bytes between fragments and between k-tiles of 64
+  const int xv = (tb * 8 + wave) * (a.D >> 4) * 1024 + lane * 16;  // B fragments: 1 KiB each
 
   f32x16_t acc[MT];
 #pragma unroll
@@ -519,7 +516,7 @@ __global__ __launch_bounds__(512, 1) void head_wide_kernel(HeadArgs a, int tok_b
   auto load_b = [&](int step, auto gc) __attribute__((always_inline)) {
     constexpr int g = decltype(gc)::value;
     step = step < last_step ? step : last_step;
-    breg[g] = __builtin_amdgcn_raw_buffer_load_b128(rx, xv, (step * 2 + (g >> 2)) * xj + (g & 3) * xt, 0);
+    breg[g] = __builtin_amdgcn_raw_buffer_load_b128(rx, xv, (step * G + g) * 1024, 0);
   };
   auto dma_w = [&](int slab, int i) __attribute__((always_inline)) {
     uint16_t* base = smem + (size_t)(slab & (NB - 1)) * ROWS * XS + wave * 8 * XS;
@@ -668,15 +665,16 @@ bool head_wide_ok(const HeadArgs& a) {
          a.n_forbidden == 0 && !a.logits_out;
 }
 
+size_t head_x_tiles_bytes(int M, int D) { return M > 64 ? (size_t)(M + 31) / 32 * 32 * D * 2 : 0; }
+
 // The wide kernel alone: partials (and, in the sorting branch, keys) of every row; sets a.nwg.
 int head_wide_logits(hipStream_t st, HeadArgs& a) {
   if (!head_wide_ok(a)) return TMX_ERR_SHAPE;
+  if (!a.x_tiles) return TMX_ERR_ARG;
   const int tok_blocks = (a.M + 255) / 256, voc_blocks = (a.V + HW::ROWS - 1) / HW::ROWS;
-  if (a.x_tiles) {
-    hipLaunchKernelGGL(head_x_tiles_kernel, dim3(a.D / 128, (a.M + 31) / 32), dim3(512), 0, st, a.x, a.x_tiles, a.M, a.D);
-    const int rc = check_launch();
-    if (rc != TMX_OK) return rc;
-  }
+  hipLaunchKernelGGL(head_x_tiles_kernel, dim3(a.D / 128, (a.M + 31) / 32), dim3(512), 0, st, a.x, a.x_tiles, a.M, a.D);
+  const int rc = check_launch();
+  if (rc != TMX_OK) return rc;
   a.nwg = voc_blocks;
   a.row_base = 0;
   int lrc;

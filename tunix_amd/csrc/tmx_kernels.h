@@ -186,7 +186,7 @@ struct AttnArgs {
 
 struct HeadArgs {
   const uint16_t* x;  // [M, D] final-normed hidden states
-  uint16_t* x_tiles;  // room for x again, rows rounded up to 32, in the wide kernel's order (null: it reads x itself)
+  uint16_t* x_tiles;  // room for x again in the wide kernel's order (head_x_tiles_bytes; needed by head_wide only)
   const uint16_t* w;  // [V, D]
   const uint16_t* w_tiles;  // the same matrix in the tile layout of head_tiles_kernel, or null
   int M, D, V;
@@ -312,6 +312,7 @@ int moe_rows(hipStream_t st, const MoeArgs& a, int E, bool down);  // its form f
 int head_sample(hipStream_t st, HeadArgs a);
 // any number of rows in 256 x 256 blocks (greedy, sampling without the sorting branch, scoring); needs
 // D % 128 == 0, no forbidden ids, no logits output; part_f / part_i sized [M][ceil(V / 256)]
+size_t head_x_tiles_bytes(int M, int D);  // 0 up to 64 rows, which head_wide does not take
 int head_wide(hipStream_t st, HeadArgs a);
 bool head_wide_ok(const HeadArgs& a);
 int head_wide_logits(hipStream_t st, HeadArgs& a);  // the wide kernel without the finalize launch
