@@ -382,6 +382,7 @@ int head_tiles_pack(hipStream_t st, const uint16_t* w, uint16_t* tiles, int V, i
 __device__ __forceinline__ void finalize_advance(const HeadArgs& a, int step) {
   if (!a.advance) return;
   if (gridDim.x > 1) {
+    asm volatile("" ::"s"(step) : "memory");
     __builtin_amdgcn_s_waitcnt(0);
     if (__hip_atomic_fetch_add(a.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
     __hip_atomic_store(a.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -567,8 +568,12 @@ __global__ __launch_bounds__(512, 1) void head_wide_kernel(HeadArgs a, int tok_b
     });
   };
 
+  // (in this order, which the counts of the waits assume)
 #pragma unroll
-  for (int i = 0; i < (NB - 1) * XR; ++i) dma_w(i / XR, i % XR);
+  for (int i = 0; i < (NB - 1) * XR; ++i) {
+    dma_w(i / XR, i % XR);
+    if (i % XR == XR - 1) __builtin_amdgcn_sched_barrier(0);
+  }
   static_for<G>([&](auto gc) __attribute__((always_inline)) { load_b(0, gc); });
   meet(IC<(NB - 2) * XR + G>{});
 #pragma unroll

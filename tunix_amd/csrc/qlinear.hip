@@ -974,6 +974,7 @@ __global__ __launch_bounds__(512, 1) void qlinear_gate_up8_kernel(QLinearArgs a)
   };
 
   dma_x(0, 0);
+  __builtin_amdgcn_sched_barrier(0);  // the slab first: the wait counts what is younger
   static_for<TPW>([&](auto jc) __attribute__((always_inline)) { load_w_tile(0, jc); });
   if constexpr (FUSE) load_l(0);
   __builtin_amdgcn_sched_barrier(0);
@@ -1402,6 +1403,7 @@ __device__ __forceinline__ void gemm_block_dma(const QLinearArgs& a, uint16_t* s
   };
 
   dma_x(0, 0);
+  __builtin_amdgcn_sched_barrier(0);  // the slab first: the wait counts what is younger
   if (tile_ok) static_for<TPW>([&](auto jc) __attribute__((always_inline)) { load_w_tile(0, IC<0>{}, jc); });
   wait_slab();
   if (DW == 2 && tile_ok)

@@ -159,12 +159,18 @@ __device__ __forceinline__ void wide_core(uint16_t* smem, __amdgpu_buffer_rsrc_t
     });
   };
 
+  // (in this order, which the counts of the waits assume)
   static_for<WB>([&](auto bc) __attribute__((always_inline)) { load_w(decltype(bc)::value, bc); });
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < (NB - 1) * MT; ++i) dma_x(i / MT, i / MT, i % MT);
+  for (int i = 0; i < (NB - 1) * MT; ++i) {
+    dma_x(i / MT, i / MT, i % MT);
+    if (i % MT == MT - 1) __builtin_amdgcn_sched_barrier(0);
+  }
   meet(IC<(NB - 2) * MT>{});
   take_w(IC<0>{});
   load_w(WB, IC<0>{});
+  __builtin_amdgcn_sched_barrier(0);
   if (active) {
     static_for<RING>([&](auto rc) __attribute__((always_inline)) { read_x(xlane + (c0 ^ nl) * 8, rc); });
     static_for<8>([&](auto pc) __attribute__((always_inline)) { dequant(IC<0>{}, pc); });
