@@ -925,7 +925,7 @@ def test_moe_route_matches_oracle(B, D, E, k):
 
 @pytest.mark.parametrize('B,D,F,E,k,group', [
     (8, 256, 256, 16, 4, 64), (32, 512, 256, 32, 8, 128), (40, 256, 512, 4, 2, 64),
-    # more than 1024 routed pairs (many-rows passes): the block kernel, hundreds of rows per expert
+    # more than 1024 routed pairs (many-rows passes): up to 128 rows of an expert at a time, hundreds of rows per expert
     (600, 256, 256, 6, 2, 64), (300, 512, 256, 9, 4, 128), (300, 256, 256, 40, 4, 64)])
 def test_moe_experts_match_oracle(B, D, F, E, k, group):
   T = G.Keep()
@@ -1153,13 +1153,14 @@ def test_adapter_sync_writes_both_operands(K, r, widths, dtype):
 @pytest.mark.parametrize('down,K,N', [(0, 256, 640), (0, 512, 128), (1, 256, 384), (1, 768, 128)])
 def test_moe_experts_row_counts(down, K, N):
   from tunix_amd import quant
-  counts = [0, 1, 15, 16, 17, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 257, 300]
+  counts = [0, 1, 15, 16, 17, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 257, 300, 1]  # whole tokens of two pairs
   E, k, group = len(counts), 2, 64
   g = torch.Generator(device=G.DEV).manual_seed(K + N)
   idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
-  P = idx.numel() // k * k
-  assert 1024 < P <= 8192
-  idx = idx[torch.randperm(idx.numel(), generator=torch.Generator().manual_seed(3))][:P].to(torch.int32).to(G.DEV)
+  P = idx.numel()
+  assert 1024 < P <= 8192 and P % k == 0
+  idx = idx[torch.randperm(P, generator=torch.Generator().manual_seed(3))].to(torch.int32).to(G.DEV)
+  assert torch.bincount(idx, minlength=E).tolist() == counts
   w = (torch.randn(K, E * N, generator=g, device=G.DEV) * 0.05).to(torch.bfloat16)
   pl = quant.PackedLinear.from_dense([w], group, G.DEV)
   dense = torch.empty(K, E * N, dtype=torch.bfloat16, device=G.DEV)

@@ -611,6 +611,7 @@ def test_scoring_clip_reaches_the_many_rows_head(stream_head):
   model = C.product_model(cfg, st, 64, 16.0)
   model.stream_head = stream_head
   s = _sampler(model, cfg, 48)
+  s.ONE_WALK_ROWS = -1  # the completions' 96 rows alone
   rng = np.random.default_rng(4)
   prompt = rng.integers(3, cfg.vocab_size, (8, 10)).astype(np.int32)
   comp = rng.integers(3, cfg.vocab_size, (8, 12)).astype(np.int32)
@@ -915,8 +916,8 @@ def test_scoring_shares_no_prompt_between_rows_whose_token_masks_differ():
 @pytest.mark.parametrize('family', ['llama3', 'moe'])
 @pytest.mark.parametrize('b,p,t', [(5, 37, 20), (1, 2, 1), (3, 1, 6), (4, 65, 3)])
 def test_scoring_in_one_walk_equals_prompt_and_completion_walks(family, b, p, t):
-  """Prompt and completion in one pass, where padding in front of the prompts is walked too and scores of prompt columns are
-  left out: the log-probs are those of two walks.  Rows of other counts take other tiles and K-slices, so sums round
+  """Prompt and completion in one pass, where padding in front of the prompts is walked too (as another token) and scores of
+  prompt columns are left out: the log-probs are those of two walks.  Rows of other counts take other tiles and K-slices, so sums round
   differently: the tolerance of the log-probs."""
   cfg = C.TOY if family == 'llama3' else OM.Config('qwen3', 2, 1024, 256, 256, 4, 64, 2, rope_theta=1_000_000, norm_eps=1e-6,
                                                    tied=False, num_experts=8, experts_per_tok=2)
@@ -972,7 +973,8 @@ def test_adapters_of_any_rank_in_steps_of_one_to_four_rows(rank, n_seq):
   rng = np.random.default_rng(rank)
   prompts = [rng.integers(3, cfg.vocab_size, 40).astype(np.int32) for _ in range(n_seq)]
   out = s(prompt_token_ids=prompts, max_generation_steps=6, temperature=0.0, eos_tokens=[-1], return_logprobs=True)
-  many = 8 // n_seq
+  many = 24 // n_seq  # 24 rows of 6 tokens: 144 rows of a pass, and no prompt walked for several rows
+  s.share_prompt_kv = False
   scored = s.per_token_logps(np.tile(np.stack(prompts), (many, 1)), np.tile(np.stack(out.tokens), (many, 1)), pad_id=0)
   assert np.abs(scored[:n_seq] - np.array(out.logprobs)).max() <= LOGPROB_TOL
 
@@ -996,6 +998,7 @@ def test_head_of_more_than_256_rows_finds_room_for_its_copy(cfg):
 def _check_head_of_many_rows(cfg, b, p, t, tol):
   model = C.product_model(cfg, C.make_state(cfg, 11, 8, norm_jitter=0.05), 64, 16.0)
   s = _sampler(model, cfg, 32)
+  s.ONE_WALK_ROWS = -1  # the head's rows are the completions' alone
   rng = np.random.default_rng(b)
   prompt = rng.integers(3, cfg.vocab_size, (b, p)).astype(np.int32)
   part = 128 // t
