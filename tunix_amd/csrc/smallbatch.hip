@@ -480,6 +480,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
 // 32 columns -> 16): q|k|v 8.0 / 9.1 -> 8.0 / 9.0, o 9.3 / 15.6 -> 7.4 / 9.6, down 11.8 / 14.4 -> 9.8 / 13.0 (less since, see
 // below and SbCopy).
 constexpr int kSbPairs = 8;  // k-tile pairs per wave requested at once
+constexpr int kSbLoraTiles = 4;  // k-tiles of A per wave requested at once
 
 // LDS: x [M][K + 8] bf16 | red [8 waves][4][16] f32 | red_t [8][4][64] f32 | t [4][64] f32 | row scratch [4 + 8 * 4] f32
 constexpr size_t kSb16TailFloats = kSbWaves * kSbMaxRows * 16 + kSbWaves * kSbMaxRows * 64 + kSbMaxRows * 64 + 4 + kSbWaves * 4;
@@ -516,7 +517,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
 
   // x . A of this wave's eighth of K, for the tiles of 16 columns of A that hold this workgroup's segment (of a rank of 16
   // half of what lies in a tile of 32 is another segment's or padding: 64 KB instead of 128 KB of A per workgroup on the 1B
-  // shape, one row / three rows: q|k|v 8.0 / 9.1 -> 7.0 / 7.8 us, o 7.5 / 9.8 -> 6.4 / 8.7); up to four (k-tile, tile) items at a time, the first four requested now.
+  // shape, one row / three rows: q|k|v 8.0 / 9.1 -> 7.0 / 7.8 us, o 7.5 / 9.8 -> 6.4 / 8.7), the first of them requested now.
   // The four lane groups of a load hold 32 consecutive steps of the contraction.
   const bool lora_here = a.a_t != nullptr;
   int q0 = 0, nq = 0;
@@ -524,23 +525,29 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
     const int n0 = (int)blockIdx.x * 16;
     const int seg = n0 >= a.seg_end[0] ? (n0 >= a.seg_end[1] ? 2 : 1) : 0;
     q0 = (seg * a.lora_r) >> 4;
-    nq = min(((seg + 1) * a.lora_r - 1) >> 4, (a.Rpad >> 4) - 1) - q0 + 1;  // 1 to 3: ranks up to 32
+    nq = min(((seg + 1) * a.lora_r - 1) >> 4, (a.Rpad >> 4) - 1) - q0 + 1;  // 1 or 2: r <= 32, and 3 r <= 64 where there are segments
   }
   const int RT = a.Rpad >> 5;
-  const int lper = (KT + kSbWaves - 1) / kSbWaves, l0 = wave * lper, l1 = min(l0 + lper, KT);
-  const int items = max(l1 - l0, 0) * nq;
-  u32x4_t ab[4][2];
-  auto load_a = [&](int it, auto ic) __attribute__((always_inline)) {
-    constexpr int i = decltype(ic)::value;
-    if (it < items) {
-      const int k = nq == 1 ? it : it / nq, qq = q0 + it - k * nq;
-      const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + ((size_t)((l0 + k) * RT + (qq >> 1)) * 4 + par) * 64 + 32 * h +
-                          (qq & 1) * 16 + n16;
+  const int lper = (KT + kSbWaves - 1) / kSbWaves, l0 = wave * lper, nk = min(lper, KT - l0);
+  u32x4_t ab[8][2];
+  // The count as a constant: straight code, whose LDS reads and products are in flight together.  With one loop for all counts
+  // rank 32 took 8.7 us at 1 x 2048 x 3072 and 20.2 at 1 x 8192 x 2048 (now 7.4 and 13.1), rank 16 7.5 and 12.8 (7.4 and 11.2).
+  auto by_nq = [&](auto&& f) __attribute__((always_inline)) {
+    if (nq == 1) f(IC<1>{});
+    else if (nq == 2) f(IC<2>{});
+  };
+  // k-tile k of this wave into slot d
+  auto load_a = [&](auto nqc, int k, auto dc) __attribute__((always_inline)) {
+    constexpr int NQ = decltype(nqc)::value, d = decltype(dc)::value;
+    if (k < nk) {
+      const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + ((size_t)(l0 + k) * RT * 4 + par) * 64 + 32 * h + n16;
 #pragma unroll
-      for (int s = 0; s < 2; ++s) ab[i][s] = ap[s * 128];
+      for (int i = 0; i < 2 * NQ; ++i) ab[d * NQ + i / 2][i % 2] = ap[((q0 + i / 2) >> 1) * 256 + ((q0 + i / 2) & 1) * 16 + i % 2 * 128];
     }
   };
-  static_for<4>([&](auto ic) __attribute__((always_inline)) { load_a(decltype(ic)::value, ic); });
+  by_nq([&](auto nqc) __attribute__((always_inline)) {
+    static_for<kSbLoraTiles>([&](auto dc) __attribute__((always_inline)) { load_a(nqc, decltype(dc)::value, dc); });
+  });
 
   // what the epilogue needs and no other launch makes
   const bool epi_thread = tid < kSbMaxRows * 16 && (tid >> 4) < M;
@@ -586,27 +593,30 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
     });
   }
   if (lora_here) {
-    f32x4_t tacc[3] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    f32x4_t tacc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     const uint16_t* lb = xs + min(n16, M - 1) * XS + l0 * 64 + par * 16 + h * 8;
-    for (int it0 = 0; it0 < items; it0 += 4) {
-      static_for<4>([&](auto ic) __attribute__((always_inline)) {
-        constexpr int i = decltype(ic)::value;
-        if (it0 + i < items) {
-          const int k = nq == 1 ? it0 + i : (it0 + i) / nq, u = it0 + i - k * nq;
+    by_nq([&](auto nqc) __attribute__((always_inline)) {
+      constexpr int NQ = decltype(nqc)::value, D = kSbLoraTiles;
+      for (int k0 = 0; k0 < nk; k0 += D) {
+        static_for<D>([&](auto dc) __attribute__((always_inline)) {
+          constexpr int d = decltype(dc)::value;
+          const int k = k0 + d;
+          if (k < nk) {
 #pragma unroll
-          for (int s = 0; s < 2; ++s) {
-            const bf16x8_t xa = *reinterpret_cast<const bf16x8_t*>(lb + k * 64 + s * 32), bb = __builtin_bit_cast(bf16x8_t, ab[i][s]);
-            if (u == 0) tacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, bb, tacc[0], 0, 0, 0);
-            else if (u == 1) tacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, bb, tacc[1], 0, 0, 0);
-            else tacc[2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, bb, tacc[2], 0, 0, 0);
+            for (int s = 0; s < 2; ++s) {
+              const bf16x8_t xa = *reinterpret_cast<const bf16x8_t*>(lb + k * 64 + s * 32);
+#pragma unroll
+              for (int u = 0; u < NQ; ++u)
+                tacc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8_t, ab[d * NQ + u][s]), tacc[u], 0, 0, 0);
+            }
           }
-          load_a(it0 + i + 4, ic);
-        }
-      });
-    }
+          load_a(nqc, k + D, dc);
+        });
+      }
+    });
     if (q == 0) {
 #pragma unroll
-      for (int u = 0; u < 3; ++u)
+      for (int u = 0; u < 2; ++u)
         if (u < nq) {
 #pragma unroll
           for (int r = 0; r < kSbMaxRows; ++r) red_t[(wave * kSbMaxRows + r) * 64 + (q0 + u) * 16 + n16] = tacc[u][r];
