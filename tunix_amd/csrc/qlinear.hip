@@ -1512,7 +1512,7 @@ static int num_splits4(int K, int N) {
 
 int qlinear_num_lora_splits(int K, int N);
 int qlinear_num_splits(int K, int N, int M) {
-  if (M > 128) return wide_plan(M, N, K, 0).nsplit;
+  if (M > 128) return wide_plan(M, N, K, 0, 0, 0).nsplit;
   if (four_wave(K, N)) return num_splits4(K, N);
   const int nblocks = (N + 127) / 128;
   const int KT = K / 64;

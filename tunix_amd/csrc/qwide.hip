@@ -485,6 +485,8 @@ __global__ __launch_bounds__(512, MT <= 4 && CT == 4 ? 4 : 1) void qlinear_mfma_
   gemm_block_wide<MT, CT>(a, smem, bx, by, bz);
 }
 
+static int lora_workgroups(const QLinearArgs& a) { return a.a_t ? ((a.M + 31) / 32 * a.n_lora_slices + 7) / 8 * 8 : 0; }
+
 template <int MT, int CT>
 static int launch_wide(hipStream_t st, QLinearArgs a) {
   static const hipError_t attr = hipFuncSetAttribute(
@@ -492,7 +494,7 @@ static int launch_wide(hipStream_t st, QLinearArgs a) {
       (int)wide_lds(MT));
   if (attr != hipSuccess) return TMX_ERR_LAUNCH;
   const int blocks = (a.N + CT * 32 - 1) / (CT * 32);
-  a.lora_wgs = a.a_t ? ((a.M + 31) / 32 * a.n_lora_slices + 7) / 8 * 8 : 0;
+  a.lora_wgs = lora_workgroups(a);
   const int row_blocks = (a.M + MT * 32 - 1) / (MT * 32);
   int S = 8;
   while (row_blocks % S) S >>= 1;  // gcd(row_blocks, 8)
@@ -620,8 +622,14 @@ int moe_rows(hipStream_t st, const MoeArgs& a, int E, bool down) {
 // gate|up 8 x 8, 715 (4 x 4: 840).
 static const int kWideTiles[][2] = {{2, 4}, {3, 4}, {4, 4}, {5, 4}, {6, 4}, {7, 4}, {8, 4}, {4, 8}, {5, 8}, {6, 8}, {7, 8}, {8, 8}};
 
+// The LoRA workgroups of a launch (1 us + 0.25 a k-tile each) come first: where they and the others make more rounds, the last of
+// the others start behind them or share a CU.  Left out of the price, tiles that fill the chip by themselves were chosen: 630 x 2048 x
+// 16384 with rank 16 in 5 x 8 tiles (256 + 24 workgroups) 54.7 us, in 7 x 8 (192 + 24) 51.0; 200 x 4096 x 2048 in 4 slices and 2 x 4
+// tiles (256 + 16) 17.5, in 3 x 4 (192 + 16) 13.4.  Over 16 matrices at 15 row counts with adapters the choice is 0.5 % off the best
+// tile in the mean, 13 % at most (4.9 and 31 % without this), without adapters 0.15 and 9 %.
+
 // What a tile in s slices costs, us; `order`: by the prices that fix the order of the sums.
-static float wide_price(int M, int N, int KT, int mt, int ct, int s, int cus, bool order) {
+static float wide_price(int M, int N, int KT, int mt, int ct, int s, int cus, int lora_wgs, float lora_us, bool order) {
   const long tiles = (long)((M + 32 * mt - 1) / (32 * mt)) * ((N + 32 * ct - 1) / (32 * ct));
   const long n = (tiles * s + cus - 1) / cus;  // workgroups of a CU
   const bool pairs = mt <= 4 && ct == 4;
@@ -631,15 +639,18 @@ static float wide_price(int M, int N, int KT, int mt, int ct, int s, int cus, bo
     return (pairs ? 8.f + (n == 1 ? 1.f : 0.92f) * n * loop : n * (8.f + loop)) + planes;
   }
   const float fixed = ct == 4 ? 3.7f + 0.78f * mt : 5.8f + 0.62f * mt, loop = steps * ((ct == 4 ? 0.4f : 0.56f) + 0.024f * mt * ct);
-  return (pairs || n == 1 ? fixed + n * loop : fixed + 1.12f * n * loop + 0.5f * (n - 1) * fixed) + planes;
+  auto rounds = [&](long k) { return pairs || k == 1 ? fixed + k * loop : fixed + 1.12f * k * loop + 0.5f * (k - 1) * fixed; };
+  const long with = (tiles * s + lora_wgs + cus - 1) / cus;
+  const float more = rounds(with), behind = rounds(n) + (with - n) * lora_us;
+  return (more < behind ? more : behind) + planes;
 }
 
-WidePlan wide_plan(int M, int N, int K, int nsplit) {
+WidePlan wide_plan(int M, int N, int K, int nsplit, int lora_wgs, int lora_kt) {
   const int cus = device_cus(), KT = K >> 6;
   WidePlan best = {8, 8, nsplit > 0 ? nsplit : 1};
   float best_cost = 1e30f;
   auto offer = [&](int mt, int ct, int s, bool order) {
-    const float cost = wide_price(M, N, KT, mt, ct, s, cus, order);
+    const float cost = wide_price(M, N, KT, mt, ct, s, cus, lora_wgs, 1.f + 0.25f * lora_kt, order);
     if (cost < best_cost) { best_cost = cost; best = {mt, ct, s}; }
   };
   for (const auto& t : kWideTiles)
@@ -658,14 +669,14 @@ WidePlan wide_plan(int M, int N, int K, int nsplit) {
 int qwide_lora_launch(hipStream_t st, QLinearArgs a) {
   static_assert(wide_lds(2) >= 8 * 16 * 64 * 4, "the accumulators of the 8 waves meet in LDS");
   if (!a.a_t || !a.sync || a.M > TMX_MAX_FILL_ROWS) return TMX_ERR_ARG;
-  a.lora_wgs = ((a.M + 31) / 32 * a.n_lora_slices + 7) / 8 * 8;
+  a.lora_wgs = lora_workgroups(a);
   hipLaunchKernelGGL((qlinear_mfma_wide_kernel<2, 4>), dim3(a.lora_wgs), dim3(512), wide_lds(2), st, a, 1, 1, 1);
   return check_launch();
 }
 
 int qwide_launch(hipStream_t st, const QLinearArgs& a) {
   if (a.sync && a.M > TMX_MAX_FILL_ROWS) return TMX_ERR_SHAPE;  // the hand-over area has a word per row tile
-  const WidePlan p = wide_plan(a.M, a.N, a.K, a.nsplit);
+  const WidePlan p = wide_plan(a.M, a.N, a.K, a.nsplit, lora_workgroups(a), a.kt_per_lora_split);
 #define TMX_WIDE_CASE(MM, CC) \
   if (p.mt == MM && p.ct == CC) return launch_wide<MM, CC>(st, a);
   TMX_WIDE_CASE(2, 4)

@@ -337,7 +337,7 @@ inline int slice_len(int KT, int s) { return ((KT + s - 1) / s + 3) / 4 * 4; }
 inline bool slices_ok(int KT, int s) { return (KT + slice_len(KT, s) - 1) / slice_len(KT, s) == s; }
 // Projections of more than 128 rows (qwide.hip): mt row tiles x ct column tiles per workgroup, K in nsplit slices
 struct WidePlan { int mt, ct, nsplit; };
-WidePlan wide_plan(int M, int N, int K, int nsplit);  // nsplit 0: its choice
+WidePlan wide_plan(int M, int N, int K, int nsplit, int lora_wgs, int lora_kt);  // nsplit 0: its choice; LoRA workgroups, k-tiles of each
 int qwide_launch(hipStream_t st, const QLinearArgs& a);
 int qwide_lora_launch(hipStream_t st, QLinearArgs a);  // the LoRA workgroups of such a launch by themselves
 // What the LoRA half of a many-rows projection hands over inside its launch.  Two areas of wide_sync_words() words take
