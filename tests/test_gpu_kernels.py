@@ -1255,6 +1255,32 @@ def test_many_rows_projection_steps(M, K, N):
   test_many_rows_projection_tiles(M, K, N)
 
 
+# planes of x . A of 2, 3, 4 and 8 k-tiles, of which a workgroup of the many-rows launch takes one, two or four: every plane is its
+# K-slice's sum, and those behind the last k-tile are zero
+@pytest.mark.parametrize('M,K,N,r', [(129, 640, 256, 8), (300, 4096, 1024, 32), (844, 1152, 320, 24), (200, 4096, 512, 64),
+                                     (333, 8192, 256, 16), (257, 128, 64, 4), (150, 2048, 64, 100)])
+def test_many_rows_lora_planes(M, K, N, r):
+  lib = _lib.lib()
+  g = torch.Generator(device=G.DEV).manual_seed(M + K)
+  rn = lambda *s: torch.randn(*s, generator=g, device=G.DEV)
+  pl = quant.PackedLinear.from_dense([rn(K, N) * 0.02], 64, G.DEV, [(rn(K, r), rn(r, N))], 2.0)
+  x = rn(M, K).to(torch.bfloat16)
+  ns, nl = lib.tmx_qlora_linear_num_splits(M, K, N), lib.tmx_qlora_linear_num_lora_splits(K, N)
+  yp = torch.empty(ns, M, N, device=G.DEV)
+  tp = torch.full((nl, M, 128), 7.0, device=G.DEV)
+  G.call('tmx_qlora_linear_planes', S(), G.p(x), G.p(pl.qweight), G.p(pl.scales), G.p(pl.lora_a_t), G.p(yp), G.p(tp), M, K, N, 64,
+         pl.r_pad, ns)
+  G.sync()
+  a = pl.lora_a_dense().double()
+  assert (tp[:, :, pl.r_pad:] == 7.0).all()
+  got, want = tp[:, :, :pl.r_pad].double(), x.double() @ a
+  assert (got.sum(0) - want).norm() <= 1e-5 * want.norm()
+  step = next(n for n in range(64, K + 64, 64) if -(-K // n) <= nl and (got[0] - x[:, :n].double() @ a[:n]).norm() <= 1e-5 * want.norm())
+  for i in range(nl):
+    part = x[:, i * step:(i + 1) * step].double() @ a[i * step:(i + 1) * step]
+    assert (got[i] - part).norm() <= 1e-5 * want.norm()
+
+
 # one and several K-slices of x . A, one to four column tiles of A, a ragged last row tile
 @pytest.mark.parametrize('M,K,N,r', [(129, 256, 96, 8), (300, 4096, 12288, 16), (161, 5120, 28672, 32), (416, 2048, 16384, 64),
                                      (1000, 4224, 4096, 24)])

@@ -348,7 +348,10 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
   else lora(IC<2>{});
 }
 
-// t = x . A of one row tile (32 rows) over one K-slice.  The 8 waves are column tiles of A (1, 2 or 4) x k-parts; a wave
+__host__ __device__ inline int lora_col_waves(const QLinearArgs& a) { return a.Rpad > 64 ? 4 : a.Rpad >> 5; }
+
+// t = x . A of one row tile (32 rows) over one K-slice (or a.lora_par short ones side by side).  The 8 waves are column tiles of
+// A (1, 2 or 4) x k-parts; a wave
 // reads its x fragments straight from global memory (32 rows, 64 bytes each per pair of loads; the column tiles of a
 // k-part hit the same lines) two k-tiles ahead, the parts meet in LDS.  Every slice leaves its f32 plane; with a
 // hand-over area (a.sync) the last slice of the row tile to arrive adds the planes in slice order and writes the
@@ -358,13 +361,13 @@ __device__ __forceinline__ void gemm_block_wide(const QLinearArgs& a, uint16_t* 
 // them is latency: about 8 us at 256 rows, hidden behind the main workgroups' loop, where a LoRA-only launch and a
 // reduction launch in front of the projection took 14 + 5 us (decode step of 256 sequences, 8 layers: 3.43 -> 3.25 ms).
 __device__ __forceinline__ void wide_lora_block(const QLinearArgs& a, float* red, int id) {
-  const int RT = (a.M + 31) >> 5, rt = id % RT, ks = id / RT;
-  if (ks >= a.n_lora_slices) return;
+  const int PS = a.lora_par, RT = (a.M + 31) >> 5, rt = id % RT, ks0 = id / RT * PS;
+  if (ks0 >= a.n_lora_slices) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, nl = lane & 31;
-  const int KT = a.K >> 6, NT = a.Rpad >> 5, NP = NT > 2 ? 4 : NT, nk = 8 / NP;
-  const int ct = wave % NP, kp = wave / NP;
+  const int KT = a.K >> 6, NT = a.Rpad >> 5, NP = lora_col_waves(a), nk = 8 / NP / PS;
+  const int ct = wave % NP, kp = wave / NP % nk, ks = ks0 + wave / NP / nk;  // (a slice past the last one has no k-tiles)
   const int k0 = ks * a.kt_per_lora_split, k1 = min(k0 + a.kt_per_lora_split, KT);
   if (a.sync_clear && ks == 0 && tid < 2) a.sync_clear[tid * kWideTiles32 + rt] = 0u;  // the next launch's area
 
@@ -418,15 +421,15 @@ __device__ __forceinline__ void wide_lora_block(const QLinearArgs& a, float* red
                                             (row * a.ldt16 + c) * 2, 0, 0x10);
     if (a.t_fin) *reinterpret_cast<f32x4_t*>(a.t_fin + (size_t)row * a.ldt + c) = f32x4_t{bf_lo(lo), bf_hi(lo), bf_lo(hi), bf_hi(hi)};
   };
-  for (int e = tid; e < 32 * quads; e += 512) {
-    const int rl = e / quads, c = (e - rl * quads) * 4, row = rt * 32 + rl;
-    if (row >= a.M) continue;
+  for (int e = tid; e < PS * 32 * quads; e += 512) {
+    const int rs = e / quads, c = (e - rs * quads) * 4, rl = rs & 31, s = rs >> 5, row = rt * 32 + rl, sl = ks0 + s;
+    if (row >= a.M || sl >= a.n_lora_slices) continue;
     const int r = (rl >> 3) * 4 + (rl & 3), ln = ((rl >> 2) & 1) * 32 + (c & 31);
     f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-    for (int p = 0; p < nk; ++p) v += *reinterpret_cast<const f32x4_t*>(red + ((p * NP + (c >> 5)) * 16 + r) * 64 + ln);
+    for (int p = s * nk; p < (s + 1) * nk; ++p) v += *reinterpret_cast<const f32x4_t*>(red + ((p * NP + (c >> 5)) * 16 + r) * 64 + ln);
     if (final_here && a.n_lora_slices == 1) finish(row, c, v);
-    else if (!final_here) *reinterpret_cast<f32x4_t*>(a.t_part + ((size_t)ks * a.M + row) * a.ldt + c) = v;
-    else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), rp, (int)((((size_t)ks * a.M + row) * a.ldt + c) * 4), 0, 0x10);
+    else if (!final_here) *reinterpret_cast<f32x4_t*>(a.t_part + ((size_t)sl * a.M + row) * a.ldt + c) = v;
+    else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), rp, (int)((((size_t)sl * a.M + row) * a.ldt + c) * 4), 0, 0x10);
   }
   if (!final_here) return;
   __builtin_amdgcn_s_waitcnt(0);  // this thread's stores are in memory
@@ -485,7 +488,15 @@ __global__ __launch_bounds__(512, MT <= 4 && CT == 4 ? 4 : 1) void qlinear_mfma_
   gemm_block_wide<MT, CT>(a, smem, bx, by, bz);
 }
 
-static int lora_workgroups(const QLinearArgs& a) { return a.a_t ? ((a.M + 31) / 32 * a.n_lora_slices + 7) / 8 * 8 : 0; }
+// Workgroups of t = x . A, and how many slices each takes: as many as leave every wave a k-tile, where nothing is handed over (the
+// f32 planes of a caller may have slices of 4 k-tiles: 844 x 4096 x 1024 with rank 32 in 432 workgroups of one slice 24.3 us, in 216 of two 16.9).
+static int lora_workgroups(QLinearArgs& a) {
+  a.lora_par = 1;
+  if (!a.a_t) return 0;
+  if (!a.sync)
+    while (8 / lora_col_waves(a) / (2 * a.lora_par) >= a.kt_per_lora_split) a.lora_par *= 2;
+  return ((a.M + 31) / 32 * ((a.n_lora_slices + a.lora_par - 1) / a.lora_par) + 7) / 8 * 8;
+}
 
 template <int MT, int CT>
 static int launch_wide(hipStream_t st, QLinearArgs a) {
@@ -674,7 +685,7 @@ int qwide_lora_launch(hipStream_t st, QLinearArgs a) {
   return check_launch();
 }
 
-int qwide_launch(hipStream_t st, const QLinearArgs& a) {
+int qwide_launch(hipStream_t st, QLinearArgs a) {
   if (a.sync && a.M > TMX_MAX_FILL_ROWS) return TMX_ERR_SHAPE;  // the hand-over area has a word per row tile
   const WidePlan p = wide_plan(a.M, a.N, a.K, a.nsplit, lora_workgroups(a), a.kt_per_lora_split);
 #define TMX_WIDE_CASE(MM, CC) \

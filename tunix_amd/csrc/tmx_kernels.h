@@ -44,6 +44,7 @@ struct QLinearArgs {
   // many-rows kernel: LoRA workgroups in front of the launch; the hand-over area of the next launch, which they
   // clear; the finished t in f32 for a consumer behind the launch [M][ldt]
   int lora_wgs;
+  int lora_par;            // K-slices of x . A that a LoRA workgroup of the many-rows launch takes side by side
   uint32_t* sync_clear;
   float* t_fin;
 };
@@ -338,7 +339,7 @@ inline bool slices_ok(int KT, int s) { return (KT + slice_len(KT, s) - 1) / slic
 // Projections of more than 128 rows (qwide.hip): mt row tiles x ct column tiles per workgroup, K in nsplit slices
 struct WidePlan { int mt, ct, nsplit; };
 WidePlan wide_plan(int M, int N, int K, int nsplit, int lora_wgs, int lora_kt);  // nsplit 0: its choice; LoRA workgroups, k-tiles of each
-int qwide_launch(hipStream_t st, const QLinearArgs& a);
+int qwide_launch(hipStream_t st, QLinearArgs a);
 int qwide_lora_launch(hipStream_t st, QLinearArgs a);  // the LoRA workgroups of such a launch by themselves
 // What the LoRA half of a many-rows projection hands over inside its launch.  Two areas of wide_sync_words() words take
 // turns: a launch uses one, which has to be zero, and clears the other.
