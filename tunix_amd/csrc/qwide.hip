@@ -8,8 +8,9 @@ namespace tmx {
 // A workgroup is 8 waves = CT column tiles of 32 x KW = 8 / CT k-parts over MT row tiles of 32.  A wave multiplies its
 // column tile against all row tiles (16 MT accumulator registers) on the 16 x 16 x 32 MFMA with the weights as A operand,
 // so a lane ends up with four consecutive columns of a row, and a dequantised weight fragment feeds 2 MT MFMAs.
-// What bounds it: at a thousand rows and more the power of the chip.  With every CU at work the clock falls from 2.39 to
-// 1.8 GHz (4096 x 4096 x 28672), and the same launch with zeros for x runs 1.27 times as fast.  Registers only and on
+// What bounds it: at a thousand rows and more the power of the chip, and the schedule for the rest.  With every CU at work the clock
+// falls from 2.39 to 1.8 GHz (4096 x 4096 x 28672: its MFMAs, 16 cycles each, are 0.64 of the launch at that clock), and the same
+// launch with zeros for x runs 1.27 times as fast.  Registers only and on
 // random bf16 the 16 x 16 x 32 MFMA sustains 2.02 PFLOP/s and the 32 x 32 x 16 one 1.77, so the former, although it takes
 // twice the issue slots.  In one round of workgroups it is the schedule: the loop below takes 2.18 us a step of 8 x 8 tiles
 // where its MFMAs alone are 1.71.  Before (32 x 32 x 16, the barrier between two steps, the transfers of a slab in one
