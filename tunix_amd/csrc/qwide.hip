@@ -523,7 +523,7 @@ static int launch_wide(hipStream_t st, QLinearArgs a) {
 // a lane and SwiGLU needs no exchange.  Sums run over K in the order of moe_stream_kernel: the same bits.
 // What bounds it at the 64 rows an expert has in a pass of 1024 tokens (128 experts of 2048 x 768, top-8) is the
 // instructions of the dequantisation (32 us of issue) beside those of the MFMAs: 92 + 63 us per layer, in chunks of 32 rows that
-// dequantised every matrix two to three times 194 + 145 us.  In this form (134 to 150 registers, one workgroup per CU): held to 128
+// dequantised every matrix two to three times 194 + 145 us.  In this form (156 registers, one workgroup per CU): held to 128
 // registers, two per CU, it spills and takes 121 us for gate | up; three or four slab buffers, 101 and 106; chunks
 // of 64 rows 125 (an expert with 65 rows streams its matrices twice).  The list of rows is read in one go by every
 // workgroup, consecutive pairs by consecutive lanes; 16 pairs per lane instead cost 23 us of down's 80.
