@@ -448,6 +448,15 @@ int tmx_decode_steps(const tmx_model_desc* model, const tmx_decode_state* state,
 int tmx_fill_ragged(const tmx_model_desc* model, const tmx_decode_state* state, void* stream, const int32_t* first_col,
                     int width, int n_rows);
 
+/* The same as a scoring pass (state->sampling_mode TMX_SAMPLE_SCORE, state->logprobs set, no logits_out): of sequence s the
+ * columns from first_col[s] to end_col[s] - 1 within the pass, n_rows in all, and the n_head rows among them from column
+ * head_col on through the head (0: none), which writes the log-prob of the token of the next column there.  Both counts are
+ * the caller's.  Serves a learner's batch: padding in front of the prompts is left out, prompt columns take no part in the head,
+ * and of the padding behind a completion, whose rows are all alike (one token at one position that looks at the same
+ * slots), the caller walks the first and repeats its log-prob. */
+int tmx_score_ragged(const tmx_model_desc* model, const tmx_decode_state* state, void* stream, const int32_t* first_col,
+                     const int32_t* end_col, int width, int n_rows, int head_col, int n_head);
+
 /* Some decode kernels hand data from one group of workgroups to another inside a launch (the
  * fused gate | up projection computes its LoRA projection once and passes it on).  The
  * receiving side waits a bounded number of polls; if a wait ever runs out the kernel carries

@@ -941,6 +941,42 @@ def test_scoring_in_one_walk_equals_prompt_and_completion_walks(family, b, p, t)
   assert np.isfinite(got[0]).all() and np.abs(got[0] - got[1]).max() <= (2 if family == 'moe' else 1) * LOGPROB_TOL
 
 
+@pytest.mark.parametrize('one', [256, -1])
+@pytest.mark.parametrize('b,p,t,limit', [(7, 37, 20, 4096), (7, 5, 1, 4096), (7, 1, 40, 4096), (40, 9, 33, 4096), (9, 30, 45, 100), (7, 20, 25, 3)])
+def test_scoring_of_padded_completions_equals_a_walk_of_every_row(one, b, p, t, limit):
+  """Of the padding behind a completion the first row is walked and its log-prob repeated, prompt columns take no part in the
+  head: the log-probs are those of walks that compute every row, in one pass and in several.  Other row counts take other
+  tiles and K-slices, so sums round differently: the tolerance of the log-probs."""
+  cfg = C.TOY
+  model = C.product_model(cfg, C.make_state(cfg, 47, 8, norm_jitter=0.05), 64, 16.0)
+  rng = np.random.default_rng(p * t)
+  prompt = rng.integers(3, cfg.vocab_size, (b, p)).astype(np.int32)
+  comp = rng.integers(3, cfg.vocab_size, (b, t)).astype(np.int32)
+  for i in range(b):
+    prompt[i, :rng.integers(0, p)] = 0
+    comp[i, t - rng.integers(0, t):] = 0
+  comp[1] = 0                     # nothing but padding
+  comp[2, t // 2] = 0             # and some inside
+  prompt[3] = 0                   # no prompt
+  prompt[4] = comp[4] = 0         # no token
+  mask = None
+  if one < 0:                     # masked tails whose tokens differ, or are no padding ids
+    mask = np.concatenate([prompt, comp], 1) != 0
+    mask[5, -(t // 2 + 1):] = mask[6, -(t // 3 + 1):] = False
+    comp[6, -(t // 3 + 1):] = 9
+  got = []
+  for ragged in (True, False):
+    s = _sampler(model, cfg, 96)
+    s.ONE_WALK_ROWS, s.MAX_FILL_ROWS = one, limit
+    s.MAX_ROWS = min(s.MAX_ROWS, limit)
+    if not ragged:
+      s._fill_ragged_ok = lambda: False
+    got.append(s.per_token_logps(prompt, comp, pad_id=0, token_mask=mask))
+  some = [i for i in range(b) if i != 4]  # (a row that sees no slot has no softmax to compare)
+  assert got[0].shape == (b, t) and np.isfinite(got[0][some]).all()
+  assert np.abs(got[0] - got[1])[some].max() <= LOGPROB_TOL
+
+
 def test_scoring_does_not_read_the_embedding_of_padding_in_front_of_prompts():
   """Padding in front of a prompt is not walked, or walked as another token: whatever its embedding holds, the log-probs are the
   same.  In one walk of prompt and completion and in two."""

@@ -47,6 +47,7 @@ SIGNATURES = {
     'tmx_moe_experts': [vp, vp, ci, vp, vp, vp, ci, ci, ci, ci, ci, ci, ci, vp, ci],
     'tmx_decode_steps': [vp, vp, vp, ci, ci],
     'tmx_fill_ragged': [vp, vp, vp, vp, ci, ci],
+    'tmx_score_ragged': [vp, vp, vp, vp, vp, ci, ci, ci, ci],
     'tmx_decode_steps_graph': [vp, vp, vp, ci, ci],
     'tmx_decode_steps_profiled': [vp, vp, vp, ci, ci, vp, vp],
     'tmx_decode_status': [vp, vp, vp],

@@ -37,6 +37,8 @@ struct Workspace {
   uint16_t* head_x;  // the many-rows head's copy of its rows: a buffer that is free by then where one is large enough
   int2* row_map;  // ragged pass: row -> (sequence, column), and the sequences' runs of rows
   int4* seg;
+  int2* head_map;  // ragged scoring pass: (sequence, column) of the head's rows, and their rows in the pass
+  int32_t* head_src;
   size_t total;
 };
 
@@ -142,6 +144,8 @@ static Workspace carve(const tmx_model_desc* m, int B, int C, char* base) {
   }
   w.row_map = (int2*)take((size_t)B * 8);
   w.seg = (int4*)take((size_t)B * 16);
+  w.head_map = (int2*)take((size_t)B * 8);
+  w.head_src = (int32_t*)take((size_t)B * 4);
   w.total = off;
   return w;
 }
@@ -175,11 +179,14 @@ extern "C" size_t tmx_decode_workspace_bytes(const tmx_model_desc* m, int batch,
   return carve(m, batch, cache_size, nullptr).total;
 }
 
-// A cache-fill pass that leaves out the padding in front of the prompts: `width` columns of every sequence, of each
-// only those from first_col on, n_rows rows in all.
+// A cache-fill or scoring pass that leaves out rows nobody needs: `width` columns of every sequence, of each only those from
+// first_col on and before end_col (null: to the last), n_rows rows in all; a scoring pass takes the n_head of them from
+// column head_col on to the head.
 struct Ragged {
   const int32_t* first_col;
   int width, n_rows;
+  const int32_t* end_col;
+  int head_col, n_head;
 };
 
 static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s, void* stream,
@@ -290,7 +297,13 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       wide_turn = 0;
     }
     if (rg) {
-      rc = plan_rows(st, rg->first_col, s->step, NSEQ, rg->width, B, L, w.row_map, w.seg);
+      RowPlan p = {};
+      p.first_col = rg->first_col; p.end_col = rg->end_col; p.step = s->step;
+      p.batch = NSEQ; p.width = rg->width; p.n_rows = B; p.buf_len = L;
+      p.row_map = w.row_map; p.seg = w.seg;
+      p.head_col = rg->head_col; p.n_head = sample ? rg->n_head : 0;
+      p.head_map = w.head_map; p.head_src = w.head_src;
+      rc = plan_rows(st, p);
       if (rc != TMX_OK) return rc;
     }
     {  // embedding gather + first input norm + this step's RoPE table
@@ -561,6 +574,15 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       a.w = (const uint16_t*)m->head;
       a.w_tiles = (const uint16_t*)m->head_tiles;
       a.M = B; a.D = D; a.V = m->vocab_size;
+      if (rg) {
+        a.M = rg->n_head;
+        a.row_map = w.head_map;
+        if (a.M < B) {  // (the residual stream has been read for the last time)
+          rc = gather_rows(st, w.xn, w.head_src, w.x, a.M, D);
+          if (rc != TMX_OK) return rc;
+          a.x = w.x;
+        }
+      }
       a.mode = s->sampling_mode;
       a.temperature = s->temperature;
       a.k0 = s->seed_hi; a.k1 = s->seed_lo;
@@ -607,8 +629,20 @@ extern "C" int tmx_fill_ragged(const tmx_model_desc* m, const tmx_decode_state* 
   if (!m || !s || !first_col) return TMX_ERR_ARG;
   if (width <= 0 || n_rows <= 0 || s->batch <= 0 || (long)n_rows > (long)width * s->batch) return TMX_ERR_SHAPE;
   if (m->num_kv_heads <= 0 || !attn_fill_ok(m->num_heads, m->num_kv_heads, m->head_dim, s->cache_size)) return TMX_ERR_UNSUPPORTED;
-  const Ragged rg = {first_col, width, n_rows};
+  const Ragged rg = {first_col, width, n_rows, nullptr, 0, 0};
   return decode_steps_impl(m, s, stream, 1, 0, nullptr, &rg);
+}
+
+extern "C" int tmx_score_ragged(const tmx_model_desc* m, const tmx_decode_state* s, void* stream, const int32_t* first_col,
+                                const int32_t* end_col, int width, int n_rows, int head_col, int n_head) {
+  if (!m || !s || !first_col || !end_col || !s->logprobs) return TMX_ERR_ARG;
+  if (s->sampling_mode != TMX_SAMPLE_SCORE) return TMX_ERR_ARG;
+  if (width <= 0 || n_rows <= 0 || s->batch <= 0 || (long)n_rows > (long)width * s->batch) return TMX_ERR_SHAPE;
+  if (head_col < 0 || n_head < 0 || n_head > n_rows) return TMX_ERR_SHAPE;
+  if (s->logits_out) return TMX_ERR_UNSUPPORTED;
+  if (m->num_kv_heads <= 0 || !attn_fill_ok(m->num_heads, m->num_kv_heads, m->head_dim, s->cache_size)) return TMX_ERR_UNSUPPORTED;
+  const Ragged rg = {first_col, width, n_rows, end_col, head_col, n_head};
+  return decode_steps_impl(m, s, stream, 1, n_head > 0, nullptr, &rg);
 }
 
 extern "C" int tmx_decode_status(const tmx_model_desc* m, const tmx_decode_state* s, void* stream) {

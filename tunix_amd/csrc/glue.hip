@@ -817,57 +817,80 @@ int advance_step(hipStream_t st, int32_t* step, int by) {
 // One workgroup: the sequences' row counts, their running sum (1024 sequences at a time), then the rows themselves by
 // binary search.  A few microseconds per pass of thousands of rows, instead of a copy from the host.
 constexpr int kPlanThreads = 1024;
-__global__ __launch_bounds__(kPlanThreads) void plan_rows_kernel(const int32_t* first_col, const int32_t* step, int batch,
-                                                                 int width, int n_rows, int buf_len, int2* row_map,
-                                                                 int4* seg, int n_seg) {
-  __shared__ int wave_n[16], wave_e[16];
-  __shared__ int e_row[TMX_MAX_FILL_ROWS];   // first row of every entry
+__global__ __launch_bounds__(kPlanThreads) void plan_rows_kernel(RowPlan p) {
+  __shared__ int wave_n[16], wave_e[16], wave_h[16];
+  __shared__ int e_row[TMX_MAX_FILL_ROWS], e_head[TMX_MAX_FILL_ROWS];  // first row of every entry, in the pass and among the head's
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int c0 = min(max(*step, 0), buf_len - 1), c1 = min(c0 + width, buf_len);
-  int rows = 0, entries = 0;
-  for (int s0 = 0; s0 < batch; s0 += kPlanThreads) {
+  const int c0 = min(max(*p.step, 0), p.buf_len - 1), c1 = min(c0 + p.width, p.buf_len);
+  int rows = 0, entries = 0, heads = 0;
+  for (int s0 = 0; s0 < p.batch; s0 += kPlanThreads) {
     const int s = s0 + tid;
-    const int first = s < batch ? max(first_col[s], c0) : c1;
-    const int n = max(c1 - first, 0);
-    int pn = n, pe = n > 0 ? 1 : 0;  // inclusive sums over the wave
+    const int first = s < p.batch ? max(p.first_col[s], c0) : c1;
+    const int end = s < p.batch && p.end_col ? min(p.end_col[s], c1) : c1;
+    const int n = max(end - first, 0), nh = p.n_head > 0 ? max(end - max(first, p.head_col), 0) : 0;
+    int pn = n, pe = n > 0 ? 1 : 0, ph = nh;  // inclusive sums over the wave
     for (int o = 1; o < 64; o <<= 1) {
-      const int an = __shfl_up(pn, o, 64), ae = __shfl_up(pe, o, 64);
-      if (lane >= o) { pn += an; pe += ae; }
+      const int an = __shfl_up(pn, o, 64), ae = __shfl_up(pe, o, 64), ah = __shfl_up(ph, o, 64);
+      if (lane >= o) { pn += an; pe += ae; ph += ah; }
     }
-    if (lane == 63) { wave_n[wave] = pn; wave_e[wave] = pe; }
+    if (lane == 63) { wave_n[wave] = pn; wave_e[wave] = pe; wave_h[wave] = ph; }
     __syncthreads();
-    int row0 = rows + pn - n, e = entries + pe - 1;
-    for (int w = 0; w < wave; ++w) { row0 += wave_n[w]; e += wave_e[w]; }
+    int row0 = rows + pn - n, e = entries + pe - 1, head0 = heads + ph - nh;
+    for (int w = 0; w < wave; ++w) { row0 += wave_n[w]; e += wave_e[w]; head0 += wave_h[w]; }
     // (a caller whose n_rows is short of the real count gets its first rows)
-    if (n > 0 && row0 < n_rows && e < n_seg) {
-      seg[e] = make_int4(s, row0, min(n, n_rows - row0), first);
+    if (n > 0 && row0 < p.n_rows && e < p.n_seg) {
+      p.seg[e] = make_int4(s, row0, min(n, p.n_rows - row0), first);
       e_row[e] = row0;
+      e_head[e] = head0;
     }
-    for (int w = 0; w < 16; ++w) { rows += wave_n[w]; entries += wave_e[w]; }
+    for (int w = 0; w < 16; ++w) { rows += wave_n[w]; entries += wave_e[w]; heads += wave_h[w]; }
     __syncthreads();
   }
-  entries = min(entries, n_seg);
-  for (int e = entries + tid; e < n_seg; e += kPlanThreads) seg[e] = make_int4(0, 0, 0, 0);
+  entries = min(entries, p.n_seg);
+  for (int e = entries + tid; e < p.n_seg; e += kPlanThreads) p.seg[e] = make_int4(0, 0, 0, 0);
   __threadfence_block();
   __syncthreads();
-  for (int m = tid; m < n_rows; m += kPlanThreads) {
-    if (entries == 0) { row_map[m] = make_int2(0, c0); continue; }
+  auto entry_of = [&](const int* begin, int i) {  // the last one that begins at or before i
     int lo = 0, hi = entries;
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
-      if (m >= e_row[mid]) lo = mid;
+      if (i >= begin[mid]) lo = mid;
       else hi = mid;
     }
-    const int4 g = seg[lo];
-    row_map[m] = make_int2(g.x, g.w + min(m - g.y, g.z - 1));  // rows past the count repeat the last one
+    return lo;
+  };
+  for (int m = tid; m < p.n_rows; m += kPlanThreads) {
+    if (entries == 0) { p.row_map[m] = make_int2(0, c0); continue; }
+    const int4 g = p.seg[entry_of(e_row, m)];
+    p.row_map[m] = make_int2(g.x, g.w + min(m - g.y, g.z - 1));  // rows past the count repeat the last one
+  }
+  for (int i = tid; i < p.n_head; i += kPlanThreads) {
+    if (entries == 0) { p.head_map[i] = make_int2(0, c0); p.head_src[i] = 0; continue; }
+    const int e = entry_of(e_head, i);
+    const int4 g = p.seg[e];
+    const int at = min(max(p.head_col - g.w, 0) + i - e_head[e], g.z - 1);  // row of the sequence in this pass
+    p.head_map[i] = make_int2(g.x, g.w + at);
+    p.head_src[i] = g.y + at;
   }
 }
 
-int plan_rows(hipStream_t st, const int32_t* first_col, const int32_t* step, int batch, int width, int n_rows,
-              int buf_len, int2* row_map, int4* seg) {
-  if (batch <= 0 || width <= 0 || n_rows <= 0 || n_rows > TMX_MAX_FILL_ROWS || buf_len <= 0) return TMX_ERR_SHAPE;
-  hipLaunchKernelGGL(plan_rows_kernel, dim3(1), dim3(kPlanThreads), 0, st, first_col, step, batch, width, n_rows, buf_len,
-                     row_map, seg, batch < n_rows ? batch : n_rows);
+int plan_rows(hipStream_t st, RowPlan p) {
+  if (p.batch <= 0 || p.width <= 0 || p.n_rows <= 0 || p.n_rows > TMX_MAX_FILL_ROWS || p.buf_len <= 0) return TMX_ERR_SHAPE;
+  if (p.n_head < 0 || p.n_head > p.n_rows || (p.n_head && (!p.head_map || !p.head_src))) return TMX_ERR_ARG;
+  p.n_seg = p.batch < p.n_rows ? p.batch : p.n_rows;
+  hipLaunchKernelGGL(plan_rows_kernel, dim3(1), dim3(kPlanThreads), 0, st, p);
+  return check_launch();
+}
+
+__global__ __launch_bounds__(256) void gather_rows_kernel(const uint16_t* x, const int32_t* src, uint16_t* out, int D) {
+  const uint4* from = reinterpret_cast<const uint4*>(x + (size_t)src[blockIdx.x] * D);
+  uint4* to = reinterpret_cast<uint4*>(out + (size_t)blockIdx.x * D);
+  for (int c = threadIdx.x; c < D >> 3; c += 256) to[c] = from[c];
+}
+
+int gather_rows(hipStream_t st, const uint16_t* x, const int32_t* src, uint16_t* out, int n, int D) {
+  if (n <= 0 || D <= 0 || D % 8) return TMX_ERR_SHAPE;
+  hipLaunchKernelGGL(gather_rows_kernel, dim3(n), dim3(256), 0, st, x, src, out, D);
   return check_launch();
 }
 

@@ -90,8 +90,8 @@ __device__ __forceinline__ void head_tile_stats(const HeadArgs& a, const f32x16_
 // The given next token of sequence row `row` of this launch (scoring), or -1.
 __device__ __forceinline__ int head_target(const HeadArgs& a, int row) {
   if (a.mode != TMX_SAMPLE_SCORE || row >= a.M) return -1;
-  const int tpp = a.tpp > 0 ? a.tpp : 1, prow = a.row_base + row;  // row of the pass
-  return a.token_buffer[(size_t)(prow / tpp) * a.buf_len + min(*a.step + prow % tpp + 1, a.buf_len - 1)];
+  const int2 at = score_row(a, a.row_base + row);
+  return a.token_buffer[(size_t)at.x * a.buf_len + min(at.y + 1, a.buf_len - 1)];
 }
 
 // The other half-wave holds the other 16 vocabulary rows of the same sequence; one half stores the result.
@@ -426,12 +426,10 @@ __global__ __launch_bounds__(256) void head_finalize_kernel(HeadArgs a) {
       best_merge(best, o);
     }
     if (a.mode == TMX_SAMPLE_SCORE) {  // teacher forcing: the token stays, only its log-prob is written
-      const int tpp = a.tpp > 0 ? a.tpp : 1;
-      const int prow = a.row_base + row;
+      const int2 at = score_row(a, a.row_base + row);
       // selective_log_softmax: logit - logsumexp, with logsumexp = max + log(sum exp(z - max))
-      const int step = *a.step, scol = step + prow % tpp + 1;
-      if (a.logprobs && scol < a.buf_len)
-        a.logprobs[(size_t)(prow / tpp) * a.buf_len + scol] = best.z - (mx + logf(se));
+      const int step = *a.step, scol = at.y + 1;
+      if (a.logprobs && scol < a.buf_len) a.logprobs[(size_t)at.x * a.buf_len + scol] = best.z - (mx + logf(se));
       finalize_advance(a, step);
       return;
     }
@@ -587,8 +585,8 @@ __global__ __launch_bounds__(512, 1) void head_wide_kernel(HeadArgs a, int tok_b
   constexpr bool score = MODE == TMX_SAMPLE_SCORE, sampling = MODE == TMX_SAMPLE_TOP_P;
   uint32_t key0 = 0, key1 = 0;
   if (sampling) threefry2x32(a.k0, a.k1, 0u, (uint32_t)*a.step, key0, key1);
-  const int tpp = a.tpp > 0 ? a.tpp : 1;
-  const int target = score ? a.token_buffer[(size_t)(tok_l / tpp) * a.buf_len + min(*a.step + tok_l % tpp + 1, a.buf_len - 1)] : -1;
+  const int2 at = score ? score_row(a, tok_l) : make_int2(0, 0);
+  const int target = score ? a.token_buffer[(size_t)at.x * a.buf_len + min(at.y + 1, a.buf_len - 1)] : -1;
   float mx = kNegBig, se = 0.f;
   Best best = {-INFINITY, -INFINITY, 0x7FFFFFFF};
   uint64_t packed = 0;  // sorting branch: the 16-bit keys of four consecutive vocabulary rows

@@ -211,6 +211,7 @@ struct HeadArgs {
   int buf_len;
   int tpp;  // tokens per pass (0: 1), score mode only: row m is sequence m / tpp at column *step + m % tpp
   int row_base;  // score mode: x holds rows row_base .. row_base + M - 1 of the pass (chunks of <= 128 rows)
+  const int2* row_map;  // score mode, ragged pass: (sequence, column) of row m, replaces step and tpp (null: none)
   int32_t* advance;    // the step counter, if the finalize launch moves it on; `arrived` counts its workgroups (zero before and after)
   uint32_t* arrived;
   int row_off;   // set by head_logits when it splits the rows over two launches: x, logits_out, sort_keys and the
@@ -296,10 +297,28 @@ int row_norm(hipStream_t st, const RowNormArgs& a, int M);
 int rope_kvwrite(hipStream_t st, const RopeArgs& a, int B);
 int swiglu(hipStream_t st, const SwigluArgs& a, int M);
 int advance_step(hipStream_t st, int32_t* step, int by);
-// Rows of a ragged pass over columns *step .. *step + width - 1: those from first_col[s] on, sequence by sequence.
-// row_map [n_rows], seg [min(batch, n_rows)] (see AttnArgs); n_rows is the caller's count of those rows.
-int plan_rows(hipStream_t st, const int32_t* first_col, const int32_t* step, int batch, int width, int n_rows,
-              int buf_len, int2* row_map, int4* seg);
+// Rows of a ragged pass over columns *step .. *step + width - 1: those from first_col[s] to end_col[s] - 1 (null: to the
+// last), sequence by sequence.  row_map [n_rows], seg [min(batch, n_rows)] (see AttnArgs); n_rows is the caller's count of
+// those rows.  With n_head > 0 also the n_head of them from column head_col on: head_map like row_map, head_src their rows.
+struct RowPlan {
+  const int32_t *first_col, *end_col, *step;
+  int batch, width, n_rows, buf_len;
+  int2* row_map;
+  int4* seg;
+  int n_seg;  // set by plan_rows
+  int head_col, n_head;
+  int2* head_map;
+  int32_t* head_src;
+};
+int plan_rows(hipStream_t st, RowPlan p);
+// out[i] = x[src[i]], rows of D values (D % 8 == 0)
+int gather_rows(hipStream_t st, const uint16_t* x, const int32_t* src, uint16_t* out, int n, int D);
+// The (sequence, column) of row m of a scoring pass, whose next token is looked for.
+__device__ __forceinline__ int2 score_row(const HeadArgs& a, int m) {
+  if (a.row_map) return a.row_map[m];
+  const int tpp = a.tpp > 0 ? a.tpp : 1;
+  return make_int2(m / tpp, *a.step + m % tpp);
+}
 int empty_launch(hipStream_t st);  // measurement aid: a kernel that does nothing
 int gqa_decode(hipStream_t st, AttnArgs a, int H);
 bool attn_fill_ok(int N, int Kh, int H, int C);  // shapes of the kernel that serves ragged passes

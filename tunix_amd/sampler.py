@@ -362,6 +362,16 @@ class Sampler:
         n_tokens -= n_lead
         st['fresh'] = False
     passes = 0
+    if sample and 'score_end' in st and n_tokens > 0 and self._fill_ragged_ok():
+      col = 0 if st.get('fresh') else st['score_col']
+      st['fresh'] = False
+      for width, rows in self._fill_passes(st['score_first'], col, n_tokens, st['score_end']):
+        self._run_score(st, col, width, rows)
+        col += width
+        passes += 1
+        if passes % self.MAX_PASSES_IN_FLIGHT == 0:
+          torch.cuda.current_stream().synchronize()
+      return
     if not sample and n_tokens > 0 and self._fill_ragged_ok():
       col = 0 if st.get('fresh') else int(st['step'].item())
       st['fresh'] = False
@@ -387,12 +397,13 @@ class Sampler:
         # thousands of short passes otherwise leaves tens of thousands of dispatches pending at once
         torch.cuda.current_stream().synchronize()
 
-  def _fill_passes(self, first, col, n_tokens):
+  def _fill_passes(self, first, col, n_tokens, ends=None):
     """(columns, rows) of the passes of a cache fill over columns col .. col + n_tokens - 1, where sequence s starts at
-    column first[s]: as few passes as the row limit allows, of about equally many rows each (a pass of few rows leaves
-    most of the chip idle), at least one column."""
+    column first[s] and ends before ends[s] (None: at the last): as few passes as the row limit allows, of about equally
+    many rows each (a pass of few rows leaves most of the chip idle), at least one column."""
     end = col + n_tokens
-    rows_upto = lambda c: int(np.maximum(c - np.maximum(first, col), 0).sum())
+    last = end if ends is None else np.minimum(ends, end)
+    rows_upto = lambda c: int(np.maximum(np.minimum(c, last) - np.maximum(first, col), 0).sum())
     total, limit = rows_upto(end), self._fill_rows()
     if total <= limit:
       yield n_tokens, total
@@ -425,6 +436,24 @@ class Sampler:
     rc = self._lib.tmx_fill_ragged(ctypes.byref(self._transformer.desc()), ctypes.byref(cs), _lib.stream(),
                                    st['first_col'].data_ptr(), width, rows)
     _lib.check(rc, 'tmx_fill_ragged')
+
+  def _run_score(self, st, col, width, rows):
+    """One pass of a scoring walk: `rows` rows over the columns col .. col + width - 1."""
+    first, end = (np.clip(st[k], col, col + width) for k in ('score_first', 'score_end'))
+    n_head = int(np.maximum(end - np.maximum(first, st['score_col']), 0).sum())
+    if rows == 0:
+      st['step'].add_(width)
+      return
+    if rows == n_head == width * st['token_buffer'].shape[0] and width >= self.MIN_BLOCK_TOKENS:
+      self.run_steps(st, 1, sample=True, tokens_per_pass=width)  # nothing to leave out
+      return
+    if st['score_span'] is None:
+      st['score_span'] = torch.from_numpy(np.stack([st['score_first'], st['score_end']])).to(self._transformer.device)
+    cs = self._c_state(st, 1, rows)
+    rc = self._lib.tmx_score_ragged(ctypes.byref(self._transformer.desc()), ctypes.byref(cs), _lib.stream(),
+                                    st['score_span'][0].data_ptr(), st['score_span'][1].data_ptr(), width, rows, st['score_col'],
+                                    n_head)
+    _lib.check(rc, 'tmx_score_ragged')
 
   def _walk_group_leaders(self, st, n):
     """Cache fill over the first n columns, which every group of st['share_group'] consecutive rows has in
@@ -517,14 +546,28 @@ class Sampler:
       st['share_group'], st['share_len'], st['share_common'] = share
     st['positions'] = torch.from_numpy(utils.build_positions_from_mask(valid).astype(np.int32)).to(dev)
     st['sampling_mode'] = 'score'
+    # What a scoring walk computes of a row: from its first token (at the latest the prompt's last column) up to the first of
+    # the equal masked tokens it ends with.  The rows of the others have the same token, position and visible slots: the log-probs
+    # behind it repeat its own.  A row with no token at all has no visible slot, and is walked whole.  Completions of half to all
+    # of their columns, prompts likewise: 16 x (256 + 512) on 8 layers of the 8B shape 46.0 -> 39.5 ms, 5 x (37 + 90) on the 1B
+    # shape 3.57 -> 3.12 ms; where nothing is padded the passes are those over all columns.
+    same = (ids == ids[:, -1:]) & ~valid
+    tail = total - np.logical_and.accumulate(same[:, ::-1], axis=1).sum(axis=1)
+    tail = np.where(valid.any(axis=1), np.maximum(tail, p - 1), total)
+    st['score_col'], st['score_span'] = p - 1, None
+    st['score_first'] = np.minimum(first, p - 1).astype(np.int32)
+    st['score_end'] = np.minimum(tail + 1, total - 1).astype(np.int32)
     if st['share_group'] == 1 and self._one_walk(b, p, t):
-      # prompt columns are scored too, and their scores left out
+      # prompt columns are scored too where the walk leaves nothing out, and their scores left out
       self.walk(st, total - 1, sample=True)
     else:
       self.walk(st, p - 1)
       self.walk(st, t, sample=True)
     self.check_device_status(st)
-    return st['logprobs'][:, p:p + t].cpu().numpy()
+    logps = st['logprobs'][:, p:p + t].cpu().numpy()
+    if self._fill_ragged_ok():
+      return np.take_along_axis(logps, np.minimum(np.arange(t), (st['score_end'] - p)[:, None]), axis=1)
+    return logps
 
   # -- the call ---------------------------------------------------------------
   def __call__(self, input_strings=None, max_generation_steps=0, max_prompt_length=None, echo=False,
