@@ -416,8 +416,8 @@ typedef struct {
                               sequences whose cache slots [0, share_len) and input_mask entries are identical
                               (the samples of one prompt); one-token decode steps then read those slots once
                               per group (see tmx_gqa_decode_attention_shared).  Ignored where the shared walk
-                              does not apply (more than 128 sequences, batch % g != 0, the 1..4-row path,
-                              tokens_per_pass > 1) */
+                              does not apply or every row by itself is faster (batch % g != 0, the 1..4-row path,
+                              tokens_per_pass > 1, short prompts) */
   int share_len;
 } tmx_decode_state;
 

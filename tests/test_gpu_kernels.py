@@ -520,6 +520,17 @@ def test_gqa_decode_attention_with_shared_prompt_slots(B, N, Kh, H, C, step, gs,
   assert lib.tmx_gqa_decode_attention_shared(S(), 1, 1, 1, 1, 1, 1, C, 1, 1, B + 1, N, Kh, H, C, gs, sl) == -4
 
 
+# Groups walked by one workgroup, shared slots and every row's own (few slots behind the prompt): one and several splits, the
+# last own block of 1 and of 32 slots, none yet, a step inside the shared slots, more rows than a query block, every group width
+@pytest.mark.parametrize('B,N,Kh,H,C,step,gs,sl', [
+    (32, 32, 8, 128, 320, 288, 8, 256), (32, 32, 8, 128, 320, 287, 8, 256), (32, 32, 8, 128, 320, 319, 8, 256),
+    (32, 32, 8, 128, 320, 255, 8, 256), (32, 32, 8, 128, 320, 100, 8, 256), (120, 32, 8, 128, 128, 101, 6, 96),
+    (96, 16, 8, 64, 200, 180, 24, 150), (48, 32, 4, 128, 160, 159, 6, 64), (40, 8, 8, 128, 160, 140, 40, 96),
+    (6, 32, 8, 64, 600, 550, 3, 512), (128, 8, 4, 128, 96, 70, 2, 40)])
+def test_gqa_group_walk(B, N, Kh, H, C, step, gs, sl):
+  test_gqa_decode_attention_with_shared_prompt_slots(B, N, Kh, H, C, step, gs, sl)
+
+
 @pytest.mark.parametrize('nseq,T,N,Kh,H,C,step', [
     (2, 40, 4, 4, 64, 64, 3), (3, 9, 8, 2, 64, 96, 50), (2, 33, 32, 8, 128, 300, 200), (1, 64, 8, 1, 128, 128, 0),
     (2, 5, 16, 8, 128, 96, 60), (1, 128, 4, 4, 128, 200, 31), (2, 3, 8, 4, 64, 64, 20),

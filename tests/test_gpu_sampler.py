@@ -267,6 +267,34 @@ def test_samples_of_one_prompt_share_its_cache_rows_and_match_oracle():
   assert np.abs(runs[True] - runs[False]).max() <= 1e-2
 
 
+def test_many_samples_of_a_prompt_share_its_cache_rows():
+  """17 prompts of 230 tokens x 8 samples, more rows than there is room for parts: one workgroup per group and kv head walks
+  the shared slots and all rows' own.  Logits are those of rows that walk their caches by themselves."""
+  cfg = OM.Config('llama3', 2, 512, 256, 512, 16, 64, 8, norm_eps=1e-5)
+  model = C.product_model(cfg, C.make_state(cfg, 31, 8, norm_jitter=0.05), 64, 16.0)
+  rng = np.random.default_rng(12)
+  ids = np.repeat(rng.integers(3, 512, (17, 230)), 8, axis=0).astype(np.int32)
+  toks = torch.from_numpy(rng.integers(3, 512, (136, 5)).astype(np.int32)).cuda()
+  runs = {}
+  for share in (True, False):
+    s = _sampler(model, cfg, 240)
+    s.share_prompt_kv = share
+    s.eos_ids = np.array([-1])
+    st = s.init_sample_state(ids, 235, True, None, 0.0, None, None, 0)
+    assert (st['share_group'], st['share_len']) == ((8, 224) if share else (1, 0))
+    s.walk(st, 229)
+    if share:  # the group's first sequence alone is read there
+      st['cache'].view(2, 2, 17, 8, 240, 8, 64)[:, :, :, 1:, :224] = float('nan')
+    steps = []
+    for step in range(5):
+      s.run_steps(st, 1, sample=True)
+      steps.append(st['logits'].clone())
+      st['token_buffer'][:, 230 + step] = toks[:, step]
+    s.check_device_status(st)
+    runs[share] = torch.stack(steps)
+  assert torch.isfinite(runs[True]).all() and (runs[True] - runs[False]).abs().max() <= 1e-2
+
+
 def test_temperature_sampling_follows_the_threefry_schedule():
   """Every generated token equals categorical(fold_in(PRNGKey(seed), decoding_step), logits / T)
   evaluated on the kernel's own logits, with decoding_step = P - 1, P, ... as in the reference

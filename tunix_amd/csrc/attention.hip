@@ -19,6 +19,7 @@
 namespace tmx {
 
 constexpr int kMaxPrefixSplits = 4;  // splits of the slots that a group of sequences shares
+constexpr int kMaxGroupSplits = 8;   // the same where the group's workgroups walk its rows' own slots too
 
 // waves per workgroup: fewer for wide groups so the merge buffers stay under 64 KiB
 template <int G>
@@ -263,9 +264,10 @@ struct TileJob {
   int split, nsp;  // this workgroup takes split `split` of nsp splits of the blocks of 32 positions
   int part;        // index of the part it writes when a row has several (nparts > 1)
   int nparts;
+  int own;         // OWN: behind the walk's positions come slots pend .. pend + own - 1 of every query row, from its own cache
 };
 
-template <int H, int G>
+template <int H, int G, bool OWN = false>
 __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& lds, const int kvh, const TileJob j) {
   constexpr int KS = H / 16;        // MFMA k-steps of the score product
   constexpr int CPR = H / 8;        // 16-byte chunks per cache row
@@ -276,7 +278,8 @@ __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& l
   const int h = lane >> 5, qi = lane & 31;
   const int lead = j.kv_row;
   const int plen = j.pend - j.pbeg;  // positions are counted from pbeg below
-  const int nblk = plen > 0 ? (plen + 31) >> 5 : 0;
+  const int nlead = plen > 0 ? (plen + 31) >> 5 : 0, nown = OWN && j.own > 0 ? (j.own + 31) >> 5 : 0;
+  const int nblk = nlead + nown * j.nrows;
   const int bps = (nblk + j.nsp - 1) / j.nsp;
   const int b_end = min((j.split + 1) * bps, nblk);
 
@@ -292,33 +295,47 @@ __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& l
 
   const uint32_t row_bytes = (uint32_t)a.Kh * H * 2;
   const uint32_t span = ((uint32_t)(a.C - 1) * a.Kh + 1) * H * 2;  // rows past the cache read zero
-  const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.kcache + ((size_t)lead * a.C * a.Kh + kvh) * H, span);
-  const __amdgpu_buffer_rsrc_t rv = make_rsrc(a.vcache + ((size_t)lead * a.C * a.Kh + kvh) * H, span);
+  // Where block blk lies: cache row, first slot, slots of the walk from there on, and the query row whose own it is
+  struct Place { int kv, pos, len, own_of; };
+  auto place = [&](int blk) __attribute__((always_inline)) {
+    if (!OWN || blk < nlead) return Place{lead, j.pbeg + blk * 32, plen - blk * 32, -1};
+    const int i = __builtin_amdgcn_readfirstlane((blk - nlead) / nown), k = blk - nlead - i * nown;
+    return Place{j.row0 + i, j.pend + k * 32, j.own - k * 32, i};
+  };
+  auto cache_of = [&](const uint16_t* cache, int row) __attribute__((always_inline)) {
+    return make_rsrc(cache + ((size_t)row * a.C * a.Kh + kvh) * H, span);
+  };
+  const __amdgpu_buffer_rsrc_t rk_lead = cache_of(a.kcache, lead), rv_lead = cache_of(a.vcache, lead);
   uint16_t* vt = reinterpret_cast<uint16_t*>(lds.tiles) + wave * 32 * H;
   // V tile transfer: load i moves rows i RPD .. i RPD + RPD - 1 of the block, the 16-byte chunks of row r
   // XOR-swizzled by r % CPR.  Row i RPD + lane / CPR has r % CPR = (i RPD) % CPR ^ lane / CPR, so the per-lane
   // part of the swizzle is one word and the rest a constant per load; the offsets are formed at the transfer
   // (kept in registers over the loop they would be spilled)
   const int vrow = (lane / CPR) * row_bytes, vswz = (lane % CPR) ^ (lane / CPR);
-  auto dma_v = [&](int blk) __attribute__((always_inline)) {
+  // OWN: a row has few slots of its own, so most of its last block lies behind them; the transfers there repeat the last one
+  auto dma_v = [&](const Place& p) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rv = OWN ? cache_of(a.vcache, p.kv) : rv_lead;
     int sw = vswz;
     asm volatile("" : "+v"(sw));
 #pragma unroll
-    for (int i = 0; i < NLD; ++i)
-      load_row_to_lds(rv, vt + i * RPD * H, vrow + ((sw ^ ((i * RPD) % CPR)) << 4), (j.pbeg + blk * 32 + i * RPD) * row_bytes);
+    for (int i = 0; i < NLD; ++i) {
+      const int r0 = OWN ? min(i * RPD, (p.len - 1) / RPD * RPD) : i * RPD;
+      load_row_to_lds(rv, vt + i * RPD * H, vrow + ((sw ^ ((i * RPD) % CPR)) << 4), (p.pos + r0) * row_bytes);
+    }
   };
   // K fragments of a block: lane (position qi, h) reads the half h of its row, 16 bytes per MFMA step
   const int koff = qi * row_bytes + h * H;
   u32x4_t kf[KS];
-  auto load_k = [&](int blk) __attribute__((always_inline)) {
+  auto load_k = [&](const Place& p) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rk = OWN ? cache_of(a.kcache, p.kv) : rk_lead;
+    const int off = OWN ? min(qi, p.len - 1) * (int)row_bytes + h * H : koff;
 #pragma unroll
     for (int t = 0; t < KS; ++t)
-      kf[t] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rk, koff + t * 16, (j.pbeg + blk * 32) * row_bytes, 0));
+      kf[t] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rk, off + t * 16, p.pos * row_bytes, 0));
   };
-  const uint8_t* mrow = a.input_mask + (size_t)lead * a.buf_len;
-  auto mask_byte = [&](int blk) __attribute__((always_inline)) {
-    const int p = j.pbeg + blk * 32 + qi;
-    return (h == 0 && p < a.buf_len) ? mrow[p] : (uint8_t)0;
+  auto mask_byte = [&](const Place& p) __attribute__((always_inline)) {
+    const int at = p.pos + qi;
+    return (h == 0 && at < a.buf_len) ? a.input_mask[(size_t)p.kv * a.buf_len + at] : (uint8_t)0;
   };
 
   f32x16_t o[HT];
@@ -330,10 +347,12 @@ __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& l
 
   int blk = j.split * bps + wave;
   uint8_t mb = 0;
+  Place at = {};
   if (blk < b_end) {
-    mb = mask_byte(blk);
-    load_k(blk);
-    dma_v(blk);
+    at = place(blk);
+    mb = mask_byte(at);
+    load_k(at);
+    dma_v(at);
   }
   for (; blk < b_end; blk += 4) {
     const bool more = blk + 4 < b_end;
@@ -352,7 +371,7 @@ __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& l
     // accumulator register r holds position 8 (r / 4) + 4 h + r % 4 of the block: with the lane's half folded
     // into the mask word and the limit, the per-register part is a compile-time constant
     const uint32_t mb2 = mbits >> (4 * h);
-    const int lim = plen - blk * 32 - 4 * h;  // plen: positions of this walk, counted from pbeg
+    const int lim = (OWN && at.own_of >= 0 && at.own_of != qi / G ? 0 : at.len) - 4 * h;  // another row's own slots: none
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int pc = (r >> 2) * 8 + (r & 3);
@@ -424,9 +443,10 @@ __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& l
     // and the other eleven waves of the CU cover the round trip.
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (more) {
-      mb = mask_byte(blk + 4);
-      load_k(blk + 4);
-      dma_v(blk + 4);
+      at = place(blk + 4);
+      mb = mask_byte(at);
+      load_k(at);
+      dma_v(at);
     }
   }
   l += __shfl_xor(l, 32, 64);
@@ -508,6 +528,7 @@ __device__ __forceinline__ bool tile_job(const AttnArgs& a, int n_group_y, int y
   const int step = min(*a.step, min(a.C, a.buf_len) - 1);
   const int shared_end = a.share_gs > 1 ? min(a.share_len, step + 1) : 0;
   j.nparts = a.nsplit + a.psplits;
+  j.own = a.nsplit ? 0 : step + 1 - shared_end;
   j.split = z;
   if (y < n_group_y) {
     if (z >= a.psplits) return false;
@@ -537,6 +558,17 @@ __global__ __launch_bounds__(256, 3) void gqa_tile_kernel(AttnArgs a, int n_grou
   __shared__ PrefixLds<H> lds;
   TileJob j;
   if (tile_job<G>(a, n_group_y, blockIdx.y, blockIdx.z, true, j)) gqa_tile_walk<H, G>(a, lds, blockIdx.x, j);
+}
+
+// Groups alone: a workgroup walks the shared slots of its group and then every query row's own, for whose blocks the other
+// rows' columns are masked (7 of 8 columns of the MFMA tile idle there, which costs nothing: it waits for memory).  Every
+// cache row is read once and, in one split, no part leaves the workgroup.  256 rows of the 8B shape in groups of 8 at 128 + 12
+// slots 36.0 us by themselves, 14.8 here; 8 layers, 24 steps of that 68.6 -> 61.8 ms.  grid (Kh, group query blocks, splits).
+template <int H, int G>
+__global__ __launch_bounds__(256, 3) void gqa_group_kernel(AttnArgs a) {
+  __shared__ PrefixLds<H> lds;
+  TileJob j;
+  if (tile_job<G>(a, gridDim.y, blockIdx.y, blockIdx.z, false, j)) gqa_tile_walk<H, G, true>(a, lds, blockIdx.x, j);
 }
 
 // The same grid with the rows' own slots on the vector-ALU walk (gqa_decode_walk) and only the shared slots on
@@ -771,10 +803,10 @@ int attn_num_splits(int B, int Kh, int C) {
   return ns;
 }
 
-// The shared walk serves one token per sequence, up to 128 sequences in whole groups, the head dimensions and
-// group widths of the tile walk, and 32-bit byte offsets per cache.
+// The shared walk serves one token per sequence, sequences in whole groups, the head dimensions and group widths of the tile
+// walk, and 32-bit byte offsets per cache.
 bool attn_share_ok(int B, int N, int Kh, int H, int C, int share_gs, int share_len) {
-  if (share_gs <= 1 || share_len < 32 || share_len > C || B <= 0 || B > 128 || B % share_gs) return false;
+  if (share_gs <= 1 || share_len < 32 || share_len > C || B <= 0 || B % share_gs) return false;
   if (Kh <= 0 || N % Kh || (H != 64 && H != 128)) return false;
   const int G = N / Kh;
   if (G != 1 && G != 2 && G != 4 && G != 8) return false;
@@ -784,12 +816,18 @@ bool attn_share_ok(int B, int N, int Kh, int H, int C, int share_gs, int share_l
 // Which kernel walks the cache of a one-token step, and in how many splits.
 struct AttnPlan {
   bool tile;    // gqa_tile_kernel (matrix pipe) or gqa_decode_kernel (vector ALU)
-  bool shared;  // tile only: prompt slots once per group
-  int nsplit;   // splits of a row's own slots
+  bool shared;  // prompt slots once per group
+  int nsplit;   // splits of a row's own slots (0: the groups' workgroups walk them too, gqa_group_kernel)
   int psplits;  // splits of the shared slots
 };
 
-static AttnPlan plan_attention(int B, int N, int Kh, int H, int C, int share_gs, int share_len) {
+static long group_workgroups(int B, int G, int Kh, int share_gs) {
+  const int rpb = 32 / G;
+  return (long)(B / share_gs) * ((share_gs + rpb - 1) / rpb) * Kh;
+}
+
+// The plan with (shared) or without the groups' shared slots walked by workgroups of their own beside the rows'.
+static AttnPlan plan_rows_walk(int B, int N, int Kh, int H, int C, bool shared, int share_gs, int share_len) {
   AttnPlan p = {false, false, attn_num_splits(B, Kh, C), 0};
   const int G = Kh > 0 && N % Kh == 0 ? N / Kh : 0;
   if ((H != 64 && H != 128) || (G != 1 && G != 2 && G != 4 && G != 8) || (size_t)C * Kh * H * 2 >= (1u << 31)) return p;
@@ -797,7 +835,7 @@ static AttnPlan plan_attention(int B, int N, int Kh, int H, int C, int share_gs,
   // sequences x 8 kv heads = 1024 workgroups: 108 against 98 us for the vector-ALU walk, four of whose workgroups
   // fit a CU); with shared prompt slots a launch reads fewer cache rows and may take two rounds.
   const long slots = 3L * device_cus(), pairs = (long)B * Kh;
-  p.shared = attn_share_ok(B, N, Kh, H, C, share_gs, share_len);
+  p.shared = shared;
   // Rows' own slots: the tile walk for 8 query heads per kv head (measured on the 30B-A3B shape, 32 sequences at
   // context 512: 10.7 + 3.0 us for walk and combine against 21.7 + 3.9 us; the vector walk's work per cache row
   // grows with the heads); up to 2 heads, and 4 heads behind shared slots, the vector walk (see gqa_shared_kernel).
@@ -810,8 +848,7 @@ static AttnPlan plan_attention(int B, int N, int Kh, int H, int C, int share_gs,
   if (p.shared && pairs > 2 * slots) p.shared = false;
   long group_wgs = 0;
   if (p.shared) {
-    const int rpb = 32 / G, qblocks = (share_gs + rpb - 1) / rpb;
-    group_wgs = (long)(B / share_gs) * qblocks * Kh;
+    group_wgs = group_workgroups(B, G, Kh, share_gs);
     // splits of the shared slots: a block of 32 positions for every other wave, while the launch stays resident
     // (measured on 256 shared slots at 64 sequences of the 8B shape: 1, 2, 4 splits -> 23.9, 22.1, 21.2 us)
     const int nblk = (share_len + 31) / 32;
@@ -831,8 +868,42 @@ static AttnPlan plan_attention(int B, int N, int Kh, int H, int C, int share_gs,
   return p;
 }
 
+// With shared prompt slots: rows by themselves, groups and rows side by side, or groups alone, whichever costs least at the
+// middle of the rollout (half of the `len` - share_len slots behind the prompt in use).  us, launches included; every walk has
+// a fixed part, cache bytes at 5.2 TB/s (4.7 in the group walk, which reads K in 16-byte pieces), and the combine launch of
+// several parts 3.4; a workgroup of the group walk takes 2.2 per round of its four waves.  Measured on cold caches, 8 kv heads of 4 query heads, rows x group, shared + own slots: rows by
+// themselves / side by side / groups alone:
+//   256 x 8, 128 + 12   36.0 /   -  / 14.8       256 x 8, 256 + 512  140.8 /   -  / 111.5     128 x 8, 256 + 24  32.0 / 18.3 / 13.9
+//   64 x 8, 256 + 32    19.9 / 13.5 / 12.0 in 4  64 x 8, 256 + 256    29.7 / 23.7 /  25.1     128 x 8, 64 + 32   15.4 / 17.8 / 12.3
+//   32 x 8, 256 + 64    17.2 / 12.4 / 10.6 in 8  48 x 8, 224 + 32     17.8 / 12.2 /  11.3     24 x 6, 64 + 24     7.0 /  9.4 /  8.7
+// (in one split but where noted).  More than 128 rows have no room for parts: groups alone in one split.
+static AttnPlan plan_attention(int B, int N, int Kh, int H, int C, int share_gs, int share_len, int len, bool must_share) {
+  const AttnPlan rows = plan_rows_walk(B, N, Kh, H, C, false, 0, 0);
+  if (!attn_share_ok(B, N, Kh, H, C, share_gs, share_len)) return rows;
+  const int G = N / Kh, own = len > share_len ? (len - share_len + 1) / 2 : 1;
+  const float us_per_slot = (float)H * 4.f / 5.2e6f;  // a K and a V row
+  AttnPlan best = rows;
+  float best_cost = 6.f + us_per_slot * B * Kh * (share_len + own) + (rows.nsplit > 1 ? 3.f : 0.f);
+  if (must_share) best_cost = 1e30f;
+  auto offer = [&](const AttnPlan& p, float cost) {
+    if (cost < best_cost) { best = p; best_cost = cost; }
+  };
+  const long wgs = group_workgroups(B, G, Kh, share_gs), slots = 3L * device_cus();
+  if (B <= 128) {
+    const AttnPlan p = plan_rows_walk(B, N, Kh, H, C, true, share_gs, share_len);
+    if (p.shared) offer(p, 9.2f + us_per_slot * ((float)B * Kh * own + (float)wgs * share_len));
+  }
+  const int rpb = 32 / G, nrows = share_gs < rpb ? share_gs : rpb;
+  const int blocks = (share_len + 31) / 32 + nrows * ((own + 31) / 32);
+  for (int z = 1; z <= (B <= 128 ? kMaxGroupSplits : 1) && (z == 1 || wgs * z <= slots); ++z) {
+    const float rounds = 2.2f * ((blocks + 4 * z - 1) / (4 * z)), bytes = 1.1f * us_per_slot * 32.f * blocks * wgs;
+    offer(AttnPlan{false, true, 0, z}, 4.4f + (rounds > bytes ? rounds : bytes) + (z > 1 ? 3.4f : 0.f));
+  }
+  return best;
+}
+
 size_t attn_partial_bytes(int B, int N, int Kh, int H, int C) {
-  const AttnPlan p = plan_attention(B, N, Kh, H, C, 0, 0);
+  const AttnPlan p = plan_rows_walk(B, N, Kh, H, C, false, 0, 0);
   // rows of two or three tokens per pass take the vector-ALU walk whatever the plan says
   const int ns = p.nsplit > attn_num_splits(B, Kh, C) ? p.nsplit : attn_num_splits(B, Kh, C);
   return ns == 1 ? 0 : (size_t)B * N * ns * (H + 2) * sizeof(float);
@@ -854,7 +925,8 @@ static int launch_tile(hipStream_t st, const AttnArgs& a, bool rows_on_tile) {
   }
   const int nz = a.nsplit > a.psplits ? a.nsplit : a.psplits;
   const dim3 grid(a.Kh, n_group_y + a.B, nz);
-  if (rows_on_tile) hipLaunchKernelGGL((gqa_tile_kernel<H, G>), grid, dim3(256), 0, st, a, n_group_y);
+  if (!a.nsplit) hipLaunchKernelGGL((gqa_group_kernel<H, G>), dim3(a.Kh, n_group_y, a.psplits), dim3(256), 0, st, a);
+  else if (rows_on_tile) hipLaunchKernelGGL((gqa_tile_kernel<H, G>), grid, dim3(256), 0, st, a, n_group_y);
   else if constexpr (G <= 4) hipLaunchKernelGGL((gqa_shared_kernel<H, G>), grid, dim3(256), 0, st, a, n_group_y);
   else return TMX_ERR_UNSUPPORTED;
   int rc = check_launch();
@@ -872,7 +944,7 @@ int gqa_decode(hipStream_t st, AttnArgs a, int H) {
   const int G = a.N / a.Kh;
   if (a.N % a.Kh) return TMX_ERR_SHAPE;
   if (a.tpp <= 1 && !a.seg) {
-    const AttnPlan p = plan_attention(a.B, a.N, a.Kh, H, a.C, a.share_gs, a.share_len);
+    const AttnPlan p = plan_attention(a.B, a.N, a.Kh, H, a.C, a.share_gs, a.share_len, a.C < a.buf_len ? a.C : a.buf_len, a.must_share);
     if (p.tile || p.shared) {
       a.nsplit = p.nsplit;
       a.psplits = p.shared ? p.psplits : 0;
@@ -959,7 +1031,7 @@ extern "C" int tmx_gqa_decode_attention_shared(void* stream, const void* q, cons
                                                int share_group, int share_len) {
   if (!q || !kcache || !vcache || !input_mask || !step || !out || !workspace) return TMX_ERR_ARG;
   if (B <= 0 || N <= 0 || Kh <= 0 || C <= 0) return TMX_ERR_SHAPE;
-  if (!plan_attention(B, N, Kh, H, C, share_group, share_len).shared) return TMX_ERR_UNSUPPORTED;
+  if (B > 128 || !plan_attention(B, N, Kh, H, C, share_group, share_len, C < buf_len ? C : buf_len, true).shared) return TMX_ERR_UNSUPPORTED;
   AttnArgs a = {};
   a.q = (const uint16_t*)q;
   a.kcache = (const uint16_t*)kcache;
@@ -970,7 +1042,7 @@ extern "C" int tmx_gqa_decode_attention_shared(void* stream, const void* q, cons
   a.out = (uint16_t*)out;
   a.partial = (float*)workspace;
   a.B = B; a.N = N; a.Kh = Kh; a.C = C;
-  a.share_gs = share_group; a.share_len = share_len;
+  a.share_gs = share_group; a.share_len = share_len; a.must_share = true;
   a.scale = 1.0f / sqrtf((float)H);
   return gqa_decode((hipStream_t)stream, a, H);
 }

@@ -289,7 +289,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
     if (rc != TMX_OK) return rc;
   }
   // samples of one prompt in consecutive rows: decode attention reads the prompt slots once per group
-  const bool share_walk = T == 1 && !rg && !small && w.attn_partial && attn_share_ok(B, N, Kh, H, C, s->share_group, s->share_len);
+  const bool share_walk = T == 1 && !rg && !small && attn_share_ok(B, N, Kh, H, C, s->share_group, s->share_len);
   // Without the head nobody reads what the last layer adds to the residual stream: it ends with its K and V rows in the cache.
   // 65 408 prompt rows on 6 layers of the Qwen3-8B shape and 32 steps at 128 sequences: 200.7 -> 180.0 ms; two passes of 2.3k
   // rows on 8 layers of the 8B shape and 8 steps 26.2 -> 24.1.

@@ -179,10 +179,11 @@ struct AttnArgs {
   int n_seg, seg_width;
   // Shared prompt slots (G samples of one prompt in consecutive rows): share_gs > 1 says that the sequences
   // come in consecutive groups of share_gs whose cache slots [0, share_len) and input_mask entries are
-  // identical.  Those slots are then walked once per group (gqa_prefix_kernel, psplits splits, from the
-  // group's first sequence), every row walks only its own slots share_len .. *step (nsplit splits), and
-  // the nsplit + psplits partial results per row are merged by the rows' walk itself or the combine kernel.
+  // identical.  Those slots are then walked once per group (psplits splits, from the group's first sequence), every row's
+  // own slots share_len .. *step by a workgroup of its own (nsplit splits) or by the group's (nsplit = 0), and
+  // the nsplit + psplits partial results per row are merged by the combine kernel.
   int share_gs, share_len, psplits;
+  bool must_share;  // never every row by itself, whatever that would cost
 };
 
 struct HeadArgs {
