@@ -1197,6 +1197,43 @@ def test_moe_experts_row_counts(down, K, N):
   assert ((got - want).abs() > 2.0 ** -6 * want.abs() + 2.0 ** -8).sum() == 0
 
 
+# The stream kernel with the rows of an expert in LDS: no row, one, as many as fit (11 of 2048 up, 18 to 32 down), one more, several
+# loads of them; waves without columns; one, two and three workgroups' room.  The reference is the f32 product.
+@pytest.mark.parametrize('down,K,N', [(0, 2048, 256), (0, 2048, 128), (0, 256, 896), (1, 768, 256), (1, 512, 128), (1, 4096, 384)])
+def test_moe_experts_of_few_rows(down, K, N):
+  from tunix_amd import quant
+  counts = [0, 1, 11, 12, 35, 2, 0, 3, 1, 4, 18, 19, 2, 1, 1, 0, 5, 1, 0, 2, 1, 1, 0, 2] + [0] * 24  # whole tokens of two pairs
+  E, k, group = len(counts), 2, 64
+  g = torch.Generator(device=G.DEV).manual_seed(K + N)
+  idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+  P = idx.numel()
+  assert P <= 1024 and P % k == 0 and P / E + 3.5 * (P / E) ** 0.5 <= 9
+  idx = idx[torch.randperm(P, generator=torch.Generator().manual_seed(3))].to(torch.int32).to(G.DEV)
+  w = (torch.randn(K, E * N, generator=g, device=G.DEV) * 0.05).to(torch.bfloat16)
+  pl = quant.PackedLinear.from_dense([w], group, G.DEV)
+  dense = torch.empty(K, E * N, dtype=torch.bfloat16, device=G.DEV)
+  G.call('tmx_int4_dequant', S(), G.p(pl.qweight), G.p(pl.scales), G.p(dense), K, E * N, group)
+  x = torch.randn(P if down else P // k, K, generator=g, device=G.DEV).to(torch.bfloat16)
+  cols = N if down else N // 2
+  out = torch.full((P + 1, cols), 7.0, dtype=torch.bfloat16, device=G.DEV)  # the last row stays
+  G.call('tmx_moe_experts', S(), G.p(x), K, G.p(pl.qweight), G.p(pl.scales), G.p(idx), P, k, E, K, N, group, down, G.p(out), cols)
+  rows = x.float() if down else x.float().repeat_interleave(k, 0)
+  want = torch.empty(P, cols, device=G.DEV)
+  rb = lambda t: t.to(torch.bfloat16).float()
+  for e in range(E):
+    mine = (idx == e).nonzero().flatten()
+    y = rows[mine] @ dense[:, e * N:(e + 1) * N].float()
+    if not down:
+      gate, up = rb(y[:, :cols]), rb(y[:, cols:])
+      y = rb(gate * rb(torch.sigmoid(gate))) * up
+    want[mine] = y
+  got = out[:P].float()
+  assert (out[P] == 7.0).all()
+  # the bounds of test_moe_experts_row_counts
+  assert (got - want).norm() <= (2e-3 if down else 6e-3) * want.norm()
+  assert ((got - want).abs() > 2.0 ** -6 * want.abs() + 2.0 ** -8).sum() == 0
+
+
 # A call of more than 1024 pairs is one launch of the many-rows kernel, a call of fewer the stream kernel: same bits, whatever the
 # distance of the rows (0: one row for all; 2^21 bytes apart: beyond 32-bit offsets), where rows of out begin, and also when the
 # last token has fewer pairs than top_k.

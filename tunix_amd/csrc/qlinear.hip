@@ -13,6 +13,7 @@
 // rounded pairwise to bf16 by the hardware converter, which reproduces the
 // reference's bf16 dequantised weight bit for bit before it enters the MFMA.
 #include <atomic>
+#include <cmath>
 
 #include "tmx_kernels.h"
 
@@ -343,12 +344,16 @@ static int launch_qlinear4(hipStream_t st, QLinearArgs a) {
 // the routing table (at most a few hundred entries) and leaves if there are none, so unrouted experts
 // are never streamed.  In decode an expert sees a handful of rows (batch x top_k pairs spread over many
 // experts), so the product is nothing but a weight stream: every wave walks its own column tiles (DOWN)
-// or gate / up tile pairs (SwiGLU in its epilogue) over all of K with no LDS and no barrier after the
+// or gate / up tile pairs (SwiGLU in its epilogue) over all of K with no barrier after the
 // compaction.  Weight tiles come through a ring of kMoeRing tiles per wave (buffer loads, scalar
-// offsets), the x fragments of the live rows straight from global memory (gathered activation rows;
-// lanes of absent rows hold zeros), one k-tile ahead; output rows are scattered.  The ring runs on
-// across the wave's tiles, so the stream never drains.  More than 32 rows of an expert are taken in
-// chunks of 32, each streaming the weights again (rare).
+// offsets), requested in front of the compaction; output rows are scattered.  The ring runs on
+// across the wave's tiles, so the stream never drains.  LDS: the expert's rows are gathered into LDS, and an absent row's
+// fragments are read from zeros; otherwise the fragments of the live rows come straight from global memory, for which the
+// compiler makes 16 exec-mask regions and 86 register fills per 8 weight tiles.  Rows that do not fit, and more than 32, are
+// taken in chunks, each streaming the weights again (rare).
+// What bounds it: the stream (128 experts of 2048 x 1536 and 768 x 2048, 32 rows of 8: 186 + 93 MB in 42.5 + 23.9 us, 4.4 + 3.9
+// TB/s with the launch) and, beside it, the dequantisation (35 ns per 512 weights of a SIMD, 23 + 12 us).  With the rows
+// looked up first and from global memory 48.5 + 29.6 us; 8 layers of that in 48 steps and the prompts 77.5 -> 72.5 ms.
 // Weight tiles that ONE wave reads once, whole cache lines per load (the routed experts, the fused gate | up
 // launch): non-temporal buffer loads (the nt bit of the cache policy).  A plain streaming read reaches 5.6-6.2 TB/s
 // on this part, a non-temporal one 6.3-7.0; the split projections and the 64-row head measured slower with it.
@@ -356,73 +361,99 @@ constexpr int kNtLoad = 2;
 
 constexpr int kMoeStreamPairs = 1024;  // most pairs of a launch (more: moe_rows)
 constexpr int kMoeRing = 4;  // divides K / 64 (K % 256 == 0), so a ring slot is k-tile % 4 in every unit
+constexpr size_t kMoeLds = 160 * 1024 - 4 * 2304;  // of a CU, less what its workgroups hold beside x
+constexpr int kMoeXZero = 256;  // zeros in front of the rows' copy in LDS: a group of k-tiles of an absent row
 
-template <bool DOWN>
-__global__ __launch_bounds__(256, 2) void moe_stream_kernel(MoeArgs m) {
-  __shared__ int rows_s[kMoeStreamPairs];
-  __shared__ int wave_cnt[4];
-  __shared__ int n_s;
+template <bool DOWN, bool LDS>
+__global__ __launch_bounds__(256, LDS ? (DOWN ? 4 : 3) : 2) void moe_stream_kernel(MoeArgs m) {
+  extern __shared__ __align__(16) uint16_t xs[];  // LDS: zeros, then x_rows rows
+  __shared__ uint16_t rows_s[kMoeStreamPairs];
+  __shared__ int wave_cnt[2][4];
   constexpr int TPU = DOWN ? 1 : 2;  // tiles per unit: one column tile, or a gate tile and its up tile
   const int e = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, nl = lane & 31;
-  int base = 0;
-  int ev = tid < m.P ? m.expert_of[tid] : -1;
-  for (int p0 = 0; p0 < m.P; p0 += 256) {  // ordered compaction of { p : expert_of[p] == e }
-    const int p = p0 + tid;
-    const bool hit = ev == e;
-    ev = p + 256 < m.P ? m.expert_of[p + 256] : -1;  // the next round's entry travels during this one's barriers
-    const unsigned long long mask = __ballot(hit);
-    if (lane == 0) wave_cnt[wave] = __popcll(mask);
-    __syncthreads();
-    int off = base;
-    for (int w = 0; w < wave; ++w) off += wave_cnt[w];
-    if (hit) rows_s[off + __popcll(mask & ((1ull << lane) - 1ull))] = p;
-    base += wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
-    __syncthreads();
-  }
-  if (tid == 0) n_s = base;
-  __syncthreads();
-  const int n = n_s;
-  if (n == 0) return;
-
   const int KT = m.K >> 6, KG = m.K / m.G, gs = __builtin_ctz(m.G >> 6);
   const int NT = m.N >> 5;
   const int units = DOWN ? NT : NT / 2;  // column tiles, or gate | up pairs (F / 32)
   // units of this wave: u = blockIdx.x + groups * (wave + 4 j), j = 0, 1, ... (groups = gridDim.x)
   const int u0 = (int)blockIdx.x + (int)gridDim.x * wave, ustride = (int)gridDim.x * 4;
-  if (u0 >= units) return;
-  const int nu = (units - u0 + ustride - 1) / ustride;
+  const int nu = u0 < units ? (units - u0 + ustride - 1) / ustride : 0;
 
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(m.qw + (size_t)e * m.qw_stride, (uint32_t)NT * KT * 1024u);
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(m.scales + (size_t)e * m.sc_stride, (uint32_t)NT * KG * 64u);
-
-  for (int c0 = 0; c0 < n; c0 += 32) {
-    const int rows = n - c0 < 32 ? n - c0 : 32;
-    // A fragments: lane (row nl, h) reads x[src][64 kt + 16 t + 8 h ..]; absent rows stay zero
-    const bool live = nl < rows;
-    const int pr = live ? rows_s[c0 + nl] : 0;
-    const uint16_t* xrow = m.x + (size_t)(DOWN ? pr : (m.pair0 + pr) / m.top_k) * m.ldx + 8 * h;
-    u32x4_t wring[kMoeRing][TPU];
-    uint16_t sring[kMoeRing][TPU];
-    // tile (unit ui of this wave, k-tile kt) into ring slot sl; past the last unit: its last tile again
-    auto load_w = [&](int ui, int kt, auto sc) __attribute__((always_inline)) {
-      constexpr int sl = decltype(sc)::value;
-      if (ui >= nu) { ui = nu - 1; kt = KT - 1; }
+  u32x4_t wring[kMoeRing][TPU];
+  uint16_t sring[kMoeRing][TPU];
+  // tile (unit ui of this wave, k-tile kt) into ring slot sl; past the last unit: its last tile again
+  auto load_w = [&](int ui, int kt, auto sc) __attribute__((always_inline)) {
+    constexpr int sl = decltype(sc)::value;
+    if (ui >= nu) { ui = nu - 1; kt = KT - 1; }
 #pragma unroll
-      for (int c = 0; c < TPU; ++c) {
-        const int nb = u0 + ui * ustride + c * units;  // the gate tile, or the up tile F / 32 further on
-        wring[sl][c] = __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, (int)((uint32_t)(nb * KT + kt) * 1024u), kNtLoad);
-        sring[sl][c] = __builtin_amdgcn_raw_buffer_load_b16(rs, nl * 2, (nb * KG + (kt >> gs)) * 64, 0);
+    for (int c = 0; c < TPU; ++c) {
+      const int nb = u0 + ui * ustride + c * units;  // the gate tile, or the up tile F / 32 further on
+      wring[sl][c] = __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, (int)((uint32_t)(nb * KT + kt) * 1024u), kNtLoad);
+      sring[sl][c] = __builtin_amdgcn_raw_buffer_load_b16(rs, nl * 2, (nb * KG + (kt >> gs)) * 64, 0);
+    }
+  };
+  auto fill_ring = [&]() __attribute__((always_inline)) {
+    static_for<kMoeRing>([&](auto sc) __attribute__((always_inline)) { load_w(0, decltype(sc)::value, sc); });
+  };
+  int ev = tid < m.P ? m.expert_of[tid] : -1;
+  __builtin_amdgcn_sched_barrier(0);
+  if (LDS && nu > 0) fill_ring();  // on the way while the rows are looked up
+  __builtin_amdgcn_sched_barrier(0);
+  int n = 0;
+  for (int p0 = 0, turn = 0; p0 < m.P; p0 += 256, turn ^= 1) {  // ordered compaction of { p : expert_of[p] == e }
+    const int p = p0 + tid;
+    const bool hit = ev == e;
+    ev = p + 256 < m.P ? m.expert_of[p + 256] : -1;  // the next round's entry travels during this one's barrier
+    const unsigned long long mask = __ballot(hit);
+    if (lane == 0) wave_cnt[turn][wave] = __popcll(mask);
+    __syncthreads();
+    int off = n;
+    for (int w = 0; w < wave; ++w) off += wave_cnt[turn][w];
+    if (hit) rows_s[off + __popcll(mask & ((1ull << lane) - 1ull))] = (uint16_t)p;
+    n += wave_cnt[turn][0] + wave_cnt[turn][1] + wave_cnt[turn][2] + wave_cnt[turn][3];
+  }
+  n = __builtin_amdgcn_readfirstlane(n);
+  if (n == 0) return;
+  __syncthreads();
+  auto x_row = [&](int r) __attribute__((always_inline)) {
+    const int pr = rows_s[r];
+    return m.x + (size_t)(DOWN ? pr : (m.pair0 + pr) / m.top_k) * m.ldx;
+  };
+  const int XS = m.K + 8;  // elements between the rows in LDS: 16 bytes of padding, rows on other banks
+  const int chunk = LDS ? m.x_rows : 32;
+  if (LDS && tid < kMoeXZero / 8) *reinterpret_cast<u32x4_t*>(xs + tid * 8) = u32x4_t{0u, 0u, 0u, 0u};
+
+  for (int c0 = 0; c0 < n; c0 += chunk) {
+    const int rows = n - c0 < chunk ? n - c0 : chunk;
+    if constexpr (LDS) {
+      if (c0) __syncthreads();
+      const int pieces = m.K >> 3;
+      for (int r = 0; r < rows; ++r) {
+        const uint16_t* src = x_row(c0 + r);
+        for (int c = tid; c < pieces; c += 256)
+          *reinterpret_cast<u32x4_t*>(xs + kMoeXZero + r * XS + c * 8) = *reinterpret_cast<const u32x4_t*>(src + c * 8);
       }
-    };
+      __syncthreads();
+    }
+    if (nu == 0) continue;
+    if (c0 || !LDS) fill_ring();
+    // A fragments: lane (row nl, h) takes x[src][64 kt + 16 t + 8 h ..]; absent rows are zero
+    const bool live = nl < rows;
+    const uint16_t* xrow = x_row(c0 + (live ? nl : 0)) + 8 * h;
+    const uint16_t* xlds = xs + (live ? kMoeXZero + nl * XS : 0) + 8 * h;
+    const int kmask = live ? ~0 : 255;  // absent rows stay inside the zeros
     u32x4_t xq[2][4];
     auto load_x = [&](int kt, int slot) __attribute__((always_inline)) {
+      const uint16_t* p = xlds + ((kt * 64) & kmask);
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        xq[slot][t] = live ? *reinterpret_cast<const u32x4_t*>(xrow + kt * 64 + 16 * t) : u32x4_t{0, 0, 0, 0};
+      for (int t = 0; t < 4; ++t) {
+        if constexpr (LDS) xq[slot][t] = *reinterpret_cast<const u32x4_t*>(p + 16 * t);
+        else xq[slot][t] = live ? *reinterpret_cast<const u32x4_t*>(xrow + kt * 64 + 16 * t) : u32x4_t{0, 0, 0, 0};
+      }
     };
-    static_for<kMoeRing>([&](auto sc) __attribute__((always_inline)) { load_w(0, decltype(sc)::value, sc); });
     load_x(0, 0);
     f32x16_t acc[TPU];
     for (int u = 0; u < nu; ++u) {
@@ -500,8 +531,30 @@ int moe_experts(hipStream_t st, const MoeArgs& a, int E, bool down) {
   const int units = down ? a.N / 32 : a.N / 64;
   int groups = units / (down ? 8 : 4);
   groups = groups < 1 ? 1 : (groups > 32 ? 32 : groups);
-  if (down) hipLaunchKernelGGL(moe_stream_kernel<true>, dim3(groups, E), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(moe_stream_kernel<false>, dim3(groups, E), dim3(256), 0, st, a);
+  // Rows in LDS: as many as leave room for the workgroups whose registers fit a CU (down: or one or two fewer), if an expert
+  // seldom has more (the mean + 3.5 sqrt(mean)), since one that has streams its matrices again.  us, from global memory / LDS, 128
+  // experts of 2048 x 768, top-8: 8 rows up 44.1 / 39.3, down 22.0 / 18.8; 32 rows 48.5 / 42.5, 29.6 / 23.9; 64 rows 51.4 / 47.6,
+  // 32.5 / 26.6; 128 rows up (two workgroups of a CU) 55.7 / 56.8, down 36.3 / 29.7.
+  const float mean = (float)a.P / E;
+  const int need = (int)ceilf(mean + 3.5f * sqrtf(mean));
+  MoeArgs m = a;
+  size_t lds = 0;
+  for (int wgs = down ? 4 : 3; wgs >= (down ? 2 : 3) && !m.x_rows; --wgs) {
+    const int rows = (int)((kMoeLds / wgs - kMoeXZero * 2) / ((a.K + 8) * 2));
+    if (need <= rows || rows >= 32) {
+      m.x_rows = rows < 32 ? rows : 32;
+      lds = (size_t)(kMoeXZero + m.x_rows * (a.K + 8)) * 2;
+    }
+  }
+  static const hipError_t attr_d = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_stream_kernel<true, true>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMoeLds / 2);
+  static const hipError_t attr_u = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_stream_kernel<false, true>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMoeLds / 2);
+  if (attr_d != hipSuccess || attr_u != hipSuccess) return TMX_ERR_LAUNCH;
+  if (down && lds) hipLaunchKernelGGL((moe_stream_kernel<true, true>), dim3(groups, E), dim3(256), lds, st, m);
+  else if (down) hipLaunchKernelGGL((moe_stream_kernel<true, false>), dim3(groups, E), dim3(256), 0, st, m);
+  else if (lds) hipLaunchKernelGGL((moe_stream_kernel<false, true>), dim3(groups, E), dim3(256), lds, st, m);
+  else hipLaunchKernelGGL((moe_stream_kernel<false, false>), dim3(groups, E), dim3(256), 0, st, m);
   return check_launch();
 }
 

@@ -76,6 +76,7 @@ struct MoeArgs {
   uint16_t* out;           // gate|up: act [P, F]; down: y [P, D]
   int ldo;
   int pair0;               // gate|up in runs of pairs: the first pair of the run (x is the whole batch's)
+  int x_rows;              // rows of an expert in LDS at a time (0: fragments from global memory); set by moe_experts
 };
 // Bytes of x from its first to its last element, and how many of them the many-rows kernel's offsets reach.
 __host__ __device__ inline size_t moe_x_bytes(const MoeArgs& a, bool down) {
