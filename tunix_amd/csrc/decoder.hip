@@ -486,8 +486,13 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
           a.router.w = (const uint16_t*)l.router_w;
           a.router.D = D; a.router.E = m->num_experts; a.router.top_k = m->experts_per_tok;
           a.router.expert_of = w.expert_of; a.router.weight_of = w.weight_of;
+          a.router.x = w.xn;
         }
+        const RouterArgs route = a.router;
+        const bool apart = moe && moe_route_rows_ok(route, B);
+        if (apart) a.router.w = nullptr;
         TMX_TRY(TMX_K_ROWNORM, row_norm(st, a, B));
+        if (apart) TMX_TRY(TMX_K_ROUTER, moe_route(st, route, B));
       }
       if (moe) {
         const int P = B * m->experts_per_tok;

@@ -167,9 +167,9 @@ __device__ __forceinline__ void add_lora8(float* o, const float* t_s, const uint
 
 // One workgroup per row: h = bf16(bf16(y + delta) + residual); xn = RMSNorm(h).
 // In embedding mode it also fills this step's RoPE sin/cos table row.
-template <int CPT>  // 8-element chunks per thread, D <= 4096 * CPT
+template <int CPT, bool ROUTE = false>  // 8-element chunks per thread, D <= 4096 * CPT; ROUTE: the row is routed here
 __global__ __launch_bounds__(512) void row_norm_kernel(RowNormArgs a) {
-  extern __shared__ __align__(16) float route_sm[];  // moe_router_lds_floats(D, E) floats when the row is routed here, else none
+  extern __shared__ __align__(16) float route_sm[];  // moe_router_lds(D, E) bytes when the row is routed here, else none
   __shared__ float smem[8];
   __shared__ float t_s[TMX_MAX_RPAD];
   __shared__ float t_stage[TMX_MAX_LORA_SPLITS * 64];
@@ -327,6 +327,12 @@ __global__ __launch_bounds__(512) void row_norm_kernel(RowNormArgs a) {
     }
   }
   if (!a.norm_w) return;
+  RouterStep ring[ROUTE ? 2 : 1];
+  if constexpr (ROUTE) {  // on the way while the row is normalised (from the start of the kernel on they would not fit its registers)
+    router_load(a.router, 0, 0, ring[0]);
+    router_load(a.router, 1, 0, ring[1]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   ss = block_sum<8>(ss, smem);
   const float rms = sqrtf(ss / (float)a.D + a.eps);
 #pragma unroll
@@ -342,17 +348,16 @@ __global__ __launch_bounds__(512) void row_norm_kernel(RowNormArgs a) {
         else o[e] = w[e] * (v[i][e] / rms);
       }
       *reinterpret_cast<uint4*>(a.xn_out + (size_t)m * a.D + n0) = pack8(o);
-      if (a.router.w) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) route_sm[n0 + e] = rbf(o[e]);
-      }
+      if constexpr (ROUTE) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(route_sm) + n0) = pack8(o);
+    } else if (ROUTE && c < moe_router_steps(a.D) * 32) {
+      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(route_sm) + c * 8) = uint4{0, 0, 0, 0};
     }
   }
-  if (a.router.w) {
+  if constexpr (ROUTE) {
     // MoE layer: the token is routed here, from the normed row this workgroup just made (no router launch, no
     // reload of xn)
     __syncthreads();
-    moe_route_token(a.router, route_sm, m);
+    moe_route_token(a.router, route_sm, m, ring);
   }
 }
 
@@ -420,8 +425,8 @@ int row_norm(hipStream_t st, const RowNormArgs& a, int M) {
     const RouterArgs& r = a.router;
     if (!a.norm_w || !r.expert_of || !r.weight_of || r.D != a.D) return TMX_ERR_ARG;
     if (r.E <= 0 || r.E % 8 || r.top_k <= 0 || r.top_k > 64 || r.top_k > r.E) return TMX_ERR_SHAPE;
-    lds = moe_router_lds_floats(a.D, r.E) * sizeof(float);
-    if (lds > 60000) return TMX_ERR_SHAPE;
+    if (!moe_router_ok(a.D, r.E)) return TMX_ERR_SHAPE;
+    lds = moe_router_lds(a.D, r.E);
   }
   // (few rows leave most CUs one workgroup each: the wider one finishes sooner)
   if (M > 128 && a.y_bf16 && !a.embed && !a.lora.t_part && !a.delta && !a.moe_y && !a.router.w && a.D <= 8192) {
@@ -431,6 +436,12 @@ int row_norm(hipStream_t st, const RowNormArgs& a, int M) {
     return check_launch();
   }
   const int cpt = (a.D / 8 + 511) / 512;
+  if (a.router.w) {
+    if (cpt <= 1) hipLaunchKernelGGL((row_norm_kernel<1, true>), dim3(M), dim3(512), lds, st, a);
+    else if (cpt <= 2) hipLaunchKernelGGL((row_norm_kernel<2, true>), dim3(M), dim3(512), lds, st, a);
+    else hipLaunchKernelGGL((row_norm_kernel<4, true>), dim3(M), dim3(512), lds, st, a);
+    return check_launch();
+  }
   if (cpt <= 1) hipLaunchKernelGGL(row_norm_kernel<1>, dim3(M), dim3(512), lds, st, a);
   else if (cpt <= 2) hipLaunchKernelGGL(row_norm_kernel<2>, dim3(M), dim3(512), lds, st, a);
   else hipLaunchKernelGGL(row_norm_kernel<4>, dim3(M), dim3(512), lds, st, a);

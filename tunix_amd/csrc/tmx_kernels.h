@@ -329,6 +329,7 @@ size_t attn_partial_bytes(int B, int N, int Kh, int H, int C);
 size_t attn_shared_partial_bytes(int B, int N, int Kh, int H, int C);
 bool attn_share_ok(int B, int N, int Kh, int H, int C, int share_gs, int share_len);
 int moe_route(hipStream_t st, const RouterArgs& a, int B);
+bool moe_route_rows_ok(const RouterArgs& a, int B);  // enough tokens for a launch of their own behind the row kernel
 int moe_experts(hipStream_t st, const MoeArgs& a, int E, bool down);
 int moe_rows(hipStream_t st, const MoeArgs& a, int E, bool down);  // its form for many rows per expert
 int head_sample(hipStream_t st, HeadArgs a);
