@@ -214,6 +214,29 @@ def test_row_norm_of_many_finished_rows(family, M, D):
       assert torch.all(xn == 7.0)
 
 
+# rows of a pass of more than 256 that still need their K-slices added and LoRA: the same bits as in calls of at most 100 rows, which
+# the test below holds against the oracle
+@pytest.mark.parametrize('D,ns,r', [(8, 1, 0), (1024, 5, 16), (2040, 4, 7), (2048, 0, 16), (2056, 3, 20), (4096, 8, 33)])
+def test_row_norm_of_many_unfinished_rows(D, ns, r):
+  M, g = 300, torch.Generator(device=G.DEV).manual_seed(D)
+  rand = lambda *shape: torch.randn(*shape, generator=g, device=G.DEV)
+  y16 = None if ns else rand(M, D).to(torch.bfloat16)
+  yp, tp = rand(max(ns, 1), M, D), rand(1, M, 128)
+  b, res, w = rand(max(r, 1), D).to(torch.bfloat16), rand(M, D).to(torch.bfloat16), rand(D).to(torch.bfloat16)
+
+  def run(lo, hi):
+    x, xn = res[lo:hi].clone(), torch.full((hi - lo, D), 7.0, dtype=torch.bfloat16, device=G.DEV)
+    yh, yq, tq = None if y16 is None else y16[lo:hi].contiguous(), yp[:, lo:hi].contiguous(), tp[:, lo:hi].contiguous()
+    G.call('tmx_lora_residual_rmsnorm', S(), None if yh is None else G.p(yh), None if ns == 0 else G.p(yq), ns, G.p(tq) if r else None, 1,
+           128, G.p(b) if r else None, r, 1.5, G.p(x), G.p(x), G.p(w), G.p(xn), hi - lo, D, 1e-6, 0)
+    G.sync()
+    return x, xn
+
+  x, xn = run(0, M)
+  parts = [run(lo, lo + 100) for lo in range(0, M, 100)]
+  assert torch.equal(x, torch.cat([p[0] for p in parts])) and torch.equal(xn, torch.cat([p[1] for p in parts]))
+
+
 @pytest.mark.parametrize('family', [0, 1])
 def test_lora_residual_rmsnorm_planes(family):
   T = G.Keep()

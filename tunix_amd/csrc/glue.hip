@@ -416,6 +416,114 @@ __global__ __launch_bounds__(256) void row_norm_plain_kernel(RowNormArgs a) {
   }
 }
 
+// The same for many rows that still need something: K-slices added (four planes at a time), LoRA from a finished t (one plane),
+// or the experts of a token.  One chunk of 8 values a thread; what the kernel above keeps in registers to have few rows'
+// loads out at once (236 of them: one workgroup of a CU, and half of its threads idle at 2048 values) is more than many rows
+// need: they wait for each other.  At most 128 registers, so 4 workgroups of 256 threads share a CU, or 2 of 512.  The same bits.
+// Measured (us back to back, the kernel above / this one, rank 16): 2048 values in 3 planes 477 rows 10.7 / 7.2, 630 rows 14.9 / 7.5, 1024
+// rows 20.7 / 9.6, 4096 rows 77 / 31; 4096 values in 2 planes 477 rows 10.3 / 8.3, 1024 rows 22.4 / 16.5; up to 256 rows of more
+// than 2048 values, a workgroup a CU, the one above (256 rows, 8 planes 8.3 / 9.1).
+template <int NT>  // threads, D <= 8 NT
+__global__ __launch_bounds__(NT, NT == 256 ? 4 : 2) void row_norm_part_kernel(RowNormArgs a) {
+  __shared__ float smem[NT / 64];
+  const int m = blockIdx.x, M = gridDim.x, n0 = threadIdx.x * 8;
+  const bool mine = n0 < a.D;
+  const int nl = mine ? n0 : 0;
+  const size_t at = (size_t)m * a.D + nl;
+  uint4 r4 = {0, 0, 0, 0}, w4 = {0, 0, 0, 0};
+  if (a.residual) r4 = *reinterpret_cast<const uint4*>(a.residual + at);
+  if (a.norm_w) w4 = *reinterpret_cast<const uint4*>(a.norm_w + nl);
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (a.moe_y) {
+    for (int j0 = 0; j0 < a.top_k; j0 += 8) {
+      uint4 yr[8];
+      float wr[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const size_t p = (size_t)m * a.top_k + min(j0 + u, a.top_k - 1);
+        yr[u] = *reinterpret_cast<const uint4*>(a.moe_y + p * a.D + nl);
+        wr[u] = a.moe_w[p];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        if (j0 + u >= a.top_k) break;
+        float y8[8];
+        unpack8(yr[u], y8);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = fmaf(wr[u], y8[e], v[e]);
+      }
+    }
+  } else if (a.y_bf16) {
+    unpack8(*reinterpret_cast<const uint4*>(a.y_bf16 + at), v);
+  } else {
+    const size_t stride = (size_t)M * a.D;
+    for (int s0 = 0; s0 < a.nsplit; s0 += 4) {
+      float4 lo[4], hi[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4* q = reinterpret_cast<const float4*>(a.y_part + (size_t)min(s0 + i, a.nsplit - 1) * stride + at);
+        lo[i] = q[0];
+        hi[i] = q[1];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (s0 + i >= a.nsplit) break;
+        v[0] += lo[i].x; v[1] += lo[i].y; v[2] += lo[i].z; v[3] += lo[i].w;
+        v[4] += hi[i].x; v[5] += hi[i].y; v[6] += hi[i].z; v[7] += hi[i].w;
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = rbf(v[e]);
+  if (a.lora.t_part) {
+    const float* t = a.lora.t_part + (size_t)m * a.lora.ldt;
+    float d[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int r0 = 0; r0 < a.lora.r; r0 += 8) {
+      uint4 b4[8];
+      float tv[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int rr = min(r0 + i, a.lora.r - 1);
+        b4[i] = *reinterpret_cast<const uint4*>(a.lora.b + (size_t)rr * a.D + nl);
+        tv[i] = r0 + i < a.lora.r ? rbf(t[rr]) : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float w[8];
+        unpack8(b4[i], w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d[e] = fmaf(tv[i], w[e], d[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = rbf(v[e] + rbf(rbf(d[e]) * a.lora.ls));
+  }
+  float ss = 0.f;
+  if (a.residual) {
+    float r8[8];
+    unpack8(r4, r8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = rbf(v[e] + r8[e]);
+  }
+  if (mine) {
+    if (a.x_out) *reinterpret_cast<uint4*>(a.x_out + at) = pack8(v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+  }
+  if (!a.norm_w) return;
+  ss = block_sum<NT / 64>(ss, smem);
+  const float rms = sqrtf(ss / (float)a.D + a.eps);
+  if (!mine) return;
+  float w[8], o[8];
+  unpack8(w4, w);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    if (a.family == TMX_FAMILY_LLAMA3) o[e] = rbf(w[e] * v[e]) / rms;
+    else o[e] = w[e] * (v[e] / rms);
+  }
+  *reinterpret_cast<uint4*>(a.xn_out + at) = pack8(o);
+}
+
 int row_norm(hipStream_t st, const RowNormArgs& a, int M) {
   if (a.D <= 0 || a.D % 8 || a.D > 4096 * 4) return TMX_ERR_SHAPE;
   if (a.lora.t_part && a.lora.r > TMX_MAX_RPAD) return TMX_ERR_SHAPE;
@@ -433,6 +541,11 @@ int row_norm(hipStream_t st, const RowNormArgs& a, int M) {
     if (a.D <= 2048) hipLaunchKernelGGL(row_norm_plain_kernel<1>, dim3(M), dim3(256), 0, st, a);
     else if (a.D <= 4096) hipLaunchKernelGGL(row_norm_plain_kernel<2>, dim3(M), dim3(256), 0, st, a);
     else hipLaunchKernelGGL(row_norm_plain_kernel<4>, dim3(M), dim3(256), 0, st, a);
+    return check_launch();
+  }
+  if (M > (a.D <= 2048 ? 128 : 256) && !a.embed && !a.delta && !a.router.w && a.D <= 4096 && (!a.lora.t_part || a.lora.nsplit == 1)) {
+    if (a.D <= 2048) hipLaunchKernelGGL(row_norm_part_kernel<256>, dim3(M), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(row_norm_part_kernel<512>, dim3(M), dim3(512), 0, st, a);
     return check_launch();
   }
   const int cpt = (a.D / 8 + 511) / 512;
