@@ -620,18 +620,18 @@ int moe_rows(hipStream_t st, const MoeArgs& a, int E, bool down) {
   return down ? launch_moe_rows<true>(st, a, E) : launch_moe_rows<false>(st, a, E);
 }
 
-// Which tile and how many K-slices.  The order in which a sum runs over K is set by the slices and by CT (one or two
-// k-parts); it follows prices of its own that stay as they are, so that a call gives the same bits whatever
-// becomes of the kernel (a greedy rollout goes another way where the two best logits are one bf16 step apart): a fixed part
-// of 8 us and steps of 0.24 us + 0.05 us per column tile and row tile.  The row tiles follow what the kernel takes now: a
-// fixed part (first slab and weights from cold caches, exchange, stores) and a time per step, both linear in the tile;
+// Which tile and how many K-slices.  The slices, which callers make room for, follow prices of their own: a fixed part
+// of 8 us and steps of 0.24 us + 0.05 us per column tile and row tile (by the prices below they would be fewer here and there, and
+// nothing gained: 256 x 4096 x 6144 unsplit instead of in 2 slices 0.4 % of a decode step slower).  The tile follows what the kernel
+// takes: a fixed part (first slab and weights from cold caches, exchange, stores) and a time per step, both linear in the tile;
 // fitted to every tile and slice count of twelve matrices of the 8B, 1B, Qwen3-8B and 30B-A3B shapes at 13 row counts from 135 to
 // 4096, they are 6 % off in the mean.  More workgroups than CUs run in rounds, whose steps are 1.12 times as long (the clock falls
 // with every CU at work) and which hide half of the fixed part; two workgroups of up to 4 x 4 tiles share a CU and hide
 // all of it.  K-slices cost their f32 planes, written here and read by the consumer.  At 256 rows of the 8B shape (us,
 // without LoRA and without the consumer's read) q|k|v runs 4 x 4 tiles in 2 slices, 20.6 (8 x 4 in 4: 21.6 and
 // twice the planes), gate|up 8 x 4 unsplit, 55 (4 x 4: 59, 8 x 8: 81), down 4 x 4 in 4, 33 (8 x 4 in 4: 43); 4096 rows of
-// gate|up 8 x 8, 715 (4 x 4: 840).
+// gate|up 8 x 8, 715 (4 x 4: 840); 3606 rows of it 8 x 8, 705 (7 x 4, which the prices of the slices would take, 789), 1024 rows
+// 8 x 8, 200 (4 x 4: 226), 400 rows of 4096 x 24576 7 x 8, 82 (7 x 4: 99).
 static const int kWideTiles[][2] = {{2, 4}, {3, 4}, {4, 4}, {5, 4}, {6, 4}, {7, 4}, {8, 4}, {4, 8}, {5, 8}, {6, 8}, {7, 8}, {8, 8}};
 
 // The LoRA workgroups of a launch (1 us + 0.25 a k-tile each) come first: where they and the others make more rounds, the last of
@@ -640,7 +640,7 @@ static const int kWideTiles[][2] = {{2, 4}, {3, 4}, {4, 4}, {5, 4}, {6, 4}, {7, 
 // tiles (256 + 16) 17.5, in 3 x 4 (192 + 16) 13.4.  Over 16 matrices at 15 row counts with adapters the choice is 0.5 % off the best
 // tile in the mean, 13 % at most (4.9 and 31 % without this), without adapters 0.15 and 9 %.
 
-// What a tile in s slices costs, us; `order`: by the prices that fix the order of the sums.
+// What a tile in s slices costs, us; `order`: by the prices that fix the slices.
 static float wide_price(int M, int N, int KT, int mt, int ct, int s, int cus, int lora_wgs, float lora_us, bool order) {
   const long tiles = (long)((M + 32 * mt - 1) / (32 * mt)) * ((N + 32 * ct - 1) / (32 * ct));
   const long n = (tiles * s + cus - 1) / cus;  // workgroups of a CU
@@ -668,10 +668,9 @@ WidePlan wide_plan(int M, int N, int K, int nsplit, int lora_wgs, int lora_kt) {
   for (const auto& t : kWideTiles)
     for (int s = nsplit > 0 ? nsplit : 1; s <= (nsplit > 0 ? nsplit : TMX_MAX_SPLITS); ++s)
       if (slices_ok(KT, s)) offer(t[0], t[1], s, true);
-  const int ct = best.ct, s = best.nsplit;
+  const int s = best.nsplit;
   best_cost = 1e30f;
-  for (const auto& t : kWideTiles)
-    if (t[1] == ct) offer(t[0], ct, s, false);
+  for (const auto& t : kWideTiles) offer(t[0], t[1], s, false);
   return best;
 }
 
