@@ -607,7 +607,7 @@ __global__ __launch_bounds__(256, 3) void gqa_shared_kernel(AttnArgs a, int n_gr
 constexpr int kFillMinTokens = 4;  // tokens per sequence and pass from which the fill kernel is used
 
 template <int H, int G>
-__global__ __launch_bounds__(256) void gqa_fill_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, 3) void gqa_fill_kernel(AttnArgs a) {
   constexpr int KS = H / 16;        // MFMA k-steps of the score product
   constexpr int CPR = H / 8;        // 16-byte chunks per cache row
   constexpr int RPD = 64 / CPR;     // rows per 1 KiB direct-to-LDS load
@@ -615,9 +615,12 @@ __global__ __launch_bounds__(256) void gqa_fill_kernel(AttnArgs a) {
   constexpr int HT = H / 32;        // hidden tiles of the output
   constexpr int TPW = 32 / G, TQ = 4 * TPW;  // tokens per wave / workgroup
   __shared__ __align__(16) uint16_t kt[2][32 * H], vt[2][32 * H];
-  const int kvh = blockIdx.x, tblk = blockIdx.z;
+  const int kvh = blockIdx.x, tblk = (int)(gridDim.z - 1 - blockIdx.z);  // the longest walks first
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = lane >> 5, qi = lane & 31;
+  // K rows: 16-byte chunk c of row r at slot c ^ r % CPR, 16 rows on 16 slots.  V rows are read transposed, 32 lanes four chunks of
+  // four consecutive rows: slot c ^ 4 (r % 4), or with 128-byte rows, of which two cover the banks, c ^ 4 (r / 2 % 2)
+  auto v_swizzle = [](int r) __attribute__((always_inline)) { return CPR == 16 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
   int seq = blockIdx.y, row_base = blockIdx.y * a.tpp, T = a.tpp, col0 = a.seg ? 0 : *a.step;
   if (a.seg) {  // ragged pass: the sequence's own rows
     const int4 g = a.seg[blockIdx.y];
@@ -643,17 +646,18 @@ __global__ __launch_bounds__(256) void gqa_fill_kernel(AttnArgs a) {
   const uint32_t span = ((uint32_t)(a.C - 1) * a.Kh + 1) * H * 2;  // rows past the cache read zero
   const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.kcache + ((size_t)seq * a.C * a.Kh + kvh) * H, span);
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(a.vcache + ((size_t)seq * a.C * a.Kh + kvh) * H, span);
-  int toff[NLD];  // tile transfer: load i of this wave moves rows (wave + 4 i) RPD .. + RPD - 1
+  int koff[NLD], voff[NLD];  // tile transfer: load i of this wave moves rows (wave + 4 i) RPD .. + RPD - 1
 #pragma unroll
   for (int i = 0; i < NLD; ++i) {
     const int row_l = (wave + 4 * i) * RPD + lane / CPR;
-    toff[i] = row_l * row_bytes + (((lane % CPR) ^ (row_l % CPR)) * 16);
+    koff[i] = row_l * row_bytes + (((lane % CPR) ^ (row_l % CPR)) * 16);
+    voff[i] = row_l * row_bytes + (((lane % CPR) ^ v_swizzle(row_l)) * 16);
   }
   auto dma_tile = [&](int blk, int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-      load_row_to_lds(rk, &kt[buf][(wave + 4 * i) * RPD * H], toff[i], blk * 32 * row_bytes);
-      load_row_to_lds(rv, &vt[buf][(wave + 4 * i) * RPD * H], toff[i], blk * 32 * row_bytes);
+      load_row_to_lds(rk, &kt[buf][(wave + 4 * i) * RPD * H], koff[i], blk * 32 * row_bytes);
+      load_row_to_lds(rv, &vt[buf][(wave + 4 * i) * RPD * H], voff[i], blk * 32 * row_bytes);
     }
   };
   // input mask of a block: lane p of the lower half fetches the byte of position 32 blk + p early,
@@ -668,6 +672,20 @@ __global__ __launch_bounds__(256) void gqa_fill_kernel(AttnArgs a) {
   for (int c = 0; c < HT; ++c)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[c][r] = 0.f;
+  // This lane's byte offsets in a tile: K, chunk KS h + t of row qi (t: XOR t << 4), and V, chunk 4 c + 2 g2 + q4 / 2 of row 4 h + k4
+  // (c: XOR c << 6; rows 8 and 16 further on: constants)
+  const int k4 = (lane & 15) >> 2, q4 = lane & 3, g2 = (lane >> 4) & 1;
+  const int kbase = qi * H * 2 + (((KS * h) ^ (qi % CPR)) << 4);
+  const int vbase = (4 * h + k4) * H * 2 + (((2 * g2 + (q4 >> 1)) ^ v_swizzle(k4)) << 4) + 8 * (q4 & 1);
+  // Scores stay unscaled, probabilities are powers of two of scale2 (score - m), one fma and one v_exp_f32 each.  m follows
+  // the largest score only when that is 2^8 ahead: any m gives the same quotient, and the accumulators are rescaled at the first
+  // block and seldom after.  Masks are looked at where a block has one or passes a token's own slot.
+  // What bounds it is the instructions beside the 24 MFMAs of a block: 537 with a mask, two multiplies and a subtraction for
+  // every score, rescaling at most blocks and accumulators moved in and out of AGPRs; about 150 so, and 165 registers, three
+  // workgroups a CU instead of two.  8 kv heads of 4 query heads, 3 x 680 tokens behind 1360: 185 -> 106 us, 16 x 192 behind 512:
+  // 82 -> 54, 128 x 32 behind 480: 98 -> 70.
+  const float scale2 = a.scale * 1.44269504089f;
+  const int first_limit = step0 + min(tblk * TQ + wave * TPW, T - 1);  // newest slot of the wave's first token
   float m = -1e30f, l = 0.f;
 
   uint8_t mb = mask_byte(0);
@@ -683,65 +701,65 @@ __global__ __launch_bounds__(256) void gqa_fill_kernel(AttnArgs a) {
     f32x16_t sacc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
-    const uint16_t* kb = &kt[buf][qi * H];
+    // (the bases are opaque here, so that one XOR each makes the addresses of a block where they are used: kept over
+    // the loop they are 24 registers, and three workgroups would not fit a CU)
+    int ka = kbase, va = vbase;
+    asm volatile("" : "+v"(ka), "+v"(va));
+    const char* kb = reinterpret_cast<const char*>(kt[buf]);
+    const char* vb = reinterpret_cast<const char*>(vt[buf]);
 #pragma unroll
     for (int t = 0; t < KS; ++t) {
-      const int slot = ((KS * h + t) ^ (qi % CPR)) * 8;  // lane (position, h) multiplies k = (H / 2) h + 8 t ..
-      const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(kb + slot);
+      const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(kb + (ka ^ (t << 4)));  // lane (position, h) multiplies k = (H / 2) h + 8 t ..
       sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, __builtin_bit_cast(bf16x8_t, qf[t]), sacc, 0, 0, 0);
     }
-    float sc[16];
-    float mn = m;
+    if (mbits != ~0u || blk * 32 + 31 > first_limit) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int pl = acc_row(r, lane), p = blk * 32 + pl;
-      const bool ok = p <= limit && ((mbits >> pl) & 1u);
-      sc[r] = ok ? sacc[r] * a.scale : -1e30f;
-      mn = fmaxf(mn, sc[r]);
+      for (int r = 0; r < 16; ++r) {
+        const int pl = acc_row(r, lane), p = blk * 32 + pl;
+        if (!(p <= limit && ((mbits >> pl) & 1u))) sacc[r] = -1e30f;
+      }
     }
+    float mn = fmaxf(sacc[0], sacc[1]);
+#pragma unroll
+    for (int r = 2; r < 16; r += 2) mn = fmaxf(fmaxf(mn, sacc[r]), sacc[r + 1]);
     mn = fmaxf(mn, __shfl_xor(mn, 32, 64));
-    const float alpha = __expf(m - mn);
-    m = mn;
-    // probabilities as bf16 pairs hi + lo (16 mantissa bits between them), so that the product
-    // keeps the precision of the one-token kernel's f32 probabilities and a scoring pass
-    // reproduces the log-probs of the rollout that generated the tokens
-    float ps = 0.f;
-    uint32_t pk[8], pl2[8];
-#pragma unroll
-    for (int r = 0; r < 16; r += 2) {
-      const float p0 = sc[r] > -1e29f ? __expf(sc[r] - mn) : 0.f;
-      const float p1 = sc[r + 1] > -1e29f ? __expf(sc[r + 1] - mn) : 0.f;
-      pk[r >> 1] = pack_bf2(p0, p1);
-      pl2[r >> 1] = pack_bf2(p0 - bf_lo(pk[r >> 1]), p1 - bf_hi(pk[r >> 1]));
-      ps += p0 + p1;
-    }
-    l = l * alpha + ps;
-    if (__any(alpha != 1.f)) {
+    if (__any((mn - m) * scale2 > 8.f)) {
+      mn = fmaxf(mn, m);
+      const float alpha = __builtin_amdgcn_exp2f((m - mn) * scale2);
+      m = mn;
+      l *= alpha;
 #pragma unroll
       for (int c = 0; c < HT; ++c)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[c][r] *= alpha;
     }
+    const float off = m > -1e29f ? -m * scale2 : 0.f;  // nothing seen yet: every score is masked, and its power of two 0
+    // probabilities as bf16 pairs hi + lo (16 mantissa bits between them), so that the product
+    // keeps the precision of the one-token kernel's f32 probabilities and a scoring pass
+    // reproduces the log-probs of the rollout that generated the tokens
     // out^T += V^T . P^T, 16 positions (accumulator registers 8 kb .. 8 kb + 7) per MFMA
 #pragma unroll
     for (int kb2 = 0; kb2 < 2; ++kb2) {
-      const u32x4_t pf = {pk[4 * kb2], pk[4 * kb2 + 1], pk[4 * kb2 + 2], pk[4 * kb2 + 3]};
-      const u32x4_t pg = {pl2[4 * kb2], pl2[4 * kb2 + 1], pl2[4 * kb2 + 2], pl2[4 * kb2 + 3]};
+      u32x4_t pf, pg;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(sacc[8 * kb2 + 2 * i], scale2, off));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(sacc[8 * kb2 + 2 * i + 1], scale2, off));
+        pf[i] = pack_bf2(p0, p1);
+        pg[i] = pack_bf2(p0 - bf_lo(pf[i]), p1 - bf_hi(pf[i]));
+        l += p0 + p1;
+      }
 #pragma unroll
       for (int c = 0; c < HT; ++c) {
         // V^T fragment: two runs of four consecutive rows of the lane's column, by the transposing LDS read
         // (see gqa_tile_walk): lane (k4, q4) of a group of 16 points at row run + 4 h + k4, columns
         // 32 c + 16 (group % 2) + 4 q4 .. + 3
         typedef short s16x4_t __attribute__((ext_vector_type(4)));
-        const int k4 = (lane & 15) >> 2, q4 = lane & 3, g2 = (lane >> 4) & 1;
         s16x4_t run[2];
 #pragma unroll
-        for (int a2 = 0; a2 < 2; ++a2) {
-          const int row = 16 * kb2 + 8 * a2 + 4 * h + k4;
-          const int chunk = 4 * c + 2 * g2 + (q4 >> 1);
+        for (int a2 = 0; a2 < 2; ++a2)
           run[a2] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(
-              &vt[buf][row * H + ((chunk ^ (row % CPR)) * 8) + 4 * (q4 & 1)]));
-        }
+              vb + (va ^ (c << 6)) + (16 * kb2 + 8 * a2) * H * 2));
         uint32_t vw[4];
         __builtin_memcpy(&vw[0], &run[0], 8);
         __builtin_memcpy(&vw[2], &run[1], 8);
