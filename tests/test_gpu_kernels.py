@@ -1142,6 +1142,16 @@ def test_small_linear_sixteen_columns(M, K, N, group, r, mode):
   test_small_linear_matches_oracle(M, K, N, group, r, mode)
 
 
+# the loads a wave keeps on the way are constants of a variant: 1, 2, 4 and 8 (pairs of) k-tiles and a remainder behind them, with
+# 0 to 2 tiles of A; K of an odd number of k-tiles takes 32 columns per workgroup
+@pytest.mark.parametrize('M,K,N,group,r,mode', [
+    (4, 2048, 64, 64, 16, 'residual'), (2, 3072, 96, 64, 32, 'plain'), (3, 4096, 64, 64, 0, 'plain'), (1, 7168, 32, 64, 16, 'norm'),
+    (1, 1088, 96, 64, 31, 'residual'), (4, 2112, 64, 64, 16, 'plain'), (2, 576, 64, 64, 0, 'norm'), (1, 4160, 64, 64, 32, 'residual'),
+    (2, 768, 128, 64, 16, 'swiglu'), (3, 1088, 64, 64, 1, 'swiglu'), (1, 2304, 128, 64, 0, 'swiglu'), (1, 4352, 64, 64, 11, 'swiglu')])
+def test_small_linear_load_depths(M, K, N, group, r, mode):
+  test_small_linear_matches_oracle(M, K, N, group, r, mode)
+
+
 def test_small_linear_rejects_what_it_cannot_take():
   lib = _lib.lib()
   one = torch.zeros(64, dtype=torch.uint8, device=G.DEV)

@@ -27,16 +27,19 @@ namespace tmx {
 
 constexpr int kSbThreads = 512, kSbWaves = 8;
 constexpr int kSbMaxRows = 4;
-constexpr int kSbMaxTiles = 8;   // k-tiles per wave requested at once
+
+// A lane offset past the end of every descriptor here: the load fetches nothing and gives zero.  Loads that some threads, or some
+// launches, have no use for take it instead of a branch: behind one the compiler no longer knows how many loads are on the way.
+constexpr int kSbNowhere = 0x7FFF0000;
 
 enum { SB_PRO_PLAIN = 0, SB_PRO_NORM = 1, SB_PRO_ATTN = 2 };
 enum { SB_EPI_PLAIN = 0, SB_EPI_RESIDUAL = 1, SB_EPI_SWIGLU = 2 };
 
 // LDS carve of sb_linear_kernel (bytes): x [M][K + 8] bf16 | red [8 waves][4][32] f32 |
-// red_t [8][4][64] f32 | t [4][64] f32 | act [4][32] f32 | row scratch [4 + 8 * 4] f32
+// red_t [8][4][64] f32 | t [4][64] f32 | act [4][32] f32 | row scratch [4 + 8 * 4] f32 | B [2][16][32] bf16 | A_next [4][32][8] bf16
 __host__ __device__ inline size_t sb_x_bytes(int M, int K) { return ((size_t)M * (K + 8) * 2 + 15) & ~(size_t)15; }
 constexpr size_t kSbTailFloats = kSbWaves * kSbMaxRows * 32 + kSbWaves * kSbMaxRows * 64 + kSbMaxRows * 64 +
-                                 kSbMaxRows * 32 + 4 + kSbWaves * 4;
+                                 kSbMaxRows * 32 + 4 + kSbWaves * 4 + 2 * 16 * 32 / 2 + 4 * 32 * 4;
 
 // t handed over as parts by the launch before: a thread adds a run of parts of four adjacent columns of a row (columns
 // 0 .. 4 nq - 1), in up to 32 runs; the runs meet in red_t [run][m][4 nq] and are added in run order.
@@ -240,7 +243,14 @@ template <int PRO> struct SbPrologue { using type = SbMerge; };
 template <> struct SbPrologue<SB_PRO_PLAIN> { using type = SbCopy; };
 template <> struct SbPrologue<SB_PRO_NORM> { using type = SbNorm; };
 
-template <int PRO, int EPI>
+// Loads return in the order they are requested, and a wait counts the ones behind: what is waited for first, the rows, is
+// requested in front of the weights, whose number NT (at least a wave's k-tiles, up to 8 at once) is a constant, as is the
+// number NA of the tiles of A, so that the wait for the rows leaves the others on the way.  Requested behind the weights ("they
+// come from farther") the norm began when the last weight had arrived.  A, which every workgroup reads whole, is 128 KiB a CU
+// beside 64 KiB of weights in gate|up of the 1B shape: requested with the weights it holds them up (11.7 us a launch at one
+// row), a k-tile at a time behind them it costs a round trip each (10.6); requested at once when half the weights are used up:
+// 9.9 (8.2 without an adapter; four rows 12.1 -> 11.3).
+template <int PRO, int EPI, int NT, int NA>
 __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
   extern __shared__ __align__(16) unsigned char sb_smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -256,60 +266,72 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
   float* t_s = red_t + kSbWaves * kSbMaxRows * 64;
   float* act_s = t_s + kSbMaxRows * 64;
   float* rms_s = act_s + kSbMaxRows * 32;  // [4] + per-wave sums [8][4]
+  uint16_t* b_s = reinterpret_cast<uint16_t*>(rms_s + 4 + kSbWaves * 4);  // [CT][16][32]
+  u32x4_t* an_s = reinterpret_cast<u32x4_t*>(b_s + 2 * 16 * 32);          // [4][32]
 
-  // column tile of this wave; its first weight tiles and scales are requested before anything else
+  // what the epilogue needs that depends on no other launch: the B values of the column tile(s) (rows 0..15 of B; a larger
+  // rank reads the rest in the epilogue), the residual, and the rows of the next projection's A
+  const bool epi_thread = tid < kSbMaxRows * 32 && (tid >> 5) < M;
+  const int em = tid >> 5, ej = tid & 31;
+  // (one 16-byte load of a wave: column tile q of B by wave q, lane (row, piece); the 32 rows of A_next by waves 2 and 3; they
+  // meet the threads that use them in LDS.  As 16 or 32 values of two bytes a thread they held up the loads behind them)
+  uint32_t res_v = 0;
+  u32x4_t aux;
+  {
+    const bool of_b = wave < CT;
+    const int n0 = ((int)blockIdx.x + wave * (EPI == SB_EPI_SWIGLU ? a.pair_off : 0)) * 32;
+    // rows k .. k + 7 of column j are 8 consecutive values in fragment order (r_pad 32): ((kb * 4 + t) * 64 + 32 h + j) * 8 with
+    // k = 64 kb + 16 t + 8 h, so the 32 rows from 32 blockIdx.x on are 2 KiB
+    const bool of_next = EPI == SB_EPI_SWIGLU && (wave >> 1) == 1 && a.a_next;
+    const void* src = of_b ? (const void*)a.lora_b : (const void*)a.a_next;
+    const uint32_t bytes = of_b ? (a.lora_b ? (uint32_t)a.lora_r * a.N * 2u : 0u) : of_next ? (uint32_t)gridDim.x * 2048u : 0u;
+    aux = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(src, bytes), of_b ? ((lane >> 2) * a.N + n0) * 2 + (lane & 3) * 16 : lane * 16,
+                                                of_b ? 0 : (int)blockIdx.x * 2048 + (wave & 1) * 1024, 0);
+    if constexpr (EPI == SB_EPI_RESIDUAL)
+      res_v = __builtin_amdgcn_raw_buffer_load_b16(make_rsrc(a.residual, (uint32_t)M * a.ldy * 2u),
+                                                   epi_thread ? (em * a.ldy + (int)blockIdx.x * 32 + ej) * 2 : kSbNowhere, 0, 0);
+  }
+  // parts of t and the rows
+  SbParts parts;
+  parts.request(a);  // handed over for single matrices only (down projection)
+  typename SbPrologue<PRO>::type pro;
+  pro.request(a);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // column tile of this wave: its first weight tiles and scales
   const int nb = EPI == SB_EPI_SWIGLU ? (int)blockIdx.x + c * a.pair_off : (int)blockIdx.x;
   const int per = (KT + KS - 1) / KS;  // k-tiles per slice
   const int kt0 = s * per, kt1 = min(kt0 + per, KT);
   const int gs = __builtin_ctz(a.G >> 6), KG = K / a.G;
   const u32x4_t* wsrc = reinterpret_cast<const u32x4_t*>(a.qw) + (size_t)nb * KT * 64 + lane;
   const uint16_t* ssrc = a.scales + (size_t)nb * KG * 32 + nl;
-  u32x4_t wr[kSbMaxTiles];
-  uint16_t sr[kSbMaxTiles];
+  u32x4_t wr[NT];
+  uint32_t sr[NT];
+  auto load_w = [&](int kt, int slot) __attribute__((always_inline)) {
+    kt = min(kt, KT - 1);
+    wr[slot] = __builtin_nontemporal_load(wsrc + (size_t)kt * 64);  // every tile is read once, by this wave
+    sr[slot] = ssrc[(size_t)(kt >> gs) * 32];
+  };
 #pragma unroll
-  for (int i = 0; i < kSbMaxTiles; ++i) {
-    if (i < per) {
-      const int kt = min(kt0 + i, KT - 1);
-      wr[i] = __builtin_nontemporal_load(wsrc + (size_t)kt * 64);  // every tile is read once, by this wave
-      sr[i] = ssrc[(size_t)(kt >> gs) * 32];
-    }
+  for (int i = 0; i < NT; ++i) load_w(kt0 + i, i);
+  // x . A: wave w takes the w-th eighth of K, i.e. the c-th part of its own slice
+  constexpr int LT = NT < 4 / (NA ? NA : 1) ? NT : 4 / (NA ? NA : 1);  // k-tiles of A per wave requested at once
+  const int lpart = (per + CT - 1) / CT, l0 = kt0 + c * lpart, nk = min(lpart, kt1 - l0);
+  u32x4_t ab[LT][NA ? NA : 1][4];  // [slot][tile of A][step]
+  // the epilogue uses the t columns of its own segment(s) only: the tiles of A that hold them
+  const int RT = a.Rpad >> 5;  // 32-column tiles of A (<= 2)
+  int q0 = 0;
+  if (NA && CT == 1) {
+    const int n0 = blockIdx.x * 32;
+    const int seg = n0 >= a.seg_end[0] ? (n0 >= a.seg_end[1] ? 2 : 1) : 0;
+    q0 = min((seg * a.lora_r) >> 5, RT - NA);
   }
-  // Everything the epilogue needs that depends on no other launch is requested now as well, so that its
-  // latency hides behind the weight stream: the B values of this thread's column(s) (rows 0..15 of B; a
-  // larger rank reads the rest in the epilogue), the residual, and the rows of the next projection's A.
-  const bool epi_thread = tid < kSbMaxRows * 32 && (tid >> 5) < M;
-  const int em = tid >> 5, ej = tid & 31;
-  uint16_t breg[CT][16];
-  uint16_t res_v = 0;
-  uint4 anx[EPI == SB_EPI_SWIGLU ? 4 : 1];  // A_next[32 blockIdx.x + 8 u .. + 7][ej], u = 0..3
-  if (epi_thread) {
-    if (a.lora_b) {
+  auto load_a = [&](int k, int slot) __attribute__((always_inline)) {
+    const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + ((size_t)min(l0 + k, KT - 1) * RT + q0) * 256 + lane;
 #pragma unroll
-      for (int q = 0; q < CT; ++q) {
-        const int n = ((int)blockIdx.x + q * (EPI == SB_EPI_SWIGLU ? a.pair_off : 0)) * 32 + ej;
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) breg[q][rr] = a.lora_b[(size_t)min(rr, a.lora_r - 1) * a.N + n];
-      }
-    }
-    if constexpr (EPI == SB_EPI_RESIDUAL) res_v = a.residual[(size_t)em * a.ldy + blockIdx.x * 32 + ej];
-    if constexpr (EPI == SB_EPI_SWIGLU) {
-      if (a.a_next) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          // rows k .. k + 7 of column ej are 8 consecutive values in fragment order (r_pad 32):
-          // ((kb * 4 + t) * 64 + 32 h + ej) * 8 with k = 64 kb + 16 t + 8 h
-          const int k = blockIdx.x * 32 + u * 8;
-          const int kb = k >> 6, rem = k & 63, t = rem >> 4, hh = (rem >> 3) & 1;
-          anx[u] = *reinterpret_cast<const uint4*>(a.a_next + ((((size_t)kb * 4 + t) * 64) + 32 * hh + ej) * 8);
-        }
-      }
-    }
-  }
-  // parts of t and the rows: requested behind the weights (which come from farther), before anything is waited for
-  SbParts parts;
-  parts.request(a);  // handed over for single matrices only (down projection)
-  typename SbPrologue<PRO>::type pro;
-  pro.request(a);
+    for (int i = 0; i < NA * 4; ++i) ab[slot][i / 4][i % 4] = ap[i * 64];
+  };
+  __builtin_amdgcn_sched_barrier(0);
 
   // ---- prologue: the activations of every row into LDS ----
   parts.finish(a, red_t);
@@ -319,79 +341,61 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
   // ---- the K-slice of this wave: its column tile, and its share of x . A ----
   const int xrow = min(nl, M - 1);  // rows beyond the batch repeat the last one (their results are dropped)
   const uint16_t* xb = xs + xrow * XS + h * 8;
-  f32x16_t acc;
+  f32x16_t acc, tacc[2];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  const bool lora_here = a.a_t != nullptr;
-  const int RT = a.Rpad >> 5;  // 32-column tiles of A (<= 2)
-  // the epilogue uses the t columns of its own segment(s) only: the tiles of A that hold them
-  int q0 = 0, q1 = RT - 1;
-  if (CT == 1 && lora_here) {
-    const int n0 = blockIdx.x * 32;
-    const int seg = n0 >= a.seg_end[0] ? (n0 >= a.seg_end[1] ? 2 : 1) : 0;
-    q0 = (seg * a.lora_r) >> 5;
-    q1 = min(((seg + 1) * a.lora_r - 1) >> 5, RT - 1);
-  }
-  f32x16_t tacc[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) tacc[q][r] = 0.f;
-  // x . A: wave w takes the w-th eighth of K, i.e. the c-th part of its own slice, so the x fragments are
-  // the ones it reads anyway.  The A tiles of a k-tile are requested one k-tile ahead.
-  const int lpart = (per + CT - 1) / CT;
-  auto mine = [&](int i) { return lora_here && i >= c * lpart && i < (c + 1) * lpart && kt0 + i < kt1; };
-  u32x4_t ab[2][2][4];  // [parity of the k-tile][tile of A][step]
-  auto load_a = [&](int i, auto pc) __attribute__((always_inline)) {
-    constexpr int p = decltype(pc)::value;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      if (q < q0 || q > q1) continue;
-      const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + ((size_t)((kt0 + i) * RT + q) * 4) * 64 + lane;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) ab[p][q][t] = ap[t * 64];
-    }
-  };
-  if (mine(0)) load_a(0, IC<0>{});
-  for (int base = 0; base < per; base += kSbMaxTiles) {
-    static_for<kSbMaxTiles>([&](auto ic) __attribute__((always_inline)) {
+  for (int r = 0; r < 16; ++r) acc[r] = tacc[0][r] = tacc[1][r] = 0.f;
+  for (int base = 0; base < per; base += NT) {
+    static_for<NT>([&](auto ic) __attribute__((always_inline)) {
       constexpr int i = decltype(ic)::value;
+      if constexpr (NA > 0 && i == NT / 2) {
+        if (base == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int d = 0; d < LT; ++d) load_a(d, d);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
       const int kt = kt0 + base + i;
       if (kt < kt1) {
-        if (mine(base + i + 1)) load_a(base + i + 1, IC<(i + 1) & 1>{});
         bf16x8_t xa[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) xa[t] = *reinterpret_cast<const bf16x8_t*>(xb + kt * 64 + t * 16);
-        const NibbleScale sc = nibble_scale(bf2f(sr[i]));
+        const NibbleScale sc = nibble_scale(bf2f((uint16_t)sr[i]));
         const uint32_t wd[4] = {wr[i].x, wr[i].y, wr[i].z, wr[i].w};
-        if (base + i + kSbMaxTiles < per) {  // slot consumed: refill it for the tile 8 further on
-          const int ktn = min(kt + kSbMaxTiles, KT - 1);
-          wr[i] = __builtin_nontemporal_load(wsrc + (size_t)ktn * 64);
-          sr[i] = ssrc[(size_t)(ktn >> gs) * 32];
-        }
+        if (base + i + NT < per) load_w(kt + NT, i);  // slot consumed: refill it for the tile NT further on
 #pragma unroll
         for (int t = 0; t < 4; ++t)
           acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[t], dequant_word(wd[t], sc), acc, 0, 0, 0);
-        if (mine(base + i)) {
-#pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            if (q < q0 || q > q1) continue;
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-              tacc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[t], __builtin_bit_cast(bf16x8_t, ab[i & 1][q][t]), tacc[q], 0, 0, 0);
-          }
-        }
       }
     });
   }
+  if constexpr (NA > 0) {
+    for (int k0 = 0; k0 < nk; k0 += LT)
+      static_for<LT>([&](auto dc) __attribute__((always_inline)) {
+        constexpr int d = decltype(dc)::value;
+        const int k = k0 + d;
+        if (k < nk) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const bf16x8_t xa = *reinterpret_cast<const bf16x8_t*>(xb + (l0 + k) * 64 + t * 16);
+#pragma unroll
+            for (int u = 0; u < NA; ++u)
+              tacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, __builtin_bit_cast(bf16x8_t, ab[d][u][t]), tacc[u], 0, 0, 0);
+          }
+          if (k + LT < nk) load_a(k + LT, d);
+        }
+      });
+  }
+  if (wave < CT) reinterpret_cast<u32x4_t*>(b_s)[wave * 64 + lane] = aux;
+  else if (EPI == SB_EPI_SWIGLU && (wave >> 1) == 1) an_s[(wave & 1) * 64 + lane] = aux;
   // rows 0..3 of a tile are accumulator registers 0..3 of the lanes with h == 0
   if (h == 0) {
 #pragma unroll
     for (int r = 0; r < kSbMaxRows; ++r) {
       red[(wave * kSbMaxRows + r) * 32 + nl] = acc[r];
-      if (!a.t_parts) {
-        red_t[(wave * kSbMaxRows + r) * 64 + nl] = tacc[0][r];
-        red_t[(wave * kSbMaxRows + r) * 64 + 32 + nl] = tacc[1][r];
+      if constexpr (NA > 0) {
+#pragma unroll
+        for (int u = 0; u < NA; ++u) red_t[(wave * kSbMaxRows + r) * 64 + (q0 + u) * 32 + nl] = tacc[u][r];
       }
     }
   }
@@ -403,7 +407,8 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
     if (m < M) {
       if (a.t_parts) {
         t = sb_parts_total(parts, red_t, m, cc);
-      } else if (lora_here) {
+      } else if (NA && (cc >> 5) >= q0 && (cc >> 5) < q0 + NA) {
+#pragma unroll
         for (int w = 0; w < kSbWaves; ++w) t += red_t[(w * kSbMaxRows + m) * 64 + cc];
       }
     }
@@ -428,7 +433,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
         const float* tp = t_s + m * 64 + seg * a.lora_r;
         float d = 0.f;
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr) d = fmaf(rr < a.lora_r ? tp[rr] : 0.f, bf2f(breg[q][rr]), d);
+        for (int rr = 0; rr < 16; ++rr) d = fmaf(rr < a.lora_r ? tp[rr] : 0.f, bf2f(b_s[(q * 16 + rr) * 32 + j]), d);
         for (int rr = 16; rr < a.lora_r; ++rr) d = fmaf(tp[rr], bf2f(a.lora_b[(size_t)rr * a.N + n]), d);
         b = rbf(b + rbf(rbf(d) * a.lora_ls));
       }
@@ -443,7 +448,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
     } else {
       const int n = blockIdx.x * 32 + j;
       float v = yv[0];
-      if constexpr (EPI == SB_EPI_RESIDUAL) v = rbf(v + bf2f(res_v));
+      if constexpr (EPI == SB_EPI_RESIDUAL) v = rbf(v + bf2f((uint16_t)res_v));
       a.y[(size_t)m * a.ldy + n] = f2bf(v);
     }
   }
@@ -455,7 +460,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
         float t = 0.f;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const uint32_t w[4] = {anx[u].x, anx[u].y, anx[u].z, anx[u].w};
+          const u32x4_t w = an_s[u * 32 + ej];
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj) {
             t = fmaf(act_s[em * 32 + u * 8 + 2 * jj], bf_lo(w[jj]), t);
@@ -477,15 +482,14 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear_kernel(SbLinearArgs a) {
 // The 16 x 16 x 32 MFMA takes them: lane (n = l % 16, q = l / 16) holds column n of k-tile 2 p + q / 2, half q % 2, so a
 // wave's load is two half tiles, and word t of the four lanes of a column is 32 consecutive steps of the contraction
 // (the x operand reads the same k).  Measured on the 1B shape at one row / three rows (trace, us per launch,
-// 32 columns -> 16): q|k|v 8.0 / 9.1 -> 8.0 / 9.0, o 9.3 / 15.6 -> 7.4 / 9.6, down 11.8 / 14.4 -> 9.8 / 13.0 (less since, see
-// below and SbCopy).
-constexpr int kSbPairs = 8;  // k-tile pairs per wave requested at once
-constexpr int kSbLoraTiles = 4;  // k-tiles of A per wave requested at once
+// 32 columns -> 16): q|k|v 8.0 / 9.1 -> 8.0 / 9.0, o 9.3 / 15.6 -> 7.4 / 9.6, down 11.8 / 14.4 -> 9.8 / 13.0 (see
+// also SbCopy); with the rows requested before the weights, and the numbers of loads constants (see sb_linear_kernel), at one row
+// 6.7 -> 6.1, 6.4 -> 5.9 and, without the x . A that is handed over, 9.0 -> 7.6.
 
-// LDS: x [M][K + 8] bf16 | red [8 waves][4][16] f32 | red_t [8][4][64] f32 | t [4][64] f32 | row scratch [4 + 8 * 4] f32
-constexpr size_t kSb16TailFloats = kSbWaves * kSbMaxRows * 16 + kSbWaves * kSbMaxRows * 64 + kSbMaxRows * 64 + 4 + kSbWaves * 4;
+// LDS: x [M][K + 8] bf16 | red [8 waves][4][16] f32 | red_t [8][4][64] f32 | t [4][64] f32 | row scratch [4 + 8 * 4] f32 | B [16][16] bf16
+constexpr size_t kSb16TailFloats = kSbWaves * kSbMaxRows * 16 + kSbWaves * kSbMaxRows * 64 + kSbMaxRows * 64 + 4 + kSbWaves * 4 + 16 * 16 / 2;
 
-template <int PRO, int EPI>
+template <int PRO, int EPI, int NT, int NQ>  // pairs of k-tiles per wave requested at once (1 to 8), tiles of 16 columns of A (0 to 2)
 __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a) {
   extern __shared__ __align__(16) unsigned char sb_smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -497,6 +501,27 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
   float* red_t = red + kSbWaves * kSbMaxRows * 16;
   float* t_s = red_t + kSbWaves * kSbMaxRows * 64;
   float* rms_s = t_s + kSbMaxRows * 64;  // [4] + per-wave sums [8][4]
+  uint16_t* b_s = reinterpret_cast<uint16_t*>(rms_s + 4 + kSbWaves * 4);  // [16][16]
+
+  // what the epilogue needs and no other launch makes
+  const bool epi_thread = tid < kSbMaxRows * 16 && (tid >> 4) < M;
+  const int em = tid >> 4, n = (int)blockIdx.x * 16 + (tid & 15);
+  uint32_t res_v = 0;
+  u32x4_t aux;  // rows 0..15 of B, by the first 32 threads (see sb_linear_kernel)
+  {
+    aux = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(a.lora_b, a.lora_b ? (uint32_t)a.lora_r * a.N * 2u : 0u),
+                                                tid < 32 ? ((tid >> 1) * a.N + (int)blockIdx.x * 16) * 2 + (tid & 1) * 16 : kSbNowhere, 0, 0);
+    if constexpr (EPI == SB_EPI_RESIDUAL)
+      res_v = __builtin_amdgcn_raw_buffer_load_b16(make_rsrc(a.residual, (uint32_t)M * a.ldy * 2u),
+                                                   epi_thread ? (em * a.ldy + n) * 2 : kSbNowhere, 0, 0);
+  }
+
+  // parts of t and the rows: in front of the weights, see sb_linear_kernel
+  SbParts parts;
+  parts.request(a);  // handed over for single matrices only (down projection)
+  typename SbPrologue<PRO>::type pro;
+  pro.request(a);
+  __builtin_amdgcn_sched_barrier(0);
 
   // weights and scales of this wave's pairs
   const int nb = (int)blockIdx.x >> 1, half16 = ((int)blockIdx.x & 1) * 16;
@@ -504,68 +529,40 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
   const int gs = __builtin_ctz(a.G >> 6), KG = K / a.G;
   const u32x4_t* wsrc = reinterpret_cast<const u32x4_t*>(a.qw) + ((size_t)nb * KT + par) * 64 + 32 * h + half16 + n16;
   const uint16_t* ssrc = a.scales + (size_t)nb * KG * 32 + half16 + n16;
-  u32x4_t wr[kSbPairs];
-  uint16_t sr[kSbPairs];
+  u32x4_t wr[NT];
+  uint32_t sr[NT];
   auto load_w = [&](int p, int slot) __attribute__((always_inline)) {
     p = min(p, KP - 1);
     wr[slot] = __builtin_nontemporal_load(wsrc + (size_t)p * 128);
     sr[slot] = ssrc[(size_t)((2 * p + par) >> gs) * 32];
   };
 #pragma unroll
-  for (int i = 0; i < kSbPairs; ++i)
-    if (i < per) load_w(p0 + i, i);
+  for (int i = 0; i < NT; ++i) load_w(p0 + i, i);
 
   // x . A of this wave's eighth of K, for the tiles of 16 columns of A that hold this workgroup's segment (of a rank of 16
   // half of what lies in a tile of 32 is another segment's or padding: 64 KB instead of 128 KB of A per workgroup on the 1B
   // shape, one row / three rows: q|k|v 8.0 / 9.1 -> 7.0 / 7.8 us, o 7.5 / 9.8 -> 6.4 / 8.7), the first of them requested now.
   // The four lane groups of a load hold 32 consecutive steps of the contraction.
-  const bool lora_here = a.a_t != nullptr;
-  int q0 = 0, nq = 0;
-  if (lora_here) {
+  constexpr int LT = NT == 1 ? 2 : 4;  // k-tiles of A per wave requested at once
+  int q0 = 0;
+  if constexpr (NQ > 0) {
     const int n0 = (int)blockIdx.x * 16;
     const int seg = n0 >= a.seg_end[0] ? (n0 >= a.seg_end[1] ? 2 : 1) : 0;
-    q0 = (seg * a.lora_r) >> 4;
-    nq = min(((seg + 1) * a.lora_r - 1) >> 4, (a.Rpad >> 4) - 1) - q0 + 1;  // 1 or 2: r <= 32, and 3 r <= 64 where there are segments
+    q0 = min((seg * a.lora_r) >> 4, (a.Rpad >> 4) - NQ);
   }
   const int RT = a.Rpad >> 5;
   const int lper = (KT + kSbWaves - 1) / kSbWaves, l0 = wave * lper, nk = min(lper, KT - l0);
-  u32x4_t ab[8][2];
-  // The count as a constant: straight code, whose LDS reads and products are in flight together.  With one loop for all counts
-  // rank 32 took 8.7 us at 1 x 2048 x 3072 and 20.2 at 1 x 8192 x 2048 (now 7.4 and 13.1), rank 16 7.5 and 12.8 (7.4 and 11.2).
-  auto by_nq = [&](auto&& f) __attribute__((always_inline)) {
-    if (nq == 1) f(IC<1>{});
-    else if (nq == 2) f(IC<2>{});
-  };
-  // k-tile k of this wave into slot d
-  auto load_a = [&](auto nqc, int k, auto dc) __attribute__((always_inline)) {
-    constexpr int NQ = decltype(nqc)::value, d = decltype(dc)::value;
-    if (k < nk) {
-      const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + ((size_t)(l0 + k) * RT * 4 + par) * 64 + 32 * h + n16;
+  u32x4_t ab[LT][NQ ? NQ : 1][2];
+  auto load_a = [&](int k, int slot) __attribute__((always_inline)) {
+    const u32x4_t* ap = reinterpret_cast<const u32x4_t*>(a.a_t) + ((size_t)min(l0 + k, KT - 1) * RT * 4 + par) * 64 + 32 * h + n16;
 #pragma unroll
-      for (int i = 0; i < 2 * NQ; ++i) ab[d * NQ + i / 2][i % 2] = ap[((q0 + i / 2) >> 1) * 256 + ((q0 + i / 2) & 1) * 16 + i % 2 * 128];
-    }
+    for (int i = 0; i < 2 * NQ; ++i) ab[slot][i / 2][i % 2] = ap[((q0 + i / 2) >> 1) * 256 + ((q0 + i / 2) & 1) * 16 + i % 2 * 128];
   };
-  by_nq([&](auto nqc) __attribute__((always_inline)) {
-    static_for<kSbLoraTiles>([&](auto dc) __attribute__((always_inline)) { load_a(nqc, decltype(dc)::value, dc); });
-  });
-
-  // what the epilogue needs and no other launch makes
-  const bool epi_thread = tid < kSbMaxRows * 16 && (tid >> 4) < M;
-  const int em = tid >> 4, n = (int)blockIdx.x * 16 + (tid & 15);
-  uint16_t breg[16], res_v = 0;
-  if (epi_thread) {
-    if (a.lora_b) {
+  if constexpr (NQ > 0) {
 #pragma unroll
-      for (int rr = 0; rr < 16; ++rr) breg[rr] = a.lora_b[(size_t)min(rr, a.lora_r - 1) * a.N + n];
-    }
-    if constexpr (EPI == SB_EPI_RESIDUAL) res_v = a.residual[(size_t)em * a.ldy + n];
+    for (int i = 0; i < LT; ++i) load_a(i, i);
   }
-
-  // parts of t and the rows: requested behind the weights (which come from farther), before anything is waited for
-  SbParts parts;
-  parts.request(a);  // handed over for single matrices only (down projection)
-  typename SbPrologue<PRO>::type pro;
-  pro.request(a);
+  __builtin_amdgcn_sched_barrier(0);
 
   // ---- prologue: the activations of every row into LDS ----
   parts.finish(a, red_t);
@@ -575,54 +572,51 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
   // ---- this wave's pairs of k-tiles ----
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   const uint16_t* xb = xs + min(n16, M - 1) * XS + par * 64 + h * 8;  // rows beyond the batch repeat the last one
-  for (int base = 0; base < per; base += kSbPairs) {
-    static_for<kSbPairs>([&](auto ic) __attribute__((always_inline)) {
+  for (int base = 0; base < per; base += NT) {
+    static_for<NT>([&](auto ic) __attribute__((always_inline)) {
       constexpr int i = decltype(ic)::value;
       const int p = p0 + base + i;
       if (p < p1) {
         bf16x8_t xa[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) xa[t] = *reinterpret_cast<const bf16x8_t*>(xb + p * 128 + t * 16);
-        const NibbleScale sc = nibble_scale(bf2f(sr[i]));
+        const NibbleScale sc = nibble_scale(bf2f((uint16_t)sr[i]));
         const uint32_t wd[4] = {wr[i].x, wr[i].y, wr[i].z, wr[i].w};
-        if (base + i + kSbPairs < per) load_w(p + kSbPairs, i);
+        if (base + i + NT < per) load_w(p + NT, i);
 #pragma unroll
         for (int t = 0; t < 4; ++t)
           acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[t], dequant_word(wd[t], sc), acc, 0, 0, 0);
       }
     });
   }
-  if (lora_here) {
-    f32x4_t tacc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  if constexpr (NQ > 0) {
+    f32x4_t tacc[NQ];
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) tacc[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const uint16_t* lb = xs + min(n16, M - 1) * XS + l0 * 64 + par * 16 + h * 8;
-    by_nq([&](auto nqc) __attribute__((always_inline)) {
-      constexpr int NQ = decltype(nqc)::value, D = kSbLoraTiles;
-      for (int k0 = 0; k0 < nk; k0 += D) {
-        static_for<D>([&](auto dc) __attribute__((always_inline)) {
-          constexpr int d = decltype(dc)::value;
-          const int k = k0 + d;
-          if (k < nk) {
+    for (int k0 = 0; k0 < nk; k0 += LT)
+      static_for<LT>([&](auto dc) __attribute__((always_inline)) {
+        constexpr int d = decltype(dc)::value;
+        const int k = k0 + d;
+        if (k < nk) {
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-              const bf16x8_t xa = *reinterpret_cast<const bf16x8_t*>(lb + k * 64 + s * 32);
+          for (int s = 0; s < 2; ++s) {
+            const bf16x8_t xa = *reinterpret_cast<const bf16x8_t*>(lb + k * 64 + s * 32);
 #pragma unroll
-              for (int u = 0; u < NQ; ++u)
-                tacc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8_t, ab[d * NQ + u][s]), tacc[u], 0, 0, 0);
-            }
+            for (int u = 0; u < NQ; ++u)
+              tacc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8_t, ab[d][u][s]), tacc[u], 0, 0, 0);
           }
-          load_a(nqc, k + D, dc);
-        });
-      }
-    });
+          if (k + LT < nk) load_a(k + LT, d);
+        }
+      });
     if (q == 0) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-        if (u < nq) {
+      for (int u = 0; u < NQ; ++u)
 #pragma unroll
-          for (int r = 0; r < kSbMaxRows; ++r) red_t[(wave * kSbMaxRows + r) * 64 + (q0 + u) * 16 + n16] = tacc[u][r];
-        }
+        for (int r = 0; r < kSbMaxRows; ++r) red_t[(wave * kSbMaxRows + r) * 64 + (q0 + u) * 16 + n16] = tacc[u][r];
     }
   }
+  if (tid < 32) reinterpret_cast<u32x4_t*>(b_s)[tid] = aux;
   if (q == 0) {  // rows 0..3 of the 16 x 16 tile: registers 0..3 of lanes 0..15
 #pragma unroll
     for (int r = 0; r < kSbMaxRows; ++r) red[(wave * kSbMaxRows + r) * 16 + n16] = acc[r];
@@ -635,7 +629,7 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
     if (m < M) {
       if (a.t_parts) {
         t = sb_parts_total(parts, red_t, m, cc);
-      } else if (lora_here && (cc >> 4) >= q0 && (cc >> 4) < q0 + nq) {
+      } else if (NQ && (cc >> 4) >= q0 && (cc >> 4) < q0 + NQ) {
 #pragma unroll
         for (int w = 0; w < kSbWaves; ++w) t += red_t[(w * kSbMaxRows + m) * 64 + cc];
       }
@@ -653,35 +647,71 @@ __global__ __launch_bounds__(kSbThreads) void sb_linear16_kernel(SbLinearArgs a)
       const float* tp = t_s + em * 64 + seg * a.lora_r;
       float d = 0.f;
 #pragma unroll
-      for (int rr = 0; rr < 16; ++rr) d = fmaf(rr < a.lora_r ? tp[rr] : 0.f, bf2f(breg[rr]), d);
+      for (int rr = 0; rr < 16; ++rr) d = fmaf(rr < a.lora_r ? tp[rr] : 0.f, bf2f(b_s[rr * 16 + (tid & 15)]), d);
       for (int rr = 16; rr < a.lora_r; ++rr) d = fmaf(tp[rr], bf2f(a.lora_b[(size_t)rr * a.N + n]), d);
       b = rbf(b + rbf(rbf(d) * a.lora_ls));
     }
-    if constexpr (EPI == SB_EPI_RESIDUAL) b = rbf(b + bf2f(res_v));
+    if constexpr (EPI == SB_EPI_RESIDUAL) b = rbf(b + bf2f((uint16_t)res_v));
     a.y[(size_t)em * a.ldy + n] = f2bf(b);
   }
 }
 
 size_t sb_linear_lds(int M, int K) { return sb_x_bytes(M, K) + kSbTailFloats * 4; }
 
-template <int PRO, int EPI>
+template <int PRO, int EPI, int NT, int NA>
 static int launch_sb(hipStream_t st, const SbLinearArgs& a, int blocks) {
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&sb_linear_kernel<PRO, EPI>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+      reinterpret_cast<const void*>(&sb_linear_kernel<PRO, EPI, NT, NA>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
   if (attr != hipSuccess) return TMX_ERR_LAUNCH;
-  hipLaunchKernelGGL((sb_linear_kernel<PRO, EPI>), dim3(blocks), dim3(kSbThreads), sb_linear_lds(a.M, a.K), st, a);
+  hipLaunchKernelGGL((sb_linear_kernel<PRO, EPI, NT, NA>), dim3(blocks), dim3(kSbThreads), sb_linear_lds(a.M, a.K), st, a);
   return check_launch();
+}
+// tiles of A that hold the columns of any workgroup's segment
+static int sb_a_tiles(const SbLinearArgs& a, bool pairs, int width) {
+  if (!a.a_t) return 0;
+  if (pairs) return a.Rpad / width;  // gate and up columns meet in a workgroup
+  int n = 1;
+  for (int seg = 0; seg < (a.seg_end[0] < a.N ? (a.seg_end[1] < a.N ? 3 : 2) : 1); ++seg) {
+    const int q0 = seg * a.lora_r / width, q1 = ((seg + 1) * a.lora_r - 1) / width;
+    if (q1 - q0 + 1 > n) n = q1 - q0 + 1;
+  }
+  return n < a.Rpad / width ? n : a.Rpad / width;
+}
+template <int PRO, int EPI, int NT>
+static int launch_sb_a(hipStream_t st, const SbLinearArgs& a, int blocks) {
+  switch (sb_a_tiles(a, EPI == SB_EPI_SWIGLU, 32)) {
+    case 0: return launch_sb<PRO, EPI, NT, 0>(st, a, blocks);
+    case 1: return launch_sb<PRO, EPI, NT, 1>(st, a, blocks);
+    default: return launch_sb<PRO, EPI, NT, 2>(st, a, blocks);
+  }
 }
 
 size_t sb_linear16_lds(int M, int K) { return sb_x_bytes(M, K) + kSb16TailFloats * 4; }
 
-template <int PRO, int EPI>
+template <int PRO, int EPI, int NT, int NQ>
 static int launch_sb16(hipStream_t st, const SbLinearArgs& a) {
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&sb_linear16_kernel<PRO, EPI>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+      reinterpret_cast<const void*>(&sb_linear16_kernel<PRO, EPI, NT, NQ>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
   if (attr != hipSuccess) return TMX_ERR_LAUNCH;
-  hipLaunchKernelGGL((sb_linear16_kernel<PRO, EPI>), dim3(a.N / 16), dim3(kSbThreads), sb_linear16_lds(a.M, a.K), st, a);
+  hipLaunchKernelGGL((sb_linear16_kernel<PRO, EPI, NT, NQ>), dim3(a.N / 16), dim3(kSbThreads), sb_linear16_lds(a.M, a.K), st, a);
   return check_launch();
+}
+template <int PRO, int EPI, int NT>
+static int launch_sb16_a(hipStream_t st, const SbLinearArgs& a) {
+  switch (sb_a_tiles(a, false, 16)) {
+    case 0: return launch_sb16<PRO, EPI, NT, 0>(st, a);
+    case 1: return launch_sb16<PRO, EPI, NT, 1>(st, a);
+    default: return launch_sb16<PRO, EPI, NT, 2>(st, a);
+  }
+}
+// as many requests at once as a wave has k-tiles (pairs), at most 8
+template <int PRO, int EPI>
+static int launch_sb16_t(hipStream_t st, const SbLinearArgs& a) {
+  const int per = ((a.K >> 7) + kSbWaves - 1) / kSbWaves;
+  if (per <= 1) return launch_sb16_a<PRO, EPI, 1>(st, a);
+  if (per <= 2) return launch_sb16_a<PRO, EPI, 2>(st, a);
+  if (per <= 4) return launch_sb16_a<PRO, EPI, 4>(st, a);
+  return launch_sb16_a<PRO, EPI, 8>(st, a);
 }
 
 bool sb_linear_ok(int M, int K, int N, int G, int rank, int rpad, bool norm) {
@@ -696,20 +726,24 @@ int sb_linear(hipStream_t st, const SbLinearArgs& a, int pro, int epi) {
   if (!sb_linear_ok(a.M, a.K, a.N, a.G, a.lora_r, a.Rpad, pro == SB_PRO_NORM)) return TMX_ERR_SHAPE;
   if (epi == SB_EPI_SWIGLU) {
     if (pro != SB_PRO_NORM || a.N % 64) return TMX_ERR_UNSUPPORTED;
-    return launch_sb<SB_PRO_NORM, SB_EPI_SWIGLU>(st, a, a.N / 64);
+    const int per = ((a.K >> 6) + kSbWaves / 2 - 1) / (kSbWaves / 2);
+    if (per <= 1) return launch_sb_a<SB_PRO_NORM, SB_EPI_SWIGLU, 1>(st, a, a.N / 64);
+    if (per <= 2) return launch_sb_a<SB_PRO_NORM, SB_EPI_SWIGLU, 2>(st, a, a.N / 64);
+    if (per <= 4) return launch_sb_a<SB_PRO_NORM, SB_EPI_SWIGLU, 4>(st, a, a.N / 64);
+    return launch_sb_a<SB_PRO_NORM, SB_EPI_SWIGLU, 8>(st, a, a.N / 64);
   }
   // whole pairs of k-tiles and segment ends on 16 columns: 16 columns per workgroup
   if (a.K % 128 == 0 && a.seg_end[0] % 16 == 0 && a.seg_end[1] % 16 == 0) {
-    if (pro == SB_PRO_NORM && epi == SB_EPI_PLAIN) return launch_sb16<SB_PRO_NORM, SB_EPI_PLAIN>(st, a);
-    if (pro == SB_PRO_ATTN && epi == SB_EPI_RESIDUAL) return launch_sb16<SB_PRO_ATTN, SB_EPI_RESIDUAL>(st, a);
-    if (pro == SB_PRO_PLAIN && epi == SB_EPI_RESIDUAL) return launch_sb16<SB_PRO_PLAIN, SB_EPI_RESIDUAL>(st, a);
-    if (pro == SB_PRO_PLAIN && epi == SB_EPI_PLAIN) return launch_sb16<SB_PRO_PLAIN, SB_EPI_PLAIN>(st, a);
+    if (pro == SB_PRO_NORM && epi == SB_EPI_PLAIN) return launch_sb16_t<SB_PRO_NORM, SB_EPI_PLAIN>(st, a);
+    if (pro == SB_PRO_ATTN && epi == SB_EPI_RESIDUAL) return launch_sb16_t<SB_PRO_ATTN, SB_EPI_RESIDUAL>(st, a);
+    if (pro == SB_PRO_PLAIN && epi == SB_EPI_RESIDUAL) return launch_sb16_t<SB_PRO_PLAIN, SB_EPI_RESIDUAL>(st, a);
+    if (pro == SB_PRO_PLAIN && epi == SB_EPI_PLAIN) return launch_sb16_t<SB_PRO_PLAIN, SB_EPI_PLAIN>(st, a);
   }
   const int blocks = a.N / 32;
-  if (pro == SB_PRO_NORM && epi == SB_EPI_PLAIN) return launch_sb<SB_PRO_NORM, SB_EPI_PLAIN>(st, a, blocks);
-  if (pro == SB_PRO_ATTN && epi == SB_EPI_RESIDUAL) return launch_sb<SB_PRO_ATTN, SB_EPI_RESIDUAL>(st, a, blocks);
-  if (pro == SB_PRO_PLAIN && epi == SB_EPI_RESIDUAL) return launch_sb<SB_PRO_PLAIN, SB_EPI_RESIDUAL>(st, a, blocks);
-  if (pro == SB_PRO_PLAIN && epi == SB_EPI_PLAIN) return launch_sb<SB_PRO_PLAIN, SB_EPI_PLAIN>(st, a, blocks);
+  if (pro == SB_PRO_NORM && epi == SB_EPI_PLAIN) return launch_sb_a<SB_PRO_NORM, SB_EPI_PLAIN, 8>(st, a, blocks);
+  if (pro == SB_PRO_ATTN && epi == SB_EPI_RESIDUAL) return launch_sb_a<SB_PRO_ATTN, SB_EPI_RESIDUAL, 8>(st, a, blocks);
+  if (pro == SB_PRO_PLAIN && epi == SB_EPI_RESIDUAL) return launch_sb_a<SB_PRO_PLAIN, SB_EPI_RESIDUAL, 8>(st, a, blocks);
+  if (pro == SB_PRO_PLAIN && epi == SB_EPI_PLAIN) return launch_sb_a<SB_PRO_PLAIN, SB_EPI_PLAIN, 8>(st, a, blocks);
   return TMX_ERR_UNSUPPORTED;
 }
 
