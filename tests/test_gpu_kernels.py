@@ -262,6 +262,29 @@ def test_lora_residual_rmsnorm_planes(family):
   G.assert_bf16_close(G.host(xn), ref, ulps=1.0, min_exact=0.99, what='norm of residual')
 
 
+@pytest.mark.parametrize('ns', [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 16, 17])
+def test_k_slices_of_every_count(ns):
+  """The planes of a split projection are added in ascending order in f32 whatever their number, in the row kernel and in the
+  rotation (whose V heads are the bare sum): bit for bit."""
+  T = G.Keep()
+  rng = np.random.default_rng(ns)
+  M, D, N, Kh, H = 3, 2304, 2, 1, 64
+  yp = rng.standard_normal((ns, M, D)).astype(np.float32)
+  want = np.zeros((M, D), np.float32)
+  for s in range(ns):
+    want = want + yp[s]
+  x_out = torch.empty(M, D, dtype=torch.bfloat16, device=G.DEV)
+  G.call('tmx_lora_residual_rmsnorm', S(), None, T.f32(yp), ns, None, 0, 0, None, 0, 0.0, None, G.p(x_out), None, None, M, D, 1e-6, 0)
+  qkv = np.ascontiguousarray(yp[:, :, :(N + 2 * Kh) * H])
+  q_out = torch.empty(M, N * H, dtype=torch.bfloat16, device=G.DEV)
+  kc, vc = [torch.zeros(M, 4, Kh, H, dtype=torch.bfloat16, device=G.DEV) for _ in range(2)]
+  G.call('tmx_rope_kv_write', S(), None, T.f32(qkv), ns, None, 0, 0, None, 0, 0.0, None, None, T.i32(np.zeros((M, 4), np.int32)),
+         T.i32([1]), 4, G.p(q_out), G.p(kc), G.p(vc), M, N, Kh, H, 4, 10_000.0, 1e-6, 0)
+  G.sync()
+  assert np.array_equal(G.host(x_out), bf16_round(want))
+  assert np.array_equal(G.host(vc)[:, 1, 0], bf16_round(want[:, (N + Kh) * H:(N + 2 * Kh) * H]))
+
+
 @pytest.mark.parametrize('family,H,N,Kh', [(0, 64, 4, 4), (0, 128, 8, 2), (1, 128, 4, 2), (1, 64, 8, 8)])
 def test_rope_kv_write(family, H, N, Kh):
   T = G.Keep()

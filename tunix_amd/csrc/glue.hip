@@ -30,7 +30,9 @@ __device__ __forceinline__ uint4 pack8(const float* o) {
 
 // Sums NS K-slice planes of 8 adjacent f32 values; all 2 * NS loads are issued before the
 // first add so that the planes' memory latencies overlap.  Planes are added in ascending
-// order whatever NS is, so every code path rounds identically.
+// order whatever NS is, so every code path rounds identically.  Every count up to 8 has its own code: a clamped index fetches
+// the last plane again (16 times 32 bytes a thread, 7 planes of 4096 values of 64 rows: 8.0 us back to back, 6.7 without; 3
+// planes 7.6 / 5.9).
 template <int NS>
 __device__ __forceinline__ void sum_planes8(const float* p, size_t stride, float* o) {
   float4 a[NS], b[NS];
@@ -62,7 +64,11 @@ __device__ __forceinline__ float sum_planes1_dyn(const float* p, size_t stride, 
   switch (ns) {
     case 1: return sum_planes1<1>(p, stride);
     case 2: return sum_planes1<2>(p, stride);
+    case 3: return sum_planes1<3>(p, stride);
     case 4: return sum_planes1<4>(p, stride);
+    case 5: return sum_planes1<5>(p, stride);
+    case 6: return sum_planes1<6>(p, stride);
+    case 7: return sum_planes1<7>(p, stride);
     case 8: return sum_planes1<8>(p, stride);
     case 16: return sum_planes1<16>(p, stride);
     case 32: return sum_planes1<32>(p, stride);
@@ -120,7 +126,11 @@ __device__ __forceinline__ void load_base8(const uint16_t* y_bf16, const float* 
   switch (nsplit) {
     case 1: sum_planes8<1>(p, stride, o); break;
     case 2: sum_planes8<2>(p, stride, o); break;
+    case 3: sum_planes8<3>(p, stride, o); break;
     case 4: sum_planes8<4>(p, stride, o); break;
+    case 5: sum_planes8<5>(p, stride, o); break;
+    case 6: sum_planes8<6>(p, stride, o); break;
+    case 7: sum_planes8<7>(p, stride, o); break;
     case 8: sum_planes8<8>(p, stride, o); break;
     case 16: sum_planes8<16>(p, stride, o); break;
     default: {
