@@ -221,7 +221,7 @@ int tmx_qlora_gate_up_swiglu(void* stream, const void* x, const void* qweight, c
                              const void* lora_a_t, const void* lora_b, void* act, int M, int K, int F,
                              int G, int r, float lora_scale);
 
-/* The same launch in the form the decode step runs at up to 64 rows with LoRA: t = x . [A_gate | A_up] is
+/* The same launch in the form the decode step runs at 33 to 64 rows with LoRA and K >= 4096: t = x . [A_gate | A_up] is
  * computed once, by K / 256 extra workgroups of the launch, and handed to the others through `workspace`
  * (tmx_qlora_gate_up_swiglu_handover_bytes(M, K, F, r) bytes, whose state block the call clears with one
  * small launch) instead of being recomputed by every workgroup; same results up to the summation order of
