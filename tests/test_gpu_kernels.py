@@ -737,6 +737,46 @@ def test_head_greedy(M, D, V, head_layout):
   assert clear.sum() == 0 or np.abs(lp[clear, step + 1] - o_lp[clear]).max() <= 1e-2
 
 
+@pytest.mark.parametrize('tiled', [False, True])
+@pytest.mark.parametrize('mode,temp', [(0, 1.0), (1, 0.7)])
+@pytest.mark.parametrize('M', [1, 2, 7, 15, 16])
+def test_head_of_few_rows_equals_its_rows_among_many(M, mode, temp, tiled):
+  """Up to 16 rows a half-wave takes a row and a lane a vocabulary row, above a lane takes 16: the same logits and tokens (equal
+  logits, forbidden ids and an infinite logit among them), the log-probs to the order of their f32 sums."""
+  rng = np.random.default_rng(M)
+  V, D, many = 416, 128, 33  # a last workgroup with one live wave
+  w = bf16_round(rng.standard_normal((V, D)).astype(np.float32))
+  x = np.abs(bf16_round(rng.standard_normal((many, D)).astype(np.float32))) + np.float32(0.5)
+  w[300] = w[17]
+  w[44] = 4.0
+  w[301] = w[45] = 8.0
+  if M == 7:
+    w[200, 3] = np.inf
+  W, X = torch.from_numpy(w).to(G.DEV, torch.bfloat16), torch.from_numpy(x).to(G.DEV, torch.bfloat16)
+  if tiled:
+    wt = torch.empty_like(W)
+    G.call('tmx_head_tiles_pack', S(), G.p(W), G.p(wt), V, D)
+  bad = torch.tensor([44, 415], dtype=torch.int32, device=G.DEV)
+  eos = torch.zeros(1, dtype=torch.int32, device=G.DEV)
+  out = []
+  for rows in (M, many):
+    tok = torch.zeros(rows, 4, dtype=torch.int32, device=G.DEV)
+    lp = torch.zeros(rows, 4, dtype=torch.float32, device=G.DEV)
+    logits = torch.zeros(rows, V, dtype=torch.float32, device=G.DEV)
+    done = torch.zeros(rows, dtype=torch.uint8, device=G.DEV)
+    ws = torch.empty(_lib.lib().tmx_head_sample_workspace_bytes(rows, V), dtype=torch.uint8, device=G.DEV)
+    step = torch.ones(1, dtype=torch.int32, device=G.DEV)
+    G.call('tmx_head_sample_tiles' if tiled else 'tmx_head_sample', S(), G.p(X), G.p(wt if tiled else W), rows, D, V, mode, temp, 3, 5,
+           G.p(step), G.p(bad), 2, G.p(eos), 1, G.p(tok), G.p(lp), G.p(done), 4, G.p(logits), G.p(ws))
+    G.sync()
+    out.append((tok[:M], lp[:M], logits[:M]))
+  assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][2], out[1][2])
+  if mode == 0:
+    assert int(out[0][0][0, 2]) == (200 if M == 7 else 45)
+  # a sum of 416 terms of at most 1 around a maximum of 1: 2^-24 relative per addition, then a logarithm near its rounding
+  assert torch.allclose(out[0][1], out[1][1], rtol=2.0 ** -22, atol=416 * 2.0 ** -24, equal_nan=True)
+
+
 def test_head_scoring_clips_logits_like_the_reference():
   """TMX_SAMPLE_SCORE follows selective_log_softmax (tunix/rl/common.py:217-221): NaN logits count
   as -1e9, the others are clipped to [-1e9, 1e9], so every score is finite.  Row 0 of x is 1e10:

@@ -26,6 +26,12 @@ namespace tmx {
 
 template <int V>
 struct HIC { static constexpr int value = V; };
+// Up to here head_kernel spreads the values of a sequence row over the lanes.  Its epilogue is a chain of 16 values a lane however
+// many rows there are, 20 threefry rounds and two logarithms each when sampling; spread out, half a value a lane and row, and a
+// reduction.  us per launch with finalize, chain / spread: 1024 x 256 head, one row greedy 12.7 / 7.8, sampling 25.5 / 8.3, 9 rows
+// 15.5 / 11.0, 16 rows 15.6 / 12.9; 128256 x 2048, one row sampling 104.6 / 91.8, 16 rows 99.7 / 97.5.  More rows would not fit the
+// slabs' LDS.
+constexpr int kHeadFewRows = 16;
 constexpr int kHXStride = 72;  // bf16 elements per LDS row of the activation tile (64 + 8 pad)
 
 // Scoring (tunix/rl/common.py:217-221, selective_log_softmax): a NaN logit counts as -1e9 and
@@ -40,51 +46,82 @@ struct RowStat {
   Best best = {-INFINITY, -INFINITY, 0x7FFFFFFF};
 };
 
-// Adds the 16 vocabulary rows of an accumulator tile (first row v0) to the statistics of sequence row `row`.
+// A vocabulary row of sequence row `row`: z, what the log-softmax runs over, and the key the best candidate is found by.
+// In sampling with sort_keys the key is z, and sort_key the 16-bit key whose ascending order is the descending order of the logit
+// (= of z, T > 0; -0 counts as +0): non-negative values count down from 0x7FFF, negative ones up from 0x8000.
+struct HeadValue { float z, key; uint32_t sort_key; };
+__device__ __forceinline__ HeadValue head_value(const HeadArgs& a, float acc, int v, int row, int target, uint32_t key0, uint32_t key1) {
+  float logit = rbf(acc);
+  if (a.logits_out) a.logits_out[(size_t)row * a.V + v] = logit;
+  for (int f = 0; f < a.n_forbidden; ++f)
+    if (a.forbidden[f] == v) logit = -INFINITY;
+  HeadValue c = {logit, logit, 0u};
+  if (a.mode == TMX_SAMPLE_SCORE) {
+    // the "best" candidate is the given next token: its z is what the log-prob needs
+    c.z = score_clip(rbf(logit / a.temperature));  // bf16 logits divided in place stay bf16 (rl/common.py:591-592)
+    c.key = (v == target) ? 0.f : -INFINITY;
+  } else if (a.mode == TMX_SAMPLE_TOP_P) {
+    c.key = c.z = logit / a.temperature;
+    if (a.sort_keys) {
+      const uint32_t zb = __float_as_uint(logit + 0.0f) >> 16;
+      c.sort_key = (zb & 0x8000u) ? zb : (~zb & 0x7FFFu);
+    } else {
+      uint32_t o0, o1;
+      threefry2x32(key0, key1, 0u, (uint32_t)(a.row_off + row) * (uint32_t)a.V + (uint32_t)v, o0, o1);
+      c.key = c.z + gumbel_from_bits(o0 ^ o1);
+    }
+  }
+  return c;
+}
+// exp(z - mx) of a z that is at most mx (the infinite maximum itself counts once, as every maximum does)
+__device__ __forceinline__ float head_exp(float z, float mx) { return z == mx ? 1.f : expf(z - mx); }
+
+// Adds the 16 vocabulary rows of an accumulator tile (first row v0) to the statistics of sequence row `row`: their maximum
+// first, so that a value takes one exponential and no branch (a running maximum takes both sides of one in most waves).
+// 128256 x 4096, greedy / sampling: 64 rows 185.5 / 191.5 -> 183.7 / 189.0 us, 256 rows 331.6 / 397.6 -> 325.9 / 393.3.
 __device__ __forceinline__ void head_tile_stats(const HeadArgs& a, const f32x16_t& acc, int v0, int row, int lane, int target,
                                                 uint32_t key0, uint32_t key1, RowStat& st) {
-  const bool score = a.mode == TMX_SAMPLE_SCORE;
   uint64_t packed = 0;
+  float z[16], mx = st.mx;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int v = v0 + acc_row(r, lane);
-    float logit = rbf(acc[r]);
-    if (a.logits_out) a.logits_out[(size_t)row * a.V + v] = logit;
-    for (int f = 0; f < a.n_forbidden; ++f)
-      if (a.forbidden[f] == v) logit = -INFINITY;
-    float z = logit, key = logit;
-    if (score) {
-      // the "best" candidate is the given next token: its z is what the log-prob needs
-      z = score_clip(rbf(logit / a.temperature));  // bf16 logits divided in place stay bf16 (rl/common.py:591-592)
-      key = (v == target) ? 0.f : -INFINITY;
-    } else if (a.mode == TMX_SAMPLE_TOP_P) {
-      z = logit / a.temperature;
-      if (a.sort_keys) {
-        // 16-bit key whose ascending order is the descending order of the logit (= of z, T > 0;
-        // -0 counts as +0): non-negative values count down from 0x7FFF, negative ones up from 0x8000
-        const uint32_t zb = __float_as_uint(logit + 0.0f) >> 16;
-        // registers 4 q .. 4 q + 3 hold four consecutive vocabulary rows: one 8-byte store
-        packed |= (uint64_t)((zb & 0x8000u) ? zb : (~zb & 0x7FFFu)) << (16 * (r & 3));
-        if ((r & 3) == 3) {
-          *reinterpret_cast<uint64_t*>(a.sort_keys + (size_t)row * a.V + v - 3) = packed;
-          packed = 0;
-        }
-        key = z;
-      } else {
-        uint32_t o0, o1;
-        threefry2x32(key0, key1, 0u, (uint32_t)(a.row_off + row) * (uint32_t)a.V + (uint32_t)v, o0, o1);
-        key = z + gumbel_from_bits(o0 ^ o1);
+    const HeadValue c = head_value(a, acc[r], v, row, target, key0, key1);
+    if (a.sort_keys) {
+      // registers 4 q .. 4 q + 3 hold four consecutive vocabulary rows: one 8-byte store
+      packed |= (uint64_t)c.sort_key << (16 * (r & 3));
+      if ((r & 3) == 3) {
+        *reinterpret_cast<uint64_t*>(a.sort_keys + (size_t)row * a.V + v - 3) = packed;
+        packed = 0;
       }
     }
-    if (z > st.mx) {
-      st.se = st.se * expf(st.mx - z) + 1.f;
-      st.mx = z;
-    } else {
-      st.se += expf(z - st.mx);
-    }
-    Best c = {key, z, v};
-    best_merge(st.best, c);
+    z[r] = c.z;
+    mx = fmaxf(mx, c.z);
+    Best b = {c.key, c.z, v};
+    best_merge(st.best, b);
   }
+  st.se *= head_exp(st.mx, mx);
+  st.mx = mx;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) st.se += head_exp(z[r], mx);
+}
+
+// Maximum / sum over the lanes of a half-wave, every lane gets it.
+__device__ __forceinline__ float half_max(float v) {
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  v = fmaxf(v, dpp_f<0x128>(v));  // row_ror:8
+  v = fmaxf(v, dpp_f<0x124>(v));  // row_ror:4
+  v = fmaxf(v, dpp_f<0x4E>(v));   // quad_perm [2,3,0,1]
+  return fmaxf(v, dpp_f<0xB1>(v));  // quad_perm [1,0,3,2]
+}
+__device__ __forceinline__ float half_sum(float v) {
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  v += dpp_f<0x128>(v);
+  v += dpp_f<0x124>(v);
+  v += dpp_f<0x4E>(v);
+  return v + dpp_f<0xB1>(v);
 }
 
 // The given next token of sequence row `row` of this launch (scoring), or -1.
@@ -132,7 +169,7 @@ __device__ __forceinline__ void head_store_partial(const HeadArgs& a, int row, i
 // stream, read once (non-temporal).  Row-major, one load touches 32 lines of 32 different DRAM
 // pages; measured on the 1.05 GB head at 64 rows: 252 us row-major, 190 us from tiles.
 template <int MT, bool TILED>
-__global__ __launch_bounds__(256, MT == 4 ? 1 : 2) void head_kernel(HeadArgs a) {
+__global__ __launch_bounds__(256, 2) void head_kernel(HeadArgs a) {
   __shared__ __align__(16) uint16_t xs[2][MT * 32][kHXStride];
   __shared__ float s_f[4][MT * 32][4];
   __shared__ int s_i[4][MT * 32];
@@ -228,12 +265,46 @@ __global__ __launch_bounds__(256, MT == 4 ? 1 : 2) void head_kernel(HeadArgs a) 
   // per-step key = fold_in(seed, step)
   uint32_t key0 = 0, key1 = 0;
   if (a.mode == TMX_SAMPLE_TOP_P) threefry2x32(a.k0, a.k1, 0u, (uint32_t)*a.step, key0, key1);
+  if (MT == 1 && a.M <= kHeadFewRows) {
+    // Few sequence rows use few lanes of the tile, 16 vocabulary rows each, one after the other: turned over in LDS (the slabs are
+    // free), so that the half-waves take a sequence row each and a lane one vocabulary row of it.
+    static_assert(4 * 32 * (kHeadFewRows + 1) * 4 <= (int)sizeof(uint16_t) * 2 * 32 * kHXStride, "the tiles of the waves take the place of the slabs");
+    float* tile_s = reinterpret_cast<float*>(&xs[0][0][0]) + wave * 32 * (kHeadFewRows + 1);
+    if (nl < kHeadFewRows) {
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int row = m * 32 + nl;
-    RowStat st;
-    if (live && row < a.M) head_tile_stats(a, acc[m], v0, row, lane, head_target(a, row), key0, key1, st);
-    head_stat_to_lds(st, h, s_f[wave][row], &s_i[wave][row]);
+      for (int r = 0; r < 16; ++r) tile_s[acc_row(r, lane) * (kHeadFewRows + 1) + nl] = acc[0][r];
+    }
+    __syncthreads();
+    for (int m0 = 0; m0 < a.M; m0 += 2) {
+      const int row = m0 + h;
+      RowStat st;
+      if (live && row < a.M) {
+        const int v = v0 + nl;
+        const HeadValue c = head_value(a, tile_s[nl * (kHeadFewRows + 1) + row], v, row, head_target(a, row), key0, key1);
+        if (a.sort_keys) a.sort_keys[(size_t)row * a.V + v] = (uint16_t)c.sort_key;
+        st.mx = fmaxf(st.mx, half_max(c.z));
+        st.se = half_sum(head_exp(c.z, st.mx));
+        const float key = half_max(c.key);
+        const uint32_t ahead = (uint32_t)(__ballot(c.key == key) >> (h * 32));
+        if (ahead) {  // (none: every key is NaN)
+          const int first = __builtin_ctz(ahead);  // equal keys: the lowest vocabulary row
+          st.best = {key, __shfl(c.z, h * 32 + first, 64), v0 + first};
+        }
+      }
+      if (nl == 0 && row < a.M) {
+        float* f = s_f[wave][row];
+        f[0] = st.mx; f[1] = st.se; f[2] = st.best.key; f[3] = st.best.z;
+        s_i[wave][row] = st.best.idx;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int row = m * 32 + nl;
+      RowStat st;
+      if (live && row < a.M) head_tile_stats(a, acc[m], v0, row, lane, head_target(a, row), key0, key1, st);
+      head_stat_to_lds(st, h, s_f[wave][row], &s_i[wave][row]);
+    }
   }
   __syncthreads();
   for (int row = threadIdx.x; row < MT * 32; row += 256)
