@@ -392,7 +392,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
         }
         if (prof) TMX_TRY(TMX_K_EMPTY, empty_launch(st));
       }
-      {  // final norm in front of the head
+      if (!head_row_ok(B, D)) {  // final norm in front of the head
         RowNormArgs a = {};
         a.y_bf16 = w.x;
         a.norm_w = (const uint16_t*)m->final_norm_w; a.xn_out = w.xn;
@@ -590,6 +590,11 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
       a.w = (const uint16_t*)m->head;
       a.w_tiles = (const uint16_t*)m->head_tiles;
       a.M = B; a.D = D; a.V = m->vocab_size;
+      if (small && head_row_ok(B, D)) {
+        a.x = w.x;
+        a.norm_w = (const uint16_t*)m->final_norm_w;
+        a.eps = m->norm_eps; a.family = m->family;
+      }
       if (rg) {
         a.M = rg->n_head;
         a.row_map = w.head_map;

@@ -158,6 +158,43 @@ __device__ __forceinline__ void head_store_partial(const HeadArgs& a, int row, i
   a.part_i[(size_t)row * a.nwg + wg] = best.idx;
 }
 
+// Statistics of the rows of a tile when they are at most R: few sequence rows use few lanes of it, 16 vocabulary rows each, one
+// after the other, so it is turned over in LDS (tile_s: 4 x 32 x (R + 1) floats), and the half-waves take a sequence row each and a
+// lane one vocabulary row of it.  Every thread of the workgroup comes here.
+template <int R, int ROWS>
+__device__ __forceinline__ void head_few_stats(const HeadArgs& a, const f32x16_t& acc, float* tile_s, int wave, int lane, bool live,
+                                               int v0, uint32_t key0, uint32_t key1, float (*s_f)[ROWS][4], int (*s_i)[ROWS]) {
+  const int h = lane >> 5, nl = lane & 31;
+  tile_s += wave * 32 * (R + 1);
+  if (nl < R) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tile_s[acc_row(r, lane) * (R + 1) + nl] = acc[r];
+  }
+  __syncthreads();
+  for (int m0 = 0; m0 < a.M; m0 += 2) {
+    const int row = m0 + h;
+    RowStat st;
+    if (live && row < a.M) {
+      const int v = v0 + nl;
+      const HeadValue c = head_value(a, tile_s[nl * (R + 1) + row], v, row, head_target(a, row), key0, key1);
+      if (a.sort_keys) a.sort_keys[(size_t)row * a.V + v] = (uint16_t)c.sort_key;
+      st.mx = fmaxf(st.mx, half_max(c.z));
+      st.se = half_sum(head_exp(c.z, st.mx));
+      const float key = half_max(c.key);
+      const uint32_t ahead = (uint32_t)(__ballot(c.key == key) >> (h * 32));
+      if (ahead) {  // (none: every key is NaN)
+        const int first = __builtin_ctz(ahead);  // equal keys: the lowest vocabulary row
+        st.best = {key, __shfl(c.z, h * 32 + first, 64), v0 + first};
+      }
+    }
+    if (nl == 0 && row < a.M) {
+      float* f = s_f[wave][row];
+      f[0] = st.mx; f[1] = st.se; f[2] = st.best.key; f[3] = st.best.z;
+      s_i[wave][row] = st.best.idx;
+    }
+  }
+}
+
 // Workgroup = 4 waves x 32 vocabulary rows.  The hidden-state k-tile x[0:M, 64 kb : 64 kb + 64]
 // is fetched once per workgroup, double-buffered in LDS and shared by the waves (MFMA B
 // fragments); head rows stream HBM -> registers through a ring of 4 k-tiles per wave.  Lane
@@ -266,37 +303,8 @@ __global__ __launch_bounds__(256, 2) void head_kernel(HeadArgs a) {
   uint32_t key0 = 0, key1 = 0;
   if (a.mode == TMX_SAMPLE_TOP_P) threefry2x32(a.k0, a.k1, 0u, (uint32_t)*a.step, key0, key1);
   if (MT == 1 && a.M <= kHeadFewRows) {
-    // Few sequence rows use few lanes of the tile, 16 vocabulary rows each, one after the other: turned over in LDS (the slabs are
-    // free), so that the half-waves take a sequence row each and a lane one vocabulary row of it.
     static_assert(4 * 32 * (kHeadFewRows + 1) * 4 <= (int)sizeof(uint16_t) * 2 * 32 * kHXStride, "the tiles of the waves take the place of the slabs");
-    float* tile_s = reinterpret_cast<float*>(&xs[0][0][0]) + wave * 32 * (kHeadFewRows + 1);
-    if (nl < kHeadFewRows) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) tile_s[acc_row(r, lane) * (kHeadFewRows + 1) + nl] = acc[0][r];
-    }
-    __syncthreads();
-    for (int m0 = 0; m0 < a.M; m0 += 2) {
-      const int row = m0 + h;
-      RowStat st;
-      if (live && row < a.M) {
-        const int v = v0 + nl;
-        const HeadValue c = head_value(a, tile_s[nl * (kHeadFewRows + 1) + row], v, row, head_target(a, row), key0, key1);
-        if (a.sort_keys) a.sort_keys[(size_t)row * a.V + v] = (uint16_t)c.sort_key;
-        st.mx = fmaxf(st.mx, half_max(c.z));
-        st.se = half_sum(head_exp(c.z, st.mx));
-        const float key = half_max(c.key);
-        const uint32_t ahead = (uint32_t)(__ballot(c.key == key) >> (h * 32));
-        if (ahead) {  // (none: every key is NaN)
-          const int first = __builtin_ctz(ahead);  // equal keys: the lowest vocabulary row
-          st.best = {key, __shfl(c.z, h * 32 + first, 64), v0 + first};
-        }
-      }
-      if (nl == 0 && row < a.M) {
-        float* f = s_f[wave][row];
-        f[0] = st.mx; f[1] = st.se; f[2] = st.best.key; f[3] = st.best.z;
-        s_i[wave][row] = st.best.idx;
-      }
-    }
+    head_few_stats<kHeadFewRows, MT * 32>(a, acc[0], reinterpret_cast<float*>(&xs[0][0][0]), wave, lane, live, v0, key0, key1, s_f, s_i);
   } else {
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
@@ -310,6 +318,133 @@ __global__ __launch_bounds__(256, 2) void head_kernel(HeadArgs a) {
   for (int row = threadIdx.x; row < MT * 32; row += 256)
     if (row < a.M) head_store_partial(a, row, blockIdx.x, s_f[0][row], &s_i[0][row], 4, MT * 32);
 }
+
+// The same for at most kHeadRows rows of at most kHeadRowD values: they fit LDS whole, [M][D + 8], so the matrix streams past them
+// without a barrier, and the norm in front of the head is taken here, by every workgroup while its first tiles are on the way (the
+// bits of row_norm_kernel: the squares of 8 values by a thread, 64 threads by a wave, the waves in order), instead of by a
+// launch of its own.  Measured (back to back with finalize, without a norm, head_kernel / this; its launch of 3.5 to 4.7 us goes as
+// well), one row and four rows, sampling: 128256 x 4096 167.6 / 160.6 and 168.6 / 162.7 us (6.5 TB/s), 128256 x 2048 92.4 / 88.1 and
+// 93.9 / 89.6, 1024 x 256 8.1 / 7.8 and 9.2 / 9.1.
+constexpr int kHeadRows = 4, kHeadRowD = 4096;
+template <int R, bool TILED>  // M <= R
+__global__ __launch_bounds__(256, 3) void head_row_kernel(HeadArgs a) {
+  extern __shared__ __align__(16) uint16_t xs[];  // [M][D + 8]
+  __shared__ float tile_s[4 * 32 * (R + 1)];
+  __shared__ float s_ss[R][8];
+  __shared__ float s_f[4][R][4];
+  __shared__ int s_i[4][R];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, nl = lane & 31;
+  const int tile = blockIdx.x * 4 + wave;
+  const bool live = tile * 32 < a.V;
+  const int v0 = live ? tile * 32 : a.V - 32;  // dead waves recompute the last tile (dropped)
+  const int D = a.D, KT = D >> 6, klast = KT - 1, XS = D + 8;
+
+  // the rows first: they are waited for first.  Loads of rows and columns that are not there fetch nothing.
+  constexpr int kNowhere = 0x7FFF0000;
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x, (uint32_t)a.M * D * 2u), rn = make_rsrc(a.norm_w, a.norm_w ? (uint32_t)D * 2u : 0u);
+  u32x4_t xq[R][2], nq[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int at = (tid + 256 * i) * 8 < D ? (tid + 256 * i) * 16 : kNowhere;
+#pragma unroll
+    for (int m = 0; m < R; ++m)
+      xq[m][i] = __builtin_amdgcn_raw_buffer_load_b128(rx, at == kNowhere ? at : m * D * 2 + at, 0, 0);
+    nq[i] = __builtin_amdgcn_raw_buffer_load_b128(rn, at, 0, 0);
+  }
+  constexpr int P = 4;
+  u32x4_t wring[P][4];
+  const u32x4_t* wsrc = TILED ? reinterpret_cast<const u32x4_t*>(a.w_tiles + (size_t)v0 * D) + lane
+                              : reinterpret_cast<const u32x4_t*>(a.w + (size_t)(v0 + nl) * D + h * 32);
+  auto load_w = [&](int kb, auto pc, auto tc) __attribute__((always_inline)) {
+    constexpr int p = decltype(pc)::value, t = decltype(tc)::value;
+    kb = kb < klast ? kb : klast;
+    wring[p][t] = TILED ? __builtin_nontemporal_load(wsrc + (size_t)kb * 256 + t * 64) : wsrc[(size_t)kb * 8 + t];
+  };
+  __builtin_amdgcn_sched_barrier(0);
+  static_for<P>([&](auto pc) __attribute__((always_inline)) {
+    static_for<4>([&](auto tc) __attribute__((always_inline)) { load_w(decltype(pc)::value, pc, tc); });
+  });
+  __builtin_amdgcn_sched_barrier(0);
+  auto unpack = [](const u32x4_t& q, float (&v)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { v[2 * e] = bf_lo(q[e]); v[2 * e + 1] = bf_hi(q[e]); }
+  };
+  auto put = [&](int m, int i, u32x4_t q) __attribute__((always_inline)) {
+    if ((tid + 256 * i) * 8 < D) *reinterpret_cast<u32x4_t*>(xs + m * XS + (tid + 256 * i) * 8) = q;
+  };
+  if (a.norm_w) {
+#pragma unroll
+    for (int m = 0; m < R; ++m)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float ss = 0.f;
+        if (m < a.M && wave * 512 + i * 2048 < D) {  // (the whole wave or none of it)
+          float v[8];
+          unpack(xq[m][i], v);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+          ss = wave_sum(ss);
+        }
+        if (lane == 0) s_ss[m][wave + 4 * i] = ss;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < R; ++m) {
+      float t = 0.f;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) t += s_ss[m][w];
+      const float rms = sqrtf(t / (float)D + a.eps);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (m < a.M && wave * 512 + i * 2048 < D) {
+          float v[8], w[8], o[8];
+          unpack(xq[m][i], v);
+          unpack(nq[i], w);
+          __builtin_amdgcn_sched_barrier(0);  // (one piece at a time: side by side their divisions take 50 registers)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) o[e] = a.family == TMX_FAMILY_LLAMA3 ? rbf(w[e] * v[e]) / rms : w[e] * (v[e] / rms);
+          put(m, i, u32x4_t{pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]), pack_bf2(o[4], o[5]), pack_bf2(o[6], o[7])});
+        }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int m = 0; m < R; ++m)
+        if (m < a.M) put(m, i, xq[m][i]);
+  }
+  __syncthreads();
+
+  f32x16_t acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  const uint16_t* xb = xs + min(nl, a.M - 1) * XS + h * 32;  // lanes past the rows repeat the last one (dropped)
+  auto step = [&](int kb, auto pc) __attribute__((always_inline)) {
+    constexpr int p = decltype(pc)::value;
+    static_for<4>([&](auto tc) __attribute__((always_inline)) {
+      constexpr int t = decltype(tc)::value;
+      const bf16x8_t xf = *reinterpret_cast<const bf16x8_t*>(xb + kb * 64 + t * 8);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wring[p][t]), xf, acc, 0, 0, 0);
+      load_w(kb + P, pc, tc);  // consumed: refill
+    });
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int kb = 0;
+  for (; kb + P <= KT; kb += P)
+    static_for<P>([&](auto pc) __attribute__((always_inline)) { step(kb + decltype(pc)::value, pc); });
+  static_for<P - 1>([&](auto pc) __attribute__((always_inline)) {
+    if (kb + decltype(pc)::value < KT) step(kb + decltype(pc)::value, pc);
+  });
+
+  uint32_t key0 = 0, key1 = 0;
+  if (a.mode == TMX_SAMPLE_TOP_P) threefry2x32(a.k0, a.k1, 0u, (uint32_t)*a.step, key0, key1);
+  head_few_stats<R, R>(a, acc, tile_s, wave, lane, live, v0, key0, key1, s_f, s_i);
+  __syncthreads();
+  if (tid < a.M) head_store_partial(a, tid, blockIdx.x, s_f[0][tid], &s_i[0][tid], 4, R);
+}
+bool head_row_ok(int M, int D) { return M <= kHeadRows && D <= kHeadRowD; }
 
 // 65 to 256 rows: the matrix still has to stream once, but a wave multiplies up to 256 sequence rows (MT = 4 or 8 tiles),
 // so the hidden states go to LDS by direct transfers (no registers) and the weights, from the tile copy, straight to
@@ -783,7 +918,14 @@ int head_logits(hipStream_t st, HeadArgs& a) {
     c.part_f = a.part_f + (size_t)r0 * a.nwg * 4;
     c.part_i = a.part_i + (size_t)r0 * a.nwg;
     int rc = TMX_OK;
-    if (c.w_tiles) {
+    if (head_row_ok(c.M, c.D)) {
+      const size_t lds = (size_t)c.M * (c.D + 8) * 2;
+#define TMX_HEAD_ROW(R) \
+  if (c.w_tiles) hipLaunchKernelGGL((head_row_kernel<R, true>), dim3(a.nwg), dim3(256), lds, st, c); \
+  else hipLaunchKernelGGL((head_row_kernel<R, false>), dim3(a.nwg), dim3(256), lds, st, c)
+      if (c.M == 1) { TMX_HEAD_ROW(1); } else if (c.M == 2) { TMX_HEAD_ROW(2); } else { TMX_HEAD_ROW(4); }
+#undef TMX_HEAD_ROW
+    } else if (c.w_tiles) {
       if (c.M <= 32) hipLaunchKernelGGL((head_kernel<1, true>), dim3(a.nwg), dim3(256), 0, st, c);
       else if (c.M <= 64) hipLaunchKernelGGL((head_kernel<2, true>), dim3(a.nwg), dim3(256), 0, st, c);
       else rc = c.M <= 128 ? launch_head_mid<4, 4, 4>(st, c) : launch_head_mid<8, 4, 4>(st, c);

@@ -188,7 +188,10 @@ struct AttnArgs {
 };
 
 struct HeadArgs {
-  const uint16_t* x;  // [M, D] final-normed hidden states
+  const uint16_t* x;  // [M, D] final-normed hidden states, or with norm_w (head_row_ok) the ones to be normed
+  const uint16_t* norm_w;  // [D] or null
+  float eps;
+  int family;
   uint16_t* x_tiles;  // room for x again in the wide kernel's order (head_x_tiles_bytes; needed by head_wide only)
   const uint16_t* w;  // [V, D]
   const uint16_t* w_tiles;  // the same matrix in the tile layout of head_tiles_kernel, or null
@@ -332,6 +335,8 @@ int moe_route(hipStream_t st, const RouterArgs& a, int B);
 bool moe_route_rows_ok(const RouterArgs& a, int B);  // enough tokens for a launch of their own behind the row kernel
 int moe_experts(hipStream_t st, const MoeArgs& a, int E, bool down);
 int moe_rows(hipStream_t st, const MoeArgs& a, int E, bool down);  // its form for many rows per expert
+// Rows that the head takes without the norm in front of it.
+bool head_row_ok(int M, int D);
 int head_sample(hipStream_t st, HeadArgs a);
 // any number of rows in 256 x 256 blocks (greedy, sampling without the sorting branch, scoring); needs
 // D % 128 == 0, no forbidden ids, no logits output; part_f / part_i sized [M][ceil(V / 256)]
