@@ -317,10 +317,10 @@ class QLoRAModel:
 
   def _lora_slots(self):
     """Where every adapter lives: {name of lora_state(): (index, (rows, columns), PackedLinear, other shapes seen to be
-    good)} and, under the index, the tmx_lora_pack_desc that writes it (src and dtype left open).  Updates are in place, so the
-    destinations stay what they are."""
+    good for these rows and columns)} and, under the index, the tmx_lora_pack_desc that writes it (src and dtype left
+    open).  Updates are in place, so the destinations stay what they are."""
     if self._slots is None:
-      out, rows = {}, []
+      out, rows, good = {}, [], {}
       for i, layer in enumerate(self.layers):
         for key, names, pre, wk in (('qkv', ('q_proj', 'k_proj', 'v_proj'), 'attn', 'w'),
                                     ('o', ('o_proj',), 'attn', 'w'),
@@ -331,9 +331,10 @@ class QLoRAModel:
             continue
           col = 0
           for j, (n, width) in enumerate(zip(names, pl.seg_cols)):
-            out[f'layers.{i}.{pre}.{n}.{wk}_lora_a'] = (len(rows), (pl.k, pl.rank), pl, set())
+            a, b = (pl.k, pl.rank), (pl.rank, width)
+            out[f'layers.{i}.{pre}.{n}.{wk}_lora_a'] = (len(rows), a, pl, good.setdefault(a, set()))
             rows.append((0, pl.lora_a_t.data_ptr(), pl.k, pl.rank, j * pl.rank, pl.r_pad, 1, 0))
-            out[f'layers.{i}.{pre}.{n}.{wk}_lora_b'] = (len(rows), (pl.rank, width), pl, set())
+            out[f'layers.{i}.{pre}.{n}.{wk}_lora_b'] = (len(rows), b, pl, good.setdefault(b, set()))
             rows.append((0, pl.lora_b.data_ptr(), pl.rank, width, col, pl.n, 0, 0))
             col += width
       self._slots = out, np.array(rows, dtype=_LORA_PACK_DESC)
