@@ -435,9 +435,10 @@ def main():
     on_tile = g_heads in (4, 8) and batch * cfg.num_kv_heads <= 3 * cus
     symbols.update({} if small else {
         f"tmx::gqa_{'tile' if on_tile else 'decode'}_kernel<{cfg.head_dim}, {g_heads}>": ['attention']})
-    # the head from its tile copy, 65 to 256 rows by head_mid_kernel, more in 256 x 256 blocks (template argument 1:
+    # the head from its tile copy, up to 4 rows by head_row_kernel, 65 to 256 rows by head_mid_kernel, more in 256 x 256 blocks (template argument 1:
     # sampling); with top_p < 1 the class also holds the three selection launches of nucleus.hip
-    head_symbol = (f'head_kernel<{min(mt, 2)}, true>' if batch <= 64 else 'head_mid_kernel<4, 4, 4>' if batch <= 128 else
+    head_symbol = (f'head_row_kernel<{1 << (batch - 1).bit_length()}, true>' if batch <= 4 and cfg.embed_dim <= 4096 else
+                   f'head_kernel<{min(mt, 2)}, true>' if batch <= 64 else 'head_mid_kernel<4, 4, 4>' if batch <= 128 else
                    'head_mid_kernel<8, 4, 4>' if batch <= 256 else 'head_wide_kernel<1>')
     symbols.update({f'tmx::{head_symbol}': ['head_sample']})
     idx = {n: i for i, n in enumerate(CLASS_NAMES)}
