@@ -68,7 +68,8 @@ const char* tmx_status_string(int status);
  * loading, before it looks up anything else.
  *   7: tmx_model_desc.head_tiles and the tmx_decode_state.share_* fields
  *   8: tmx_lora_pack and tmx_fill_ragged; tokens_per_pass up to TMX_MAX_FILL_ROWS / batch (128 before);
- *      tmx_qlora_linear needs a larger workspace for more than 128 rows */
+ *      tmx_qlora_linear needs a larger workspace for more than 128 rows; tmx_score_ragged was added to it later: the
+ *      rest is as it was, and a library without it fails at the look-up of its name */
 #define TMX_ABI_VERSION 8
 int tmx_abi_version(void);
 
