@@ -577,6 +577,40 @@ def test_gqa_group_walk(B, N, Kh, H, C, step, gs, sl):
   test_gqa_decode_attention_with_shared_prompt_slots(B, N, Kh, H, C, step, gs, sl)
 
 
+# One and several splits of a group, groups beside rows; shared slots that end inside a block of 32 and inside a transfer of 4 rows,
+# whose other rows are the leader's own
+@pytest.mark.parametrize('victim', [0, 1])  # the leader's own slots, a follower's
+@pytest.mark.parametrize('B,N,Kh,H,C,step,gs,sl', [
+    (32, 32, 8, 128, 320, 290, 8, 256), (120, 32, 8, 128, 128, 101, 6, 90), (96, 16, 8, 64, 200, 180, 24, 150),
+    (48, 32, 4, 128, 160, 159, 6, 50), (6, 4, 4, 128, 200, 150, 3, 63), (8, 8, 2, 64, 96, 70, 4, 33)])
+def test_own_slots_that_are_not_finite_stay_with_their_sequence(B, N, Kh, H, C, step, gs, sl, victim):
+  """K or V rows of one sequence of every group overflow behind the prompt: its siblings' results do not change by a bit."""
+  T = G.Keep()
+  g = torch.Generator(device=G.DEV).manual_seed(B + C)
+  new = lambda *shape: torch.randn(*shape, generator=g, device=G.DEV).to(torch.bfloat16)
+  q, k, v = new(B, N, H), new(B, C, Kh, H), new(B, C, Kh, H)
+  for t in (k, v):
+    t[:, :sl] = t[::gs, :sl].repeat_interleave(gs, 0)
+  lib = _lib.lib()
+  ws = torch.empty(lib.tmx_gqa_decode_shared_workspace_bytes(B, N, Kh, H, C), dtype=torch.uint8, device=G.DEV)
+  mask, at = T.u8(np.ones((B, C))), T.i32([step])
+
+  def attend(k, v):
+    out = torch.empty(B, N * H, dtype=torch.bfloat16, device=G.DEV)
+    G.call('tmx_gqa_decode_attention_shared', S(), G.p(q), G.p(k), G.p(v), mask, at, C, G.p(out), G.p(ws), B, N, Kh, H, C, gs, sl)
+    return out
+
+  want = attend(k, v)
+  assert torch.isfinite(want).all()
+  hit = torch.arange(B, device=G.DEV) % gs == victim
+  for value in (float('nan'), float('inf')):
+    bad_k, bad_v = k.clone(), v.clone()
+    bad_k[hit, sl:step + 1], bad_v[hit, sl:step + 1] = value, value
+    for got in (attend(bad_k, v), attend(k, bad_v)):
+      assert torch.equal(got[~hit], want[~hit]), (value, victim)
+    assert not torch.isfinite(got[hit]).any(1).any()  # and it was one of the values that count
+
+
 @pytest.mark.parametrize('nseq,T,N,Kh,H,C,step', [
     (2, 40, 4, 4, 64, 64, 3), (3, 9, 8, 2, 64, 96, 50), (2, 33, 32, 8, 128, 300, 200), (1, 64, 8, 1, 128, 128, 0),
     (2, 5, 16, 8, 128, 96, 60), (1, 128, 4, 4, 128, 200, 31), (2, 3, 8, 4, 64, 64, 20),

@@ -295,6 +295,38 @@ def test_many_samples_of_a_prompt_share_its_cache_rows():
   assert torch.isfinite(runs[True]).all() and (runs[True] - runs[False]).abs().max() <= 1e-2
 
 
+def test_a_sample_that_overflows_leaves_the_others_of_its_prompt_alone():
+  """More rows than there is room for parts, heads of the 8B shape: a sample reads a token whose embedding row overflows.  Its own
+  logits are lost, those of every other sample are, bit for bit, those of a batch in which it read another token."""
+  cfg = OM.Config('llama3', 2, 512, 256, 512, 4, 128, 1, norm_eps=1e-5)
+  model = C.product_model(cfg, C.make_state(cfg, 33, 8, norm_jitter=0.05), 64, 16.0)
+  model.embed[7] = float('inf')
+  rng = np.random.default_rng(13)
+  ids = np.repeat(rng.integers(8, 512, (17, 70)), 8, axis=0).astype(np.int32)
+  toks = torch.from_numpy(rng.integers(8, 512, (136, 5)).astype(np.int32)).cuda()
+  victims = torch.tensor([3, 8, 63, 135], device='cuda')
+  runs = []
+  for overflow in (False, True):
+    s = _sampler(model, cfg, 80)
+    s.eos_ids = np.array([-1])
+    st = s.init_sample_state(ids, 75, True, None, 0.0, None, None, 0)
+    assert (st['share_group'], st['share_len']) == (8, 64)
+    s.walk(st, 69)
+    steps = []
+    for step in range(5):
+      s.run_steps(st, 1, sample=True)
+      steps.append(st['logits'].clone())
+      st['token_buffer'][:, 70 + step] = toks[:, step]
+      if overflow and step == 1:
+        st['token_buffer'][victims, 70 + step] = 7
+    s.check_device_status(st)
+    runs.append(torch.stack(steps))
+  others = torch.ones(136, dtype=torch.bool, device='cuda')
+  others[victims] = False
+  assert torch.isfinite(runs[0]).all() and not torch.isfinite(runs[1][2:, victims]).any()
+  assert torch.equal(runs[1][:, others], runs[0][:, others])
+
+
 def test_temperature_sampling_follows_the_threefry_schedule():
   """Every generated token equals categorical(fold_in(PRNGKey(seed), decoding_step), logits / T)
   evaluated on the kernel's own logits, with decoding_step = P - 1, P, ... as in the reference

@@ -294,7 +294,6 @@ __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& l
   __syncthreads();
 
   const uint32_t row_bytes = (uint32_t)a.Kh * H * 2;
-  const uint32_t span = ((uint32_t)(a.C - 1) * a.Kh + 1) * H * 2;  // rows past the cache read zero
   // Where block blk lies: cache row, first slot, slots of the walk from there on, and the query row whose own it is
   struct Place { int kv, pos, len, own_of; };
   auto place = [&](int blk) __attribute__((always_inline)) {
@@ -302,36 +301,34 @@ __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& l
     const int i = __builtin_amdgcn_readfirstlane((blk - nlead) / nown), k = blk - nlead - i * nown;
     return Place{j.row0 + i, j.pend + k * 32, j.own - k * 32, i};
   };
-  auto cache_of = [&](const uint16_t* cache, int row) __attribute__((always_inline)) {
-    return make_rsrc(cache + ((size_t)row * a.C * a.Kh + kvh) * H, span);
+  // Rows from slot `end` on read zero and fetch nothing.  That is the end of the walk, not of the cache: a probability of 0 does
+  // not cover a row that is not finite, and behind the shared slots lie the leader's own, which no other sequence may see.
+  auto cache_of = [&](const uint16_t* cache, int row, int end) __attribute__((always_inline)) {
+    return make_rsrc(cache + ((size_t)row * a.C * a.Kh + kvh) * H, end > 0 ? ((uint32_t)(end - 1) * a.Kh + 1) * H * 2 : 0u);
   };
-  const __amdgpu_buffer_rsrc_t rk_lead = cache_of(a.kcache, lead), rv_lead = cache_of(a.vcache, lead);
+  const __amdgpu_buffer_rsrc_t rk_lead = cache_of(a.kcache, lead, j.pend), rv_lead = cache_of(a.vcache, lead, j.pend);
   uint16_t* vt = reinterpret_cast<uint16_t*>(lds.tiles) + wave * 32 * H;
   // V tile transfer: load i moves rows i RPD .. i RPD + RPD - 1 of the block, the 16-byte chunks of row r
   // XOR-swizzled by r % CPR.  Row i RPD + lane / CPR has r % CPR = (i RPD) % CPR ^ lane / CPR, so the per-lane
   // part of the swizzle is one word and the rest a constant per load; the offsets are formed at the transfer
   // (kept in registers over the loop they would be spilled)
   const int vrow = (lane / CPR) * row_bytes, vswz = (lane % CPR) ^ (lane / CPR);
-  // OWN: a row has few slots of its own, so most of its last block lies behind them; the transfers there repeat the last one
   auto dma_v = [&](const Place& p) __attribute__((always_inline)) {
-    const __amdgpu_buffer_rsrc_t rv = OWN ? cache_of(a.vcache, p.kv) : rv_lead;
+    const __amdgpu_buffer_rsrc_t rv = OWN ? cache_of(a.vcache, p.kv, p.pos + p.len) : rv_lead;
     int sw = vswz;
     asm volatile("" : "+v"(sw));
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int r0 = OWN ? min(i * RPD, (p.len - 1) / RPD * RPD) : i * RPD;
-      load_row_to_lds(rv, vt + i * RPD * H, vrow + ((sw ^ ((i * RPD) % CPR)) << 4), (p.pos + r0) * row_bytes);
-    }
+    for (int i = 0; i < NLD; ++i)
+      load_row_to_lds(rv, vt + i * RPD * H, vrow + ((sw ^ ((i * RPD) % CPR)) << 4), (p.pos + i * RPD) * row_bytes);
   };
   // K fragments of a block: lane (position qi, h) reads the half h of its row, 16 bytes per MFMA step
   const int koff = qi * row_bytes + h * H;
   u32x4_t kf[KS];
   auto load_k = [&](const Place& p) __attribute__((always_inline)) {
-    const __amdgpu_buffer_rsrc_t rk = OWN ? cache_of(a.kcache, p.kv) : rk_lead;
-    const int off = OWN ? min(qi, p.len - 1) * (int)row_bytes + h * H : koff;
+    const __amdgpu_buffer_rsrc_t rk = OWN ? cache_of(a.kcache, p.kv, p.pos + p.len) : rk_lead;
 #pragma unroll
     for (int t = 0; t < KS; ++t)
-      kf[t] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rk, off + t * 16, p.pos * row_bytes, 0));
+      kf[t] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rk, koff + t * 16, p.pos * row_bytes, 0));
   };
   auto mask_byte = [&](const Place& p) __attribute__((always_inline)) {
     const int at = p.pos + qi;
@@ -371,7 +368,8 @@ __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& l
     // accumulator register r holds position 8 (r / 4) + 4 h + r % 4 of the block: with the lane's half folded
     // into the mask word and the limit, the per-register part is a compile-time constant
     const uint32_t mb2 = mbits >> (4 * h);
-    const int lim = (OWN && at.own_of >= 0 && at.own_of != qi / G ? 0 : at.len) - 4 * h;  // another row's own slots: none
+    const bool mine = !OWN || at.own_of < 0 || at.own_of == qi / G;  // shared slots, or this query row's own
+    const int lim = (mine ? at.len : 0) - 4 * h;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int pc = (r >> 2) * 8 + (r & 3);
@@ -413,29 +411,42 @@ __device__ __forceinline__ void gqa_tile_walk(const AttnArgs& a, PrefixLds<H>& l
       int lsw = (2 * g2 + (q4 >> 1)) ^ (4 * h + k4), lbase = (4 * h + k4) * H + 4 * (q4 & 1);
       asm volatile("" : "+v"(lsw), "+v"(lbase));
       typedef short s16x4_t __attribute__((ext_vector_type(4)));
-#pragma unroll
-      for (int kb2 = 0; kb2 < 2; ++kb2) {
+      // acc += V^T . P^T of hidden tile c over positions 16 kb2 .. 16 kb2 + 15 of the block
+      auto add_pv = [&](int c, int kb2, f32x16_t acc) __attribute__((always_inline)) {
         const u32x4_t pf = {pk[4 * kb2], pk[4 * kb2 + 1], pk[4 * kb2 + 2], pk[4 * kb2 + 3]};
         const u32x4_t pg = {pl2[4 * kb2], pl2[4 * kb2 + 1], pl2[4 * kb2 + 2], pl2[4 * kb2 + 3]};
+        s16x4_t run[2];
+#pragma unroll
+        for (int a2 = 0; a2 < 2; ++a2) {
+          const int row0 = 16 * kb2 + 8 * a2;  // the run without the lane's 4 h + k4
+          const uint16_t* src = vt + lbase + row0 * H + ((lsw ^ (4 * c) ^ (row0 % CPR)) << 3);
+          run[a2] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) s16x4_t*)(src));
+        }
+        uint32_t vw[4];
+        __builtin_memcpy(&vw[0], &run[0], 8);
+        __builtin_memcpy(&vw[2], &run[1], 8);
+        const u32x4_t vf = {vw[0], vw[1], vw[2], vw[3]};
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf),
+                                                      __builtin_bit_cast(bf16x8_t, pf), acc, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf),
+                                                       __builtin_bit_cast(bf16x8_t, pg), acc, 0, 0, 0);
+      };
+      if constexpr (OWN) {
+        // The columns of the other rows keep what they have: their probabilities of 0 would make NaN of a value of this row that
+        // is not finite.  One hidden tile at a time, whose sum so far waits in 16 registers.
 #pragma unroll
         for (int c = 0; c < HT; ++c) {
-          s16x4_t run[2];
+          const f32x16_t sum = add_pv(c, 1, add_pv(c, 0, o[c]));
 #pragma unroll
-          for (int a2 = 0; a2 < 2; ++a2) {
-            const int row0 = 16 * kb2 + 8 * a2;  // the run without the lane's 4 h + k4
-            const uint16_t* src = vt + lbase + row0 * H + ((lsw ^ (4 * c) ^ (row0 % CPR)) << 3);
-            run[a2] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) s16x4_t*)(src));
-          }
-          uint32_t vw[4];
-          __builtin_memcpy(&vw[0], &run[0], 8);
-          __builtin_memcpy(&vw[2], &run[1], 8);
-          const u32x4_t vf = {vw[0], vw[1], vw[2], vw[3]};
-          o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf),
-                                                         __builtin_bit_cast(bf16x8_t, pf), o[c], 0, 0, 0);
-          o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf),
-                                                         __builtin_bit_cast(bf16x8_t, pg), o[c], 0, 0, 0);
+          for (int r = 0; r < 16; ++r) o[c][r] = mine ? sum[r] : o[c][r];
+          asm volatile("" : "+v"(o[c]));  // now: at the end of the loop all four tiles' old and new sums would be alive
         }
+      } else {
+#pragma unroll
+        for (int kb2 = 0; kb2 < 2; ++kb2)
+#pragma unroll
+          for (int c = 0; c < HT; ++c) o[c] = add_pv(c, kb2, o[c]);
       }
     }
     // the tile's reads are complete before the next transfer overwrites it.  The next block's K rows are
@@ -563,7 +574,9 @@ __global__ __launch_bounds__(256, 3) void gqa_tile_kernel(AttnArgs a, int n_grou
 // Groups alone: a workgroup walks the shared slots of its group and then every query row's own, for whose blocks the other
 // rows' columns are masked (7 of 8 columns of the MFMA tile idle there, which costs nothing: it waits for memory).  Every
 // cache row is read once and, in one split, no part leaves the workgroup.  256 rows of the 8B shape in groups of 8 at 128 + 12
-// slots 36.0 us by themselves, 14.8 here; 8 layers, 24 steps of that 68.6 -> 61.8 ms.  grid (Kh, group query blocks, splits).
+// slots 36.0 us by themselves, 14.8 here; 8 layers, 24 steps of that 68.6 -> 61.8 ms.  That a sequence whose values are not
+finite leaves the others' sums alone (the select behind every tile of V^T . P^T) is 1.1 of 14.2 us in the step.  grid (Kh, group
+query blocks, splits).
 template <int H, int G>
 __global__ __launch_bounds__(256, 3) void gqa_group_kernel(AttnArgs a) {
   __shared__ PrefixLds<H> lds;
