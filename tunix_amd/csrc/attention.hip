@@ -575,8 +575,8 @@ __global__ __launch_bounds__(256, 3) void gqa_tile_kernel(AttnArgs a, int n_grou
 // rows' columns are masked (7 of 8 columns of the MFMA tile idle there, which costs nothing: it waits for memory).  Every
 // cache row is read once and, in one split, no part leaves the workgroup.  256 rows of the 8B shape in groups of 8 at 128 + 12
 // slots 36.0 us by themselves, 14.8 here; 8 layers, 24 steps of that 68.6 -> 61.8 ms.  That a sequence whose values are not
-finite leaves the others' sums alone (the select behind every tile of V^T . P^T) is 1.1 of 14.2 us in the step.  grid (Kh, group
-query blocks, splits).
+// finite leaves the others' sums alone (the select behind every tile of V^T . P^T) is 1.1 of 14.2 us in the step.  grid (Kh, group
+// query blocks, splits).
 template <int H, int G>
 __global__ __launch_bounds__(256, 3) void gqa_group_kernel(AttnArgs a) {
   __shared__ PrefixLds<H> lds;
