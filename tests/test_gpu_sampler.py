@@ -267,10 +267,11 @@ def test_samples_of_one_prompt_share_its_cache_rows_and_match_oracle():
   assert np.abs(runs[True] - runs[False]).max() <= 1e-2
 
 
-def test_many_samples_of_a_prompt_share_its_cache_rows():
+@pytest.mark.parametrize('n,h,kh', [(16, 64, 8), (16, 128, 4)])
+def test_many_samples_of_a_prompt_share_its_cache_rows(n, h, kh):
   """17 prompts of 230 tokens x 8 samples, more rows than there is room for parts: one workgroup per group and kv head walks
   the shared slots and all rows' own.  Logits are those of rows that walk their caches by themselves."""
-  cfg = OM.Config('llama3', 2, 512, 256, 512, 16, 64, 8, norm_eps=1e-5)
+  cfg = OM.Config('llama3', 2, 512, 256, 512, n, h, kh, norm_eps=1e-5)
   model = C.product_model(cfg, C.make_state(cfg, 31, 8, norm_jitter=0.05), 64, 16.0)
   rng = np.random.default_rng(12)
   ids = np.repeat(rng.integers(3, 512, (17, 230)), 8, axis=0).astype(np.int32)
@@ -284,7 +285,7 @@ def test_many_samples_of_a_prompt_share_its_cache_rows():
     assert (st['share_group'], st['share_len']) == ((8, 224) if share else (1, 0))
     s.walk(st, 229)
     if share:  # the group's first sequence alone is read there
-      st['cache'].view(2, 2, 17, 8, 240, 8, 64)[:, :, :, 1:, :224] = float('nan')
+      st['cache'].view(2, 2, 17, 8, 240, kh, h)[:, :, :, 1:, :224] = float('nan')
     steps = []
     for step in range(5):
       s.run_steps(st, 1, sample=True)
@@ -298,27 +299,28 @@ def test_many_samples_of_a_prompt_share_its_cache_rows():
 def test_a_sample_that_overflows_leaves_the_others_of_its_prompt_alone():
   """More rows than there is room for parts, heads of the 8B shape: a sample reads a token whose embedding row overflows.  Its own
   logits are lost, those of every other sample are, bit for bit, those of a batch in which it read another token."""
-  cfg = OM.Config('llama3', 2, 512, 256, 512, 4, 128, 1, norm_eps=1e-5)
+  cfg = OM.Config('llama3', 2, 512, 256, 512, 16, 128, 4, norm_eps=1e-5)
   model = C.product_model(cfg, C.make_state(cfg, 33, 8, norm_jitter=0.05), 64, 16.0)
   model.embed[7] = float('inf')
   rng = np.random.default_rng(13)
-  ids = np.repeat(rng.integers(8, 512, (17, 70)), 8, axis=0).astype(np.int32)
+  ids = np.repeat(rng.integers(8, 512, (17, 230)), 8, axis=0).astype(np.int32)
   toks = torch.from_numpy(rng.integers(8, 512, (136, 5)).astype(np.int32)).cuda()
   victims = torch.tensor([3, 8, 63, 135], device='cuda')
   runs = []
   for overflow in (False, True):
-    s = _sampler(model, cfg, 80)
+    s = _sampler(model, cfg, 240)
     s.eos_ids = np.array([-1])
-    st = s.init_sample_state(ids, 75, True, None, 0.0, None, None, 0)
-    assert (st['share_group'], st['share_len']) == (8, 64)
-    s.walk(st, 69)
+    st = s.init_sample_state(ids, 235, True, None, 0.0, None, None, 0)
+    assert (st['share_group'], st['share_len']) == (8, 224)
+    s.walk(st, 229)
+    st['cache'].view(2, 2, 17, 8, 240, 4, 128)[:, :, :, 1:, :224] = float('nan')  # the group's first sequence alone is read there
     steps = []
     for step in range(5):
       s.run_steps(st, 1, sample=True)
       steps.append(st['logits'].clone())
-      st['token_buffer'][:, 70 + step] = toks[:, step]
+      st['token_buffer'][:, 230 + step] = toks[:, step]
       if overflow and step == 1:
-        st['token_buffer'][victims, 70 + step] = 7
+        st['token_buffer'][victims, 230 + step] = 7
     s.check_device_status(st)
     runs.append(torch.stack(steps))
   others = torch.ones(136, dtype=torch.bool, device='cuda')

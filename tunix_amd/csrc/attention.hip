@@ -19,7 +19,6 @@
 namespace tmx {
 
 constexpr int kMaxPrefixSplits = 4;  // splits of the slots that a group of sequences shares
-constexpr int kMaxGroupSplits = 8;   // the same where the group's workgroups walk its rows' own slots too
 
 // waves per workgroup: fewer for wide groups so the merge buffers stay under 64 KiB
 template <int G>
@@ -573,15 +572,15 @@ __global__ __launch_bounds__(256, 3) void gqa_tile_kernel(AttnArgs a, int n_grou
 
 // Groups alone: a workgroup walks the shared slots of its group and then every query row's own, for whose blocks the other
 // rows' columns are masked (7 of 8 columns of the MFMA tile idle there, which costs nothing: it waits for memory).  Every
-// cache row is read once and, in one split, no part leaves the workgroup.  256 rows of the 8B shape in groups of 8 at 128 + 12
+// cache row is read once and no part leaves the workgroup.  256 rows of the 8B shape in groups of 8 at 128 + 12
 // slots 36.0 us by themselves, 14.8 here; 8 layers, 24 steps of that 68.6 -> 61.8 ms.  That a sequence whose values are not
 // finite leaves the others' sums alone (the select behind every tile of V^T . P^T) is 1.1 of 14.2 us in the step.  grid (Kh, group
-// query blocks, splits).
+// query blocks).
 template <int H, int G>
 __global__ __launch_bounds__(256, 3) void gqa_group_kernel(AttnArgs a) {
   __shared__ PrefixLds<H> lds;
   TileJob j;
-  if (tile_job<G>(a, gridDim.y, blockIdx.y, blockIdx.z, false, j)) gqa_tile_walk<H, G, true>(a, lds, blockIdx.x, j);
+  if (tile_job<G>(a, gridDim.y, blockIdx.y, 0, false, j)) gqa_tile_walk<H, G, true>(a, lds, blockIdx.x, j);
 }
 
 // The same grid with the rows' own slots on the vector-ALU walk (gqa_decode_walk) and only the shared slots on
@@ -902,12 +901,17 @@ static AttnPlan plan_rows_walk(int B, int N, int Kh, int H, int C, bool shared, 
 // With shared prompt slots: rows by themselves, groups and rows side by side, or groups alone, whichever costs least at the
 // middle of the rollout (half of the `len` - share_len slots behind the prompt in use).  us, launches included; every walk has
 // a fixed part, cache bytes at 5.2 TB/s (4.7 in the group walk, which reads K in 16-byte pieces), and the combine launch of
-// several parts 3.4; a workgroup of the group walk takes 2.2 per round of its four waves.  Measured on cold caches, 8 kv heads of 4 query heads, rows x group, shared + own slots: rows by
-// themselves / side by side / groups alone:
-//   256 x 8, 128 + 12   36.0 /   -  / 14.8       256 x 8, 256 + 512  140.8 /   -  / 111.5     128 x 8, 256 + 24  32.0 / 18.3 / 13.9
-//   64 x 8, 256 + 32    19.9 / 13.5 / 12.0 in 4  64 x 8, 256 + 256    29.7 / 23.7 /  25.1     128 x 8, 64 + 32   15.4 / 17.8 / 12.3
-//   32 x 8, 256 + 64    17.2 / 12.4 / 10.6 in 8  48 x 8, 224 + 32     17.8 / 12.2 /  11.3     24 x 6, 64 + 24     7.0 /  9.4 /  8.7
-// (in one split but where noted).  More than 128 rows have no room for parts: groups alone in one split.
+// several parts 3; a workgroup of the group walk takes 2.2 (1.6 at head dimension 64) per round of its four waves.  Groups side by
+// side with rows need room for parts, which more than 128 rows have not.  Measured as a whole step of a layer (us), rows x group, shared +
+// most own slots, heads of the 8B shape where not noted: rows by themselves / side by side / groups alone:
+//   64 x 8, 256 + 64   151.4 / 146.8 / 150.5   64 x 8, 256 + 256  146.3 / 139.9 / 157.3   48 x 8, 224 + 32   151.9 / 149.8 / 151.6
+//   128 x 8, 256 + 24  278.2 / 262.8 / 262.5   128 x 8, 64 + 32   208.2 / 210.1 / 203.9   128 x 4, 128 + 24  265.6 / 263.3 / 255.0
+//   120 x 3, 200 + 24  328.1 / 324.6 / 323.2   40 x 2, 100 + 24   159.1 / 160.6 / 159.2   24 x 6, 64 + 24    109.6 / 112.1 / 112.4
+//   1B 64 x 8, 256 + 64  98.1 / 95.3 / 95.6    1B 128 x 8, 128 + 32  145.6 / 145.8 / 140.2    1B 32 x 8, 64 + 32  72.9 / 76.4 / 75.6
+//   30B-A3B 32 x 8, 256 + 48  164.4 / 163.4 / 165.8   30B-A3B 64 x 8, 128 + 32  197.0 / 199.2 / 197.8
+// Groups alone in several splits, merged by the combine kernel, came within 1 % of the better of the two in each of these.
+// By themselves on cold caches, 2 to 32 kv heads of 1 to 8 heads, head dimensions 64 and 128, 32 to 128 rows, the choice is within
+// 10 % of the best in 52 of 56 shapes and 20 % off at most (4 kv heads of 8, 64 x 4, 96 + 32: 8.9 against 7.4 by themselves).
 static AttnPlan plan_attention(int B, int N, int Kh, int H, int C, int share_gs, int share_len, int len, bool must_share) {
   const AttnPlan rows = plan_rows_walk(B, N, Kh, H, C, false, 0, 0);
   if (!attn_share_ok(B, N, Kh, H, C, share_gs, share_len)) return rows;
@@ -919,17 +923,15 @@ static AttnPlan plan_attention(int B, int N, int Kh, int H, int C, int share_gs,
   auto offer = [&](const AttnPlan& p, float cost) {
     if (cost < best_cost) { best = p; best_cost = cost; }
   };
-  const long wgs = group_workgroups(B, G, Kh, share_gs), slots = 3L * device_cus();
+  const long wgs = group_workgroups(B, G, Kh, share_gs);
   if (B <= 128) {
     const AttnPlan p = plan_rows_walk(B, N, Kh, H, C, true, share_gs, share_len);
     if (p.shared) offer(p, 9.2f + us_per_slot * ((float)B * Kh * own + (float)wgs * share_len));
   }
   const int rpb = 32 / G, nrows = share_gs < rpb ? share_gs : rpb;
   const int blocks = (share_len + 31) / 32 + nrows * ((own + 31) / 32);
-  for (int z = 1; z <= (B <= 128 ? kMaxGroupSplits : 1) && (z == 1 || wgs * z <= slots); ++z) {
-    const float rounds = 2.2f * ((blocks + 4 * z - 1) / (4 * z)), bytes = 1.1f * us_per_slot * 32.f * blocks * wgs;
-    offer(AttnPlan{false, true, 0, z}, 4.4f + (rounds > bytes ? rounds : bytes) + (z > 1 ? 3.4f : 0.f));
-  }
+  const float rounds = (H == 64 ? 1.6f : 2.2f) * ((blocks + 3) / 4), bytes = 1.1f * us_per_slot * 32.f * blocks * wgs;
+  offer(AttnPlan{false, true, 0, 1}, 4.4f + (rounds > bytes ? rounds : bytes));
   return best;
 }
 
@@ -956,7 +958,7 @@ static int launch_tile(hipStream_t st, const AttnArgs& a, bool rows_on_tile) {
   }
   const int nz = a.nsplit > a.psplits ? a.nsplit : a.psplits;
   const dim3 grid(a.Kh, n_group_y + a.B, nz);
-  if (!a.nsplit) hipLaunchKernelGGL((gqa_group_kernel<H, G>), dim3(a.Kh, n_group_y, a.psplits), dim3(256), 0, st, a);
+  if (!a.nsplit) hipLaunchKernelGGL((gqa_group_kernel<H, G>), dim3(a.Kh, n_group_y), dim3(256), 0, st, a);
   else if (rows_on_tile) hipLaunchKernelGGL((gqa_tile_kernel<H, G>), grid, dim3(256), 0, st, a, n_group_y);
   else if constexpr (G <= 4) hipLaunchKernelGGL((gqa_shared_kernel<H, G>), grid, dim3(256), 0, st, a, n_group_y);
   else return TMX_ERR_UNSUPPORTED;

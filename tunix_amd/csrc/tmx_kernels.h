@@ -182,7 +182,7 @@ struct AttnArgs {
   // come in consecutive groups of share_gs whose cache slots [0, share_len) and input_mask entries are
   // identical.  Those slots are then walked once per group (psplits splits, from the group's first sequence), every row's
   // own slots share_len .. *step by a workgroup of its own (nsplit splits) or by the group's (nsplit = 0), and
-  // the nsplit + psplits partial results per row are merged by the combine kernel.
+  // the nsplit + psplits partial results per row are merged by the combine kernel (the group's workgroups leave one, the result).
   int share_gs, share_len, psplits;
   bool must_share;  // never every row by itself, whatever that would cost
 };
