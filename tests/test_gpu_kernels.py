@@ -1346,17 +1346,22 @@ def test_moe_experts_row_counts(down, K, N):
   assert ((got - want).abs() > 2.0 ** -6 * want.abs() + 2.0 ** -8).sum() == 0
 
 
-# The stream kernel with the rows of an expert in LDS: no row, one, as many as fit (11 of 2048 up, 18 to 32 down), one more, several
-# loads of them; waves without columns; one, two and three workgroups' room.  The reference is the f32 product.
-@pytest.mark.parametrize('down,K,N', [(0, 2048, 256), (0, 2048, 128), (0, 256, 896), (1, 768, 256), (1, 512, 128), (1, 4096, 384)])
-def test_moe_experts_of_few_rows(down, K, N):
+# The stream kernel with the rows of an expert in LDS: no row, one, as many as fit, one more, which then all come from global
+# memory, and 32 and more of those; waves without columns.  `fit`: rows that LDS has room for beside 512 bytes of zeros, in four
+# workgroups of a CU (down), three (gate | up, of which 32 rows of 256 would leave room) or, of 4096 values, two.  The reference is
+# the f32 product.
+@pytest.mark.parametrize('down,K,N,fit', [(0, 2048, 256, 12), (0, 2048, 128, 12), (0, 256, 896, 32), (1, 768, 256, 24), (1, 512, 128, 32), (1, 4096, 384, 9)])
+def test_moe_experts_of_few_rows(down, K, N, fit):
   from tunix_amd import quant
-  counts = [0, 1, 11, 12, 35, 2, 0, 3, 1, 4, 18, 19, 2, 1, 1, 0, 5, 1, 0, 2, 1, 1, 0, 2] + [0] * 24  # whole tokens of two pairs
+  wgs = 3 if not down else 2 if K == 4096 else 4
+  assert min(((160 * 1024 - 4 * 2304) // wgs - 512) // ((K + 8) * 2), 32) == fit
+  counts = [0, 1, fit, fit + 1, 2, 0, 3, 1, 31, 32, 33, 2, 0, 1, 35] + [0] * 45  # whole tokens of two pairs
   E, k, group = len(counts), 2, 64
   g = torch.Generator(device=G.DEV).manual_seed(K + N)
   idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
   P = idx.numel()
-  assert P <= 1024 and P % k == 0 and P / E + 3.5 * (P / E) ** 0.5 <= 9
+  need = int(np.ceil(P / E + 3.5 * (P / E) ** 0.5))
+  assert P <= 1024 and P % k == 0 and need <= fit and (K < 4096 or need > 6)  # (6 rows of 4096 would fit three workgroups)
   idx = idx[torch.randperm(P, generator=torch.Generator().manual_seed(3))].to(torch.int32).to(G.DEV)
   w = (torch.randn(K, E * N, generator=g, device=G.DEV) * 0.05).to(torch.bfloat16)
   pl = quant.PackedLinear.from_dense([w], group, G.DEV)

@@ -347,13 +347,17 @@ static int launch_qlinear4(hipStream_t st, QLinearArgs a) {
 // or gate / up tile pairs (SwiGLU in its epilogue) over all of K with no barrier after the
 // compaction.  Weight tiles come through a ring of kMoeRing tiles per wave (buffer loads, scalar
 // offsets), requested in front of the compaction; output rows are scattered.  The ring runs on
-// across the wave's tiles, so the stream never drains.  LDS: the expert's rows are gathered into LDS, and an absent row's
-// fragments are read from zeros; otherwise the fragments of the live rows come straight from global memory, for which the
-// compiler makes 16 exec-mask regions and 86 register fills per 8 weight tiles.  Rows that do not fit, and more than 32, are
-// taken in chunks, each streaming the weights again (rare).
+// across the wave's tiles, so the stream never drains; a slot is refilled when its tile has been multiplied, into the same registers
+// (requested before that it takes others, and the copies between them drain the ring once a group).  LDS: up to x_rows rows of the
+// expert are gathered into LDS; the fragments of more come straight from global memory, 32 rows at a time, so the weights
+// are streamed again for each 32 rows only, whatever fits LDS.
 // What bounds it: the stream (128 experts of 2048 x 1536 and 768 x 2048, 32 rows of 8: 186 + 93 MB in 42.5 + 23.9 us, 4.4 + 3.9
 // TB/s with the launch) and, beside it, the dequantisation (35 ns per 512 weights of a SIMD, 23 + 12 us).  With the rows
 // looked up first and from global memory 48.5 + 29.6 us; 8 layers of that in 48 steps and the prompts 77.5 -> 72.5 ms.
+// Uneven routing (128 experts, top-8, gate|up + down; from global memory alone / in chunks of the rows that fit LDS, each streaming
+// again / so): 16 tokens alike 31.4 + 17.0 / 48.5 + 16.5 / 28.0 + 15.1, 32 alike 39.3 + 21.8 / 83.6 + 29.1 / 41.1 + 22.5, 32 in eights
+// 41.8 + 24.1 / 50.2 + 20.2 / 37.4 + 19.5, 64 in eights 49.9 + 32.9 / 71.5 + 27.0 / 46.2 + 25.0; even routing of 32 53.8 + 30.6 /
+// 49.9 + 25.4 / 47.8 + 24.8.
 // Weight tiles that ONE wave reads once, whole cache lines per load (the routed experts, the fused gate | up
 // launch): non-temporal buffer loads (the nt bit of the cache policy).  A plain streaming read reaches 5.6-6.2 TB/s
 // on this part, a non-temporal one 6.3-7.0; the split projections and the 64-row head measured slower with it.
@@ -362,11 +366,11 @@ constexpr int kNtLoad = 2;
 constexpr int kMoeStreamPairs = 1024;  // most pairs of a launch (more: moe_rows)
 constexpr int kMoeRing = 4;  // divides K / 64 (K % 256 == 0), so a ring slot is k-tile % 4 in every unit
 constexpr size_t kMoeLds = 160 * 1024 - 4 * 2304;  // of a CU, less what its workgroups hold beside x
-constexpr int kMoeXZero = 256;  // zeros in front of the rows' copy in LDS: a group of k-tiles of an absent row
+constexpr int kMoeXZero = 64 * kMoeRing;  // zeros in front of the rows' copy in LDS: a group of k-tiles of an absent row
 
 template <bool DOWN, bool LDS>
 __global__ __launch_bounds__(256, LDS ? (DOWN ? 4 : 3) : 2) void moe_stream_kernel(MoeArgs m) {
-  extern __shared__ __align__(16) uint16_t xs[];  // LDS: zeros, then x_rows rows
+  extern __shared__ __align__(16) uint16_t xs[];  // LDS: zeros, then up to x_rows rows
   __shared__ uint16_t rows_s[kMoeStreamPairs];
   __shared__ int wave_cnt[2][4];
   constexpr int TPU = DOWN ? 1 : 2;  // tiles per unit: one column tile, or a gate tile and its up tile
@@ -383,7 +387,7 @@ __global__ __launch_bounds__(256, LDS ? (DOWN ? 4 : 3) : 2) void moe_stream_kern
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(m.qw + (size_t)e * m.qw_stride, (uint32_t)NT * KT * 1024u);
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(m.scales + (size_t)e * m.sc_stride, (uint32_t)NT * KG * 64u);
   u32x4_t wring[kMoeRing][TPU];
-  uint16_t sring[kMoeRing][TPU];
+  uint32_t sring[kMoeRing][TPU];
   // tile (unit ui of this wave, k-tile kt) into ring slot sl; past the last unit: its last tile again
   auto load_w = [&](int ui, int kt, auto sc) __attribute__((always_inline)) {
     constexpr int sl = decltype(sc)::value;
@@ -423,36 +427,21 @@ __global__ __launch_bounds__(256, LDS ? (DOWN ? 4 : 3) : 2) void moe_stream_kern
     return m.x + (size_t)(DOWN ? pr : (m.pair0 + pr) / m.top_k) * m.ldx;
   };
   const int XS = m.K + 8;  // elements between the rows in LDS: 16 bytes of padding, rows on other banks
-  const int chunk = LDS ? m.x_rows : 32;
-  if (LDS && tid < kMoeXZero / 8) *reinterpret_cast<u32x4_t*>(xs + tid * 8) = u32x4_t{0u, 0u, 0u, 0u};
 
-  for (int c0 = 0; c0 < n; c0 += chunk) {
-    const int rows = n - c0 < chunk ? n - c0 : chunk;
-    if constexpr (LDS) {
-      if (c0) __syncthreads();
-      const int pieces = m.K >> 3;
-      for (int r = 0; r < rows; ++r) {
-        const uint16_t* src = x_row(c0 + r);
-        for (int c = tid; c < pieces; c += 256)
-          *reinterpret_cast<u32x4_t*>(xs + kMoeXZero + r * XS + c * 8) = *reinterpret_cast<const u32x4_t*>(src + c * 8);
-      }
-      __syncthreads();
-    }
-    if (nu == 0) continue;
-    if (c0 || !LDS) fill_ring();
-    // A fragments: lane (row nl, h) takes x[src][64 kt + 16 t + 8 h ..]; absent rows are zero
+  // rows c0 .. c0 + rows - 1 (at most 32) times this wave's units, whose first tiles are on the way
+  auto walk = [&](auto from_lds, int c0, int rows) __attribute__((always_inline)) {
+    // A fragments: lane (row nl, h) takes x[src][64 kt + 16 t + 8 h ..].  Absent rows, whose results go nowhere, are zeros in LDS
+    // (repeated rows cost the matrix pipe power, and all CUs clock: 64 tokens 56 + 28.5 us, with zeros 52 + 26.8); from memory
+    // they are the first one again.
+    constexpr bool lds = decltype(from_lds)::value;
     const bool live = nl < rows;
-    const uint16_t* xrow = x_row(c0 + (live ? nl : 0)) + 8 * h;
-    const uint16_t* xlds = xs + (live ? kMoeXZero + nl * XS : 0) + 8 * h;
-    const int kmask = live ? ~0 : 255;  // absent rows stay inside the zeros
+    const uint16_t* const xfirst = (lds ? xs + (live ? kMoeXZero + nl * XS : 0) : x_row(c0 + (live ? nl : 0))) + 8 * h;
+    const int xstep = lds && !live ? 0 : 64 * kMoeRing;  // from group to group of k-tiles
+    const uint16_t* xp = xfirst;
     u32x4_t xq[2][4];
-    auto load_x = [&](int kt, int slot) __attribute__((always_inline)) {
-      const uint16_t* p = xlds + ((kt * 64) & kmask);
+    auto load_x = [&](int sl, int slot) __attribute__((always_inline)) {  // k-tile sl of the group at xp
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        if constexpr (LDS) xq[slot][t] = *reinterpret_cast<const u32x4_t*>(p + 16 * t);
-        else xq[slot][t] = live ? *reinterpret_cast<const u32x4_t*>(xrow + kt * 64 + 16 * t) : u32x4_t{0, 0, 0, 0};
-      }
+      for (int t = 0; t < 4; ++t) xq[slot][t] = *reinterpret_cast<const u32x4_t*>(xp + sl * 64 + 16 * t);
     };
     load_x(0, 0);
     f32x16_t acc[TPU];
@@ -465,42 +454,61 @@ __global__ __launch_bounds__(256, LDS ? (DOWN ? 4 : 3) : 2) void moe_stream_kern
         static_for<kMoeRing>([&](auto sc) __attribute__((always_inline)) {
           constexpr int sl = decltype(sc)::value;
           const int kt = k0 + sl;
-          load_x(kt + 1 < KT ? kt + 1 : 0, (sl & 1) ^ 1);  // the next k-tile (of the next unit: the same rows)
-          u32x4_t wc[TPU];
-          float s_c[TPU];
-#pragma unroll
-          for (int c = 0; c < TPU; ++c) { wc[c] = wring[sl][c]; s_c[c] = bf2f(sring[sl][c]); }
-          // slot consumed: refill it with the tile kMoeRing steps on in the wave's unit-major order
-          if (kt + kMoeRing < KT) load_w(u, kt + kMoeRing, sc);
-          else load_w(u + 1, kt + kMoeRing - KT, sc);
+          if constexpr (sl == kMoeRing - 1) xp = kt + 1 < KT ? xp + xstep : xfirst;
+          load_x((sl + 1) % kMoeRing, (sl & 1) ^ 1);  // the next k-tile (of the next unit: the same rows)
 #pragma unroll
           for (int c = 0; c < TPU; ++c) {
-            const NibbleScale sc = nibble_scale(s_c[c]);
-            const uint32_t wd[4] = {wc[c].x, wc[c].y, wc[c].z, wc[c].w};
+            const NibbleScale scale = nibble_scale(bf2f((uint16_t)sring[sl][c]));
+            const u32x4_t wd = wring[sl][c];
 #pragma unroll
             for (int t = 0; t < 4; ++t)
               acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, xq[sl & 1][t]),
-                                                               dequant_word(wd[t], sc), acc[c], 0, 0, 0);
+                                                               dequant_word(wd[t], scale), acc[c], 0, 0, 0);
           }
+          __builtin_amdgcn_sched_barrier(0);
+          // slot consumed: refill it with the tile kMoeRing steps on in the wave's unit-major order
+          if (kt + kMoeRing < KT) load_w(u, kt + kMoeRing, sc);
+          else load_w(u + 1, kt + kMoeRing - KT, sc);
+          __builtin_amdgcn_sched_barrier(0);
         });
       }
       // epilogue of the unit
       const int ut = u0 + u * ustride;
+      int le = lane;
+      asm volatile("" : "+v"(le));  // (the output rows are looked up here: kept over the loop they would not fit the registers)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int row = acc_row(r, lane);
+        const int row = acc_row(r, le);
         if (row >= rows) continue;
         const int p = rows_s[c0 + row];
         if (DOWN) {
-          m.out[(size_t)p * m.ldo + ut * 32 + nl] = f2bf(acc[0][r]);
+          m.out[(size_t)p * m.ldo + ut * 32 + (le & 31)] = f2bf(acc[0][r]);
         } else {
           const float g = rbf(acc[0][r]), up = rbf(acc[TPU - 1][r]);
           const float sg = rbf(1.f / (1.f + expf(-g)));
-          m.out[(size_t)p * m.ldo + ut * 32 + nl] = f2bf(rbf(g * sg) * up);
+          m.out[(size_t)p * m.ldo + ut * 32 + (le & 31)] = f2bf(rbf(g * sg) * up);
         }
       }
     }
+  };
+
+  if (!LDS || n > m.x_rows) {
+    if (nu == 0) return;
+    for (int c0 = 0; c0 < n; c0 += 32) {
+      fill_ring();
+      walk(IC<0>{}, c0, n - c0 < 32 ? n - c0 : 32);
+    }
+    return;
   }
+  if (tid < kMoeXZero / 8) *reinterpret_cast<u32x4_t*>(xs + tid * 8) = u32x4_t{0u, 0u, 0u, 0u};
+  const int pieces = m.K >> 3;
+  for (int r = 0; r < n; ++r) {
+    const uint16_t* src = x_row(r);
+    for (int c = tid; c < pieces; c += 256)
+      *reinterpret_cast<u32x4_t*>(xs + kMoeXZero + r * XS + c * 8) = *reinterpret_cast<const u32x4_t*>(src + c * 8);
+  }
+  __syncthreads();
+  if (nu > 0) walk(IC<1>{}, 0, n);
 }
 
 int moe_experts(hipStream_t st, const MoeArgs& a, int E, bool down) {
@@ -531,8 +539,8 @@ int moe_experts(hipStream_t st, const MoeArgs& a, int E, bool down) {
   const int units = down ? a.N / 32 : a.N / 64;
   int groups = units / (down ? 8 : 4);
   groups = groups < 1 ? 1 : (groups > 32 ? 32 : groups);
-  // Rows in LDS: as many as leave room for the workgroups whose registers fit a CU (down: or one or two fewer), if an expert
-  // seldom has more (the mean + 3.5 sqrt(mean)), since one that has streams its matrices again.  us, from global memory / LDS, 128
+  // Rows in LDS: as many as leave room for the workgroups whose registers fit a CU (down: or one or two fewer), if at even routing an
+  // expert seldom has more (the mean + 3.5 sqrt(mean)), since one that has reads all its rows from global memory.  us, from global memory / LDS, 128
   // experts of 2048 x 768, top-8: 8 rows up 44.1 / 39.3, down 22.0 / 18.8; 32 rows 48.5 / 42.5, 29.6 / 23.9; 64 rows 51.4 / 47.6,
   // 32.5 / 26.6; 128 rows up (two workgroups of a CU) 55.7 / 56.8, down 36.3 / 29.7.
   const float mean = (float)a.P / E;
