@@ -1069,6 +1069,22 @@ def test_moe_route_matches_oracle(B, D, E, k):
       np.testing.assert_array_equal(got_idx[b], want_idx[b])
       np.testing.assert_allclose(got_w[b], want_w[b], atol=2 * G.ulp_bf16(want_w[b]).max())
   np.testing.assert_allclose(got_w.sum(-1), 1.0, atol=0.02)
+
+
+# one workgroup a token, and 16 tokens a workgroup; a group of four experts and a last lane of fewer
+@pytest.mark.parametrize('B,E,k', [(5, 128, 8), (300, 128, 8), (257, 72, 64), (290, 8, 3)])
+def test_moe_route_of_equal_scores_takes_the_lower_experts_first(B, E, k):
+  """Scores that are multiples of 1/16 (exact in bf16, many of them equal): the order is that of lax.top_k."""
+  T = G.Keep()
+  rng = np.random.default_rng(B + E)
+  x, rw = rng.integers(-1, 2, (B, 256)).astype(np.float32), rng.integers(-1, 2, (256, E)).astype(np.float32) / 16
+  idx = torch.full((B, k), -1, dtype=torch.int32, device=G.DEV)
+  wt = torch.zeros(B, k, dtype=torch.float32, device=G.DEV)
+  G.call('tmx_moe_route', S(), T.bf(x), T.bf(rw), B, 256, E, k, G.p(idx), G.p(wt))
+  G.sync()
+  scores = x @ rw
+  assert np.abs(scores).max() < 16 and (np.diff(np.sort(scores, axis=-1), axis=-1) == 0).any(-1).mean() > 0.5
+  np.testing.assert_array_equal(idx.cpu().numpy(), np.argsort(-scores, axis=-1, kind='stable')[:, :k])
   assert (got_idx >= 0).all() and (got_idx < E).all()
   assert all(len(set(r)) == k for r in got_idx)
 

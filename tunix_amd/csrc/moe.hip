@@ -83,22 +83,22 @@ __global__ __launch_bounds__(kRouterThreads) void moe_router_rows_kernel(RouterA
     // the place of expert e: larger probabilities, and equal ones of a lower id.  As integers (they are not negative), those are
     // the ones above v - 1 in front of its group of four, above v behind, and in the group the equal ones are looked up.  Two
     // experts of a lane at a time share the broadcast reads, whose latency is what this takes
-    const int* pi = reinterpret_cast<const int*>(p);
+    auto bits = [](float v) { return __float_as_int(v); };
     for (int e1 = lane; e1 < (a.E + 63) / 64 * 64; e1 += 128) {
-      const int ee[2] = {min(e1, a.E - 1), min(e1 + 64, a.E - 1)}, v[2] = {pi[ee[0]], pi[ee[1]]};
+      const int ee[2] = {min(e1, a.E - 1), min(e1 + 64, a.E - 1)}, v[2] = {bits(p[ee[0]]), bits(p[ee[1]])};
       int place[2] = {0, 0};
 #pragma unroll 8
       for (int j = 0; j < a.E; j += 4) {
-        const int4 u = *reinterpret_cast<const int4*>(pi + j);
+        const f32x4_t u = *reinterpret_cast<const f32x4_t*>(p + j);
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
           const int t = v[k] - (j + 3 < ee[k] ? 1 : 0);
-          place[k] += (u.x > t) + (u.y > t) + (u.z > t) + (u.w > t);
+          place[k] += (bits(u[0]) > t) + (bits(u[1]) > t) + (bits(u[2]) > t) + (bits(u[3]) > t);
         }
       }
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        for (int j = ee[k] & ~3; j < ee[k]; ++j) place[k] += pi[j] == v[k];
+        for (int j = ee[k] & ~3; j < ee[k]; ++j) place[k] += bits(p[j]) == v[k];
         if (e1 + 64 * k < a.E && place[k] < a.top_k) {
           a.expert_of[(size_t)b * a.top_k + place[k]] = ee[k];
           sel[place[k]] = p[ee[k]];
