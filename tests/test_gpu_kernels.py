@@ -1069,6 +1069,8 @@ def test_moe_route_matches_oracle(B, D, E, k):
       np.testing.assert_array_equal(got_idx[b], want_idx[b])
       np.testing.assert_allclose(got_w[b], want_w[b], atol=2 * G.ulp_bf16(want_w[b]).max())
   np.testing.assert_allclose(got_w.sum(-1), 1.0, atol=0.02)
+  assert (got_idx >= 0).all() and (got_idx < E).all()
+  assert all(len(set(r)) == k for r in got_idx)
 
 
 # one workgroup a token, and 16 tokens a workgroup; a group of four experts and a last lane of fewer
@@ -1085,8 +1087,6 @@ def test_moe_route_of_equal_scores_takes_the_lower_experts_first(B, E, k):
   scores = x @ rw
   assert np.abs(scores).max() < 16 and (np.diff(np.sort(scores, axis=-1), axis=-1) == 0).any(-1).mean() > 0.5
   np.testing.assert_array_equal(idx.cpu().numpy(), np.argsort(-scores, axis=-1, kind='stable')[:, :k])
-  assert (got_idx >= 0).all() and (got_idx < E).all()
-  assert all(len(set(r)) == k for r in got_idx)
 
 
 @pytest.mark.parametrize('B,D,F,E,k,group', [
