@@ -46,6 +46,14 @@ struct Workspace {
 // split-free k-way projection plus a SwiGLU launch is faster (8B shape, 128 rows: 1.76 against 2.18 ms per step)
 static const int kFusedGateUpMaxRows = 64;
 
+// The fused gate | up launch computes x . A once and hands it to its workgroups where that is no slower than every workgroup's own:
+// its wait has to be over before their epilogue, and what it takes out of the loop is worth it at two row tiles.  us per launch, own
+// / handed over: K = 4096, 14336 hidden units, in the step: 23 rows 20.3 / 21.0, 64 rows 29.2 / 29.4; back to back 32 rows 20.7 /
+// 22.5, 64 rows 28.9 / 29.3; K = 2048 32 rows 12.9 / 15.9, 64 rows 18.6 / 20.3.
+static bool gate_up_hands_over(const tmx_model_desc* m, int B) {
+  return m->num_experts == 0 && B > 32 && B <= kFusedGateUpMaxRows && m->embed_dim >= 4096 && m->embed_dim % 256 == 0;
+}
+
 struct Splits { int qkv, o, gate_up, down; };
 
 // One to four sequences, one token each, dense layers of either family whose shapes fit the small-batch
@@ -118,7 +126,7 @@ static Workspace carve(const tmx_model_desc* m, int B, int C, char* base) {
     w.delta = (uint16_t*)take(B <= 128 ? (size_t)B * D * 2 : 0);
     w.dsync = take(B <= 128 ? qlinear_delta_sync_bytes(B, TMX_MAX_RPAD) : 0);
   }
-  w.gu_sync = take(B <= kFusedGateUpMaxRows && m->num_experts == 0 && D % 256 == 0 ? qlinear_gate_up_sync_bytes(B, (int)D) : 0);
+  w.gu_sync = take(gate_up_hands_over(m, B) ? qlinear_gate_up_sync_bytes(B, (int)D) : 0);
   const bool small = B <= kSmallBatchMaxRows && m->num_experts == 0;
   w.sb_tparts = (float*)take(small ? (F / 32 + 1) * (size_t)B * 32 * 4 : 0);
   w.sb_attn_partial = (float*)take(small ? sb_attn_partial_bytes(B, m->num_heads, m->num_kv_heads, m->head_dim, C) : 0);
@@ -284,7 +292,7 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
                         w.y_part, wl, B, l.K, l.N, l.G, l.r_pad, nsplit, fused);
   };
   // the hand-over words of the fused gate | up launch start at zero (the kernel leaves them so)
-  if (!moe && B <= kFusedGateUpMaxRows && w.gu_sync && n_steps > 0) {
+  if (w.gu_sync && n_steps > 0) {
     rc = zero_words(st, (uint32_t*)w.gu_sync, 64);
     if (rc != TMX_OK) return rc;
   }
@@ -519,14 +527,9 @@ static int decode_steps_impl(const tmx_model_desc* m, const tmx_decode_state* s,
         TMX_TRY(TMX_K_ROWNORM, row_norm(st, a, B));
       } else {
         if (fused_gu) {
-          // x . A once per launch, handed to the workgroups, where that is no slower than every workgroup's own: its wait has to be
-          // over before their epilogue, and what it takes out of the loop is worth it at two row tiles.  us per launch, own / handed
-          // over: K = 4096, 14336 hidden units, in the step: 23 rows 20.3 / 21.0, 64 rows 29.2 / 29.4; back to back 32 rows 20.7 /
-          // 22.5, 64 rows 28.9 / 29.3; K = 2048 32 rows 12.9 / 15.9, 64 rows 18.6 / 20.3.
-          void* gu_sync = B > 32 && D >= 4096 ? w.gu_sync : nullptr;
           TMX_TRY(TMX_K_GATE_UP, qlinear_gate_up_swiglu(
               st, w.xn, D, l.gate_up.qweight, l.gate_up.scales, l.gate_up.lora_a_t, l.gate_up.lora_b,
-              l.gate_up.rank, l.gate_up.lora_scale, w.act, B, D, F, l.gate_up.G, gu_sync, w.status));
+              l.gate_up.rank, l.gate_up.lora_scale, w.act, B, D, F, l.gate_up.G, w.gu_sync, w.status));
         } else {
         const bool gu16 = sp.gate_up == 1;
         {
