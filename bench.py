@@ -15,6 +15,7 @@ Prints one JSON line.
 import argparse
 import ctypes
 import json
+import math
 import os
 import sys
 import time
@@ -389,18 +390,24 @@ def main():
     dense = [('qkv_linear', 'qkv'), ('o_linear', 'o')]
     symbols = {}
     if cfg.num_experts:
-      symbols['tmx::moe_stream_kernel<false>'] = ['gate_up_linear']
-      symbols['tmx::moe_stream_kernel<true>'] = ['down_linear']
+      # the second argument: rows of an expert in LDS, where at even routing they seldom exceed what three workgroups (gate | up) or
+      # two to four (down) leave room for
+      mean = batch * cfg.num_experts_per_tok / cfg.num_experts
+      need = math.ceil(mean + 3.5 * math.sqrt(mean))
+      fit = lambda k, wgs: ((160 * 1024 - 4 * 2304) // wgs - 512) // ((k + 8) * 2)
+      lds = lambda k, wgs: str(any(fit(k, w) >= min(need, 32) for w in wgs)).lower()
+      symbols[f'tmx::moe_stream_kernel<false, {lds(cfg.embed_dim, (3,))}>'] = ['gate_up_linear']
+      symbols[f'tmx::moe_stream_kernel<true, {lds(cfg.hidden_dim, (4, 3, 2))}>'] = ['down_linear']
     else:
       gu = layer0['gate_up']
       fused = (tot_cnt[CLASS_NAMES.index('swiglu')] == 0 and gu.k % 256 == 0 and gu.k < 8192)
       if fused:
         lora = gu.lora_a_t is not None
         if batch <= 64 and gu.k % 512 == 0:   # 8 waves per workgroup, activation slab by direct-to-LDS loads
-          # LoRA mode: 0 none, 1 every workgroup multiplies x by A itself, 2 a few workgroups do it once and
-          # hand t over (K / 256 <= 32 producers that fit beside the F / 64 main workgroups within 256)
+          # LoRA mode: 0 none, 1 every workgroup multiplies x by A itself, 2 (33 rows and 4096 columns on) a few workgroups do it
+          # once and hand t over (K / 256 <= 32 producers that fit beside the F / 64 main workgroups within 256)
           cus = torch.cuda.get_device_properties(0).multi_processor_count
-          mode = 0 if not lora else (2 if gu.k // 256 <= 32 and cfg.hidden_dim // 64 + gu.k // 256 <= cus else 1)
+          mode = 0 if not lora else (2 if batch > 32 and gu.k >= 4096 and gu.k // 256 <= 32 and cfg.hidden_dim // 64 + gu.k // 256 <= cus else 1)
           sym = f'tmx::qlinear_gate_up8_kernel<{mt}, {mode}>'
         else:
           sym = f'tmx::qlinear_gate_up_kernel<{mt}>' if lora else f'tmx::qlinear_mfma4_kernel<{mt}>'
@@ -423,9 +430,17 @@ def main():
     small = batch <= 4 and not cfg.num_experts and tot_cnt[CLASS_NAMES.index('rope_kvwrite')] == 0
     if small:
       # 1..4 rows: five launches per layer, norm / LoRA / residual / SwiGLU inside the projections
-      # (template arguments: prologue 0 plain, 1 norm, 2 attention merge; epilogue 0 plain, 1 residual, 2 SwiGLU)
-      symbols = {'tmx::sb_linear16_kernel<1, 0>': ['qkv_linear'], 'tmx::sb_linear16_kernel<2, 1>': ['o_linear'],
-                 'tmx::sb_linear_kernel<1, 2>': ['gate_up_linear'], 'tmx::sb_linear16_kernel<0, 1>': ['down_linear'],
+      # (template arguments: prologue 0 plain, 1 norm, 2 attention merge; epilogue 0 plain, 1 residual, 2 SwiGLU; k-tiles or pairs of
+      # them that a wave requests at once; tiles of A that hold a workgroup's segment, none where x . A is handed over)
+      ahead = lambda tiles: next(n for n in (1, 2, 4, 8) if tiles <= n or n == 8)
+      def sb16(pl, pro, epi, own_a=True):
+        spans = [((i + 1) * pl.rank - 1) // 16 - i * pl.rank // 16 + 1 for i in range(len(pl.seg_cols))]
+        a_tiles = min(max(spans), pl.r_pad // 16) if own_a and pl.lora_a_t is not None else 0
+        return f'tmx::sb_linear16_kernel<{pro}, {epi}, {ahead(-(-pl.k // 1024))}, {a_tiles}>'
+      gu = layer0['gate_up']
+      symbols = {sb16(layer0['qkv'], 1, 0): ['qkv_linear'], sb16(layer0['o'], 2, 1): ['o_linear'],
+                 f'tmx::sb_linear_kernel<1, 2, {ahead(-(-gu.k // 256))}, {gu.r_pad // 32 if gu.lora_a_t is not None else 0}>': ['gate_up_linear'],
+                 sb16(layer0['down'], 0, 1, False): ['down_linear'],
                  f'tmx::sb_attn_kernel<{cfg.head_dim}, {cfg.num_heads // cfg.num_kv_heads}>': ['attention']}
     # the walk of the run without shared slots: on the matrix pipe for 4 or 8 query heads per kv head while three
     # workgroups per CU hold every (sequence, kv head) pair at once (+ gqa_combine_kernel where a row is split),
