@@ -661,6 +661,33 @@ def test_gqa_attention_rows(nseq, T, N, Kh, H, C, step):
     assert np.abs(got[:, t] - ref).max() < 2e-2, (t, np.abs(got[:, t] - ref).max())
 
 
+@pytest.mark.parametrize('T,N,Kh,H', [(40, 8, 2, 128), (70, 4, 2, 64)])
+def test_rows_that_see_a_score_of_nan_are_nan(T, N, Kh, H):
+  """Softmax over a visible NaN is NaN, as in the reference: the tokens from the slot on, of its kv head and sequence.  The others,
+  tokens of the same blocks among them, do not change by a bit; behind the mask a NaN key changes nothing."""
+  K = G.Keep()
+  n_seq, C, step, slot = 2, 128, 20, 37
+  g = torch.Generator(device=G.DEV).manual_seed(T)
+  new = lambda *shape: torch.randn(*shape, generator=g, device=G.DEV).to(torch.bfloat16)
+  q, k, v = new(n_seq * T, N, H), new(n_seq, C, Kh, H), new(n_seq, C, Kh, H)
+  ws = torch.empty(max(_lib.lib().tmx_gqa_decode_workspace_bytes(n_seq * T, N, Kh, H, C), 4), dtype=torch.uint8, device=G.DEV)
+  bad = k.clone()
+  bad[1, slot, 0] = float('nan')
+
+  def attend(k, mask):
+    out = torch.empty(n_seq, T, Kh, N // Kh, H, dtype=torch.bfloat16, device=G.DEV)
+    G.call('tmx_gqa_attention_rows', S(), G.p(q), G.p(k), G.p(v), K.u8(mask), K.i32([step]), C, G.p(out), G.p(ws), n_seq, T, N, Kh, H, C)
+    return out
+
+  mask = np.ones((n_seq, C))
+  want, got = attend(k, mask), attend(bad, mask)
+  hit = torch.zeros(n_seq, T, Kh, dtype=torch.bool, device=G.DEV)
+  hit[1, slot - step:, 0] = True
+  assert torch.isnan(got[hit]).all() and torch.equal(got[~hit], want[~hit])
+  mask[1, slot] = 0
+  assert torch.equal(attend(bad, mask), attend(k, mask))
+
+
 def _head_inputs(M, D, V, seed):
   rng = np.random.default_rng(seed)
   x = bf16_round(rng.standard_normal((M, D)).astype(np.float32))

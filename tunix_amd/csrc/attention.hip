@@ -691,7 +691,8 @@ __global__ __launch_bounds__(256, 3) void gqa_fill_kernel(AttnArgs a) {
   const int vbase = (4 * h + k4) * H * 2 + (((2 * g2 + (q4 >> 1)) ^ v_swizzle(k4)) << 4) + 8 * (q4 & 1);
   // Scores stay unscaled, probabilities are powers of two of scale2 (score - m), one fma and one v_exp_f32 each.  m follows
   // the largest score only when that is 2^8 ahead: any m gives the same quotient, and the accumulators are rescaled at the first
-  // block and seldom after.  Masks are looked at where a block has one or passes a token's own slot.
+  // block and seldom after.  Masks are looked at where a block has one or passes a token's own slot.  A visible score of NaN makes
+  // its row NaN, as the softmax of the reference does (with a comparison per score it had counted as masked).
   // What bounds it is the instructions beside the 24 MFMAs of a block: 537 with a mask, two multiplies and a subtraction for
   // every score, rescaling at most blocks and accumulators moved in and out of AGPRs; about 150 so, and 165 registers, three
   // workgroups a CU instead of two.  8 kv heads of 4 query heads, 3 x 680 tokens behind 1360: 185 -> 106 us, 16 x 192 behind 512:
