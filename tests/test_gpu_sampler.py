@@ -296,6 +296,27 @@ def test_many_samples_of_a_prompt_share_its_cache_rows(n, h, kh):
   assert torch.isfinite(runs[True]).all() and (runs[True] - runs[False]).abs().max() <= 1e-2
 
 
+# what a row's own slots are at most beside 64 shared ones, and whether the groups' workgroups walk them
+@pytest.mark.parametrize('new,groups', [(38, True), (506, False)])
+def test_many_samples_with_long_completions_walk_by_themselves(new, groups):
+  """160 rows of the 8B shape's heads in groups of 8, a short prompt: its slots, read once per group, are worth less than what the group
+  walk takes longer for many slots of the rows' own.  Which walk it was shows where all but a group's first row have other values in
+  their shared slots: at the first step the rows of a group are the same otherwise."""
+  cfg = OM.Config('llama3', 1, 512, 256, 512, 32, 128, 8, norm_eps=1e-5)
+  model = C.product_model(cfg, C.make_state(cfg, 35, 8, norm_jitter=0.05), 64, 16.0)
+  ids = np.repeat(np.random.default_rng(14).integers(3, 512, (20, 70)), 8, axis=0).astype(np.int32)
+  s = _sampler(model, cfg, 64 + new)
+  s.eos_ids = np.array([-1])
+  st = s.init_sample_state(ids, 64 + new, True, None, 0.0, None, None, 0)
+  assert (st['share_group'], st['share_len']) == (8, 64)
+  s.walk(st, 69)
+  st['cache'].view(1, 2, 20, 8, 64 + new, 8, 128)[:, :, :, 1:, :64] = 8
+  s.run_steps(st, 1, sample=True)
+  s.check_device_status(st)
+  off = (st['logits'].view(20, 8, 512) - st['logits'].view(20, 8, 512)[:, :1]).abs().amax(2)[:, 1:]
+  assert off.max() <= 1e-2 if groups else off.min() > 0.1
+
+
 def test_a_sample_that_overflows_leaves_the_others_of_its_prompt_alone():
   """More rows than there is room for parts, heads of the 8B shape: a sample reads a token whose embedding row overflows.  Its own
   logits are lost, those of every other sample are, bit for bit, those of a batch in which it read another token."""

@@ -574,8 +574,8 @@ __global__ __launch_bounds__(256, 3) void gqa_tile_kernel(AttnArgs a, int n_grou
 // rows' columns are masked (7 of 8 columns of the MFMA tile idle there, which costs nothing: it waits for memory).  Every
 // cache row is read once and no part leaves the workgroup.  256 rows of the 8B shape in groups of 8 at 128 + 12
 // slots 36.0 us by themselves, 14.8 here; 8 layers, 24 steps of that 68.6 -> 61.8 ms.  That a sequence whose values are not
-// finite leaves the others' sums alone (the select behind every tile of V^T . P^T) is 1.1 of 14.2 us in the step.  grid (Kh, group
-// query blocks).
+// finite leaves the others' sums alone (the select behind every tile of V^T . P^T) is 1.1 of 14.2 us in the step, and where most
+// slots are a row's own 7.8 of 77.5 (256 rows in groups of 32, 256 + 256 slots; by themselves 97).  grid (Kh, group query blocks).
 template <int H, int G>
 __global__ __launch_bounds__(256, 3) void gqa_group_kernel(AttnArgs a) {
   __shared__ PrefixLds<H> lds;
@@ -913,26 +913,42 @@ static AttnPlan plan_rows_walk(int B, int N, int Kh, int H, int C, bool shared, 
 // Groups alone in several splits, merged by the combine kernel, came within 1 % of the better of the two in each of these.
 // By themselves on cold caches, 2 to 32 kv heads of 1 to 8 heads, head dimensions 64 and 128, 32 to 128 rows, the choice is within
 // 10 % of the best in 52 of 56 shapes and 20 % off at most (4 kv heads of 8, 64 x 4, 96 + 32: 8.9 against 7.4 by themselves).
+// More than 128 rows have prices of their own, of these two walks at many rows and through whole rollouts: rows by themselves run
+// in several rounds, whose starts and ends are hidden (12 + 0.88 of the bytes; with 8 heads on the vector walk, whose arithmetic
+// it waits for, 1.42), and a CU takes a wave's K pieces one after the other, 3.4 per 128 slots of 128 values for every group of the
+// fullest CU.  The launch through the rollout, us, by themselves / groups alone (with the prices above the second was taken
+// everywhere but at 1B 160 x 8, 64 + 512):
+//   160 x 8, 64 + 512  48.9 / 60.7    160 x 8, 256 + 512  72.3 / 65.8    136 x 8, 64 + 256  31.0 / 34.7    136 x 8, 64 + 64   21.6 / 15.7
+//   256 x 8, 64 + 512  67.1 / 70.9    256 x 8, 256 + 512  98.3 / 77.8    256 x 8, 64 + 256  45.8 / 40.8    160 x 4, 64 + 512  49.0 / 53.7
+//   384 x 8, 64 + 512  96.6 / 110.4   256 x 4, 128 + 512  76.8 / 71.7    256 x 2, 64 + 128  35.7 / 29.6    160 x 2, 64 + 512  49.0 / 48.2
+//   1B 256 x 8, 64 + 512  41.6 / 36.6   1B 160 x 8, 64 + 128  19.1 / 12.9   30B-A3B 160 x 8, 64 + 512  28.2 / 35.2   256 x 8, 128 + 512  66.8 / 39.1
 static AttnPlan plan_attention(int B, int N, int Kh, int H, int C, int share_gs, int share_len, int len, bool must_share) {
   const AttnPlan rows = plan_rows_walk(B, N, Kh, H, C, false, 0, 0);
   if (!attn_share_ok(B, N, Kh, H, C, share_gs, share_len)) return rows;
   const int G = N / Kh, own = len > share_len ? (len - share_len + 1) / 2 : 1;
   const float us_per_slot = (float)H * 4.f / 5.2e6f;  // a K and a V row
+  const float row_bytes = us_per_slot * B * Kh * (share_len + own);
   AttnPlan best = rows;
-  float best_cost = 6.f + us_per_slot * B * Kh * (share_len + own) + (rows.nsplit > 1 ? 3.f : 0.f);
+  float best_cost = 6.f + row_bytes + (rows.nsplit > 1 ? 3.f : 0.f);
+  if (B > 128 && !rows.tile) best_cost = 12.f + (G == 8 ? 1.42f : 0.88f) * row_bytes;
   if (must_share) best_cost = 1e30f;
   auto offer = [&](const AttnPlan& p, float cost) {
     if (cost < best_cost) { best = p; best_cost = cost; }
   };
+  const AttnPlan groups = {false, true, 0, 1};
   const long wgs = group_workgroups(B, G, Kh, share_gs);
+  const int rpb = 32 / G, nrows = share_gs < rpb ? share_gs : rpb;
   if (B <= 128) {
     const AttnPlan p = plan_rows_walk(B, N, Kh, H, C, true, share_gs, share_len);
     if (p.shared) offer(p, 9.2f + us_per_slot * ((float)B * Kh * own + (float)wgs * share_len));
+    const int blocks = (share_len + 31) / 32 + nrows * ((own + 31) / 32);
+    const float rounds = (H == 64 ? 1.6f : 2.2f) * ((blocks + 3) / 4), bytes = 1.1f * us_per_slot * 32.f * blocks * wgs;
+    offer(groups, 4.4f + (rounds > bytes ? rounds : bytes));
+  } else {
+    const float slots = share_len + (float)nrows * own, per_cu = (wgs + device_cus() - 1) / device_cus();
+    const float pieces = 3.4f / 128.f * (H / 128.f) * slots * per_cu, bytes = 1.2f * us_per_slot * slots * wgs;
+    offer(groups, 6.4f + (pieces > bytes ? pieces : bytes));
   }
-  const int rpb = 32 / G, nrows = share_gs < rpb ? share_gs : rpb;
-  const int blocks = (share_len + 31) / 32 + nrows * ((own + 31) / 32);
-  const float rounds = (H == 64 ? 1.6f : 2.2f) * ((blocks + 3) / 4), bytes = 1.1f * us_per_slot * 32.f * blocks * wgs;
-  offer(AttnPlan{false, true, 0, 1}, 4.4f + (rounds > bytes ? rounds : bytes));
   return best;
 }
 
