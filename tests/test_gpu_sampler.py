@@ -1060,6 +1060,31 @@ def test_scoring_of_padded_completions_equals_a_walk_of_every_row(one, b, p, t, 
   assert np.abs(got[0] - got[1])[some].max() <= LOGPROB_TOL
 
 
+@pytest.mark.parametrize('one', [256, -1])
+@pytest.mark.parametrize('b,p,t,limit', [(7, 37, 20, 4096), (7, 5, 1, 4096), (7, 1, 40, 4096), (40, 9, 33, 4096), (9, 30, 45, 100), (7, 20, 25, 3)])
+def test_scoring_that_leaves_out_whatever_it_can_equals_a_walk_of_every_row(one, b, p, t, limit, monkeypatch):
+  """The same where a model this small would not leave out rows: the saving is less than the plan of the rows costs."""
+  monkeypatch.setattr(Sampler, 'LEAVE_OUT_US', -1.0)
+  test_scoring_of_padded_completions_equals_a_walk_of_every_row(one, b, p, t, limit)
+
+
+@pytest.mark.parametrize('t,padded,left_out', [(16, False, False), (16, True, False), (500, False, False), (500, True, True)])
+def test_scoring_leaves_out_rows_where_that_saves_time(t, padded, left_out):
+  """Few rows are walked whole, padding and prompt columns too: to plan without them costs more than they do."""
+  cfg = OM.Config('llama3', 2, 1024, 1024, 4096, 16, 64, 4, norm_eps=1e-5)
+  model = C.product_model(cfg, C.make_state(cfg, 47, 8, norm_jitter=0.05), 64, 16.0)
+  s = _sampler(model, cfg, 600)
+  rng = np.random.default_rng(3)
+  prompt, comp = rng.integers(3, 1024, (6, 8)).astype(np.int32), rng.integers(3, 1024, (6, t)).astype(np.int32)
+  if padded:
+    comp[:, 2:] = 0
+  whole = []
+  steps = s.run_steps
+  s.run_steps = lambda *a, **k: (whole.append(k), steps(*a, **k))
+  assert np.isfinite(s.per_token_logps(prompt, comp, pad_id=0)).all()
+  assert whole == ([] if left_out else [{'sample': True, 'tokens_per_pass': t + 7}])
+
+
 def test_scoring_does_not_read_the_embedding_of_padding_in_front_of_prompts():
   """Padding in front of a prompt is not walked, or walked as another token: whatever its embedding holds, the log-probs are the
   same.  In one walk of prompt and completion and in two."""

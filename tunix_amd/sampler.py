@@ -437,16 +437,30 @@ class Sampler:
                                    st['first_col'].data_ptr(), width, rows)
     _lib.check(rc, 'tmx_fill_ragged')
 
+  # What a scoring pass has to save by the rows it leaves out, us: the plan of the rows, its copy to the device and the head's rows
+  # gathered take 45 to 50.  Whole / left out: toy, 4 x (16 + 16) without padding 452 / 504, 1B shape of 16 layers, 1 x (36 + 27)
+  # without 1465 / 1515, half of it padding 1462 / 1417, 8 x (24 + 24) with an eighth of padding 2711 / 2625, 8B shape of 8 layers, 2 x
+  # (48 + 64) without 2111 / 2050.
+  LEAVE_OUT_US = 40
+
+  def _left_out_us(self, rows, head_rows):
+    """About what `rows` rows fewer in the layers and `head_rows` fewer in the head save, us."""
+    c = self._transformer.config
+    layer = c.embed_dim * (2 * (c.num_heads + c.num_kv_heads) * c.head_dim + 3 * c.hidden_dim * (c.num_experts_per_tok if c.num_experts else 1))
+    return 1.2e-9 * c.num_layers * layer * rows + 1e-9 * c.vocab_size * c.embed_dim * head_rows
+
   def _run_score(self, st, col, width, rows):
     """One pass of a scoring walk: `rows` rows over the columns col .. col + width - 1."""
-    first, end = (np.clip(st[k], col, col + width) for k in ('score_first', 'score_end'))
-    n_head = int(np.maximum(end - np.maximum(first, st['score_col']), 0).sum())
+    n_head = int(np.maximum(np.minimum(st['score_end'], col + width) - np.maximum(st['score_first'], max(col, st['score_col'])), 0).sum())
     if rows == 0:
       st['step'].add_(width)
       return
-    if rows == n_head == width * st['token_buffer'].shape[0] and width >= self.MIN_BLOCK_TOKENS:
-      self.run_steps(st, 1, sample=True, tokens_per_pass=width)  # nothing to leave out
+    whole = width * st['token_buffer'].shape[0]
+    if (width >= self.MIN_BLOCK_TOKENS and whole <= self._fill_rows()
+        and self._left_out_us(whole - rows, whole - n_head) < self.LEAVE_OUT_US):
+      self.run_steps(st, 1, sample=True, tokens_per_pass=width)
       return
+    st['score_cut'] = True
     if st['score_span'] is None:
       st['score_span'] = torch.from_numpy(np.stack([st['score_first'], st['score_end']])).to(self._transformer.device)
     cs = self._c_state(st, 1, rows)
@@ -550,13 +564,15 @@ class Sampler:
     # the equal masked tokens it ends with.  The rows of the others have the same token, position and visible slots: the log-probs
     # behind it repeat its own.  A row with no token at all has no visible slot, and is walked whole.  Completions of half to all
     # of their columns, prompts likewise: 16 x (256 + 512) on 8 layers of the 8B shape 46.0 -> 39.5 ms, 5 x (37 + 90) on the 1B
-    # shape 3.57 -> 3.12 ms; where nothing is padded the passes are those over all columns.
-    same = (ids == ids[:, -1:]) & ~valid
-    tail = total - np.logical_and.accumulate(same[:, ::-1], axis=1).sum(axis=1)
-    tail = np.where(valid.any(axis=1), np.maximum(tail, p - 1), total)
-    st['score_col'], st['score_span'] = p - 1, None
+    # shape 3.57 -> 3.12 ms; where that is worth less than its plan the passes are those over all columns (LEAVE_OUT_US).
+    st['score_col'], st['score_span'], st['score_cut'] = p - 1, None, False
     st['score_first'] = np.minimum(first, p - 1).astype(np.int32)
-    st['score_end'] = np.minimum(tail + 1, total - 1).astype(np.int32)
+    st['score_end'] = np.full(b, total - 1, np.int32)
+    if not valid[:, -1].all():
+      same = (ids == ids[:, -1:]) & ~valid
+      tail = total - np.logical_and.accumulate(same[:, ::-1], axis=1).sum(axis=1)
+      tail = np.where(valid.any(axis=1), np.maximum(tail, p - 1), total)
+      st['score_end'] = np.minimum(tail + 1, total - 1).astype(np.int32)
     if st['share_group'] == 1 and self._one_walk(b, p, t):
       # prompt columns are scored too where the walk leaves nothing out, and their scores left out
       self.walk(st, total - 1, sample=True)
@@ -565,7 +581,7 @@ class Sampler:
       self.walk(st, t, sample=True)
     self.check_device_status(st)
     logps = st['logprobs'][:, p:p + t].cpu().numpy()
-    if self._fill_ragged_ok():
+    if st['score_cut']:
       return np.take_along_axis(logps, np.minimum(np.arange(t), (st['score_end'] - p)[:, None]), axis=1)
     return logps
 
