@@ -916,8 +916,8 @@ static AttnPlan plan_rows_walk(int B, int N, int Kh, int H, int C, bool shared, 
 // More than 128 rows have prices of their own, of these two walks at many rows and through whole rollouts: rows by themselves run
 // in several rounds, whose starts and ends are hidden (12 + 0.88 of the bytes; with 8 heads on the vector walk, whose arithmetic
 // it waits for, 1.42), and a CU takes a wave's K pieces one after the other, 3.4 per 128 slots of 128 values for every group of the
-// fullest CU.  The launch through the rollout, us, by themselves / groups alone (with the prices above the second was taken
-// everywhere but at 1B 160 x 8, 64 + 512):
+// fullest CU.  The launch through the rollout, us, by themselves / groups alone (the prices above took the second in all of
+// them):
 //   160 x 8, 64 + 512  48.9 / 60.7    160 x 8, 256 + 512  72.3 / 65.8    136 x 8, 64 + 256  31.0 / 34.7    136 x 8, 64 + 64   21.6 / 15.7
 //   256 x 8, 64 + 512  67.1 / 70.9    256 x 8, 256 + 512  98.3 / 77.8    256 x 8, 64 + 256  45.8 / 40.8    160 x 4, 64 + 512  49.0 / 53.7
 //   384 x 8, 64 + 512  96.6 / 110.4   256 x 4, 128 + 512  76.8 / 71.7    256 x 2, 64 + 128  35.7 / 29.6    160 x 2, 64 + 512  49.0 / 48.2
